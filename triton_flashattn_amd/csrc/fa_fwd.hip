@@ -29,6 +29,11 @@ namespace fa {
 // The K/V stream of a row-broadcast bias (kinds 6, 7) is tiled like that of ALiBi, in steps of 32
 // keys: the bias values of a block need the registers that 64-key steps spend on a second block of
 // scores.
+// Sum of a lane's exponentials of a block (or half of one) beyond which their reference point is raised: far from what overflows the
+// element type of P and the fp32 accumulators, and high, so that scores that grow along the keys (a distance
+// penalty on the way to the diagonal) raise it seldom.
+template <typename T> constexpr float kRaise = __is_same(T, _Float16) ? 0x1p14f : 0x1p32f;
+
 constexpr int fwd_stream_kind(int bias) { return bias >= 5 ? 6 : bias; }
 
 template <typename T, int D, int BIAS, bool CAUSAL>
@@ -109,6 +114,17 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
     KeyStream<T, D, fwd_stream_kind(BIAS)> ks_;
     ks_.init(smem, kp, vp, bp, p.sk.s, p.sv.s, p.sbias.m, p.sbias.n, M, N, mw, wave, lane);
 
+    // raises the reference point of this row's exponentials to mx (log2 units) where it is lower
+    auto raise = [&](float mx) {
+        const float alpha = mx > m_i ? fast_exp2(m_i - mx) : 1.f;
+        m_i = mx > m_i ? mx : m_i;
+        l_i *= alpha;
+#pragma unroll
+        for (int db = 0; db < C::DB; db++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) o_acc[db][i] *= alpha;
+    };
+
     // One step of the K/V stream.  Interior steps (every key in range and visible to every row of
     // the work-group) run with STEP_MASKED = false: no range checks, no mask arithmetic.  BV: the
     // bias slices come by copy (rows that allow aligned 16-byte chunks), else element by element.
@@ -126,23 +142,100 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
         const unsigned k_rows = ks_.k_addr(k) + rows_l, v_cols = ks_.v_addr(k) + cols_l;  // operand reads by address
         const unsigned char* b_lds = ks_.b_lds(k);
         static_assert(TB == 0 || C::NH == 1, "a bias slot covers one 32-key block");
-        // The step is consumed 32 keys at a time, each block with its own softmax step.  In interior
-        // steps of more than one block all score products are issued up front: the MFMAs of the later
-        // blocks then run while the vector pipeline works on the first.
-        constexpr bool PRE = !STEP_MASKED && C::NH > 1;
-        f32x16 s_pre[C::NH];
-        if constexpr (PRE) {
+        // Interior steps of two blocks (no bias): the matrix instructions of one block are issued between
+        // the exponentials of the other, S of block 1 under the exponentials of block 0 and the PV product
+        // of block 0 under those of block 1, one fenced slot per two score elements.  Their LDS operands are
+        // fetched a phase ahead; head dim 256 has no registers for that and fetches them one slot ahead.  (Bound by
+        // the matrix and the vector pipeline together: per block 512 clocks of the one and about 440 of the other
+        // at D = 128.  With the maximum gone and this order, B=2 H=16 M=N=4096 bf16 without a bias takes 0.257 ms
+        // where it took 0.274 at D = 128, 0.570 / 0.609 ms at B=4 H=32 D = 64, 0.330 / 0.355 at H=8 D = 256.)
+        if constexpr (!STEP_MASKED && C::NH == 2) {
+            constexpr int NS = C::KSTEPS, NP = 2 * C::DB;  // matrix instructions of S and of PV per block
+            constexpr bool AHEAD = D <= 128;
+            constexpr int NSS = AHEAD ? NS : NS / 8, NPS = AHEAD ? NP : NP / 8;  // operands fetched at a time
+            T8 ka[2][NSS], va[2][NPS];
+            f32x16 sc[2];
+            auto load_k = [&](int nb, int slot) {  // operands slot * NSS .. of S of block nb
 #pragma unroll
-            for (int nb = 0; nb < C::NH; nb++) {
+                for (int i = 0; i < NSS; i++)
+                    ka[AHEAD ? nb : slot & 1][i] = SW::template row8_at<T8>(k_rows, nb * 32, slot * NSS + i);
+            };
+            auto load_v = [&](int nb, int slot) {
 #pragma unroll
-                for (int i = 0; i < 16; i++) s_pre[nb][i] = 0.f;
-#pragma unroll
-                for (int ks = 0; ks < C::KSTEPS; ks++) {
-                    T8 a = SW::template row8_at<T8>(k_rows, nb * 32, ks);
-                    s_pre[nb] = mfma32(a, qreg[ks], s_pre[nb]);
+                for (int i = 0; i < NPS; i++) {
+                    const int at = slot * NPS + i;
+                    va[AHEAD ? 0 : slot & 1][i] = SW::template col8_at<T8>(v_cols, nb * 32 + (at / C::DB) * 16, at % C::DB);
                 }
-            }
+            };
+            // the matrix instructions of slot j of 8 of S and of PV
+            auto mma_s = [&](int nb, int j) {
+                if (!AHEAD && j < 7) load_k(nb, j + 1);
+#pragma unroll
+                for (int ks = j * NS / 8; ks < (j + 1) * NS / 8; ks++)
+                    sc[nb] = mfma32(ka[AHEAD ? nb : j & 1][AHEAD ? ks : ks - j * NSS], qreg[ks], sc[nb]);
+            };
+            auto mma_pv = [&](int nb, const T8 (&pv)[2], int j) {
+                if (!AHEAD && j < 7) load_v(nb, j + 1);
+#pragma unroll
+                for (int i = j * NP / 8; i < (j + 1) * NP / 8; i++)
+                    o_acc[i % C::DB] = mfma32(va[AHEAD ? 0 : j & 1][AHEAD ? i : i - j * NPS], pv[i / C::DB], o_acc[i % C::DB]);
+            };
+            // the exponentials of a block against the current m_i; after(j) is called behind pair j of 8
+            auto exps = [&](const f32x16& x, T8 (&out)[2], auto&& after) {
+                float rs = 0.f;
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+#pragma unroll
+                    for (int e = 0; e < 2; e++) {
+                        const int i = 2 * j + e;
+                        const float pv = fast_exp2(__builtin_fmaf(x[i], qk_scale, -m_i));
+                        rs += pv;
+                        out[i >> 3][i & 7] = (T)pv;
+                    }
+                    after(j);
+                }
+                return rs;
+            };
+            auto settle = [&](const f32x16& x, T8 (&out)[2], float rs) {
+                if (__builtin_amdgcn_ballot_w64(!(rs <= kRaise<T>)) != 0) {
+                    float mx = -INFINITY;
+#pragma unroll
+                    for (int i = 0; i < 16; i++) mx = fmaxf(mx, x[i]);
+                    raise(pair_max(mx) * qk_scale);
+                    rs = exps(x, out, [](int) {});
+                }
+                l_i += rs;
+            };
+            load_k(0, 0);
+            if (AHEAD) load_k(1, 0);
+#pragma unroll
+            for (int nb = 0; nb < 2; nb++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) sc[nb][i] = 0.f;
+#pragma unroll
+            for (int j = 0; j < 8; j++) mma_s(0, j);
             issue_ahead();  // in the shadow of the MFMAs just issued
+            if (!AHEAD) load_k(1, 0);
+            if (AHEAD) load_v(0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            T8 p0[2], p1[2];
+            float rs = exps(sc[0], p0, [&](int j) {
+                __builtin_amdgcn_sched_barrier(0);
+                mma_s(1, j);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            if (!AHEAD) load_v(0, 0);
+            settle(sc[0], p0, rs);
+            rs = exps(sc[1], p1, [&](int j) {
+                __builtin_amdgcn_sched_barrier(0);
+                mma_pv(0, p0, j);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            load_v(1, 0);
+            settle(sc[1], p1, rs);
+#pragma unroll
+            for (int j = 0; j < 8; j++) mma_pv(1, p1, j);
+            return;
         }
 #pragma unroll
         for (int nb = 0; nb < C::NH; nb++) {
@@ -157,30 +250,30 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
 
         // ---- S^T = K Q^T : s[i] is key n0 + nh + 8 (i/4) + 4 g + i%4, query my_m ----
         f32x16 s;
-        if constexpr (PRE) {
-            s = s_pre[nb];
-        } else {
 #pragma unroll
-            for (int i = 0; i < 16; i++) s[i] = 0.f;
+        for (int i = 0; i < 16; i++) s[i] = 0.f;
 #pragma unroll
-            for (int ks = 0; ks < C::KSTEPS; ks++) {
-                T8 a = SW::template row8_at<T8>(k_rows, nh, ks);
-                s = mfma32(a, qreg[ks], s);
-            }
-            if (nb == 0) issue_ahead();  // in the shadow of the MFMAs just issued
+        for (int ks = 0; ks < C::KSTEPS; ks++) {
+            T8 a = SW::template row8_at<T8>(k_rows, nh, ks);
+            s = mfma32(a, qreg[ks], s);
         }
+        if (nb == 0) issue_ahead();  // in the shadow of the MFMAs just issued
 
         // ---- online softmax step.  `masked` steps (ragged edge, causal diagonal) and a
         // non-positive scale follow the reference's arithmetic term by term: scaled score,
         // plus additive -1e6 terms in log2 units, plus bias (flash_attention.py:39-53).  Interior
         // steps skip the mask terms and fold the scale into the exponent.
-        // The running maximum m_i is only raised when a step exceeds it by more than 2^8: the
-        // reference point of the exponentials is arbitrary (out = acc / l and LSE = m + log2 l
-        // do not depend on it), so a stale one costs nothing but saves rescaling O every step.
-        T8 pb[2];
+        // The reference point m_i of the exponentials is arbitrary (out = acc / l and LSE = m + log2 l do
+        // not depend on it), so no running maximum is kept: the exponentials are taken against the m_i at
+        // hand, and only when the sum of a lane's 8 or 16 of them exceeds kRaise (or is no number, as at
+        // the first keys, where m_i is -inf) is m_i raised to the maximum, O rescaled and they are taken
+        // again.  The test is one comparison on a sum that is needed anyway.
         auto softmax_step = [&](auto masked_tag) {
             constexpr bool MASKED = decltype(masked_tag)::value;
-            float mx = -INFINITY;
+            // units of s[i] below: raw dot product (no bias), natural (float bias), log2 (MASKED, bool masks)
+            constexpr bool RAW = !MASKED && BIAS == 0;
+            constexpr bool NAT = !MASKED && BIAS >= 2 && !BOOLROW;
+            const float to_log2 = RAW ? qk_scale : (NAT ? kLog2e : 1.f);
             const float mf = (float)my_m, nf0 = (float)(key0 + n0 + nh + 4 * g);  // ALiBi: row and first key as floats
 #pragma unroll
             for (int q4 = 0; q4 < 4; q4++) {
@@ -208,71 +301,72 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
 #pragma unroll
                     for (int e = 0; e < 4; e++) bv[e] = w[e];
                 }
+                if constexpr (!RAW) {
 #pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const int i = q4 * 4 + e;
-                    float x;
-                    if constexpr (MASKED) {
-                        x = __fmul_rn(s[i], qk_scale);
-                        const int n = n0 + nh + nl + e;
-                        float t = (n >= N) ? kMask : 0.f;
-                        if (CAUSAL) t += (my_m < n) ? kMask : 0.f;
-                        float add = 0.f;
-                        if (BIAS == 1) add = keep[e] ? 0.f : kMask;
-                        if (BOOLROW) add = bv[e];
-                        if (BIAS >= 2 && !BOOLROW) add = __fmul_rn(bv[e], kLog2e);
-                        if (BIAS != 0) add = (n >= N) ? kMask : add;  // out-of-range bias reads as masked
-                        x = __fadd_rn(x, __fadd_rn(t, add));
-                    } else if constexpr (BIAS == 0) {
-                        x = s[i];                                    // raw score, scale folded below
-                    } else if constexpr (BIAS == 1) {
-                        x = keep[e] ? s[i] * qk_scale : s[i] * qk_scale + kMask;
-                    } else if constexpr (BOOLROW) {
-                        x = s[i] * qk_scale + bv[e];
-                    } else {
-                        x = s[i] * p.sm_scale + bv[e];               // natural units
+                    for (int e = 0; e < 4; e++) {
+                        const int i = q4 * 4 + e;
+                        float x;
+                        if constexpr (MASKED) {
+                            x = __fmul_rn(s[i], qk_scale);
+                            const int n = n0 + nh + nl + e;
+                            float t = (n >= N) ? kMask : 0.f;
+                            if (CAUSAL) t += (my_m < n) ? kMask : 0.f;
+                            float add = 0.f;
+                            if (BIAS == 1) add = keep[e] ? 0.f : kMask;
+                            if (BOOLROW) add = bv[e];
+                            if (BIAS >= 2 && !BOOLROW) add = __fmul_rn(bv[e], kLog2e);
+                            if (BIAS != 0) add = (n >= N) ? kMask : add;  // out-of-range bias reads as masked
+                            x = __fadd_rn(x, __fadd_rn(t, add));
+                        } else if constexpr (BIAS == 1) {
+                            x = keep[e] ? s[i] * qk_scale : s[i] * qk_scale + kMask;
+                        } else if constexpr (BOOLROW) {
+                            x = s[i] * qk_scale + bv[e];
+                        } else {
+                            x = s[i] * p.sm_scale + bv[e];
+                        }
+                        s[i] = x;
                     }
-                    s[i] = x;
-                    mx = fmaxf(mx, x);
                 }
-            }
-            // units of x: log2 (MASKED, bool bias), raw dot product (no bias), natural (float bias)
-            constexpr bool RAW = !MASKED && BIAS == 0;
-            constexpr bool NAT = !MASKED && BIAS >= 2 && !BOOLROW;
-            const float to_log2 = RAW ? qk_scale : (NAT ? kLog2e : 1.f);
-            mx = pair_max(mx) * to_log2;
-            const bool raise = mx > m_i + 8.f;
-            if (__builtin_amdgcn_ballot_w64(raise) != 0) {
-                const float m_new = raise ? mx : m_i;
-                const float alpha = fast_exp2(m_i - m_new);
-                m_i = m_new;
-                l_i *= alpha;
-#pragma unroll
-                for (int db = 0; db < C::DB; db++)
-#pragma unroll
-                    for (int i = 0; i < 16; i++) o_acc[db][i] *= alpha;
             }
             // ---- P and O^T += V^T P^T (A = V^T gathered down the columns of the V rows), 16 keys
             // at a time: the MFMAs of the first 16 keys run while the exponentials of the second 16
-            // are computed ----
-            float rs = 0.f;
+            // are computed (head dim 256: all 32 at once, there are no registers for a second copy of the
+            // rescaling) ----
+            constexpr int PARTS = D <= 128 ? 2 : 1, PL = 16 / PARTS;
 #pragma unroll
-            for (int kk = 0; kk < 2; kk++) {
+            for (int part = 0; part < PARTS; part++) {
+                float pv[PL], rs;
+                auto exps = [&]() {
+                    rs = 0.f;
 #pragma unroll
-                for (int i = kk * 8; i < kk * 8 + 8; i++) {
-                    float pv;
-                    if constexpr (RAW || NAT) pv = fast_exp2(__builtin_fmaf(s[i], to_log2, -m_i));
-                    else pv = fast_exp2(s[i] - m_i);
-                    rs += pv;
-                    pb[kk][i & 7] = (T)pv;
+                    for (int j = 0; j < PL; j++) {
+                        const int i = part * PL + j;
+                        if constexpr (RAW || NAT) pv[j] = fast_exp2(__builtin_fmaf(s[i], to_log2, -m_i));
+                        else pv[j] = fast_exp2(s[i] - m_i);
+                        rs += pv[j];
+                    }
+                };
+                exps();
+                if (__builtin_amdgcn_ballot_w64(!(rs <= kRaise<T>)) != 0) {
+                    float mx = -INFINITY;
+#pragma unroll
+                    for (int i = part * PL; i < 16; i++) mx = fmaxf(mx, s[i]);
+                    raise(pair_max(mx) * to_log2);
+                    exps();
                 }
+                l_i += rs;  // per-lane partial sum; the two halves of a row are added at the end
 #pragma unroll
-                for (int db = 0; db < C::DB; db++) {
-                    T8 a = SW::template col8_at<T8>(v_cols, nh + kk * 16, db);
-                    o_acc[db] = mfma32(a, pb[kk], o_acc[db]);
+                for (int kk = part * 2 / PARTS; kk < (part + 1) * 2 / PARTS; kk++) {
+                    T8 pb;
+#pragma unroll
+                    for (int j = 0; j < 8; j++) pb[j] = (T)pv[kk * 8 + j - part * PL];
+#pragma unroll
+                    for (int db = 0; db < C::DB; db++) {
+                        T8 a = SW::template col8_at<T8>(v_cols, nh + kk * 16, db);
+                        o_acc[db] = mfma32(a, pb, o_acc[db]);
+                    }
                 }
             }
-            l_i += rs;  // per-lane partial sum; the two halves of a row are added at the end
         };
         if constexpr (STEP_MASKED && D > 128) {
             // (head dim 256: one form of the softmax step in the edge loop; a second copy of the
