@@ -3,8 +3,8 @@ the fp32 oracle with the tolerances of the parity tests (out max-abs 2e-2, gradi
 import pytest
 import torch
 
-from oracle.attention_oracle import attention_forward
-from triton_flashattn_amd import flash_attention_fn
+from oracle.attention_oracle import attention_backward, attention_forward
+from triton_flashattn_amd import AlibiBias, flash_attention_fn
 
 pytestmark = pytest.mark.gpu
 
@@ -37,3 +37,57 @@ def test_forward_reference_point_of_growing_scores(gpu_device, D, dtype):
         # so a weight by 1e-3 and the output (values up to 4) by less than the tolerance
         err = (out.float() - ref).abs().max().item()
         assert err <= 2e-2, (slope, N, causal, bias_kind, err)
+
+
+def rel_l2(a, b):
+    """||a - b|| / ||b||, measured against an RMS floor of 1e-3 where the reference is zero up to rounding."""
+    return ((a.float() - b).norm() / b.norm().clamp_min(1e-3 * b.numel() ** 0.5)).item()
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("bias_kind", [None, "dense", "row", "alibi", "bool"])
+def test_backward_ragged_tiles_with_low_scores(gpu_device, D, bias_kind):
+    """Keys past N and rows past M run through the unmasked steps of the backward kernels: their probabilities,
+    2^(0 - LSE) with an LSE far below zero, overflow, and nothing of them may reach a result."""
+    g = torch.Generator().manual_seed(D)
+    for M, N, causal in [(517, 130, False), (450, 321, False), (333, 1, False), (389, 389, True), (97, 640, False)]:
+        if bias_kind == "alibi" and N == 1:
+            continue
+        mk = lambda n: torch.randn(1, n, 2, D, generator=g)
+        q, k, v, do = mk(M), mk(N), mk(N), mk(M)
+        # scores of about -144, with an ordinary spread: were a weight near one, its dS = P (dP - delta) would be the
+        # difference of two nearly equal numbers, and delta carries the rounding of the bf16 output, 2^-8 of |o| |do|
+        q[..., 0], k[..., 0], scale = 34.0, -34.0 - torch.rand(1, N, 2, generator=g) / 4, 0.125
+        q, k, v = (t.bfloat16().to(gpu_device).requires_grad_(True) for t in (q, k, v))
+        do = do.bfloat16().to(gpu_device)
+        bias, dense, grad_of = None, None, None
+        if bias_kind in ("dense", "row"):
+            shape = (1, 2, M if bias_kind == "dense" else 1, N)
+            bias = (torch.randn(shape, generator=g) - 100.0).bfloat16().to(gpu_device).requires_grad_(True)
+            dense, grad_of = bias.detach(), bias
+        elif bias_kind == "alibi":
+            slopes = torch.tensor([0.02, 0.1], device=gpu_device).requires_grad_(True)
+            bias, grad_of = AlibiBias(slopes), slopes
+            dense = bias.materialize(M, N).detach()
+        elif bias_kind == "bool":
+            bias = dense = (torch.rand(1, 2, M, N, generator=g) > 0.3).index_fill(3, torch.tensor([0]), True).to(gpu_device)
+        out = flash_attention_fn(q, k, v, bias, causal, scale)
+        wanted = [q, k, v] + ([] if grad_of is None else [grad_of])
+        grads = torch.autograd.grad(out, wanted, do)
+        full = None if dense is None else dense.expand(1, 2, M, N)
+        o, lse = attention_forward(q.detach(), k.detach(), v.detach(), full, causal, scale)
+        dq, dk, dv, db, _ = attention_backward(do, q.detach(), k.detach(), v.detach(), o, lse, full, causal, scale)
+        assert (out.float() - o).abs().max().item() <= 2 ** -7 * v.abs().max().item(), (M, N)  # P and out in bf16
+        for name, a, b in zip("qkv", grads, (dq, dk, dv)):
+            assert rel_l2(a, b) <= 5e-2, (name, M, N, causal)
+        if bias_kind == "dense":
+            assert rel_l2(grads[3], db) <= 5e-2, (M, N)
+        elif bias_kind == "row":
+            # a sum over M rows of terms that the kernel rounds nowhere: bounded by the size of its terms, and where
+            # they vanish (one key: dP - delta is the rounding of two equal sums of D products) by M such roundings
+            limit = 1e-2 * db.abs().sum(2).max() + M * D * 2 ** -22
+            assert (grads[3].float() - db.sum(2, keepdim=True)).abs().max() <= limit, (M, N)
+        elif bias_kind == "alibi":
+            i, j = torch.arange(M, device=gpu_device)[:, None], torch.arange(N, device=gpu_device)[None, :]
+            terms = db[0] * -(i * (N / M) - j).abs()
+            assert (grads[3] - terms.sum((1, 2))).abs().max() <= 1e-2 * terms.abs().sum((1, 2)).max(), (M, N)
