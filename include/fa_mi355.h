@@ -105,7 +105,11 @@ typedef struct fa_fwd_args {
  *            dbias_strides[2] == 0, and dbias_strides[0] / [1] == 0 where the bias was broadcast over
  *            batches / heads too.  The kernels sum dS over the rows (and a second small kernel over
  *            the broadcast batches / heads), so no (B, H, M, N) gradient is ever written.  No
- *            counterpart in the reference, which leaves that reduction to autograd. */
+ *            counterpart in the reference, which leaves that reduction to autograd;
+ *   shared   the gradient of a bias that batches and / or heads share but query rows do not:
+ *            dbias_strides[0] and / or [1] are 0, [2] is not, and bias_strides are 0 in the same places.  A kernel
+ *            of its own sums dS over the pairs that share the bias, in fp32 and in a fixed order; scratch as
+ *            fa_bwd_args_workspace_bytes() says. */
 typedef struct fa_bwd_args {
     fa_problem p;
     const void *q, *k, *v, *o, *dout, *bias;
@@ -131,6 +135,11 @@ int fa_fwd(const fa_fwd_args *args, void *stream);
 /* Bytes of scratch the backward needs for this problem: delta, (B, H, M) fp32
  * (flash_attention.py:689), followed by the partial sums of the reduced dbias layouts. */
 size_t fa_bwd_workspace_bytes(const fa_problem *p);
+
+/* The same for given arguments (only p, dbias and its strides, and the strides of the bias are looked at): adds what
+ * the gradient of a shared bias needs when its pairs are split between work-groups.  Equal to
+ * fa_bwd_workspace_bytes(&args->p) for every other layout of dbias. */
+size_t fa_bwd_args_workspace_bytes(const fa_bwd_args *args);
 
 /* Scratch with which fa_fwd splits the keys of a query tile between several work-groups and merges
  * their softmaxes (the outputs of the shares in fp32, and their LSEs); 0 when the

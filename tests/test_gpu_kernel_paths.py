@@ -91,3 +91,30 @@ def test_backward_ragged_tiles_with_low_scores(gpu_device, D, bias_kind):
             i, j = torch.arange(M, device=gpu_device)[:, None], torch.arange(N, device=gpu_device)[None, :]
             terms = db[0] * -(i * (N / M) - j).abs()
             assert (grads[3] - terms.sum((1, 2))).abs().max() <= 1e-2 * terms.abs().sum((1, 2)).max(), (M, N)
+
+
+@pytest.mark.parametrize("D", [16, 32, 64, 128, 256])
+def test_gradient_of_a_shared_bias(gpu_device, D):
+    """A bias shared by batches and / or heads: its gradient is summed over the pairs in one kernel, in tiles of 128
+    rows and 64 keys, the pairs split between work-groups where the tiles are few (all cases but the last two)."""
+    g = torch.Generator().manual_seed(D)
+    cases = [((1, 3, 128, 64), 5, 3, torch.bfloat16, False), ((1, 2, 129, 65), 7, 2, torch.float32, False),
+             ((2, 1, 197, 197), 2, 3, torch.float16, True), ((1, 1, 2, 3), 3, 3, torch.float32, False),
+             ((1, 1, 127, 333), 2, 5, torch.bfloat16, False), ((1, 1, 64, 64), 1, 2, torch.float32, True)]
+    if D <= 64:
+        cases += [((1, 8, 520, 520), 2, 8, torch.float32, True), ((1, 8, 300, 770), 3, 8, torch.bfloat16, False)]
+    for shape, B, H, bias_dtype, causal in cases:
+        M, N = shape[2:]
+        dtype = torch.float16 if bias_dtype == torch.float16 else torch.bfloat16
+        mk = lambda n: torch.randn(B, n, H, D, generator=g).to(dtype).to(gpu_device).requires_grad_(True)
+        q, k, v, do = mk(M), mk(N), mk(N), mk(M).detach()
+        bias = torch.randn(shape, generator=g).to(bias_dtype).to(gpu_device).requires_grad_(True)
+        out = flash_attention_fn(q, k, v, bias, causal)
+        grads = torch.autograd.grad(out, (q, k, v, bias), do)
+        again = torch.autograd.grad(flash_attention_fn(q, k, v, bias, causal), bias, do)[0]
+        assert torch.equal(grads[3], again)
+        full = bias.detach().expand(B, H, M, N)
+        o, lse = attention_forward(q.detach(), k.detach(), v.detach(), full, causal)
+        dq, dk, dv, db, _ = attention_backward(do, q.detach(), k.detach(), v.detach(), o, lse, full, causal)
+        for name, a, b in zip(("dq", "dk", "dv", "dbias"), grads, (dq, dk, dv, db.sum_to_size(shape))):
+            assert rel_l2(a, b) <= 5e-2, (name, shape, B, H, causal, rel_l2(a, b))

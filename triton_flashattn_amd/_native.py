@@ -48,7 +48,7 @@ class FaBwdArgs(ctypes.Structure):
 
 
 EXPORTS = ("fa_abi_version", "fa_strerror", "fa_fwd", "fa_fwd_workspace_bytes", "fa_bwd_workspace_bytes", "fa_bwd", "fa_bwd_stages",
-           "fa_bwd_noalloc")
+           "fa_bwd_noalloc", "fa_bwd_args_workspace_bytes")
 FA_STAGE_PREP, FA_STAGE_MAIN, FA_STAGE_DQ, FA_STAGE_ALL, FA_STAGE_DQ_FROM_DBIAS = 1, 2, 4, 7, 8
 FA_NOALLOC_MAX_ROWS = 1 << 20
 FA_ERR_WORKSPACE = -6
@@ -82,6 +82,8 @@ def load():
     lib.fa_fwd_workspace_bytes.argtypes = [ctypes.POINTER(FaProblem)]
     lib.fa_bwd_workspace_bytes.restype = ctypes.c_size_t
     lib.fa_bwd_workspace_bytes.argtypes = [ctypes.POINTER(FaProblem)]
+    lib.fa_bwd_args_workspace_bytes.restype = ctypes.c_size_t
+    lib.fa_bwd_args_workspace_bytes.argtypes = [ctypes.POINTER(FaBwdArgs)]
     lib.fa_bwd.restype = ctypes.c_int
     lib.fa_bwd.argtypes = [ctypes.POINTER(FaBwdArgs), ctypes.c_void_p]
     lib.fa_bwd_stages.restype = ctypes.c_int

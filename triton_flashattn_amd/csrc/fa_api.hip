@@ -15,9 +15,11 @@ namespace fa {
 // one object file per head dimension defines these (fa_fwd.hip, fa_bwd.hip with -DFA_HEAD_DIM)
 template <int D> hipError_t launch_fwd_d(const FwdParams& p, int dtype, int bias, bool causal, hipStream_t st);
 template <int D> hipError_t launch_bwd_d(const BwdParams& p, int dtype, int bias, bool causal, int dbias, int stages, hipStream_t st);
+template <int D> hipError_t launch_bwd_shared_d(const BwdParams& p, int dtype, hipStream_t st);
 #define FA_DECLARE_D(D)                                                                                         \
     template <> hipError_t launch_fwd_d<D>(const FwdParams& p, int dtype, int bias, bool causal, hipStream_t st); \
-    template <> hipError_t launch_bwd_d<D>(const BwdParams& p, int dtype, int bias, bool causal, int dbias, int stages, hipStream_t st);
+    template <> hipError_t launch_bwd_d<D>(const BwdParams& p, int dtype, int bias, bool causal, int dbias, int stages, hipStream_t st); \
+    template <> hipError_t launch_bwd_shared_d<D>(const BwdParams& p, int dtype, hipStream_t st);
 FA_DECLARE_D(16)
 FA_DECLARE_D(32)
 FA_DECLARE_D(64)
@@ -42,6 +44,16 @@ static hipError_t launch_bwd(const BwdParams& p, int D, int dtype, int bias, boo
         case 64: return launch_bwd_d<64>(p, dtype, bias, causal, dbias, stages, st);
         case 128: return launch_bwd_d<128>(p, dtype, bias, causal, dbias, stages, st);
         case 256: return launch_bwd_d<256>(p, dtype, bias, causal, dbias, stages, st);
+    }
+    return hipErrorNotSupported;
+}
+static hipError_t launch_bwd_shared(const BwdParams& p, int D, int dtype, hipStream_t st) {
+    switch (D) {
+        case 16: return launch_bwd_shared_d<16>(p, dtype, st);
+        case 32: return launch_bwd_shared_d<32>(p, dtype, st);
+        case 64: return launch_bwd_shared_d<64>(p, dtype, st);
+        case 128: return launch_bwd_shared_d<128>(p, dtype, st);
+        case 256: return launch_bwd_shared_d<256>(p, dtype, st);
     }
     return hipErrorNotSupported;
 }
@@ -212,7 +224,8 @@ size_t dq_share_bytes(const fa_problem& p) {
     return s.n_splits <= 1 ? 0 : align256((size_t)s.n_splits * p.B * p.H * p.M * p.D * sizeof(float));
 }
 
-// How dbias is laid out: 0 none, 1 dense (B, H, M, N), 2 reduced in the kernels; -1 = not acceptable
+// How dbias is laid out: 0 none, 1 dense (B, H, M, N), 2 summed over the query rows in the kernels, 3 of a bias that
+// batches or heads share; -1 = not acceptable
 int dbias_mode(const fa_bwd_args* a) {
     const fa_problem& p = a->p;
     if (!a->dbias) return 0;
@@ -220,10 +233,37 @@ int dbias_mode(const fa_bwd_args* a) {
     const int64_t* s = a->dbias_strides;
     const bool red_b = p.B > 1 && s[0] == 0, red_h = p.H > 1 && s[1] == 0, red_m = p.M > 1 && s[2] == 0;
     if (!red_b && !red_h && !red_m) return 1;
-    // a reduction over batches or heads alone would need an (M, N) accumulator per output slice
-    if (!red_m && p.M > 1) return -1;
     if (p.N > 1 && s[3] == 0) return -1;
+    if (!red_m && p.M > 1) {
+        // the bias itself must be the one that is shared: its tile is read once for all pairs
+        return (red_b && a->bias_strides[0] != 0) || (red_h && a->bias_strides[1] != 0) ? -1 : 3;
+    }
     return 2;
+}
+
+// tiles of the gradient of a shared bias, over all of its slices
+int64_t shared_tiles(const fa_bwd_args* a) {
+    const fa_problem& p = a->p;
+    return (int64_t)((p.M + fa::kSharedTileM - 1) / fa::kSharedTileM) * ((p.N + fa::kSharedTileN - 1) / fa::kSharedTileN) *
+           (a->dbias_strides[0] == 0 ? 1 : p.B) * (a->dbias_strides[1] == 0 ? 1 : p.H);
+}
+// Work-groups that split the (batch, head) pairs of a tile of a shared bias's gradient between them: as many as fill
+// the GPU, one per CU (LDS).
+int shared_splits(const fa_bwd_args* a) {
+    const fa_problem& p = a->p;
+    const bool red_b = a->dbias_strides[0] == 0, red_h = a->dbias_strides[1] == 0;
+    const int64_t tiles = shared_tiles(a);
+    const int64_t pairs = (int64_t)(red_b ? p.B : 1) * (red_h ? p.H : 1);
+    int64_t n = compute_units() / tiles;
+    n = n < pairs ? n : pairs;
+    return n < 1 ? 1 : (int)n;
+}
+// the shares of such a gradient in fp32, whole tiles (0 when nothing is split)
+size_t shared_share_bytes(const fa_bwd_args* a) {
+    if (dbias_mode(a) != 3) return 0;
+    const int n = shared_splits(a);
+    if (n == 1) return 0;
+    return align256((size_t)shared_tiles(a) * n * fa::kSharedTileM * fa::kSharedTileN * sizeof(float));
 }
 
 }  // namespace
@@ -309,6 +349,12 @@ size_t fa_bwd_workspace_bytes(const fa_problem* p) {
     return align256(delta_floats(*p) * sizeof(float)) + align256(partial_floats(*p) * sizeof(float)) + dq_share_bytes(*p);
 }
 
+size_t fa_bwd_args_workspace_bytes(const fa_bwd_args* a) {
+    if (!a) return 0;
+    const size_t base = fa_bwd_workspace_bytes(&a->p);
+    return base == 0 ? 0 : base + shared_share_bytes(a);
+}
+
 }  // extern "C"
 
 namespace {
@@ -329,6 +375,7 @@ int bwd_enqueue(const fa_bwd_args* a, void* stream, int stages, float* delta) {
     if (a->dbias && (p.bias_dtype == FA_BIAS_NONE || p.bias_dtype == FA_BIAS_BOOL)) return FA_ERR_DTYPE;
     const int db_mode = dbias_mode(a);
     if (db_mode < 0) return FA_ERR_LAYOUT;
+    if (db_mode == 3 && shared_tiles(a) >= (1ll << 26)) return FA_ERR_SHAPE;  // its grid is one-dimensional too
     st = first_bad({qkv_layout(a->q, a->q_strides, p.B, p.M, p.H), qkv_layout(a->k, a->k_strides, p.B, p.N, p.H),
                     qkv_layout(a->v, a->v_strides, p.B, p.N, p.H), qkv_layout(a->o, a->o_strides, p.B, p.M, p.H),
                     qkv_layout(a->dout, a->do_strides, p.B, p.M, p.H),
@@ -339,8 +386,10 @@ int bwd_enqueue(const fa_bwd_args* a, void* stream, int stages, float* delta) {
     float* partials = nullptr;
     int dq_splits = 1, dq_keys = 0;  // (the entry point without allocations does not split: its scratch is small)
     void* part_dq = nullptr;
+    int splits = 1;  // work-groups per tile of a shared bias's gradient
     if (!delta) {
-        size_t need = fa_bwd_workspace_bytes(&p);
+        const size_t share_bytes = need_dkv ? shared_share_bytes(a) : 0;
+        size_t need = fa_bwd_workspace_bytes(&p) + share_bytes;
         if (!a->workspace || a->workspace_bytes < need || reinterpret_cast<uintptr_t>(a->workspace) % 256 != 0)
             return FA_ERR_WORKSPACE;
         delta = static_cast<float*>(a->workspace);
@@ -350,6 +399,11 @@ int bwd_enqueue(const fa_bwd_args* a, void* stream, int stages, float* delta) {
             dq_splits = s.n_splits;
             dq_keys = s.keys_per_split;
             part_dq = reinterpret_cast<char*>(partials) + align256(partial_floats(p) * sizeof(float));
+        }
+        if (share_bytes > 0) {
+            splits = shared_splits(a);
+            // (a shared bias has no column sums: its shares stand behind everything else)
+            partials = reinterpret_cast<float*>(static_cast<char*>(a->workspace) + fa_bwd_workspace_bytes(&p));
         }
     } else {
         partials = delta + FA_NOALLOC_MAX_ROWS;
@@ -382,8 +436,11 @@ int bwd_enqueue(const fa_bwd_args* a, void* stream, int stages, float* delta) {
     k.n_ntiles = (p.N + bn - 1) / bn;
     k.waves_per_role = bn / 32;
     k.n_mtiles = (p.M + fa::fwd_block_m() - 1) / fa::fwd_block_m();
+    k.causal = p.causal != 0; k.bias_kind = p.bias_dtype; k.shared_splits = splits;
+    k.shared_tiles = db_mode == 3 ? (int)shared_tiles(a) : 0;
     hipError_t e = fa::launch_bwd(k, p.D, p.dtype, p.bias_dtype, p.causal != 0, db_mode, stages,
                                   static_cast<hipStream_t>(stream));
+    if (e == hipSuccess && db_mode == 3 && need_dkv) e = fa::launch_bwd_shared(k, p.D, p.dtype, static_cast<hipStream_t>(stream));
     if (e == hipErrorNotSupported) return FA_ERR_UNSUPPORTED;
     return e == hipSuccess ? FA_OK : FA_ERR_LAUNCH;
 }

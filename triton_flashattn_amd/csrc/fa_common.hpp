@@ -23,6 +23,8 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 
+template <bool V> struct BoolTag { static constexpr bool value = V; };  // a compile-time flag as an argument
+
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kMask = -1.0e6f;  // additive mask term, in log2 units
 

@@ -13,6 +13,9 @@ struct Strides4 {
     int64_t b, h, m, n;
 };
 
+// tile of the gradient of a shared bias (fa_bwd_shared.hip): query rows, keys
+constexpr int kSharedTileM = 128, kSharedTileN = 64;
+
 // keys of a row-broadcast bias that the forward and dQ kernels keep in LDS (as fp32)
 constexpr int kRowBiasKeys = 4096;
 
@@ -70,6 +73,9 @@ struct BwdParams {
     void* part_dq;
     int row_bias_kind;  // 0, or the element kind (1 bool, 2 fp16, 3 bf16, 4 fp32) of a bias with stride 0 along M:
                         // the dK/dV kernel reads it as one value per key, the dQ kernel stages it in LDS
+    int causal, bias_kind;  // for the kernel of a shared bias, which has no variants: 1 if causal; 2 fp16, 3 bf16, 4 fp32
+    int shared_tiles;   // ... tiles of its gradient, over all slices
+    int shared_splits;  // ... work-groups that share the (batch, head) pairs of a tile (1: it stores the gradient itself)
     int dq_makes_delta; // the dQ kernel runs before the dK/dV kernel and forms delta itself (and stores it),
                         // in place of fa_bwd_prep_kernel and bit for bit like it
 };

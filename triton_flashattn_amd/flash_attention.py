@@ -172,16 +172,12 @@ class _HipBackend:
         if noalloc:
             if workspace is not None or stages != _native.FA_STAGE_ALL:
                 raise ValueError("fa_bwd_noalloc takes no workspace and runs every stage")
-        elif workspace is None:
-            workspace = self.bwd_workspace(q, k, bias, causal, sm_scale, alibi)
         a.q, a.k, a.v, a.o, a.dout, a.lse = (q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
                                              do.data_ptr(), lse.data_ptr())
         for name, t in (("dq", dq), ("dk", dk), ("dv", dv)):
             if t is not None:
                 setattr(a, name, t.data_ptr())
                 setattr(a, name + "_strides", _strides4(t))
-        if workspace is not None:
-            a.workspace, a.workspace_bytes = workspace.data_ptr(), workspace.numel()
         a.q_strides, a.k_strides, a.v_strides, a.o_strides = _strides4(q), _strides4(k), _strides4(v), _strides4(o)
         a.do_strides = _strides4(do)
         if bias is not None:
@@ -193,6 +189,13 @@ class _HipBackend:
             if not alibi:
                 a.dbias_strides = _strides4(dbias)
         with torch.cuda.device(dev):
+            if workspace is None and not noalloc:
+                nbytes = int(lib.fa_bwd_args_workspace_bytes(ctypes.byref(a)))
+                if nbytes == 0:
+                    raise _native.NativeLibraryError("libfa_mi355: problem rejected by fa_bwd_args_workspace_bytes")
+                workspace = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+            if workspace is not None:
+                a.workspace, a.workspace_bytes = workspace.data_ptr(), workspace.numel()
             stream = torch.cuda.current_stream(dev).cuda_stream
             if noalloc:
                 _native.check(lib.fa_bwd_noalloc(ctypes.byref(a), ctypes.c_void_p(stream)))
@@ -359,8 +362,8 @@ def _flash_attn_fwd(q, k, v, bias, causal, sm_scale):
 def _flash_attn_bwd(do, q, k, v, o, bias, causal, sm_scale, lse, dq, dk, dv, dbias):
     """Writes dq, dk, dv (and dbias when not None) in place; they may be strided views.  A dq that
     is None skips the dQ kernel, dk and dv that are both None (with no dbias) the dK/dV kernel.
-    dbias: a dense (B, H, M, N) tensor, or the gradient of a row-broadcast bias (B or 1, H or 1, 1,
-    N), reduced inside the kernels, or for an AlibiBias the H slope gradients."""
+    dbias: a dense (B, H, M, N) tensor, or the gradient of a bias broadcast over some of batches, heads and
+    query rows, with size 1 there, summed inside the kernels, or for an AlibiBias the H slope gradients."""
     B, M, H, D = q.shape
     N = k.shape[1]
     do, q, k, v, o = (_as_kernel_layout(t) for t in (do, q, k, v, o))
@@ -392,38 +395,11 @@ def _flash_attn_bwd(do, q, k, v, o, bias, causal, sm_scale, lse, dq, dk, dv, dbi
 
 
 def _bias_grad_like(bias, B, H, M, N):
-    """(tensor to hand to the kernels, function that turns it into the gradient of `bias`).
-    bias is the 4-D view of the caller's bias.  A bias that is broadcast over the query rows gets
-    its gradient reduced in the kernels; one that is only broadcast over batches or heads (it keeps
-    its M rows) goes through _bwd_bias_over_batches instead, marked by (None, None)."""
-    full = (B, H, M, N)
-    if bias.shape[2] == 1 and bias.shape[3] == N:
-        return torch.empty(bias.shape, dtype=bias.dtype, device=bias.device), (lambda t: t)
-    if tuple(bias.shape) == full:
-        return _empty_padded_rows(full, bias.dtype, bias.device), (lambda t: t)
-    return None, None
-
-
-def _bwd_bias_over_batches(do, q, k, v, o, bias, causal, sm_scale, lse, dq, dk, dv):
-    """The backward for a trainable bias of shape (1 or B, 1 or H, M, N) that is broadcast over
-    batches and / or heads: its gradient is the sum of dS over those dimensions, and a tile of an
-    (M, N) accumulator per output slice does not fit the kernels.  The kernels therefore run one
-    batch at a time, each writing its dS densely into ONE (1, H, M, N) scratch tensor, which is added
-    into an fp32 accumulator of the bias's shape in a fixed order (batches in sequence, heads by a
-    torch sum over a dimension: no atomics): the peak is one batch slice plus the accumulator, not
-    (B, H, M, N), and the sum is formed in fp32 whatever the bias's dtype.  Returns the gradient."""
-    B, M, H, _ = q.shape
-    N = k.shape[1]
-    over_b, over_h = bias.shape[0] == 1, bias.shape[1] == 1
-    acc = torch.zeros(bias.shape, dtype=torch.float32, device=bias.device)
-    scratch = _empty_padded_rows((1, H, M, N), bias.dtype, bias.device)
-    none = lambda t, b: None if t is None else t[b:b + 1]
-    for b in range(B):
-        _flash_attn_bwd(do[b:b + 1], q[b:b + 1], k[b:b + 1], v[b:b + 1], o[b:b + 1], bias[0:1] if over_b else bias[b:b + 1],
-                        causal, sm_scale, lse[b:b + 1], none(dq, b), none(dk, b), none(dv, b), scratch)
-        # (an in-place add of the 16-bit scratch to the fp32 accumulator converts on the fly: no fp32 copy)
-        acc[0 if over_b else b].add_(scratch.sum(dim=1, keepdim=True, dtype=torch.float32)[0] if over_h else scratch[0])
-    return acc.to(bias.dtype)
+    """The tensor that the kernels write the gradient of `bias`, the 4-D view of the caller's, into.  One that is
+    broadcast over the query rows, or over batches or heads, is summed over them in the kernels."""
+    if tuple(bias.shape) == (B, H, M, N):
+        return _empty_padded_rows(bias.shape, bias.dtype, bias.device)
+    return torch.empty(bias.shape, dtype=bias.dtype, device=bias.device)
 
 
 # --------------------------------------------------------------------------------------------
@@ -493,22 +469,18 @@ class FlashAttentionFn(torch.autograd.Function):
         dq = torch.empty_like(q) if need_q else None
         dk = torch.empty_like(k) if (need_k or need_v) else None
         dv = torch.empty_like(v) if (need_k or need_v) else None
-        dbias, finish = None, None
+        dbias = None
         if ctx.alibi:
             bias = AlibiBias(bias)
             if ctx.is_bias_trainable:
-                dbias, finish = torch.empty_like(bias.slopes), (lambda t: t)
+                dbias = torch.empty_like(bias.slopes)
         elif ctx.is_bias_trainable:
-            dbias, finish = _bias_grad_like(bias, B, H, M, N)
-        if ctx.is_bias_trainable and finish is None:
-            dbias = _bwd_bias_over_batches(_pad_head_dim(do, D), q, k, v, o, bias, ctx.causal, ctx.sm_scale, lse, dq, dk, dv)
-            finish = lambda t: t
-        elif dq is not None or dk is not None or dbias is not None:
+            dbias = _bias_grad_like(bias, B, H, M, N)
+        if dq is not None or dk is not None or dbias is not None:
             _flash_attn_bwd(_pad_head_dim(do, D), q, k, v, o, bias, ctx.causal, ctx.sm_scale, lse, dq, dk, dv, dbias)
         dq = dq if (dq is None or d_qk == D) else dq[..., :d_qk]
         dk = dk if (dk is None or not need_k) else (dk if d_qk == D else dk[..., :d_qk])
         dv = dv if (dv is None or not need_v) else (dv if d_v == D else dv[..., :d_v])
-        dbias = None if dbias is None else finish(dbias)
         grads = [dq, dk if need_k else None, dv if need_v else None, None, None, None, None]
         if dbias is not None:
             grads[6 if ctx.alibi else 3] = dbias
@@ -556,22 +528,17 @@ class FlashAttentionQKVPackedFn(torch.autograd.Function):
         qkv, o, lse, bias = ctx.saved_tensors
         B, S, _, H, _ = qkv.shape
         dqkv = torch.empty_like(qkv) if ctx.needs_input_grad[0] else None
-        dbias, finish = None, None
+        dbias = None
         if ctx.alibi:
             bias = AlibiBias(bias)
             if ctx.is_bias_trainable:
-                dbias, finish = torch.empty_like(bias.slopes), (lambda t: t)
+                dbias = torch.empty_like(bias.slopes)
         elif ctx.is_bias_trainable:
-            dbias, finish = _bias_grad_like(bias, B, H, S, S)
+            dbias = _bias_grad_like(bias, B, H, S, S)
         g = (None, None, None) if dqkv is None else (dqkv[:, :, 0], dqkv[:, :, 1], dqkv[:, :, 2])
-        if ctx.is_bias_trainable and finish is None:
-            dbias = _bwd_bias_over_batches(do, qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2], o, bias, ctx.causal, ctx.sm_scale,
-                                           lse, g[0], g[1], g[2])
-            finish = lambda t: t
-        elif dqkv is not None or dbias is not None:
+        if dqkv is not None or dbias is not None:
             _flash_attn_bwd(do, qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2], o, bias, ctx.causal, ctx.sm_scale, lse,
                             g[0], g[1], g[2], dbias)
-        dbias = None if dbias is None else finish(dbias)
         grads = [dqkv, None, None, None, None]
         if dbias is not None:
             grads[4 if ctx.alibi else 1] = dbias
@@ -643,18 +610,13 @@ def _op_bwd(do: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
             bias_grad: bool) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     B, M, H, D = q.shape
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    dbias, finish = None, None
     b4 = _check_bias(bias, q, k)
     if b4 is not None:
         b4 = _bias_kernel_layout(b4)
-    if bias_grad:
-        dbias, finish = _bias_grad_like(b4, B, H, M, k.shape[1])
-    if bias_grad and finish is None:
-        dbias, finish = _bwd_bias_over_batches(do, q, k, v, o, b4, causal, sm_scale, lse, dq, dk, dv), (lambda t: t)
-    else:
-        _flash_attn_bwd(do, q, k, v, o, b4, causal, sm_scale, lse, dq, dk, dv, dbias)
+    dbias = _bias_grad_like(b4, B, H, M, k.shape[1]) if bias_grad else None
+    _flash_attn_bwd(do, q, k, v, o, b4, causal, sm_scale, lse, dq, dk, dv, dbias)
     # an operator cannot return None: no bias gradient is an empty tensor
-    return dq, dk, dv, (finish(dbias).reshape(bias.shape).contiguous() if bias_grad else q.new_empty((0,)))
+    return dq, dk, dv, (dbias.reshape(bias.shape).contiguous() if bias_grad else q.new_empty((0,)))
 
 
 @_op_bwd.register_fake
