@@ -132,6 +132,11 @@ const char *fa_strerror(int status);
  * Replaces _flash_attn_fwd, flash_attention.py:649-685 (bias pre-scale :660-663 included). */
 int fa_fwd(const fa_fwd_args *args, void *stream);
 
+/* fa_fwd for q and k of head dim d_qk and v (and o) of head dim d_v, multiples of 8 no larger than p.D <= 128: computed
+ * at p.D with zeros in the missing columns, without padded copies.  (8, 8) .. (p.D, p.D); for p.D = 256 only p.D itself
+ * (FA_ERR_HEAD_DIM).  No counterpart in the reference, which takes powers of two (flash_attention.py:776). */
+int fa_fwd_dims(const fa_fwd_args *args, int d_qk, int d_v, void *stream);
+
 /* Bytes of scratch the backward needs for this problem: delta, (B, H, M) fp32
  * (flash_attention.py:689), followed by the partial sums of the reduced dbias layouts. */
 size_t fa_bwd_workspace_bytes(const fa_problem *p);
@@ -177,6 +182,10 @@ enum fa_bwd_stage {
  * FA_STAGE_DQ alone recomputes dS from q, k, v and the bias and never reads dbias, unless
  * FA_STAGE_DQ_FROM_DBIAS is added.  Both routes agree within the rounding of dS to 16 bits. */
 int fa_bwd_stages(const fa_bwd_args *args, void *stream, int stages);
+
+/* fa_bwd_stages for head dims as in fa_fwd_dims (q, k, dq, dk: d_qk; v, o, dout, dv: d_v).  Not for the gradient of a
+ * shared bias (FA_ERR_HEAD_DIM). */
+int fa_bwd_stages_dims(const fa_bwd_args *args, int d_qk, int d_v, void *stream, int stages);
 
 /* fa_bwd for callers that cannot allocate device memory (HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  No counterpart in the reference, whose launcher allocates

@@ -93,6 +93,14 @@ float* scratch_on_current_device() {
 
 namespace {
 
+// Head dims of q / k and of v below the kernel's, p.D: whole 16-byte chunks.  (The kernels of head dim 256 form the
+// offsets of their copies in the loop and take their full width only; the kernel of a shared bias's gradient has both
+// operands of its products in LDS and so no zeros for the missing columns.)
+bool dims_ok(const fa_problem& p, int d_qk, int d_v) {
+    if (d_qk == p.D && d_v == p.D) return true;
+    return p.D <= 128 && d_qk >= 8 && d_v >= 8 && d_qk <= p.D && d_v <= p.D && d_qk % 8 == 0 && d_v % 8 == 0;
+}
+
 bool head_dim_ok(int d) { return d == 16 || d == 32 || d == 64 || d == 128 || d == 256; }
 
 int check_problem(const fa_problem& p) {
@@ -300,11 +308,14 @@ size_t fa_fwd_workspace_bytes(const fa_problem* p) {
     return align256((size_t)s.n_splits * rows * p->D * sizeof(float)) + align256((size_t)s.n_splits * rows * sizeof(float));
 }
 
-int fa_fwd(const fa_fwd_args* a, void* stream) {
+int fa_fwd(const fa_fwd_args* a, void* stream) { return a ? fa_fwd_dims(a, a->p.D, a->p.D, stream) : FA_ERR_NULL; }
+
+int fa_fwd_dims(const fa_fwd_args* a, int d_qk, int d_v, void* stream) {
     if (!a) return FA_ERR_NULL;
     const fa_problem& p = a->p;
     int st = check_problem(p);
     if (st != FA_OK) return st;
+    if (!dims_ok(p, d_qk, d_v)) return FA_ERR_HEAD_DIM;
     if (!a->q || !a->k || !a->v || !a->o || !a->lse) return FA_ERR_NULL;
     if ((p.bias_dtype != FA_BIAS_NONE) != (a->bias != nullptr)) return FA_ERR_NULL;
     st = first_bad({qkv_layout(a->q, a->q_strides, p.B, p.M, p.H), qkv_layout(a->k, a->k_strides, p.B, p.N, p.H),
@@ -316,6 +327,7 @@ int fa_fwd(const fa_fwd_args* a, void* stream) {
     k.sq = s3(a->q_strides); k.sk = s3(a->k_strides); k.sv = s3(a->v_strides); k.so = s3(a->o_strides);
     k.B = p.B; k.H = p.H; k.M = p.M; k.N = p.N;
     k.sm_scale = p.sm_scale;
+    k.d_qk = d_qk; k.d_v = d_v;
     if (a->bias && p.bias_dtype != FA_BIAS_ALIBI) {
         k.sbias = s4(a->bias_strides);
         k.bias_vec = bias_vec_ok(a->bias, a->bias_strides, p) ? 1 : 0;
@@ -360,13 +372,14 @@ size_t fa_bwd_args_workspace_bytes(const fa_bwd_args* a) {
 namespace {
 
 // `delta` NULL: the scratch is the caller's workspace; else the workspace fields are ignored
-int bwd_enqueue(const fa_bwd_args* a, void* stream, int stages, float* delta) {
+int bwd_enqueue(const fa_bwd_args* a, int d_qk, int d_v, void* stream, int stages, float* delta) {
     if (!a) return FA_ERR_NULL;
     if (stages <= 0 || (stages & ~(FA_STAGE_ALL | FA_STAGE_DQ_FROM_DBIAS))) return FA_ERR_UNSUPPORTED;
     if ((stages & FA_STAGE_DQ_FROM_DBIAS) && !(stages & FA_STAGE_DQ)) return FA_ERR_UNSUPPORTED;
     const fa_problem& p = a->p;
     int st = check_problem(p);
     if (st != FA_OK) return st;
+    if (!dims_ok(p, d_qk, d_v)) return FA_ERR_HEAD_DIM;
     if (!a->q || !a->k || !a->v || !a->o || !a->dout || !a->lse) return FA_ERR_NULL;
     // outputs of stages that do not run may be NULL
     const bool need_dq = (stages & FA_STAGE_DQ) != 0, need_dkv = (stages & FA_STAGE_MAIN) != 0;
@@ -375,6 +388,7 @@ int bwd_enqueue(const fa_bwd_args* a, void* stream, int stages, float* delta) {
     if (a->dbias && (p.bias_dtype == FA_BIAS_NONE || p.bias_dtype == FA_BIAS_BOOL)) return FA_ERR_DTYPE;
     const int db_mode = dbias_mode(a);
     if (db_mode < 0) return FA_ERR_LAYOUT;
+    if (db_mode == 3 && (d_qk != p.D || d_v != p.D)) return FA_ERR_HEAD_DIM;
     if (db_mode == 3 && shared_tiles(a) >= (1ll << 26)) return FA_ERR_SHAPE;  // its grid is one-dimensional too
     st = first_bad({qkv_layout(a->q, a->q_strides, p.B, p.M, p.H), qkv_layout(a->k, a->k_strides, p.B, p.N, p.H),
                     qkv_layout(a->v, a->v_strides, p.B, p.N, p.H), qkv_layout(a->o, a->o_strides, p.B, p.M, p.H),
@@ -431,6 +445,7 @@ int bwd_enqueue(const fa_bwd_args* a, void* stream, int stages, float* delta) {
     }
     k.B = p.B; k.H = p.H; k.M = p.M; k.N = p.N;
     k.sm_scale = p.sm_scale;
+    k.d_qk = d_qk; k.d_v = d_v;
     int bn = fa::bwd_block_n(p.D);
     if (bn <= 0) return FA_ERR_UNSUPPORTED;
     k.n_ntiles = (p.N + bn - 1) / bn;
@@ -449,9 +464,15 @@ int bwd_enqueue(const fa_bwd_args* a, void* stream, int stages, float* delta) {
 
 extern "C" {
 
-int fa_bwd_stages(const fa_bwd_args* a, void* stream, int stages) { return bwd_enqueue(a, stream, stages, nullptr); }
+int fa_bwd_stages_dims(const fa_bwd_args* a, int d_qk, int d_v, void* stream, int stages) {
+    return bwd_enqueue(a, d_qk, d_v, stream, stages, nullptr);
+}
 
-int fa_bwd(const fa_bwd_args* a, void* stream) { return bwd_enqueue(a, stream, FA_STAGE_ALL, nullptr); }
+int fa_bwd_stages(const fa_bwd_args* a, void* stream, int stages) {
+    return a ? bwd_enqueue(a, a->p.D, a->p.D, stream, stages, nullptr) : FA_ERR_NULL;
+}
+
+int fa_bwd(const fa_bwd_args* a, void* stream) { return fa_bwd_stages(a, stream, FA_STAGE_ALL); }
 
 int fa_bwd_noalloc(const fa_bwd_args* a, void* stream) {
     if (!a) return FA_ERR_NULL;
@@ -461,7 +482,7 @@ int fa_bwd_noalloc(const fa_bwd_args* a, void* stream) {
         return FA_ERR_TOO_LARGE;
     float* delta = fa::scratch_on_current_device();
     if (!delta) return FA_ERR_LAUNCH;
-    return bwd_enqueue(a, stream, FA_STAGE_ALL, delta);
+    return bwd_enqueue(a, a->p.D, a->p.D, stream, FA_STAGE_ALL, delta);
 }
 
 }  // extern "C"

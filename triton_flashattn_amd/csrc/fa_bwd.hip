@@ -29,7 +29,7 @@ __global__ __launch_bounds__(256) void fa_bwd_prep_kernel(const BwdParams p) {
     const int64_t row = (int64_t)blockIdx.x * RPB + threadIdx.x / LPR;
     const int c = threadIdx.x % LPR;
     float acc = 0.f;
-    if (row < rows) {
+    if (row < rows && c * 8 < p.d_v) {
         const int m = (int)(row % p.M);
         const int bh = (int)(row / p.M);
         const int b = bh / p.H, h = bh % p.H;
@@ -117,10 +117,9 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
 #pragma unroll
     for (int ks = 0; ks < C::KSTEPS; ks++) {
         i32x4 rq = {0, 0, 0, 0}, rd = {0, 0, 0, 0};
-        if (!FROM_DS && my_m < M) {
-            rq = gld16(qp + (int64_t)my_m * p.sq.s + ks * 16 + 8 * g);
-            rd = gld16(dop + (int64_t)my_m * p.sdo.s + ks * 16 + 8 * g);
-        }
+        const int d = ks * 16 + 8 * g;
+        if (!FROM_DS && my_m < M && d < p.d_qk) rq = gld16(qp + (int64_t)my_m * p.sq.s + d);
+        if (!FROM_DS && my_m < M && d < p.d_v) rd = gld16(dop + (int64_t)my_m * p.sdo.s + d);
         qreg[ks] = as_vec<T8>(rq);
         doreg[ks] = as_vec<T8>(rd);
     }
@@ -140,7 +139,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
 #pragma unroll
         for (int ks = 0; ks < C::KSTEPS; ks++) {
             i32x4 ro = {0, 0, 0, 0};
-            if (my_m < M) ro = gld16(op + (int64_t)my_m * p.so.s + ks * 16 + 8 * g);
+            if (my_m < M && ks * 16 + 8 * g < p.d_v) ro = gld16(op + (int64_t)my_m * p.so.s + ks * 16 + 8 * g);
             const T8 ov = as_vec<T8>(ro);
             float a = 0.f;
 #pragma unroll
@@ -174,7 +173,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
     const unsigned rows_l = SW::rows_lane(lane), cols_l = SW::cols_lane(lane);
     KeyStream<T, D, stream_kind(BIAS), !FROM_DS> ks_;
     ks_.init(smem, kp, vp, bp, p.sk.s, p.sv.s, FROM_DS ? p.sdbias.m : p.sbias.m, FROM_DS ? p.sdbias.n : p.sbias.n, M, N,
-             mw, wave, lane);
+             mw, wave, lane, p.d_qk, p.d_v);
 
     // One step of the K/V stream.  Interior steps (every key in range and visible to every row of
     // the work-group) run with STEP_MASKED = false: no range checks, no mask arithmetic.  BV: the
@@ -400,7 +399,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
     T* op = reinterpret_cast<T*>(p.dq) + (int64_t)b * p.sdq.b + (int64_t)h * p.sdq.h;
     for (int c = lane; c < 32 * CPR; c += 64) {
         int row = c / CPR, ch = c % CPR;
-        if (mw + row < M) gst16(op + (int64_t)(mw + row) * p.sdq.s + ch * 8, lds_read16(o_lds + row * OS + ch * 8));
+        if (mw + row < M && ch * 8 < p.d_qk) gst16(op + (int64_t)(mw + row) * p.sdq.s + ch * 8, lds_read16(o_lds + row * OS + ch * 8));
     }
 }
 
@@ -413,7 +412,7 @@ template <typename T, int D> __global__ __launch_bounds__(256) void fa_bwd_dq_su
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int64_t row = idx / TPR;
     const int c = (int)(idx % TPR);
-    if (row >= rows) return;
+    if (row >= rows || c * 8 >= p.d_qk) return;
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     for (int s = 0; s < p.dq_splits; s++) {
         const float* src = reinterpret_cast<const float*>(p.part_dq) + (s * rows + row) * D + c * 8;
@@ -627,7 +626,7 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
 #pragma unroll
         for (int ks = 0; ks < C::KSTEPS; ks++) {
             i32x4 v = {0, 0, 0, 0};
-            if (my_n < N) v = gld16(src + ks * 16 + 8 * g);
+            if (my_n < N && ks * 16 + 8 * g < (s_wave ? p.d_qk : p.d_v)) v = gld16(src + ks * 16 + 8 * g);
             opreg[ks] = as_vec<T8>(v);
         }
     }
@@ -675,10 +674,10 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
         c_idx[i] = (kb * C::QD + i) % C::NQD;
         const int c = c_idx[i] * 64 + lane;
         const int row = c / CPR, src = (c % CPR) ^ SW::f(row);
-        cq_off[i] = (unsigned)(row * (int)p.sq.s * 2 + src * 16);
-        cdo_off[i] = (unsigned)(row * (int)p.sdo.s * 2 + src * 16);
+        cq_off[i] = (unsigned)(row * (int)p.sq.s * 2 + live_chunk(src, p.d_qk / 8) * 16);
+        cdo_off[i] = (unsigned)(row * (int)p.sdo.s * 2 + live_chunk(src, p.d_v / 8) * 16);
     }
-    auto issue_rows = [&](const T* base, int64_t row_stride, const unsigned (&off)[C::QD], int mb, unsigned dst) {
+    auto issue_rows = [&](const T* base, int64_t row_stride, int chunks, const unsigned (&off)[C::QD], int mb, unsigned dst) {
         // a block past the end is the last row over and over: offsets never go negative
         const int m0 = mb * BMI < M ? mb * BMI : M - 1;
         const uint64_t blk = uniform_ptr(base + (int64_t)m0 * row_stride);
@@ -695,7 +694,7 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
                 int row = c / CPR;
                 const int src = (c % CPR) ^ SW::f(row);
                 row = row < M - m0 ? row : M - 1 - m0;
-                o = (unsigned)(row * (int)row_stride * 2 + src * 16);
+                o = (unsigned)(row * (int)row_stride * 2 + live_chunk(src, chunks) * 16);
             }
             lds_copy16(blk, o, dst + c_idx[i] * 1024);
         }
@@ -729,11 +728,11 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
     // block mb of Q with its LSE (QD + 1 copies) / block mb of dO with its delta (QD + 1 copies);
     // all four waves of a role copy the 32 or 64 floats, which keeps their counts alike
     auto issue_q = [&](int mb) {
-        issue_rows(qp, p.sq.s, cq_off, mb, lds_base + (mb % C::NQB) * C::Q_BYTES);
+        issue_rows(qp, p.sq.s, p.d_qk / 8, cq_off, mb, lds_base + (mb % C::NQB) * C::Q_BYTES);
         issue_stat(lsep, mb, lds_base + C::OFF_LSE + (mb % C::NQB) * C::STAT_BYTES);
     };
     auto issue_do = [&](int mb) {
-        issue_rows(dop, p.sdo.s, cdo_off, mb, lds_base + C::OFF_DO + (mb % C::NDOB) * C::Q_BYTES);
+        issue_rows(dop, p.sdo.s, p.d_v / 8, cdo_off, mb, lds_base + C::OFF_DO + (mb % C::NDOB) * C::Q_BYTES);
         issue_stat(deltap, mb, lds_base + C::OFF_DELTA + (mb % C::NDOB) * C::STAT_BYTES);
     };
     // Issuing a copy stalls the wave while the memory pipeline of the CU is backed up, so the
@@ -1329,12 +1328,13 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
         T* dst = s_wave ? reinterpret_cast<T*>(p.dv) + (int64_t)b * p.sdv.b + (int64_t)h * p.sdv.h + (int64_t)my_n * p.sdv.s
                         : reinterpret_cast<T*>(p.dk) + (int64_t)b * p.sdk.b + (int64_t)h * p.sdk.h + (int64_t)my_n * p.sdk.s;
         const float out_scale = s_wave ? 1.f : p.sm_scale;
+        const int d_out = s_wave ? p.d_v : p.d_qk;
 #pragma unroll
         for (int db = 0; db < C::DB; db++) {
 #pragma unroll
             for (int q4 = 0; q4 < 4; q4++) {
                 const int d = db * 32 + 8 * q4 + 4 * g;
-                if (d < D) {
+                if (d < d_out) {
                     T4 o4;
 #pragma unroll
                     for (int e = 0; e < 4; e++) o4[e] = (T)(acc[db][q4 * 4 + e] * out_scale);

@@ -308,6 +308,11 @@ __device__ __forceinline__ void stage_row_bias(float* row_lds, const void* bias,
     __syncthreads();
 }
 
+// A head dim below the kernel's (a multiple of 8): a copy that would fetch a chunk behind the end of a row fetches
+// the first one again.  Such a chunk meets zeros in the operand of the product that sits in registers (Q, dO, K or V
+// rows are loaded with zeros there), or makes columns of the result that are not stored.
+__device__ __forceinline__ int live_chunk(int chunk, int chunks) { return chunk < chunks ? chunk : 0; }
+
 // Tiling of the forward and the dQ kernel: a work-group owns 128 query rows (4 waves x 32 rows) and streams
 // keys in steps of NH blocks of 32.  K and V rows of a step and the bias slice of each wave reach
 // LDS through direct global -> LDS copies issued ahead of their use.  With a bias: steps of 32
@@ -366,6 +371,7 @@ template <typename T, int D, int BIAS, bool WITH_V = true> struct KeyStream {
     const E* bp;              // (batch, head) slices
     int64_t sk, sv, sbm, sbn; // row strides of K and V, row and key stride of the bias (elements)
     int M, N, mw, lane;
+    int k_chunks, v_chunks;   // 16-byte chunks of a row of K and of V (fewer than CPR: a head dim below the kernel's)
     // LEAN (rows of LEAN_CPR chunks): the per-lane offsets of the KD copies are formed from three
     // per-lane constants when a copy is issued, instead of being held in 3 KD registers that such a
     // kernel does not have: a copy of chunk c = 64 ci + l reads row r0 + q (r0 = (64 / CPR) ci, q =
@@ -395,9 +401,11 @@ template <typename T, int D, int BIAS, bool WITH_V = true> struct KeyStream {
     // (row c / CPR, LDS chunk c % CPR holds global chunk (c % CPR) ^ f(row)).  Each wave issues KD
     // of them (more than once where a step has fewer than four).
     __device__ __forceinline__ void init(unsigned char* smem_, const T* kp_, const T* vp_, const E* bp_, int64_t sk_,
-                                         int64_t sv_, int64_t sbm_, int64_t sbn_, int M_, int N_, int mw_, int wave, int lane_) {
+                                         int64_t sv_, int64_t sbm_, int64_t sbn_, int M_, int N_, int mw_, int wave, int lane_,
+                                         int d_k, int d_v) {
         smem = smem_; kp = kp_; vp = vp_; bp = bp_; sk = sk_; sv = sv_; sbm = sbm_; sbn = sbn_;
         M = M_; N = N_; mw = mw_; lane = lane_;
+        k_chunks = d_k / 8; v_chunks = d_v / 8;
         wave = __builtin_amdgcn_readfirstlane(wave);  // the same in every lane: keep it scalar
         bias_lds = smem + C::KV_BYTES + wave * C::NBS * C::BSLOT;
         lds_kv = lds_addr_of(smem);
@@ -415,8 +423,8 @@ template <typename T, int D, int BIAS, bool WITH_V = true> struct KeyStream {
                 c_idx[i] = (wave * C::KD + i) % C::NKD;
                 const int c = c_idx[i] * 64 + lane;
                 const int row = c / C::CPR, src = (c % C::CPR) ^ SW::f(row);
-                k_off[i] = (unsigned)(row * (int)sk * 2 + src * 16);
-                v_off[i] = (unsigned)(row * (int)sv * 2 + src * 16);
+                k_off[i] = (unsigned)(row * (int)sk * 2 + live_chunk(src, k_chunks) * 16);
+                v_off[i] = (unsigned)(row * (int)sv * 2 + live_chunk(src, v_chunks) * 16);
             }
         }
     }
@@ -463,8 +471,8 @@ template <typename T, int D, int BIAS, bool WITH_V = true> struct KeyStream {
                 int row = c / C::CPR;
                 const int src = (c % C::CPR) ^ SW::f(row);
                 row = row < N - n0 ? row : N - 1 - n0;
-                ko = (unsigned)(row * (int)sk * 2 + src * 16);
-                vo = (unsigned)(row * (int)sv * 2 + src * 16);
+                ko = (unsigned)(row * (int)sk * 2 + live_chunk(src, k_chunks) * 16);
+                vo = (unsigned)(row * (int)sv * 2 + live_chunk(src, v_chunks) * 16);
             }
             lds_copy16(kt, ko, k_dst + ci * 1024);
             if constexpr (WITH_V) lds_copy16(vt, vo, v_dst + ci * 1024);

@@ -92,7 +92,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
 #pragma unroll
     for (int ks = 0; ks < C::KSTEPS; ks++) {
         i32x4 raw = {0, 0, 0, 0};
-        if (my_m < M) raw = gld16(qp + (int64_t)my_m * p.sq.s + ks * 16 + 8 * g);
+        if (my_m < M && ks * 16 + 8 * g < p.d_qk) raw = gld16(qp + (int64_t)my_m * p.sq.s + ks * 16 + 8 * g);
         qreg[ks] = as_vec<T8>(raw);
     }
 
@@ -112,7 +112,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
 
     const unsigned rows_l = SW::rows_lane(lane), cols_l = SW::cols_lane(lane);
     KeyStream<T, D, fwd_stream_kind(BIAS)> ks_;
-    ks_.init(smem, kp, vp, bp, p.sk.s, p.sv.s, p.sbias.m, p.sbias.n, M, N, mw, wave, lane);
+    ks_.init(smem, kp, vp, bp, p.sk.s, p.sv.s, p.sbias.m, p.sbias.n, M, N, mw, wave, lane, p.d_qk, p.d_v);
 
     // raises the reference point of this row's exponentials to mx (log2 units) where it is lower
     auto raise = [&](float mx) {
@@ -459,7 +459,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
     T* op = reinterpret_cast<T*>(p.o) + (int64_t)b * p.so.b + (int64_t)h * p.so.h;
     for (int c = lane; c < 32 * CPR; c += 64) {
         int row = c / CPR, ch = c % CPR;
-        if (mw + row < M) gst16(op + (int64_t)(mw + row) * p.so.s + ch * 8, lds_read16(o_lds + row * OS + ch * 8));
+        if (mw + row < M && ch * 8 < p.d_v) gst16(op + (int64_t)(mw + row) * p.so.s + ch * 8, lds_read16(o_lds + row * OS + ch * 8));
     }
 }
 
@@ -472,7 +472,7 @@ template <typename T, int D> __global__ __launch_bounds__(256) void fa_fwd_merge
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int64_t row = idx / TPR;
     const int c = (int)(idx % TPR);
-    if (row >= rows) return;
+    if (row >= rows || c * 8 >= p.d_v) return;
     float mx = -INFINITY;
     for (int s = 0; s < p.n_splits; s++) mx = fmaxf(mx, p.part_lse[s * rows + row]);
     float sum = 0.f;
