@@ -118,3 +118,73 @@ def test_gradient_of_a_shared_bias(gpu_device, D):
         dq, dk, dv, db, _ = attention_backward(do, q.detach(), k.detach(), v.detach(), o, lse, full, causal)
         for name, a, b in zip(("dq", "dk", "dv", "dbias"), grads, (dq, dk, dv, db.sum_to_size(shape))):
             assert rel_l2(a, b) <= 5e-2, (name, shape, B, H, causal, rel_l2(a, b))
+
+
+@pytest.mark.parametrize("d_qk,d_v", [(8, 8), (24, 24), (40, 56), (80, 80), (96, 40), (72, 120), (64, 128)])
+def test_head_dims_below_the_kernels(gpu_device, d_qk, d_v):
+    """Head dims that are whole 16-byte chunks run at the next head dim of the kernels without padded copies: both
+    directions, plain, split over the keys, with masks and causal, and nothing is written past a row."""
+    g = torch.Generator().manual_seed(d_qk)
+    for B, M, N, H, causal, kind in [(2, 130, 130, 2, True, None), (1, 77, 200, 3, False, "dense"), (2, 64, 333, 2, False, "bool"),
+                                     (1, 40, 2200, 1, False, None), (2, 257, 257, 2, False, None)]:
+        mk = lambda n, d: torch.randn(B, n, H, d, generator=g).bfloat16().to(gpu_device).requires_grad_(True)
+        # (the tensors are slices of wider ones, whose other columns hold NaN)
+        wide = lambda n, d: torch.cat([mk(n, d).detach(), torch.full((B, n, H, 8), float("nan"), device=gpu_device, dtype=torch.bfloat16)], -1)
+        q, k, v, do = (wide(M, d_qk)[..., :d_qk].requires_grad_(True), wide(N, d_qk)[..., :d_qk].requires_grad_(True),
+                       wide(N, d_v)[..., :d_v].requires_grad_(True), mk(M, d_v).detach())
+        bias = None
+        if kind == "dense":
+            bias = torch.randn(B, H, M, N, generator=g).bfloat16().to(gpu_device).requires_grad_(True)
+        elif kind == "bool":
+            bias = (torch.rand(B, H, M, N, generator=g) > 0.3).index_fill(3, torch.tensor([0]), True).to(gpu_device)
+        out = flash_attention_fn(q, k, v, bias, causal)
+        wanted = [q, k, v] + ([bias] if kind == "dense" else [])
+        grads = torch.autograd.grad(out, wanted, do)
+        b = None if bias is None else bias.detach()
+        o, lse = attention_forward(q.detach(), k.detach(), v.detach(), b, causal)
+        dq, dk, dv, db, _ = attention_backward(do, q.detach(), k.detach(), v.detach(), o, lse, b, causal)
+        assert out.shape == o.shape and (out.float() - o).abs().max().item() <= 2e-2
+        for name, a, ref in zip(("dq", "dk", "dv", "dbias"), grads, (dq, dk, dv, db)):
+            assert a.shape == ref.shape and rel_l2(a, ref) <= 5e-2, (name, M, N, causal, kind)
+
+
+def test_host_path_equals_the_autograd_classes(gpu_device):
+    """flash_attention_fn goes through the C++ host path; FlashAttentionFn, called directly, through Python and ctypes:
+    the same kernels on the same arguments, bit for bit, for every kind of bias, layout and set of wanted gradients."""
+    from triton_flashattn_amd.flash_attention import FlashAttentionFn, FlashAttentionQKVPackedFn, flash_attention_qkvpacked_fn
+    dev, g = gpu_device, torch.Generator().manual_seed(0)
+    B, M, N, H, D = 2, 75, 131, 4, 64
+    rnd = lambda *s: torch.randn(*s, generator=g).bfloat16().to(dev)
+    slopes = torch.tensor([0.5, 0.1, 0.02, 0.01], device=dev)
+    biases = [None, rnd(B, H, M, N), rnd(1, H, M, N).float(), rnd(H, 1, N).half(), rnd(N), rnd(M, N), rnd(B, 1, 1, N) > -1.0, slopes]
+    for i, bias in enumerate(biases):
+        for want in ((1, 1, 1, 1), (1, 0, 0, 0), (0, 1, 0, 1), (0, 0, 1, 0), (0, 0, 0, 1)):
+            if want == (0, 0, 0, 1) and (bias is None or bias.dtype == torch.bool):
+                continue
+            # sequence-major, head-major, and rows that the kernels cannot read in place
+            q = rnd(B, M, H, D) if i % 3 == 0 else rnd(B, H, M, D).transpose(1, 2) if i % 3 == 1 else rnd(B, M, H, D + 2)[..., :D]
+            inputs = [q, rnd(B, N, H, D), rnd(B, N, H, D)]
+            is_alibi = bias is slopes
+            extra = None if bias is None else bias.clone()
+            leaves = []
+            for t, w in zip(inputs + ([] if extra is None or extra.dtype == torch.bool else [extra]), want):
+                t.requires_grad_(bool(w))
+                if w:
+                    leaves.append(t)
+            do = rnd(B, M, H, D) if i % 2 else rnd(B, M, H, 1).expand(B, M, H, D)
+            ours = flash_attention_fn(*inputs, AlibiBias(extra) if is_alibi else extra, False)
+            ref = FlashAttentionFn.apply(*inputs, None if is_alibi else extra, False, None, extra if is_alibi else None)
+            assert "AttentionNode" in ours.grad_fn.name()
+            assert torch.equal(ours, ref)
+            for a, b in zip(torch.autograd.grad(ours, leaves, do), torch.autograd.grad(ref, leaves, do)):
+                assert a.shape == b.shape and a.dtype == b.dtype and torch.equal(a, b), (i, want)
+    qkv = rnd(B, M, 3, H, D).requires_grad_(True)
+    for bias in (None, rnd(1, H, M, M).requires_grad_(True)):
+        leaves, do = [qkv] + ([] if bias is None else [bias]), rnd(B, M, H, D)
+        ours, ref = flash_attention_qkvpacked_fn(qkv, bias, True), FlashAttentionQKVPackedFn.apply(qkv, bias, True, None, None)
+        for a, b in zip((ours,) + torch.autograd.grad(ours, leaves, do), (ref,) + torch.autograd.grad(ref, leaves, do)):
+            assert torch.equal(a, b)
+    with torch.no_grad():
+        assert torch.equal(flash_attention_qkvpacked_fn(qkv, None, True), ours.detach() * 0 + flash_attention_qkvpacked_fn(qkv.detach(), None, True))
+    with pytest.raises(ValueError):
+        flash_attention_fn(qkv[:, :, 0], qkv[:, :5, 1], qkv[:, :5, 2], None, True)

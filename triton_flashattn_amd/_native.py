@@ -1,12 +1,15 @@
-"""ctypes binding of libfa_mi355.so (the C ABI declared in include/fa_mi355.h).
+"""ctypes binding of libfa_mi355.so (the C ABI declared in include/fa_mi355.h), and the loader of the C++ host
+path built on the same library (csrc/torch_host.cpp).
 
-There is no fallback: if the library is missing or a call fails, an exception is raised.
+There is no fallback: if a library is missing or a call fails, an exception is raised.
 """
 import ctypes
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libfa_mi355.so")
+HOST_PATH = os.path.join(_HERE, "_torch_host.so")
 ABI_VERSION = 3
 
 FA_F16, FA_BF16 = 0, 1
@@ -48,7 +51,7 @@ class FaBwdArgs(ctypes.Structure):
 
 
 EXPORTS = ("fa_abi_version", "fa_strerror", "fa_fwd", "fa_fwd_workspace_bytes", "fa_bwd_workspace_bytes", "fa_bwd", "fa_bwd_stages",
-           "fa_bwd_noalloc", "fa_bwd_args_workspace_bytes")
+           "fa_bwd_noalloc", "fa_bwd_args_workspace_bytes", "fa_fwd_dims", "fa_bwd_stages_dims")
 FA_STAGE_PREP, FA_STAGE_MAIN, FA_STAGE_DQ, FA_STAGE_ALL, FA_STAGE_DQ_FROM_DBIAS = 1, 2, 4, 7, 8
 FA_NOALLOC_MAX_ROWS = 1 << 20
 FA_ERR_WORKSPACE = -6
@@ -56,6 +59,7 @@ FA_ERR_TOO_LARGE = -9
 FA_ERR_HEAD_STRIDE = -10
 
 _lib = None
+_host = None
 
 
 class NativeLibraryError(RuntimeError):
@@ -99,3 +103,17 @@ def load():
 def check(status):
     if status != 0:
         raise NativeLibraryError("libfa_mi355: %s (status %d)" % (load().fa_strerror(status).decode(), status))
+
+
+def host():
+    """The C++ host path, loaded once."""
+    global _host
+    if _host is None:
+        load()
+        if not os.path.exists(HOST_PATH):
+            raise NativeLibraryError("%s is missing: build it with `python -m triton_flashattn_amd.build`" % HOST_PATH)
+        spec = importlib.util.spec_from_file_location("triton_flashattn_amd._torch_host", HOST_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _host = module
+    return _host

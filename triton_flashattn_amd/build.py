@@ -1,4 +1,5 @@
-"""Builds libfa_mi355.so (HIP kernels + C ABI) for gfx950 next to this file.
+"""Builds libfa_mi355.so (HIP kernels + C ABI) for gfx950 and _torch_host.so (the host path on top of it, C++ against
+the installed PyTorch) next to this file.
 
 Usage: python -m triton_flashattn_amd.build [-j N]
 hipcc cross-compiles without a GPU, so this runs anywhere the ROCm toolchain is installed.
@@ -7,11 +8,13 @@ import os
 import re
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libfa_mi355.so")
+HOST = os.path.join(HERE, "_torch_host.so")
 HEAD_DIMS = (128, 64, 256, 32, 16)  # longest compiles first
 # (source, head dim or None): the kernel files are compiled once per head dimension
 UNITS = [(f, d) for f in ("fa_bwd.hip", "fa_fwd.hip", "fa_bwd_shared.hip") for d in HEAD_DIMS] + [("fa_api.hip", None)]
@@ -54,6 +57,22 @@ def _scratch_users(log):
     return out
 
 
+def _build_host():
+    """csrc/torch_host.cpp: host code only, so the host compiler builds it.  It links against libfa_mi355.so beside it."""
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-w", "-DUSE_ROCM=1", "-D__HIP_PLATFORM_AMD__=1",
+           "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI), "-DTORCH_EXTENSION_NAME=_torch_host"]
+    cmd += ["-I" + p for p in include_paths() + [os.path.join(os.path.dirname(os.path.dirname(HIPCC)), "include"),
+                                                 sysconfig.get_paths()["include"]]]
+    cmd += [os.path.join(CSRC, "torch_host.cpp"), "-o", HOST, "-L" + torch_lib, "-L" + HERE, "-l:libfa_mi355.so", "-ltorch",
+            "-ltorch_cpu", "-ltorch_python", "-ltorch_hip", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("torch_host.cpp failed:\n" + res.stdout + res.stderr)
+
+
 def build(jobs=8, verbose=False):
     with ThreadPoolExecutor(max_workers=max(1, jobs)) as ex:
         results = list(ex.map(_compile, UNITS))
@@ -73,6 +92,7 @@ def build(jobs=8, verbose=False):
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError("link failed:\n" + res.stdout + res.stderr)
+    _build_host()
     return LIB
 
 

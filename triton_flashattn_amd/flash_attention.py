@@ -205,7 +205,8 @@ class _HipBackend:
             # allocator re-issues it to later work on the same stream only, so it may be dropped
 
 
-_backend = _HipBackend()
+_HIP = _HipBackend()
+_backend = _HIP
 
 
 # --------------------------------------------------------------------------------------------
@@ -559,6 +560,14 @@ def _split_bias(bias):
     return (None, bias.slopes) if isinstance(bias, AlibiBias) else (bias, None)
 
 
+def _host_attention(q, k, v, bias, slopes, causal, sm_scale):
+    """The call through the C++ host path (csrc/torch_host.cpp), which does on the GPU what the autograd functions
+    above do; None where it declines: then they run, and raise whatever is to be raised."""
+    if _backend is not _HIP or not isinstance(q, torch.Tensor) or not q.is_cuda or torch.compiler.is_compiling():
+        return None
+    return _native.host().attention(q, k, v, bias, slopes, causal, sm_scale)
+
+
 def flash_attention_fn(q, k, v, bias=None, causal=False, sm_scale=None):
     """out = softmax(q k^T * sm_scale + bias) v, differentiable in q, k, v and a float bias.
 
@@ -568,18 +577,22 @@ def flash_attention_fn(q, k, v, bias=None, causal=False, sm_scale=None):
     """
     q, k, v = _autocast_inputs(q, k, v)
     bias, slopes = _split_bias(bias)
-    return FlashAttentionFn.apply(q, k, v, bias, causal, sm_scale, slopes)
+    out = _host_attention(q, k, v, bias, slopes, causal, sm_scale)
+    return FlashAttentionFn.apply(q, k, v, bias, causal, sm_scale, slopes) if out is None else out
 
 
 def flash_attention_qkvpacked_fn(qkv, bias=None, causal=False, sm_scale=None):
     """Self-attention on a packed qkv (B, seqlen, 3, H, D); bias as for flash_attention_fn with
     M = N = seqlen.  The gradient comes back packed in one tensor.  Returns out (B, seqlen, H, D)."""
     (qkv,) = _autocast_inputs(qkv)
+    tensor_bias, slopes = _split_bias(bias)
+    out = _host_attention(qkv, None, None, tensor_bias, slopes, causal, sm_scale)
+    if out is not None:
+        return out
     if isinstance(qkv, torch.Tensor) and qkv.dim() == 5 and qkv.shape[2] == 3 and qkv.shape[-1] not in _HEAD_DIMS:
         # a head dim that needs padding: the packed layout is lost anyway
         return flash_attention_fn(qkv[:, :, 0], qkv[:, :, 1], qkv[:, :, 2], bias, causal, sm_scale)
-    bias, slopes = _split_bias(bias)
-    return FlashAttentionQKVPackedFn.apply(qkv, bias, causal, sm_scale, slopes)
+    return FlashAttentionQKVPackedFn.apply(qkv, tensor_bias, causal, sm_scale, slopes)
 
 
 # --------------------------------------------------------------------------------------------
