@@ -188,3 +188,45 @@ def test_host_path_equals_the_autograd_classes(gpu_device):
         assert torch.equal(flash_attention_qkvpacked_fn(qkv, None, True), ours.detach() * 0 + flash_attention_qkvpacked_fn(qkv.detach(), None, True))
     with pytest.raises(ValueError):
         flash_attention_fn(qkv[:, :, 0], qkv[:, :5, 1], qkv[:, :5, 2], None, True)
+
+
+def test_host_path_with_hooks_views_and_transforms(gpu_device):
+    """What programs put around an autograd function: saved-tensor hooks whose tensors come back elsewhere or changed,
+    a bias written to before the backward, tracing and transforms.  (What a hook may hand back wrongly is turned into
+    an error on the host; nothing is launched for it.)"""
+    dev, g = gpu_device, torch.Generator().manual_seed(0)
+    B, S, H, D = 2, 75, 4, 64
+    rnd = lambda *s: torch.randn(*s, generator=g).bfloat16().to(dev)
+    q, k, v = (rnd(B, S, H, D).requires_grad_(True) for _ in range(3))
+    do, bias = rnd(B, S, H, D), rnd(H, S, S)
+    want = torch.autograd.grad(flash_attention_fn(q, k, v, bias), (q, k, v), do)
+    # through host memory and back, and as tensors of another layout
+    with torch.autograd.graph.save_on_cpu():
+        out = flash_attention_fn(q, k, v, bias)
+    for a, b in zip(torch.autograd.grad(out, (q, k, v), do), want):
+        assert torch.equal(a, b)
+    strided = lambda t: t.transpose(1, 2).contiguous().transpose(1, 2) if t.dim() == 4 and t.shape[-1] == D else t
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, strided):
+        out = flash_attention_fn(q, k, v, bias)
+    for a, b in zip(torch.autograd.grad(out, (q, k, v), do), want):
+        assert torch.equal(a, b)
+    for spoil in (lambda t: t.cpu(), lambda t: t[:, :7], lambda t: t.float() if t.dtype == torch.bfloat16 else t.bfloat16(),
+                  lambda t: t.cpu() if t.dim() == 3 else t, lambda t: t[0]):
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, spoil):
+            out = flash_attention_fn(q, k, v, bias)
+        with pytest.raises(ValueError):
+            out.backward(do)
+    # a bias with a missing dimension is read again by the backward, where the kernels can read it in place
+    bias = rnd(H, 1, S)
+    out = flash_attention_fn(q, k, v, bias)
+    bias.add_(1)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.backward(do)
+    # a trace runs the kernels on the inputs it is given later
+    call = lambda a, b, c: flash_attention_fn(a, b, c, None, True)
+    one, other = [rnd(B, S, H, D) for _ in range(3)], [rnd(B, S, H, D) for _ in range(3)]
+    traced = torch.jit.trace(call, one, check_trace=False)
+    assert torch.equal(traced(*other), call(*other))
+    # a transform is refused, also where it wraps none of the arguments
+    with pytest.raises(RuntimeError):
+        torch.func.vmap(lambda x: call(*one) * x)(rnd(3, 1))

@@ -225,9 +225,46 @@ struct AttentionNode : torch::autograd::Function<AttentionNode> {
         c.sm_scale = sm_scale;
         return c;
     }
+    // A saved tensor is whatever the unpack hook of a program hands back: every extent the kernels use is taken from
+    // q and k, so whatever else they read has to agree with them.
+    static void check_saved(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& o, const Tensor& lse, const Tensor& bias4,
+                            const Tensor& slopes, const Tensor& dout) {
+        const bool packed = !k.defined();
+        const auto dev = dout.device();
+        const auto dt = dout.scalar_type();
+        for (const Tensor* t : {&q, &k, &v, &o, &lse, &bias4, &slopes})
+            TORCH_CHECK_VALUE(!t->defined() || t->device() == dev, "flash_attention: all tensors must be on the same device");
+        TORCH_CHECK_VALUE(dev.type() == c10::DeviceType::CUDA && (dt == at::kHalf || dt == at::kBFloat16) &&
+                              (packed ? q.dim() == 5 && q.size(2) == 3 : q.dim() == 4 && k.dim() == 4 && v.dim() == 4),
+                          "flash_attention: a saved tensor came back with another shape");
+        const int64_t B = q.size(0), M = q.size(1), H = q.size(packed ? 3 : 2), d_qk = q.size(packed ? 4 : 3);
+        const int64_t N = packed ? M : k.size(1), d_v = packed ? d_qk : v.size(3);
+        auto expect = [&](const Tensor& t, const char* name, at::IntArrayRef shape, at::ScalarType type) {
+            TORCH_CHECK_VALUE(t.sizes() == shape && t.scalar_type() == type, name, " has shape ", t.sizes(), " and type ",
+                              t.scalar_type(), ", the kernels need ", shape, " and ", type);
+        };
+        expect(q, "q", packed ? at::IntArrayRef({B, M, 3, H, d_qk}) : at::IntArrayRef({B, M, H, d_qk}), dt);
+        if (!packed) {
+            expect(k, "k", {B, N, H, d_qk}, dt);
+            expect(v, "v", {B, N, H, d_v}, dt);
+        }
+        expect(o, "o", {B, M, H, d_v}, dt);
+        expect(dout, "do", {B, M, H, d_v}, dt);
+        expect(lse, "lse", {B, H, M}, at::kFloat);
+        TORCH_CHECK_VALUE(lse.is_contiguous(), "lse must be a dense float32 tensor of shape (B, H, M)");
+        if (slopes.defined()) expect(slopes, "slopes", {H}, at::kFloat);
+        if (bias4.defined()) {
+            const int64_t want[4] = {B, H, M, N};
+            bool fits = bias4.dim() == 4 && bias_kind(bias4) >= 0;
+            for (int i = 0; fits && i < 4; i++) fits = bias4.size(i) == want[i] || bias4.size(i) == 1;
+            TORCH_CHECK_VALUE(fits, "bias has shape ", bias4.sizes(), ", which does not broadcast to ", at::IntArrayRef(want, 4));
+        }
+    }
     static variable_list backward(AutogradContext* ctx, const variable_list& grads) {
         const variable_list saved = ctx->get_saved_variables();
-        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &o = saved[3], &lse = saved[4];
+        const Tensor &q = saved[0], &k = saved[1], &v = saved[2], &lse = saved[4];
+        check_saved(q, k, v, saved[3], lse, saved[5], saved[6], grads[0]);
+        const Tensor o = kernel_layout(saved[3]);
         const Call c = make(q, k, v, saved[5], saved[6], ctx->saved_data["causal"].toBool(), ctx->saved_data["sm_scale"].toDouble());
         const bool packed = !k.defined();
         // (the edges that exist are numbered in the order of the arguments)
@@ -280,6 +317,10 @@ std::optional<Tensor> unpack(PyObject* x) {
 py::object attention(py::handle q_, py::handle k_, py::handle v_, py::handle bias_, py::handle slopes_, py::handle causal_, py::handle scale_) {
     auto uq = unpack(q_.ptr()), uk = unpack(k_.ptr()), uv = unpack(v_.ptr()), ub = unpack(bias_.ptr()), us = unpack(slopes_.ptr());
     if (!uq || !uk || !uv || !ub || !us || !uq->defined() || c10::impl::dispatch_mode_enabled()) return py::none();
+    // a trace would not see the kernels; a transform is for the classes to refuse, whichever tensors it wraps
+    if (c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Tracer) ||
+        c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode))
+        return py::none();
     if (!PyBool_Check(causal_.ptr()) || !(scale_.is_none() || PyFloat_Check(scale_.ptr()))) return py::none();
     const Tensor q = *uq, k = *uk, v = *uv, bias = *ub, slopes = *us;
     const bool causal = causal_.ptr() == Py_True, packed = !k.defined();
@@ -323,7 +364,9 @@ py::object attention(py::handle q_, py::handle k_, py::handle v_, py::handle bia
     py::gil_scoped_release no_gil;
     Tensor out;
     {
-        at::AutoDispatchBelowADInplaceOrView below;  // views and copies of the bias are none of autograd's business
+        // (views and copies of the bias have no edges; but a view shares the version of the tensor it is taken from, so
+        // that the backward notices when that has been written to in the meantime)
+        at::AutoGradMode no_grad(false);
         if (bias.defined()) {
             bias4 = bias;
             if (bias.dim() < 4) {
