@@ -230,3 +230,43 @@ def test_host_path_with_hooks_views_and_transforms(gpu_device):
     # a transform is refused, also where it wraps none of the arguments
     with pytest.raises(RuntimeError):
         torch.func.vmap(lambda x: call(*one) * x)(rnd(3, 1))
+
+
+@pytest.mark.parametrize("kind", [None, "row", "bool", "dense", "alibi"])
+def test_few_rows_against_many_keys(gpu_device, kind):
+    """Few query tiles split their keys into up to 32 shares, short tiles into shares of 256 keys: both directions at
+    the edges of that rule (no share, two, ragged last ones, 32, and rounding that leaves fewer than asked for), with
+    whole shares behind the end of a sequence, masked by False or by a bias of -inf.  A dense bias takes the dQ
+    kernel that reads dS, split as well."""
+    g = torch.Generator().manual_seed(5)
+    for B, M, N, H, D in [(1, 1, 511, 2, 64), (1, 1, 513, 2, 128), (2, 7, 1111, 1, 32), (1, 1, 8191, 1, 128), (1, 16, 8448, 2, 64),
+                          (3, 130, 1700, 2, 128), (1, 256, 2049, 3, 16), (2, 257, 4096, 1, 64), (1, 5, 2304, 1, 256), (1, 64, 2560, 8, 128)]:
+        mk = lambda n: torch.randn(B, n, H, D, generator=g).bfloat16().to(gpu_device)
+        q, k, v, do = mk(M), mk(N), mk(N), mk(M)
+        bias, dense, grad_of = None, None, []
+        # (the last sequence ends inside the first share, and its last keys are whole masked shares)
+        ends = torch.tensor([N - 3] * (B - 1) + [max(1, min(200, N // 2))])
+        live = (torch.arange(N)[None] < ends[:, None])[:, None, None].to(gpu_device)
+        if kind == "row":
+            bias = dense = torch.zeros(B, 1, 1, N, device=gpu_device).masked_fill(~live, float("-inf"))
+        elif kind == "bool":
+            bias = dense = live
+        elif kind == "dense":
+            bias = torch.randn(B, H, M, N, generator=g).bfloat16().to(gpu_device).masked_fill(~live, float("-inf"))
+            # ... and one sequence starts with masked keys
+            bias[0, :, :, :min(300, N // 3) if B > 1 else 33] = float("-inf")
+            bias = dense = bias.requires_grad_(True)
+            grad_of = [bias]
+        elif kind == "alibi":
+            bias = AlibiBias(torch.linspace(0.01, 0.3, H).to(gpu_device))
+            dense = bias.materialize(M, N)
+        ins = [t.requires_grad_(True) for t in (q, k, v)]
+        out = flash_attention_fn(q, k, v, bias, False)
+        grads = torch.autograd.grad(out, ins + grad_of, do)
+        q, k, v = (t.detach() for t in ins)
+        full = None if dense is None else dense.detach().expand(B, H, M, N)
+        o, lse = attention_forward(q, k, v, full, False)
+        want = attention_backward(do, q, k, v, o, lse, full, False)[:3 + len(grad_of)]
+        assert (out.float() - o).abs().max().item() <= 2e-2, (kind, B, M, N, H, D)
+        for name, a, b in zip(("dq", "dk", "dv", "dbias"), grads, want):
+            assert rel_l2(a, b) <= 5e-2, (name, kind, B, M, N, H, D, rel_l2(a, b))

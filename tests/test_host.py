@@ -417,3 +417,26 @@ def test_abi_status_codes_and_workspace():
                               bias_dtype=0, causal=0, sm_scale=0.1)
     assert lib.fa_bwd_noalloc(ctypes.byref(big), None) == _native.FA_ERR_TOO_LARGE  # beyond the static scratch
     assert lib.fa_bwd_noalloc(None, None) == -1
+
+
+def test_key_shares_of_few_query_tiles():
+    """How many shares the forward splits its keys into (from the size of its scratch): at least two and at most 32, never
+    more than there are runs of 256 keys, nothing when the tiles are enough."""
+    lib = _native.load()
+    pad = lambda x: (x + 255) // 256 * 256
+
+    def shares(B, H, M, N, D, bias=0):
+        p = _native.FaProblem(B=B, H=H, M=M, N=N, D=D, dtype=_native.FA_BF16, bias_dtype=bias, causal=0, sm_scale=0.1)
+        size = lib.fa_fwd_workspace_bytes(ctypes.byref(p))
+        rows = B * H * M
+        return 1 if size == 0 else [s for s in range(2, 64) if pad(s * rows * D * 4) + pad(s * rows * 4) == size]
+
+    for bias in (0, 1, 3, 5):
+        assert shares(1, 8, 1, 448, 64, bias) == 1 and shares(1, 8, 1, 512, 64, bias) == [2]
+        assert shares(1, 8, 1, 65536, 128, bias) == [32]
+        assert shares(8, 16, 1, 4097, 128, bias) == [4] and shares(32, 16, 1, 4097, 128, bias) == 1
+        for N in range(200, 9000, 97):
+            n = shares(1, 2, 3, N, 64, bias)
+            assert n == 1 or (len(n) == 1 and 2 <= n[0] <= 32 and (n[0] - 1) * 256 < N), (bias, N, n)
+    assert shares(1, 8, 1, 2048, 64) == [8]
+    assert shares(2, 8, 1024, 1024, 64) == 1     # long tiles: shares of at least 16 steps

@@ -206,8 +206,14 @@ int compute_units() {
 }
 
 // Keys of a query tile split between work-groups when the query tiles alone leave the GPU half empty
-// (fewer than two work-groups per CU): as many splits as it takes to get there, at most four, each
-// with at least 16 steps of the K/V stream.  The answer depends on the current device (its CU
+// (fewer than two work-groups per CU): as many splits as it takes to get there, each with at least 16
+// steps of the K/V stream.  A few short tiles (at most one per four CUs, at most 256 query rows) go down
+// to shares of 256 keys: their shares of the output are small next to the keys that they have read, and without
+// that a token decoded against a long cache runs on a handful of CUs.  Beyond 32 shares the merge costs more than the
+// last of them bring.  One query row, D = 128, us per call, at most 4 shares of at least 16 steps / this rule / 64 shares
+// allowed: B=1 H=8 N=1024 19.2 / 11.9 / 11.9, N=4096 22.8 / 15.4 / 15.4, N=16384 87 / 30 / 38.  Where the line lies: 256 keys
+// at 256 tiles (B=16 H=16 N=700 D=64) 16.0 -> 18.5, at 1024 rows (B=2 H=8 M=N=1024 D=64) 14.8 -> 18.2.
+// The answer depends on the current device (its CU
 // count): a size query and the launch it sizes must run with the same device current.
 struct FwdSplit {
     int n_splits, keys_per_split;
@@ -220,10 +226,12 @@ FwdSplit fwd_split(const fa_problem& p) {
     const int bk = p.bias_dtype == FA_BIAS_NONE ? 64 : 32;  // keys per step of the forward kernel
     const int n_steps = (p.N + bk - 1) / bk;
     int s = (int)(full / wgs);
-    s = s > 4 ? 4 : s;
-    while (s > 1 && n_steps / s < 16) s--;
+    s = s > 32 ? 32 : s;
+    const int min_steps = p.M <= 256 && 8 * wgs <= full ? 256 / bk : 16;
+    while (s > 1 && n_steps / s < min_steps) s--;
     if (s <= 1) return {1, 0};
-    return {s, ((n_steps + s - 1) / s * bk + 63) / 64 * 64};  // whole steps of either kernel tiling
+    const int keys = ((n_steps + s - 1) / s * bk + 63) / 64 * 64;  // whole steps of either kernel tiling
+    return {(p.N + keys - 1) / keys, keys};                        // (rounded up, they may need fewer shares: none is empty)
 }
 
 // the shares of dq of a dQ kernel that splits its keys like the forward (0 when it does not)

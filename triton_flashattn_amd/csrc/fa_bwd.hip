@@ -414,6 +414,7 @@ template <typename T, int D> __global__ __launch_bounds__(256) void fa_bwd_dq_su
     const int c = (int)(idx % TPR);
     if (row >= rows || c * 8 >= p.d_qk) return;
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
     for (int s = 0; s < p.dq_splits; s++) {
         const float* src = reinterpret_cast<const float*>(p.part_dq) + (s * rows + row) * D + c * 8;
         const f32x4 lo = *reinterpret_cast<const f32x4*>(src), hi = *reinterpret_cast<const f32x4*>(src + 4);
@@ -1402,10 +1403,12 @@ template <typename T, int D> static hipError_t launch_all(const BwdParams& p, in
     // launch and a pass over o and do; the dK/dV kernel then reads the delta it has stored.
     const bool dq_first = (stages & 5) == 5 && !from_ds;
     auto launch_dq = [&](bool makes_delta) -> hipError_t {
-        // the one-product form runs at the rate of the dS stream and gains nothing from more work-groups
+        // The one-product form runs at the rate of the dS stream: it gains from more work-groups only where the tiles
+        // leave half of the CUs without one, that is where they are split in four or more (D = 128, H=8, N=8192, whole training
+        // step, ms: M=64 0.153 -> 0.079, M=512 0.204 -> 0.154; one tile per CU, H=32 M=1024: this kernel 0.137 -> 0.161).
         BwdParams pq = p;
         pq.dq_makes_delta = makes_delta ? 1 : 0;
-        if (from_ds) pq.dq_splits = 1;
+        if (from_ds && pq.dq_splits < 4) pq.dq_splits = 1;
         dim3 qgrid((unsigned)(pq.n_mtiles * pq.dq_splits * pq.B * pq.H));
         if (from_ds && bias == DS_BIAS) {
             if (causal) hipLaunchKernelGGL((fa_bwd_dq_kernel<T, D, DS_BIAS, true, true>), qgrid, dim3(256), 0, st, pq);

@@ -103,7 +103,9 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
     }
 
     const float qk_scale = p.sm_scale * kLog2e;
-    float m_i = -INFINITY, l_i = 0.f;
+    // (the lowest number, not -inf: keys whose bias is -inf then have exponentials of 0 also where no other key has been
+    // seen yet, as in a share of the keys that is padding from end to end)
+    float m_i = -3.402823466e38f, l_i = 0.f;
     f32x16 o_acc[C::DB];
 #pragma unroll
     for (int db = 0; db < C::DB; db++)
@@ -265,9 +267,8 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
         // steps skip the mask terms and fold the scale into the exponent.
         // The reference point m_i of the exponentials is arbitrary (out = acc / l and LSE = m + log2 l do
         // not depend on it), so no running maximum is kept: the exponentials are taken against the m_i at
-        // hand, and only when the sum of a lane's 8 or 16 of them exceeds kRaise (or is no number, as at
-        // the first keys, where m_i is -inf) is m_i raised to the maximum, O rescaled and they are taken
-        // again.  The test is one comparison on a sum that is needed anyway.
+        // hand, and only when the sum of a lane's 8 or 16 of them exceeds kRaise (as at the first keys, where m_i is
+        // the lowest number) or is no number is m_i raised to the maximum, O rescaled and they are taken again.  The test is one comparison on a sum that is needed anyway.
         auto softmax_step = [&](auto masked_tag) {
             constexpr bool MASKED = decltype(masked_tag)::value;
             // units of s[i] below: raw dot product (no bias), natural (float bias), log2 (MASKED, bool masks)
@@ -412,9 +413,10 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
 
     // ---- epilogue (flash_attention.py:188-194) ----
     const float l_tot = pair_sum(l_i);
-    const float inv_l = 1.f / l_tot;
-    // one of several shares of the keys: output and LSE go to this share's slice of the scratch
+    // one of several shares of the keys: output and LSE go to this share's slice of the scratch (a share without a
+    // visible key: zeros, and an LSE of -inf, which gives it no weight)
     const bool shared = p.n_splits > 1;
+    const float inv_l = shared && l_tot == 0.f ? 0.f : 1.f / l_tot;
     float* lse_out = shared ? p.part_lse + ((int64_t)split * p.B * p.H + bh) * M : p.lse + ((int64_t)b * p.H + h) * M;
     // (the row index passes through an empty asm so that the store address is formed here and not
     // kept in two registers across the loops)
@@ -473,12 +475,16 @@ template <typename T, int D> __global__ __launch_bounds__(256) void fa_fwd_merge
     const int64_t row = idx / TPR;
     const int c = (int)(idx % TPR);
     if (row >= rows || c * 8 >= p.d_v) return;
+    // (unrolled: up to 32 shares, whose loads would be a chain of latencies)
     float mx = -INFINITY;
+#pragma unroll 8
     for (int s = 0; s < p.n_splits; s++) mx = fmaxf(mx, p.part_lse[s * rows + row]);
     float sum = 0.f;
+#pragma unroll 8
     for (int s = 0; s < p.n_splits; s++) sum += fast_exp2(p.part_lse[s * rows + row] - mx);
     const float lse = mx + fast_log2(sum);
     float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
     for (int s = 0; s < p.n_splits; s++) {
         const float w = fast_exp2(p.part_lse[s * rows + row] - lse);
         const float* src = reinterpret_cast<const float*>(p.part_o) + (s * rows + row) * D + c * 8;
