@@ -352,8 +352,11 @@ template <int D, int BIAS> struct StreamCfg {
     __device__ static __forceinline__ int bswz(int row) {
         return ES == 4 ? ((row >> 1) & 7) : (ES == 2 ? ((row >> 2) & 3) : ((row >> 3) & 1));
     }
-    // two work-groups per CU whenever registers and LDS allow it
-    static constexpr int MIN_BLOCKS = (D <= 128 && LDS_BYTES <= 81920) ? 2 : 1;
+    // two work-groups per CU whenever registers and LDS allow it, three with a byte mask up to head dim 64: a step of such
+    // a kernel is short next to its waits, and three of its rings fit LDS (those of a 16-bit bias do not).  D = 64, us, two
+    // -> three: forward B=8 H=12 S=1024 51.7 -> 47.6, B=16 H=8 S=2048 250 -> 238; forward and backward, causal, B=8 H=12
+    // S=1024 144.7 -> 140.4.  (Head dims up to 32 stayed below 168 registers on their own: no change.)
+    static constexpr int MIN_BLOCKS = D <= 64 && BIAS == 1 ? 3 : (D <= 128 && LDS_BYTES <= 81920) ? 2 : 1;
 };
 
 // The copy machinery of the kernels tiled by StreamCfg (forward, dQ): one object per thread.
@@ -604,7 +607,7 @@ template <typename T, int D, int BIAS, bool WITH_V = true> struct KeyStream {
                     }
                 }
             } else {
-                constexpr int RB = D >= 128 ? 4 : 16;  // as many as the registers of the kernel allow
+                constexpr int RB = D >= 128 ? 4 : (D == 64 && BIAS == 1 ? 8 : 16);  // as many as the registers of the kernel allow (16: 190 at D = 64)
                 const int key = lane & 31;
                 int n = k * C::BK + key;
                 n = n < N ? n : N - 1;
