@@ -208,6 +208,31 @@ def test_broadcast_bias_and_reduced_gradient(oracle_backend):
         assert all(st == 0 for st, n, w in zip(fwd_call[2], (1,) * (4 - bias.dim()) + tuple(shape), (B, H, M, N)) if n == 1 and w > 1)
 
 
+def test_gradient_of_a_bias_of_every_broadcast_shape(oracle_backend):
+    """Every combination of full and size-1 dimensions.  One value for all keys of a row has no gradient buffer that
+    the kernels could write (its keys would share one address): the forward takes such a bias, the backward raises."""
+    q, k, v = _qkv()
+    B, M, N, H = 2, 6, 9, 2
+    do = torch.randn(B, M, H, 16).bfloat16()
+    for mask in range(16):
+        full = tuple(s if mask >> i & 1 else 1 for i, s in enumerate((B, H, M, N)))
+        for shape in {full[i:] for i in range(4) if all(s == 1 for s in full[:i])}:
+            ins = [t.clone().requires_grad_(True) for t in (q, k, v)]
+            bias = torch.randn(shape).bfloat16().requires_grad_(True)
+            for call in (flash_attention_fn, flash_attention_op):
+                out = call(*ins, bias) if call is flash_attention_fn else call(*[t.clone() for t in ins], bias)
+                oracle_backend.calls.clear()
+                if shape[-1] == 1:
+                    with pytest.raises(RuntimeError, match="size 1 along the keys"):
+                        torch.autograd.grad(out, bias, do)
+                    assert oracle_backend.calls == []
+                    continue
+                got = torch.autograd.grad(out, bias, do)[0]
+                want = reference_grads(q, k, v, bias.detach().expand(B, H, M, N), do, False, 16 ** -0.5)["dbias"]
+                want = want.sum_to_size((1,) * (4 - len(shape)) + tuple(shape)).reshape(shape)
+                assert got.shape == bias.shape and torch.allclose(got.float(), want, atol=3e-2, rtol=3e-2), shape
+
+
 def test_alibi_bias_matches_materialized(oracle_backend):
     B, M, N, H, D = 1, 8, 16, 4, 16
     q, k, v = _qkv(B, M, N, H, D)
@@ -409,7 +434,11 @@ def test_abi_status_codes_and_workspace():
     assert lib.fa_bwd(ctypes.byref(b), None) == -6            # no workspace
     b.dbias = base
     assert lib.fa_bwd(ctypes.byref(b), None) == -4            # dbias without a float bias
-    b.dbias = None
+    b.bias, b.p.bias_dtype = base, _native.FA_BIAS_BF16
+    for strides in ((1200, 400, 4, 0), (0, 400, 4, 0), (0, 0, 0, 0)):   # a gradient whose keys share one address
+        b.dbias_strides[:] = strides
+        assert lib.fa_bwd(ctypes.byref(b), None) == -5, strides
+    b.bias, b.dbias, b.p.bias_dtype = None, None, _native.FA_BIAS_NONE
     assert lib.fa_bwd_stages(ctypes.byref(b), None, 16) == -7                       # unknown stage bit
     assert lib.fa_bwd_stages(ctypes.byref(b), None, _native.FA_STAGE_DQ_FROM_DBIAS) == -7   # modifier alone
     big = _native.FaBwdArgs()

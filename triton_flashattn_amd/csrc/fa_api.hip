@@ -248,8 +248,8 @@ int dbias_mode(const fa_bwd_args* a) {
     if (p.bias_dtype == FA_BIAS_ALIBI) return 2;
     const int64_t* s = a->dbias_strides;
     const bool red_b = p.B > 1 && s[0] == 0, red_h = p.H > 1 && s[1] == 0, red_m = p.M > 1 && s[2] == 0;
+    if (p.N > 1 && s[3] == 0) return -1;  // nothing sums over the keys: they would all store to one address
     if (!red_b && !red_h && !red_m) return 1;
-    if (p.N > 1 && s[3] == 0) return -1;
     if (!red_m && p.M > 1) {
         // the bias itself must be the one that is shared: its tile is read once for all pairs
         return (red_b && a->bias_strides[0] != 0) || (red_h && a->bias_strides[1] != 0) ? -1 : 3;

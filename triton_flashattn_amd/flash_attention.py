@@ -397,7 +397,11 @@ def _flash_attn_bwd(do, q, k, v, o, bias, causal, sm_scale, lse, dq, dk, dv, dbi
 
 def _bias_grad_like(bias, B, H, M, N):
     """The tensor that the kernels write the gradient of `bias`, the 4-D view of the caller's, into.  One that is
-    broadcast over the query rows, or over batches or heads, is summed over them in the kernels."""
+    broadcast over the query rows, or over batches or heads, is summed over them in the kernels; one with a single
+    value for all keys of a row is refused (nothing sums over the keys)."""
+    if bias.shape[3] != N:
+        raise RuntimeError("the gradient of a bias of size 1 along the keys is not supported: expand it to %d keys "
+                           "(bias shape %s)" % (N, tuple(bias.shape)))
     if tuple(bias.shape) == (B, H, M, N):
         return _empty_padded_rows(bias.shape, bias.dtype, bias.device)
     return torch.empty(bias.shape, dtype=bias.dtype, device=bias.device)
