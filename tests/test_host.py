@@ -4,6 +4,7 @@ above the C ABI runs without a GPU; nothing here launches a kernel."""
 import ctypes
 import os
 import re
+import subprocess
 
 import pytest
 import torch
@@ -469,3 +470,34 @@ def test_key_shares_of_few_query_tiles():
             assert n == 1 or (len(n) == 1 and 2 <= n[0] <= 32 and (n[0] - 1) * 256 < N), (bias, N, n)
     assert shares(1, 8, 1, 2048, 64) == [8]
     assert shares(2, 8, 1024, 1024, 64) == 1     # long tiles: shares of at least 16 steps
+
+
+def test_order_of_a_causal_grid(tmp_path):
+    """The order is a permutation; a kernel that fits one work-group to a CU takes its tiles longest first whatever the
+    grid (a list schedule that ends later leaves the chip idle); two to a CU, the sums of the pairs are as even as
+    can be."""
+    src, exe = tmp_path / "order.cpp", tmp_path / "order"
+    src.write_text('''
+#include <cstdio>
+#include <initializer_list>
+#include "%s"
+int main() {
+    for (int per_cu = 1; per_cu <= 3; per_cu++)
+        for (int n : {1, 31, 32, 33, 48, 63, 64, 65, 200}) {
+            for (int slot = 0; slot < n; slot++) std::printf("%%d ", fa::causal_place(slot, n, 32, per_cu));
+            std::printf("\\n");
+        }
+}
+''' % os.path.join(ROOT, "triton_flashattn_amd", "csrc", "fa_order.hpp"))
+    subprocess.run(["g++", "-std=c++17", str(src), "-o", str(exe)], check=True)
+    lines = subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.splitlines()
+    orders = [[int(x) for x in line.split()] for line in lines]
+    for i, order in enumerate(orders):
+        per_cu, n = i // 9 + 1, len(order)
+        assert sorted(order) == list(range(n))
+        if per_cu == 1 or n <= 32 or n > 64:
+            assert order == list(range(n)), (per_cu, n)
+        else:
+            # place x has n - x units of work; work-groups i and 32 + i share CU i
+            load = [n - order[c] + (n - order[32 + c] if 32 + c < n else 0) for c in range(32)]
+            assert max(load) <= n + 1, (n, load)

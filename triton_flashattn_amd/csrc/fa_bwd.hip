@@ -80,7 +80,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
     const int r = lane & 31, g = lane >> 5;
 
     int mt, bh;
-    decode_block<CAUSAL, CAUSAL>(blockIdx.x, p.n_mtiles * p.dq_splits, p.B * p.H, mt, bh);
+    decode_block<CAUSAL, C>(blockIdx.x, p.n_mtiles * p.dq_splits, p.B * p.H, mt, bh);
     // With the keys split between work-groups (never when causal) this one sees keys key0 ..
     // key0 + N - 1 as if they were all there are (its dq is a share, summed afterwards); only ALiBi
     // needs to know better.

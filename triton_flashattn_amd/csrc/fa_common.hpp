@@ -11,6 +11,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "fa_order.hpp"
+
 namespace fa {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -652,16 +654,13 @@ template <typename T, int D, int BIAS, bool WITH_V = true> struct KeyStream {
 // comes before tile t + 1 of any; the causal kernels, whose tiles are numbered longest first,
 // so start all long tiles before any short one (a greedy schedule with the longest jobs first
 // ends near the average load, one that mixes them ends up to one long tile later).
-// PAIRED (with TILE_MAJOR, two work-groups to a CU): a grid of at most two work-groups per CU starts all at
-// once, so its order does not balance it but decides which two tiles share a CU: the first 256 are the longest,
-// longest first, the others follow shortest first (forward at B=1 H=16 M=N=4096 D=128: 0.086 -> 0.083 ms, at B=4 H=8
-// M=N=1024 D=64 dQ 0.025 -> 0.023; a larger grid is balanced by its order).
-template <bool TILE_MAJOR = false, bool PAIRED = false>
+// CFG (with TILE_MAJOR): the kernel's configuration, whose MIN_BLOCKS work-groups fit a CU (causal_place).
+struct OnePerCu { static constexpr int MIN_BLOCKS = 1; };
+template <bool TILE_MAJOR = false, typename CFG = OnePerCu>
 __device__ __forceinline__ void decode_block(int id, int n_tiles, int BH, int& tile, int& bh) {
     if ((BH & 7) == 0) {
         const int xcd = id & 7, per_xcd = BH >> 3;
-        int slot = id >> 3;
-        if (PAIRED && n_tiles * per_xcd <= 64 && slot >= 32) slot = n_tiles * per_xcd + 31 - slot;
+        const int slot = causal_place(id >> 3, n_tiles * per_xcd, kCusPerXcd, TILE_MAJOR ? CFG::MIN_BLOCKS : 1);
         if (TILE_MAJOR) {
             tile = slot / per_xcd;
             bh = (slot % per_xcd) * 8 + xcd;
@@ -670,7 +669,7 @@ __device__ __forceinline__ void decode_block(int id, int n_tiles, int BH, int& t
             tile = slot % n_tiles;
         }
     } else if (TILE_MAJOR) {
-        if (PAIRED && n_tiles * BH <= 512 && id >= 256) id = n_tiles * BH + 255 - id;
+        id = causal_place(id, n_tiles * BH, kXcds * kCusPerXcd, CFG::MIN_BLOCKS);
         tile = id / BH;
         bh = id % BH;
     } else {

@@ -57,7 +57,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
     const int r = lane & 31, g = lane >> 5;
 
     int mt, bh;
-    decode_block<CAUSAL, CAUSAL>(blockIdx.x, p.n_mtiles * p.n_splits, p.B * p.H, mt, bh);
+    decode_block<CAUSAL, C>(blockIdx.x, p.n_mtiles * p.n_splits, p.B * p.H, mt, bh);
     // With the keys split between work-groups (never when causal) this one sees keys key0 ..
     // key0 + N - 1 as if they were all there are; only ALiBi needs to know better.
     const int split = mt % p.n_splits;
