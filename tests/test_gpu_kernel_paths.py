@@ -39,6 +39,34 @@ def test_forward_reference_point_of_growing_scores(gpu_device, D, dtype):
         assert err <= 2e-2, (slope, N, causal, bias_kind, err)
 
 
+@pytest.mark.parametrize("D", [16, 32, 64, 128, 256])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_forward_of_biases_that_grow_along_the_keys(gpu_device, D, dtype):
+    """The rules for raising the reference point under a distance penalty: rows that grow in every block, in every few,
+    up to the diagonal and down behind it, all the way or not at all, with a ragged last step and rows that start masked."""
+    g = torch.Generator().manual_seed(D)
+    H = 6
+    slopes = torch.tensor([3.0, 0.7, 0.2, 0.05, 0.0, -0.5])
+    for M, N, causal in [(333, 333, True), (256, 256, True), (150, 1000, False), (130, 321, False)]:
+        q, k, v = (torch.randn(1, n, H, D, generator=g).to(dtype).to(gpu_device) for n in (M, N, N))
+        penalty = AlibiBias(slopes.abs().to(gpu_device))
+        dist = penalty.materialize(M, N)
+        row = slopes[None, :, None, None].to(gpu_device) * torch.arange(N, device=gpu_device)
+        masked = dist.clone()
+        masked[..., :70] = float("-inf")
+        if causal:
+            masked[..., torch.arange(M) < 70, 0] = 0.0
+        for name, bias, dense in [("alibi", penalty, dist), ("tensor", dist.to(dtype), dist.to(dtype)), ("fp32", dist, dist),
+                                  ("row", row, row), ("row16", row.to(dtype), row.to(dtype)), ("masked", masked, masked)]:
+            with torch.no_grad():
+                out = flash_attention_fn(q, k, v, bias, causal)
+            ref, _ = attention_forward(q, k, v, dense.expand(1, H, M, N), causal)
+            # biases reach 3000: a bias times log2 e and its fp32 sum with the score are off by 2^-12 at most, a weight by
+            # 2e-4, the output (values up to 4.5) by 1e-3 and by its own rounding
+            err = (out.float() - ref).abs().max().item()
+            assert err <= 2e-2, (name, M, N, causal, err)
+
+
 def rel_l2(a, b):
     """||a - b|| / ||b||, measured against an RMS floor of 1e-3 where the reference is zero up to rounding."""
     return ((a.float() - b).norm() / b.norm().clamp_min(1e-3 * b.numel() ** 0.5)).item()

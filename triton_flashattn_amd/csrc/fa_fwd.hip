@@ -26,14 +26,35 @@
 
 namespace fa {
 
-// The K/V stream of a row-broadcast bias (kinds 6, 7) is tiled like that of ALiBi, in steps of 32
-// keys: the bias values of a block need the registers that 64-key steps spend on a second block of
-// scores.
 // Sum of a lane's exponentials of a block (or half of one) beyond which their reference point is raised: far from what overflows the
 // element type of P and the fp32 accumulators, and high, so that scores that grow along the keys (a distance
 // penalty on the way to the diagonal) raise it seldom.
 template <typename T> constexpr float kRaise = __is_same(T, _Float16) ? 0x1p14f : 0x1p32f;
 
+// Biases that grow along the keys block after block (a distance penalty: ALiBi, its tensor, slope * key index in a
+// row-broadcast bias).  Taking the exponentials first and again once their sum is over the limit then costs a second set
+// of them per raise, in the heads with steep slopes in every block.
+//   kRowMax  the maximum of each block is formed first, and the reference point raised when it lies 2^8 above: ALiBi, where
+//            every row grows towards its diagonal: causal, and where a block's matrix work is small next to it (D <= 64).
+//   kAfter   the maximum is formed first in the block that follows a raise, as long as that raises again.  Not where the
+//            branch itself costs more than it saves: it takes 2 to 5 % from the causal kernels of a bias tile up to D = 128
+//            and from the row-broadcast ones at 128.
+//   kSum     neither.
+// Forward, us, kSum -> the rule here (B=2 H=16 M=N=2048 or, marked *, B=1 H=16 M=N=4096):
+//   ALiBi causal D=32* 93.2 -> 71.4, D=64* 94.3 -> 82.4, D=128* 120.1 -> 112.8; not causal D=32 60.7 -> 54.0, D=64 72.0 -> 64.1,
+//   D=128 95.7 -> 93.1, M=1024 N=8192 H=32 173 -> 170; as a bf16 tensor D=32 67.1 -> 61.6, fp16 D=64 74.0 -> 67.4, causal
+//   D=256 175 -> 166; slope * key as a row D=32 60.7 -> 56.8, causal B=8 D=64 115.3 -> 107.9.  Biases without a trend lose at most
+//   2 % (row-broadcast not causal D=32 79.3 -> 80.7*, D=64 97.8 -> 99.3*).
+enum Growth { kSum, kAfter, kRowMax };
+constexpr Growth growth_rule(int bias, int D, bool causal) {
+    return bias == 5 && (causal || D <= 64)                               ? kRowMax
+           : (bias >= 2 && bias <= 5 && !(causal && D <= 128)) || (bias == 6 && D != 128) ? kAfter
+                                                                                          : kSum;
+}
+
+// The K/V stream of a row-broadcast bias (kinds 6, 7) is tiled like that of ALiBi, in steps of 32
+// keys: the bias values of a block need the registers that 64-key steps spend on a second block of
+// scores.
 constexpr int fwd_stream_kind(int bias) { return bias >= 5 ? 6 : bias; }
 
 template <typename T, int D, int BIAS, bool CAUSAL>
@@ -57,7 +78,9 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
     const int r = lane & 31, g = lane >> 5;
 
     int mt, bh;
-    decode_block<CAUSAL, C>(blockIdx.x, p.n_mtiles * p.n_splits, p.B * p.H, mt, bh);
+    // (ALiBi, and a row-broadcast bias up to D = 64: longest first in any grid, pairing took 4 to 8 % from them)
+    constexpr bool PAIRS = !(BIAS == 5 || (BIAS == 6 && D <= 64));
+    decode_block<CAUSAL, typename std::conditional<PAIRS, C, OnePerCu>::type>(blockIdx.x, p.n_mtiles * p.n_splits, p.B * p.H, mt, bh);
     // With the keys split between work-groups (never when causal) this one sees keys key0 ..
     // key0 + N - 1 as if they were all there are; only ALiBi needs to know better.
     const int split = mt % p.n_splits;
@@ -106,6 +129,8 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
     // (the lowest number, not -inf: keys whose bias is -inf then have exponentials of 0 also where no other key has been
     // seen yet, as in a share of the keys that is padding from end to end)
     float m_i = -3.402823466e38f, l_i = 0.f;
+    constexpr Growth GROWTH = growth_rule(BIAS, D, CAUSAL);
+    bool rising = GROWTH == kRowMax;  // (the same in every lane) the next block's maximum is formed before its exponentials
     f32x16 o_acc[C::DB];
 #pragma unroll
     for (int db = 0; db < C::DB; db++)
@@ -334,6 +359,15 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
             // are computed (head dim 256: all 32 at once, there are no registers for a second copy of the
             // rescaling) ----
             constexpr int PARTS = D <= 128 ? 2 : 1, PL = 16 / PARTS;
+            if (GROWTH != kSum && rising) {
+                float mx = -INFINITY;
+#pragma unroll
+                for (int i = 0; i < 16; i++) mx = fmaxf(mx, s[i]);
+                mx = pair_max(mx) * to_log2;
+                const bool higher = __builtin_amdgcn_ballot_w64(mx > m_i + 8.f) != 0;
+                if (higher) raise(mx);
+                if (GROWTH == kAfter) rising = higher;
+            }
 #pragma unroll
             for (int part = 0; part < PARTS; part++) {
                 float pv[PL], rs;
@@ -348,12 +382,13 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
                     }
                 };
                 exps();
-                if (__builtin_amdgcn_ballot_w64(!(rs <= kRaise<T>)) != 0) {
+                if (GROWTH != kRowMax && __builtin_amdgcn_ballot_w64(!(rs <= kRaise<T>)) != 0) {
                     float mx = -INFINITY;
 #pragma unroll
                     for (int i = part * PL; i < 16; i++) mx = fmaxf(mx, s[i]);
                     raise(pair_max(mx) * to_log2);
                     exps();
+                    if (GROWTH == kAfter) rising = true;
                 }
                 l_i += rs;  // per-lane partial sum; the two halves of a row are added at the end
 #pragma unroll
