@@ -148,6 +148,35 @@ def test_gradient_of_a_shared_bias(gpu_device, D):
             assert rel_l2(a, b) <= 5e-2, (name, shape, B, H, causal, rel_l2(a, b))
 
 
+@pytest.mark.parametrize("D", [16, 32, 64, 128, 256])
+def test_pairs_that_share_a_bias(gpu_device, D):
+    """The walk over the (batch, head) pairs of a tile: several pairs to a work-group, over heads and batches, shares that
+    start in the middle of a batch, an empty last share, one, two and three pairs without shares; rows that are accessed
+    four elements at a time and rows that are not (odd lengths, a padded pitch, transposed)."""
+    g = torch.Generator().manual_seed(D)
+    cases = [((1, 1, 300, 300), 6, 8, torch.bfloat16, True), ((300, 300), 3, 16, torch.float32, False),
+             ((2, 1, 260, 200), 2, 24, torch.bfloat16, False), ((1, 8, 300, 300), 7, 8, torch.float32, False),
+             ((1, 16, 300, 200), 3, 16, torch.float16, False), ((1, 24, 260, 129), 2, 24, torch.bfloat16, False),
+             ((3, 1, 1000, 310), 3, 2, torch.bfloat16, False), ((1, 33, 130, 257), 4, 33, torch.float32, False)]
+    for i, (shape, B, H, bias_dtype, causal) in enumerate(cases):
+        M, N = shape[-2:]
+        dtype = torch.float16 if bias_dtype == torch.float16 else torch.bfloat16
+        mk = lambda n: torch.randn(B, n, H, D, generator=g).to(dtype).to(gpu_device).requires_grad_(True)
+        q, k, v, do = mk(M), mk(N), mk(N), mk(M).detach()
+        bias = torch.randn(shape, generator=g).to(bias_dtype).to(gpu_device)
+        if i % 3 == 1:
+            bias = torch.nn.functional.pad(bias, (0, 4))[..., :N]
+        elif i % 3 == 2:
+            bias = bias.transpose(-1, -2).contiguous().transpose(-1, -2)
+        bias.requires_grad_(True)
+        got = torch.autograd.grad(flash_attention_fn(q, k, v, bias, causal), bias, do)[0]
+        full = bias.detach().expand(B, H, M, N)
+        o, lse = attention_forward(q.detach(), k.detach(), v.detach(), full, causal)
+        want = attention_backward(do, q.detach(), k.detach(), v.detach(), o, lse, full, causal)[3].sum_to_size(shape)
+        # (the terms are rounded once each, in the products: the sum over the pairs adds no error of its own)
+        assert got.shape == want.shape and rel_l2(got, want) <= 2e-2, (shape, B, H, causal, rel_l2(got, want))
+
+
 @pytest.mark.parametrize("d_qk,d_v", [(8, 8), (24, 24), (40, 56), (80, 80), (96, 40), (72, 120), (64, 128)])
 def test_head_dims_below_the_kernels(gpu_device, d_qk, d_v):
     """Head dims that are whole 16-byte chunks run at the next head dim of the kernels without padded copies: both

@@ -168,6 +168,13 @@ bool bias_vec_ok(const void* ptr, const int64_t s[4], const fa_problem& p) {
     return true;
 }
 
+// rows of bias or dbias may be accessed four elements at a time, at multiples of four
+bool bias_quads_ok(const void* ptr, const int64_t s[4], const fa_problem& p) {
+    const int es = bias_elem_size(p.bias_dtype);
+    return es > 1 && s[3] == 1 && reinterpret_cast<uintptr_t>(ptr) % (4 * es) == 0 && (p.B == 1 || s[0] % 4 == 0) &&
+           (p.H == 1 || s[1] % 4 == 0) && (p.M == 1 || s[2] % 4 == 0);
+}
+
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // With FA_MI355_VERBOSE set in the environment, says once per process on stderr when a bias cannot
@@ -460,7 +467,11 @@ int bwd_enqueue(const fa_bwd_args* a, int d_qk, int d_v, void* stream, int stage
     k.waves_per_role = bn / 32;
     k.n_mtiles = (p.M + fa::fwd_block_m() - 1) / fa::fwd_block_m();
     k.causal = p.causal != 0; k.bias_kind = p.bias_dtype; k.shared_splits = splits;
-    k.shared_tiles = db_mode == 3 ? (int)shared_tiles(a) : 0;
+    if (db_mode == 3) {
+        k.shared_tiles = (int)shared_tiles(a);
+        k.bias_quads = bias_quads_ok(a->bias, a->bias_strides, p) ? 1 : 0;
+        k.dbias_quads = bias_quads_ok(a->dbias, a->dbias_strides, p) ? 1 : 0;
+    }
     hipError_t e = fa::launch_bwd(k, p.D, p.dtype, p.bias_dtype, p.causal != 0, db_mode, stages,
                                   static_cast<hipStream_t>(stream));
     if (e == hipSuccess && db_mode == 3 && need_dkv) e = fa::launch_bwd_shared(k, p.D, p.dtype, static_cast<hipStream_t>(stream));

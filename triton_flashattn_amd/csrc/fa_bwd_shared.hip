@@ -15,7 +15,13 @@
 // between work-groups, whose shares in fp32 a second kernel adds in a fixed order.
 // Measured: 32 batches, 12 heads, M=N=197, D=64, fp32 table: 0.023 ms and 0.005 for the shares; 24 batches, 16 heads,
 // M=N=577: 0.122 ms (0.167 with addresses formed from the indices and every copy behind the barrier).  Before, one
-// backward per batch with its dS written and added up: the whole training step at 32 batches took 2.1 ms, now 0.26.
+// backward per batch with its dS written and added up: the whole training step at 32 batches took 2.1 ms, now 0.11.
+// Few pairs: a tile then costs what stands around its pairs.  With the bias and the gradient accessed one element at a
+// time, each load behind the one before, and products formed for a pair behind the last that was 10 us of a tile at
+// D = 128 (2 us per pair); whole training steps with bf16 tables, two batches, us, one backward per batch / that / now:
+// H=16 M=N=4096 D=64 2575 / 2734 / 1868, H=16 M=N=2048 D=128 723 / 849 / 616, causal 698 / 550 / 389, D=256 causal
+// 860 / 972 / 731, D=256 1106 / 1594 / 1318: there the four slices of a pair are what bounds it, 1.5 us each, whatever
+// the order of their copies, products and tiles.
 #include "fa_common.hpp"
 #include "fa_params.hpp"
 
@@ -36,18 +42,45 @@ template <int D> struct SharedCfg {
     static constexpr int STAGES = 3;
 };
 
-// element (m, n .. n + 3) of slice (bo, ho) of the gradient
+// elements (m, n .. n + 3) of slice (bo, ho) of the gradient
+template <typename E> __device__ __forceinline__ void store_grad4(const BwdParams& p, int64_t at, int n, f32x4 v) {
+    typedef E E4 __attribute__((ext_vector_type(4)));
+    E* dst = reinterpret_cast<E*>(p.dbias) + at;
+    if (p.dbias_quads && n + 4 <= p.N) {
+        const E4 w = {(E)v[0], (E)v[1], (E)v[2], (E)v[3]};
+        *reinterpret_cast<E4*>(dst) = w;
+        return;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        if (n + e < p.N) dst[(int64_t)e * p.sdbias.n] = (E)v[e];
+}
 __device__ __forceinline__ void store_grad4(const BwdParams& p, int bo, int ho, int m, int n, f32x4 v) {
     if (m >= p.M) return;
     const int64_t at = (int64_t)bo * p.sdbias.b + (int64_t)ho * p.sdbias.h + (int64_t)m * p.sdbias.m + (int64_t)n * p.sdbias.n;
+    if (p.bias_kind == 2) store_grad4<_Float16>(p, at, n, v);
+    else if (p.bias_kind == 3) store_grad4<__bf16>(p, at, n, v);
+    else store_grad4<float>(p, at, n, v);
+}
+
+// A lane's 16 elements of a bias row in log2 units: i is key n + 8 (i/4) + i%4.  The kind is chosen once around all loads:
+// chosen per element, each load waits for the one before it.
+template <typename E> __device__ __forceinline__ void load_bias16(const BwdParams& p, int64_t row, int n, bool quads, float (&out)[16]) {
+    typedef E E4 __attribute__((ext_vector_type(4)));
+    const E* src = reinterpret_cast<const E*>(p.bias) + row;
+    E4 raw[4];
+    if (quads) {
 #pragma unroll
-    for (int e = 0; e < 4; e++) {
-        if (n + e >= p.N) break;
-        const int64_t i = at + (int64_t)e * p.sdbias.n;
-        if (p.bias_kind == 2) reinterpret_cast<_Float16*>(p.dbias)[i] = (_Float16)v[e];
-        else if (p.bias_kind == 3) reinterpret_cast<__bf16*>(p.dbias)[i] = (__bf16)v[e];
-        else reinterpret_cast<float*>(p.dbias)[i] = v[e];
+        for (int q4 = 0; q4 < 4; q4++) raw[q4] = *reinterpret_cast<const E4*>(src + n + 8 * q4);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int at = n + 8 * (i / 4) + i % 4;
+            raw[i / 4][i % 4] = src[(int64_t)(at < p.N ? at : p.N - 1) * p.sbias.n];
+        }
     }
+#pragma unroll
+    for (int i = 0; i < 16; i++) out[i] = (float)raw[i / 4][i % 4] * kLog2e;
 }
 
 // Output slice and tile number `tile` (slice-major, rows of tiles inside a slice).
@@ -95,19 +128,14 @@ __global__ __launch_bounds__(512, 2) void fa_bwd_shared_bias_kernel(const BwdPar
 
     // causal: a tile above the diagonal has no dS
     if (r0 < r1 && !(p.causal && n0 > m0 + kSharedM - 1)) {
-        // the bias of the tile in log2 units: register i is key n0 + nb + 8 (i/4) + 4 g + i%4
+        // the bias of the tile: register i is key n0 + nb + 8 (i/4) + 4 g + i%4
         float bias2[16];
         {
             const int64_t row = (int64_t)at.bo * p.sbias.b + (int64_t)at.ho * p.sbias.h + (int64_t)(my_m < M ? my_m : M - 1) * p.sbias.m;
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                int n = n0 + nb + 8 * (i / 4) + 4 * g + i % 4;
-                const int64_t j = row + (int64_t)(n < N ? n : N - 1) * p.sbias.n;
-                const float v = p.bias_kind == 2 ? (float)reinterpret_cast<const _Float16*>(p.bias)[j]
-                                : p.bias_kind == 3 ? (float)reinterpret_cast<const __bf16*>(p.bias)[j]
-                                                   : reinterpret_cast<const float*>(p.bias)[j];
-                bias2[i] = v * kLog2e;
-            }
+            const bool quads = p.bias_quads && n0 + kSharedN <= N;
+            if (p.bias_kind == 2) load_bias16<_Float16>(p, row, n0 + nb + 4 * g, quads, bias2);
+            else if (p.bias_kind == 3) load_bias16<__bf16>(p, row, n0 + nb + 4 * g, quads, bias2);
+            else load_bias16<float>(p, row, n0 + nb + 4 * g, quads, bias2);
         }
         // Copies: of the 1 KB pieces of a tensor's tile this wave issues NQ (Q, dO) or NK (K, V); lane l of piece ci
         // fetches the chunk at tile position 64 ci + l.  Rows past the end re-read the last one: what they give
@@ -236,6 +264,23 @@ __global__ __launch_bounds__(512, 2) void fa_bwd_shared_bias_kernel(const BwdPar
             const int half = j / C::KS, ks = j % C::KS;
             x[half] = mfma32(ops[2 * half][ks], ops[2 * half + 1][ks], x[half]);
         };
+        // element i of the dS of the pair whose scores are in `cur`
+        auto add_ds = [&](const f32x16 (&cur)[2], int i, auto masked_tag) __attribute__((always_inline)) {
+            float x = __builtin_fmaf(cur[0][i], qk_scale, bias2[i]);
+            if (decltype(masked_tag)::value && my_m < n0 + nb + 8 * (i / 4) + 4 * g + i % 4) x += kMask;
+            acc[i] = __builtin_fmaf(fast_exp2(x - lse), cur[1][i] - delta, acc[i]);
+        };
+        // the products of a slice of the head dim, the copies of a stage between them
+        auto slice = [&](f32x16 (&x)[2]) __attribute__((always_inline)) {
+            begin();
+            settle();
+#pragma unroll
+            for (int j = 0; j < 2 * C::KS || j < C::COPIES; j++) {
+                if (j < 2 * C::KS) mma(x, j);
+                if (j < C::COPIES) copy(j);
+            }
+            advance();
+        };
         // One pair: the products of the NEXT one are issued between the element-wise work of this one, whose scores
         // are in `cur` (what bounds a pass would otherwise be the sum of the two and of the LDS reads).
         auto pair_step = [&](f32x16 (&cur)[2], f32x16 (&next)[2], auto masked_tag) __attribute__((always_inline)) {
@@ -246,13 +291,8 @@ __global__ __launch_bounds__(512, 2) void fa_bwd_shared_bias_kernel(const BwdPar
 #pragma unroll
             for (int j = 0; j < 8; j++) {
                 __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                for (int e = 0; e < 2; e++) {
-                    const int i = 2 * j + e;
-                    float x = __builtin_fmaf(cur[0][i], qk_scale, bias2[i]);
-                    if (decltype(masked_tag)::value && my_m < n0 + nb + 8 * (i / 4) + 4 * g + i % 4) x += kMask;
-                    acc[i] = __builtin_fmaf(fast_exp2(x - lse), cur[1][i] - delta, acc[i]);
-                }
+                add_ds(cur, 2 * j, masked_tag);
+                add_ds(cur, 2 * j + 1, masked_tag);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int k = j * 2 * C::KS / 8; k < (j + 1) * 2 * C::KS / 8; k++) mma(next, k);
@@ -263,34 +303,31 @@ __global__ __launch_bounds__(512, 2) void fa_bwd_shared_bias_kernel(const BwdPar
             __builtin_amdgcn_sched_barrier(0);
             lse = lse_next;
             delta = delta_next;
-            // further slices of the head dim
 #pragma unroll
-            for (int c = 1; c < C::CHUNKS; c++) {
-                begin();
-#pragma unroll
-                for (int j = 0; j < 2 * C::KS; j++) mma(next, j);
-                issue();
-            }
+            for (int c = 1; c < C::CHUNKS; c++) slice(next);
         };
         issue();
         issue();
 #pragma unroll
         for (int i = 0; i < 16; i++) xa[0][i] = xa[1][i] = 0.f;
 #pragma unroll
-        for (int c = 0; c < C::CHUNKS; c++) {
-            begin();
-#pragma unroll
-            for (int j = 0; j < 2 * C::KS; j++) mma(xa, j);
-            issue();
-        }
+        for (int c = 0; c < C::CHUNKS; c++) slice(xa);
         lse = lse_next;
         delta = delta_next;
         auto walk = [&](auto masked_tag) {
+            int n = r1 - r0;  // pairs whose dS is due
 #pragma unroll 1
-            for (int n = r1 - r0; n > 0; n -= 2) {
+            for (; n > 2; n -= 2) {
                 pair_step(xa, xb, masked_tag);
-                if (n > 1) pair_step(xb, xa, masked_tag);
+                pair_step(xb, xa, masked_tag);
             }
+            if (n == 2) {
+                pair_step(xa, xb, masked_tag);
+                xa[0] = xb[0];
+                xa[1] = xb[1];
+            }
+#pragma unroll
+            for (int i = 0; i < 16; i++) add_ds(xa, i, masked_tag);  // the last one: no products behind it
         };
         if (masked) walk(BoolTag<true>{});
         else walk(BoolTag<false>{});

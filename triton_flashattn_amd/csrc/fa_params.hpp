@@ -76,6 +76,7 @@ struct BwdParams {
     int row_bias_kind;  // 0, or the element kind (1 bool, 2 fp16, 3 bf16, 4 fp32) of a bias with stride 0 along M:
                         // the dK/dV kernel reads it as one value per key, the dQ kernel stages it in LDS
     int causal, bias_kind;  // for the kernel of a shared bias, which has no variants: 1 if causal; 2 fp16, 3 bf16, 4 fp32
+    int bias_quads, dbias_quads;  // ... four consecutive elements of its rows / of its gradient's may be accessed at once
     int shared_tiles;   // ... tiles of its gradient, over all slices
     int shared_splits;  // ... work-groups that share the (batch, head) pairs of a tile (1: it stores the gradient itself)
     int dq_makes_delta; // the dQ kernel runs before the dK/dV kernel and forms delta itself (and stores it),
