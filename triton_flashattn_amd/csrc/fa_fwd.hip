@@ -37,8 +37,8 @@ template <typename T> constexpr float kRaise = __is_same(T, _Float16) ? 0x1p14f 
 //   kRowMax  the maximum of each block is formed first, and the reference point raised when it lies 2^8 above: ALiBi, where
 //            every row grows towards its diagonal: causal, and where a block's matrix work is small next to it (D <= 64).
 //   kAfter   the maximum is formed first in the block that follows a raise, as long as that raises again.  Not where the
-//            branch itself costs more than it saves: it takes 2 to 5 % from the causal kernels of a bias tile up to D = 128
-//            and from the row-broadcast ones at 128.
+//            branch itself costs more than it saves: it takes 2 to 5 % from the causal kernels of a bias tile up to D = 64
+//            and from those of a tile or a row-broadcast bias at 128 (B=1 H=16 M=N=4096 bf16 tensor 186.5 -> 190.7).
 //   kSum     neither.
 // Forward, us, kSum -> the rule here (B=2 H=16 M=N=2048 or, marked *, B=1 H=16 M=N=4096):
 //   ALiBi causal D=32* 93.2 -> 71.4, D=64* 94.3 -> 82.4, D=128* 120.1 -> 112.8; not causal D=32 60.7 -> 54.0, D=64 72.0 -> 64.1,
@@ -47,9 +47,9 @@ template <typename T> constexpr float kRaise = __is_same(T, _Float16) ? 0x1p14f 
 //   2 % (row-broadcast not causal D=32 79.3 -> 80.7*, D=64 97.8 -> 99.3*).
 enum Growth { kSum, kAfter, kRowMax };
 constexpr Growth growth_rule(int bias, int D, bool causal) {
-    return bias == 5 && (causal || D <= 64)                               ? kRowMax
-           : (bias >= 2 && bias <= 5 && !(causal && D <= 128)) || (bias == 6 && D != 128) ? kAfter
-                                                                                          : kSum;
+    if (bias == 5) return causal || D <= 64 ? kRowMax : kAfter;
+    const bool tile = bias >= 2 && bias <= 4;
+    return (tile && D <= 64 && !causal) || (bias == 6 && D <= 64) || ((tile || bias == 6) && D > 128) ? kAfter : kSum;
 }
 
 // The K/V stream of a row-broadcast bias (kinds 6, 7) is tiled like that of ALiBi, in steps of 32
