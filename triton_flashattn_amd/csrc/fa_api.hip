@@ -342,7 +342,7 @@ int fa_fwd_dims(const fa_fwd_args* a, int d_qk, int d_v, void* stream) {
     k.sq = s3(a->q_strides); k.sk = s3(a->k_strides); k.sv = s3(a->v_strides); k.so = s3(a->o_strides);
     k.B = p.B; k.H = p.H; k.M = p.M; k.N = p.N;
     k.sm_scale = p.sm_scale;
-    k.d_qk = d_qk; k.d_v = d_v;
+    k.d_qk = d_qk; k.d_v = d_v; k.qk_inv = (256 + d_qk / 8 - 1) / (d_qk / 8);
     if (a->bias && p.bias_dtype != FA_BIAS_ALIBI) {
         k.sbias = s4(a->bias_strides);
         k.bias_vec = bias_vec_ok(a->bias, a->bias_strides, p) ? 1 : 0;
@@ -460,7 +460,7 @@ int bwd_enqueue(const fa_bwd_args* a, int d_qk, int d_v, void* stream, int stage
     }
     k.B = p.B; k.H = p.H; k.M = p.M; k.N = p.N;
     k.sm_scale = p.sm_scale;
-    k.d_qk = d_qk; k.d_v = d_v;
+    k.d_qk = d_qk; k.d_v = d_v; k.qk_inv = (256 + d_qk / 8 - 1) / (d_qk / 8);
     int bn = fa::bwd_block_n(p.D);
     if (bn <= 0) return FA_ERR_UNSUPPORTED;
     k.n_ntiles = (p.N + bn - 1) / bn;

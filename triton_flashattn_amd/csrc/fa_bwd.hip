@@ -113,15 +113,20 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
 
     // Q^T and dO^T as B operands: column my_m, k = d
     const T* dop = reinterpret_cast<const T*>(p.dout) + (int64_t)b * p.sdo.b + (int64_t)h * p.sdo.h;
+    const LiveChunks chunks{p.d_qk / 8, p.qk_inv};
     T8 qreg[C::KSTEPS], doreg[C::KSTEPS];
 #pragma unroll
     for (int ks = 0; ks < C::KSTEPS; ks++) {
         i32x4 rq = {0, 0, 0, 0}, rd = {0, 0, 0, 0};
         const int d = ks * 16 + 8 * g;
-        if (!FROM_DS && my_m < M && d < p.d_qk) rq = gld16(qp + (int64_t)my_m * p.sq.s + d);
+        if (!FROM_DS && my_m < M) rq = gld16(qp + (int64_t)my_m * p.sq.s + (D <= 128 ? chunks.wrap(2 * ks + g) * 8 : d));
         if (!FROM_DS && my_m < M && d < p.d_v) rd = gld16(dop + (int64_t)my_m * p.sdo.s + d);
         qreg[ks] = as_vec<T8>(rq);
         doreg[ks] = as_vec<T8>(rd);
+    }
+    if (D <= 128 && !FROM_DS && p.d_qk < D) {
+#pragma unroll
+        for (int ks = 0; ks < C::KSTEPS; ks++) qreg[ks] = chunks.part<T>(qreg[ks], 2 * ks + g, C::CPR);
     }
     // LSE (log2 units) and delta of this lane's query row
     float lse_i = 0.f, delta_i = 0.f;
@@ -173,7 +178,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
     const unsigned rows_l = SW::rows_lane(lane), cols_l = SW::cols_lane(lane);
     KeyStream<T, D, stream_kind(BIAS), !FROM_DS> ks_;
     ks_.init(smem, kp, vp, bp, p.sk.s, p.sv.s, FROM_DS ? p.sdbias.m : p.sbias.m, FROM_DS ? p.sdbias.n : p.sbias.n, M, N,
-             mw, wave, lane, p.d_qk, p.d_v);
+             mw, wave, lane, chunks, p.d_v / 8);
 
     // One step of the K/V stream.  Interior steps (every key in range and visible to every row of
     // the work-group) run with STEP_MASKED = false: no range checks, no mask arithmetic.  BV: the

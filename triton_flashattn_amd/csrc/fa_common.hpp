@@ -310,10 +310,29 @@ __device__ __forceinline__ void stage_row_bias(float* row_lds, const void* bias,
     __syncthreads();
 }
 
-// A head dim below the kernel's (a multiple of 8): a copy that would fetch a chunk behind the end of a row fetches
-// the first one again.  Such a chunk meets zeros in the operand of the product that sits in registers (Q, dO, K or V
-// rows are loaded with zeros there), or makes columns of the result that are not stored.
+// A head dim below the kernel's (a multiple of 8): a copy that would fetch a chunk behind the end of a row fetches a live
+// one again.  Such a chunk meets zeros in the operand of the product that sits in registers (dO, K or V rows are loaded with
+// zeros there), or makes columns of the result that are not stored.
 __device__ __forceinline__ int live_chunk(int chunk, int chunks) { return chunk < chunks ? chunk : 0; }
+
+// S = K Q^T of the forward and the dQ kernel is formed differently: a key may hold infinities (scores of -inf, weights of
+// zero), and 0 * inf would make all of its row NaN.  Chunk c behind the end of a K row is its chunk c mod `live`, and the
+// parts of a chunk of Q that meet the same chunk of K are halves, quarters ... of it that add up to it: no product is formed
+// that the sum over the live chunks does not have (halving is exact, but for fp16 numbers below 2^-13, whose error is at
+// most 2^-25).  inv: 256 / live, rounded up.
+struct LiveChunks {
+    int live, inv;
+    __device__ __forceinline__ int turn(int c) const { return (c * inv) >> 8; }  // c / live, for c and live up to 16
+    __device__ __forceinline__ int wrap(int c) const { return c - turn(c) * live; }
+    // what is left of chunk wrap(c) of Q (8 elements) for place c of `places`
+    template <typename T, typename V8> __device__ __forceinline__ V8 part(V8 q, int c, int places) const {
+        const int last = turn(places - 1 - wrap(c)), i = turn(c);  // places of this chunk: 0 .. last
+        const float w = __builtin_bit_cast(float, (127 - (i < last ? i + 1 : last)) << 23);
+#pragma unroll
+        for (int e = 0; e < 8; e++) q[e] = (T)((float)q[e] * w);
+        return q;
+    }
+};
 
 // Tiling of the forward and the dQ kernel: a work-group owns 128 query rows (4 waves x 32 rows) and streams
 // keys in steps of NH blocks of 32.  K and V rows of a step and the bias slice of each wave reach
@@ -376,7 +395,6 @@ template <typename T, int D, int BIAS, bool WITH_V = true> struct KeyStream {
     const E* bp;              // (batch, head) slices
     int64_t sk, sv, sbm, sbn; // row strides of K and V, row and key stride of the bias (elements)
     int M, N, mw, lane;
-    int k_chunks, v_chunks;   // 16-byte chunks of a row of K and of V (fewer than CPR: a head dim below the kernel's)
     // LEAN (rows of LEAN_CPR chunks): the per-lane offsets of the KD copies are formed from three
     // per-lane constants when a copy is issued, instead of being held in 3 KD registers that such a
     // kernel does not have: a copy of chunk c = 64 ci + l reads row r0 + q (r0 = (64 / CPR) ci, q =
@@ -407,10 +425,9 @@ template <typename T, int D, int BIAS, bool WITH_V = true> struct KeyStream {
     // of them (more than once where a step has fewer than four).
     __device__ __forceinline__ void init(unsigned char* smem_, const T* kp_, const T* vp_, const E* bp_, int64_t sk_,
                                          int64_t sv_, int64_t sbm_, int64_t sbn_, int M_, int N_, int mw_, int wave, int lane_,
-                                         int d_k, int d_v) {
+                                         LiveChunks k_chunks, int v_chunks) {
         smem = smem_; kp = kp_; vp = vp_; bp = bp_; sk = sk_; sv = sv_; sbm = sbm_; sbn = sbn_;
         M = M_; N = N_; mw = mw_; lane = lane_;
-        k_chunks = d_k / 8; v_chunks = d_v / 8;
         wave = __builtin_amdgcn_readfirstlane(wave);  // the same in every lane: keep it scalar
         bias_lds = smem + C::KV_BYTES + wave * C::NBS * C::BSLOT;
         lds_kv = lds_addr_of(smem);
@@ -428,7 +445,7 @@ template <typename T, int D, int BIAS, bool WITH_V = true> struct KeyStream {
                 c_idx[i] = (wave * C::KD + i) % C::NKD;
                 const int c = c_idx[i] * 64 + lane;
                 const int row = c / C::CPR, src = (c % C::CPR) ^ SW::f(row);
-                k_off[i] = (unsigned)(row * (int)sk * 2 + live_chunk(src, k_chunks) * 16);
+                k_off[i] = (unsigned)(row * (int)sk * 2 + k_chunks.wrap(src) * 16);
                 v_off[i] = (unsigned)(row * (int)sv * 2 + live_chunk(src, v_chunks) * 16);
             }
         }
@@ -472,12 +489,10 @@ template <typename T, int D, int BIAS, bool WITH_V = true> struct KeyStream {
                 // formed here and not kept in registers across the loops)
                 int lane_here = lane;
                 asm volatile("" : "+v"(lane_here));
-                const int c = ci * 64 + lane_here;
-                int row = c / C::CPR;
-                const int src = (c % C::CPR) ^ SW::f(row);
-                row = row < N - n0 ? row : N - 1 - n0;
-                ko = (unsigned)(row * (int)sk * 2 + live_chunk(src, k_chunks) * 16);
-                vo = (unsigned)(row * (int)sv * 2 + live_chunk(src, v_chunks) * 16);
+                int over = (ci * 64 + lane_here) / C::CPR - (N - 1 - n0);
+                over = over > 0 ? over : 0;
+                ko -= (unsigned)(over * (int)sk * 2);
+                vo -= (unsigned)(over * (int)sv * 2);
             }
             lds_copy16(kt, ko, k_dst + ci * 1024);
             if constexpr (WITH_V) lds_copy16(vt, vo, v_dst + ci * 1024);

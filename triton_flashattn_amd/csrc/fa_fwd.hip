@@ -111,12 +111,17 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
                        (int64_t)b * p.sbias.b + (int64_t)h * p.sbias.h + (int64_t)key0 * p.sbias.n, p.sbias.n, N, tid);
 
     // Q^T as B operand: column my_m, k = d
+    const LiveChunks chunks{p.d_qk / 8, p.qk_inv};
     T8 qreg[C::KSTEPS];
 #pragma unroll
     for (int ks = 0; ks < C::KSTEPS; ks++) {
         i32x4 raw = {0, 0, 0, 0};
-        if (my_m < M && ks * 16 + 8 * g < p.d_qk) raw = gld16(qp + (int64_t)my_m * p.sq.s + ks * 16 + 8 * g);
+        if (my_m < M) raw = gld16(qp + (int64_t)my_m * p.sq.s + (D <= 128 ? chunks.wrap(2 * ks + g) : 2 * ks + g) * 8);
         qreg[ks] = as_vec<T8>(raw);
+    }
+    if (D <= 128 && p.d_qk < D) {
+#pragma unroll
+        for (int ks = 0; ks < C::KSTEPS; ks++) qreg[ks] = chunks.part<T>(qreg[ks], 2 * ks + g, C::CPR);
     }
 
     int n_steps = (N + BK - 1) / BK;
@@ -139,7 +144,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
 
     const unsigned rows_l = SW::rows_lane(lane), cols_l = SW::cols_lane(lane);
     KeyStream<T, D, fwd_stream_kind(BIAS)> ks_;
-    ks_.init(smem, kp, vp, bp, p.sk.s, p.sv.s, p.sbias.m, p.sbias.n, M, N, mw, wave, lane, p.d_qk, p.d_v);
+    ks_.init(smem, kp, vp, bp, p.sk.s, p.sv.s, p.sbias.m, p.sbias.n, M, N, mw, wave, lane, chunks, p.d_v / 8);
 
     // raises the reference point of this row's exponentials to mx (log2 units) where it is lower
     auto raise = [&](float mx) {

@@ -39,7 +39,8 @@ struct FwdParams {
     int n_splits, keys_per_split;
     void* part_o;
     float* part_lse;
-    int d_qk, d_v;  // head dims of the tensors: multiples of 8, at most the kernel's (which is computed with zeros there)
+    int d_qk, d_v;  // head dims of the tensors: multiples of 8, at most the kernel's
+    int qk_inv;     // 256 / (d_qk / 8), rounded up (LiveChunks)
     int row_bias_kind;  // 0, or the element kind (1 bool, 2 fp16, 3 bf16, 4 fp32) of a bias with stride 0 along M
                         // whose keys (of one split) fit the kernel's LDS row: staged once, not streamed
 };
@@ -62,7 +63,7 @@ struct BwdParams {
     Strides4 sbias, sdbias;
     int B, H, M, N;
     float sm_scale;
-    int d_qk, d_v;  // as in FwdParams
+    int d_qk, d_v, qk_inv;  // as in FwdParams
     int n_ntiles;   // key tiles of the dK/dV kernel
     int waves_per_role;  // 32-key blocks per key tile of the dK/dV kernel
     int n_mtiles;   // query tiles of the dQ kernel
