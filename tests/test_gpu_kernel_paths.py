@@ -316,6 +316,24 @@ def test_host_path_with_hooks_views_and_transforms(gpu_device):
         torch.func.vmap(lambda x: call(*one) * x)(rnd(3, 1))
 
 
+def test_host_path_raises_what_the_launchers_raise(gpu_device):
+    """A problem that the library refuses (2^28 keys, as views of one: nothing is allocated or launched) is a
+    NativeLibraryError, in the forward and in the backward, which meets it through a hook; no memory is an OutOfMemoryError."""
+    from triton_flashattn_amd import _native
+    q, k, v = (torch.randn(1, n, 1, 64, device=gpu_device).bfloat16().requires_grad_(True) for n in (3, 1, 1))
+    many = lambda t: t.detach().expand(1, 1 << 28, 1, 64) if t.shape == k.shape else t
+    with torch.no_grad(), pytest.raises(_native.NativeLibraryError, match="bad shape"):
+        flash_attention_fn(q, many(k), many(v))
+    with pytest.raises(_native.NativeLibraryError, match="bad shape"):
+        flash_attention_fn(q, many(k), many(v))
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, many):
+        out = flash_attention_fn(q, k, v)
+    with pytest.raises(_native.NativeLibraryError, match="bad shape"):
+        torch.autograd.grad(out, q, torch.ones_like(out))
+    with torch.no_grad(), pytest.raises(torch.OutOfMemoryError):
+        flash_attention_fn(q.expand(1 << 12, 3, 1 << 18, 64), k.expand(1 << 12, 1, 1 << 18, 64), v.expand(1 << 12, 1, 1 << 18, 64))
+
+
 @pytest.mark.parametrize("kind", [None, "row", "bool", "dense", "alibi"])
 def test_few_rows_against_many_keys(gpu_device, kind):
     """Few query tiles split their keys into up to 32 shares, short tiles into shares of 256 keys: both directions at

@@ -11,6 +11,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/forward_grad.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -100,7 +101,16 @@ void set_bias_strides(int64_t (&dst)[4], const Tensor& b, const Call& c) {
     const int64_t want[4] = {c.B(), c.H(), c.M(), c.N()};
     for (int i = 0; i < 4; i++) dst[i] = b.size(i) == 1 && want[i] > 1 ? 0 : b.stride(i);
 }
-void check(int status) { TORCH_CHECK(status == FA_OK, "libfa_mi355: ", fa_strerror(status), " (status ", status, ")"); }
+// NativeLibraryError, as _native.check raises it; from a node of the backward it reaches the caller as it is
+void check(int status) {
+    if (status == FA_OK) return;
+    py::gil_scoped_acquire gil;
+    const std::string text = "libfa_mi355: " + std::string(fa_strerror(status)) + " (status " + std::to_string(status) + ")";
+    PyErr_SetString(py::module_::import("triton_flashattn_amd._native").attr("NativeLibraryError").ptr(), text.c_str());
+    python_error error;
+    error.persist();
+    throw error;
+}
 void* current_stream(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 Tensor scratch(size_t bytes, const Tensor& like) {
     return at::empty({(int64_t)bytes}, like.options().dtype(at::kByte));
