@@ -268,8 +268,14 @@ def test_host_path_equals_the_autograd_classes(gpu_device):
         ours, ref = flash_attention_qkvpacked_fn(qkv, bias, True), FlashAttentionQKVPackedFn.apply(qkv, bias, True, None, None)
         for a, b in zip((ours,) + torch.autograd.grad(ours, leaves, do), (ref,) + torch.autograd.grad(ref, leaves, do)):
             assert torch.equal(a, b)
+    # without gradients the host path goes below autograd
     with torch.no_grad():
-        assert torch.equal(flash_attention_qkvpacked_fn(qkv, None, True), ours.detach() * 0 + flash_attention_qkvpacked_fn(qkv.detach(), None, True))
+        assert torch.equal(flash_attention_qkvpacked_fn(qkv, None, True), FlashAttentionQKVPackedFn.apply(qkv, None, True, None, None))
+        for bias in biases:
+            for q in (rnd(B, M, H, D), rnd(B, H, M, D).transpose(1, 2), rnd(B, M, H, D + 2)[..., :D]):
+                k, v, is_alibi = rnd(B, N, H, D), rnd(B, N, H, D), bias is slopes
+                ref = FlashAttentionFn.apply(q, k, v, None if is_alibi else bias, False, None, bias if is_alibi else None)
+                assert torch.equal(flash_attention_fn(q, k, v, AlibiBias(bias) if is_alibi else bias, False), ref)
     with pytest.raises(ValueError):
         flash_attention_fn(qkv[:, :, 0], qkv[:, :5, 1], qkv[:, :5, 2], None, True)
 
