@@ -124,10 +124,13 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
         qreg[ks] = as_vec<T8>(rq);
         doreg[ks] = as_vec<T8>(rd);
     }
-    if (D <= 128 && !FROM_DS && p.d_qk < D) {
+    auto split_q = [&]() {
+        if (D <= 128 && !FROM_DS && p.d_qk < D) {
 #pragma unroll
-        for (int ks = 0; ks < C::KSTEPS; ks++) qreg[ks] = chunks.part<T>(qreg[ks], 2 * ks + g, C::CPR);
-    }
+            for (int ks = 0; ks < C::KSTEPS; ks++) qreg[ks] = chunks.part(qreg[ks], 2 * ks + g, C::CPR);
+        }
+    };
+    if constexpr (TB != 0) split_q();  // (kernels of a bias tile have no registers for it later)
     // LSE (log2 units) and delta of this lane's query row
     float lse_i = 0.f, delta_i = 0.f;
     if (!FROM_DS && my_m < M) {
@@ -350,6 +353,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
         // steps ahead.  Waiting for them here, before the first copy, keeps the loops free of it.
         wait_vmcnt<0>();
         ks_.template prologue<BV>();
+        if constexpr (TB == 0) split_q();  // (while the first copies are on their way)
         // the leading fast steps whose copies stay inside the tensors issue them without clamps
         const int n_lean = (BV || TB == 0) ? ks_.lean_steps(n_fast, m0 + BM) : 0;
         int k = 0;

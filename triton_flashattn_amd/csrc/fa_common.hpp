@@ -316,21 +316,27 @@ __device__ __forceinline__ void stage_row_bias(float* row_lds, const void* bias,
 __device__ __forceinline__ int live_chunk(int chunk, int chunks) { return chunk < chunks ? chunk : 0; }
 
 // S = K Q^T of the forward and the dQ kernel is formed differently: a key may hold infinities (scores of -inf, weights of
-// zero), and 0 * inf would make all of its row NaN.  Chunk c behind the end of a K row is its chunk c mod `live`, and the
-// parts of a chunk of Q that meet the same chunk of K are halves, quarters ... of it that add up to it: no product is formed
-// that the sum over the live chunks does not have (halving is exact, but for fp16 numbers below 2^-13, whose error is at
-// most 2^-25).  inv: 256 / live, rounded up.
+// zero), and 0 * inf would make all of its row NaN.  Chunk c behind the end of a K row is its chunk c mod `live`, and what
+// meets it is a number of the sign of Q there (0 for 0) instead of zero, so that no product has a value or a sign that the
+// sum over the live chunks does not have:
+//   bf16  the smallest normal number, or what Q has below it.  The sum is off by 2^-126 of a key.
+//   fp16  has no such room (2^-24).  The parts of Q that meet the same chunk of K are halves, quarters ... of it that add up
+//         to it; exact, but for numbers below 2^-13, which are off by at most 2^-25.
+// (Halving bf16 too, through fp32, took 1 us of the 17 of a forward at B=8 H=16 M=N=257 D=80.)
 struct LiveChunks {
-    int live, inv;
+    int live, inv;  // inv: 256 / live, rounded up
     __device__ __forceinline__ int turn(int c) const { return (c * inv) >> 8; }  // c / live, for c and live up to 16
     __device__ __forceinline__ int wrap(int c) const { return c - turn(c) * live; }
-    // what is left of chunk wrap(c) of Q (8 elements) for place c of `places`
-    template <typename T, typename V8> __device__ __forceinline__ V8 part(V8 q, int c, int places) const {
+    // what stands at place c of `places`, from chunk wrap(c) of Q (8 elements)
+    __device__ __forceinline__ f16x8 part(f16x8 q, int c, int places) const {
         const int last = turn(places - 1 - wrap(c)), i = turn(c);  // places of this chunk: 0 .. last
-        const float w = __builtin_bit_cast(float, (127 - (i < last ? i + 1 : last)) << 23);
-#pragma unroll
-        for (int e = 0; e < 8; e++) q[e] = (T)((float)q[e] * w);
-        return q;
+        return q * (_Float16)__builtin_bit_cast(float, (127 - (i < last ? i + 1 : last)) << 23);
+    }
+    __device__ __forceinline__ bf16x8 part(bf16x8 q, int c, int) const {
+        typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
+        const u16x8 bits = __builtin_bit_cast(u16x8, q), least = (unsigned short)0x0080;
+        const u16x8 tiny = (bits & (unsigned short)0x8000) | __builtin_elementwise_min(bits & (unsigned short)0x7fff, least);
+        return c < live ? q : __builtin_bit_cast(bf16x8, tiny);
     }
 };
 

@@ -119,10 +119,13 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
         if (my_m < M) raw = gld16(qp + (int64_t)my_m * p.sq.s + (D <= 128 ? chunks.wrap(2 * ks + g) : 2 * ks + g) * 8);
         qreg[ks] = as_vec<T8>(raw);
     }
-    if (D <= 128 && p.d_qk < D) {
+    auto split_q = [&]() {
+        if (D <= 128 && p.d_qk < D) {
 #pragma unroll
-        for (int ks = 0; ks < C::KSTEPS; ks++) qreg[ks] = chunks.part<T>(qreg[ks], 2 * ks + g, C::CPR);
-    }
+            for (int ks = 0; ks < C::KSTEPS; ks++) qreg[ks] = chunks.part(qreg[ks], 2 * ks + g, C::CPR);
+        }
+    };
+    if constexpr (TB != 0) split_q();  // (kernels of a bias tile have no registers for it later)
 
     int n_steps = (N + BK - 1) / BK;
     if (CAUSAL) {
@@ -393,7 +396,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
                     for (int i = part * PL; i < 16; i++) mx = fmaxf(mx, s[i]);
                     raise(pair_max(mx) * to_log2);
                     exps();
-                    if (GROWTH == kAfter) rising = true;
+                    if (GROWTH == kAfter) rising = k > 0;  // (the first block always raises)
                 }
                 l_i += rs;  // per-lane partial sum; the two halves of a row are added at the end
 #pragma unroll
@@ -435,6 +438,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
         // steps ahead.  Waiting for them here, before the first copy, keeps the loops free of it.
         wait_vmcnt<0>();
         ks_.template prologue<BV>();
+        if constexpr (TB == 0) split_q();  // (while the first copies are on their way)
         // the leading fast steps whose copies stay inside the tensors issue them without clamps
         const int n_lean = (BV || TB == 0) ? ks_.lean_steps(n_fast, m0 + BM) : 0;
         int k = 0;
