@@ -98,7 +98,7 @@ typedef struct fa_fwd_args {
  * the bias is trainable, flash_attention.py:693,799) are outputs and are fully overwritten:
  * unlike the reference's dbias they need no zero fill by the caller.
  *
- * dbias of a float bias comes in two layouts, told apart by dbias_strides:
+ * dbias of a float bias comes in three layouts, told apart by dbias_strides (the key stride is 0 in none of them):
  *   dense    (B, H, M, N), every stride of a dimension larger than 1 non-zero: dbias = dS, as the
  *            reference stores it (flash_attention.py:307-308);
  *   reduced  the gradient of a bias that was broadcast over the query rows, (B or 1, H or 1, 1, N):
@@ -115,7 +115,8 @@ typedef struct fa_bwd_args {
     const void *q, *k, *v, *o, *dout, *bias;
     const float *lse;             /* as written by fa_fwd */
     void *dq, *dk, *dv, *dbias;   /* dbias NULL = bias not trainable */
-    void *workspace;              /* fa_bwd_workspace_bytes() bytes, 256-byte aligned */
+    void *workspace;              /* fa_bwd_args_workspace_bytes() bytes, 256-byte aligned (fa_bwd_workspace_bytes() do
+                                     unless dbias is of the shared layout) */
     size_t workspace_bytes;
     int64_t q_strides[4], k_strides[4], v_strides[4], o_strides[4], do_strides[4];
     int64_t dq_strides[4], dk_strides[4], dv_strides[4];
@@ -133,8 +134,9 @@ const char *fa_strerror(int status);
 int fa_fwd(const fa_fwd_args *args, void *stream);
 
 /* fa_fwd for q and k of head dim d_qk and v (and o) of head dim d_v, multiples of 8 no larger than p.D <= 128: computed
- * at p.D with zeros in the missing columns, without padded copies.  (8, 8) .. (p.D, p.D); for p.D = 256 only p.D itself
- * (FA_ERR_HEAD_DIM).  No counterpart in the reference, which takes powers of two (flash_attention.py:776). */
+ * at p.D as with zeros in the missing columns, without padded copies.  (8, 8) .. (p.D, p.D); for p.D = 256 only p.D itself
+ * (FA_ERR_HEAD_DIM).  Infinities in k give what they give at p.D; one in dout makes gradients NaN that zero-padded copies
+ * would leave infinite.  No counterpart in the reference, which takes powers of two (flash_attention.py:776). */
 int fa_fwd_dims(const fa_fwd_args *args, int d_qk, int d_v, void *stream);
 
 /* Bytes of scratch the backward needs for this problem: delta, (B, H, M) fp32

@@ -95,7 +95,7 @@ namespace {
 
 // Head dims of q / k and of v below the kernel's, p.D: whole 16-byte chunks.  (The kernels of head dim 256 form the
 // offsets of their copies in the loop and take their full width only; the kernel of a shared bias's gradient has both
-// operands of its products in LDS and so no zeros for the missing columns.)
+// operands of its products in LDS and so nothing to put against the missing columns.)
 bool dims_ok(const fa_problem& p, int d_qk, int d_v) {
     if (d_qk == p.D && d_v == p.D) return true;
     return p.D <= 128 && d_qk >= 8 && d_v >= 8 && d_qk <= p.D && d_v <= p.D && d_qk % 8 == 0 && d_v % 8 == 0;
@@ -300,12 +300,13 @@ const char* fa_strerror(int status) {
         case FA_OK: return "ok";
         case FA_ERR_NULL: return "a required pointer is NULL";
         case FA_ERR_SHAPE: return "bad shape: a dimension is < 1, too large, or causal with M != N";
-        case FA_ERR_HEAD_DIM: return "head dimension must be one of 16, 32, 64, 128, 256";
+        case FA_ERR_HEAD_DIM: return "head dimension must be one of 16, 32, 64, 128, 256; d_qk and d_v that equal it, or (up to 128, not "
+                                       "with the gradient of a bias that batches or heads share) multiples of 8 below it";
         case FA_ERR_DTYPE: return "unsupported dtype / bias dtype (or dbias requested for a bool bias)";
         case FA_ERR_LAYOUT:
-            return "layout: head-dim stride must be 1 and pointers/strides 16-byte aligned; a dbias broadcast over "
-                   "batches or heads must be broadcast over the query rows too";
-        case FA_ERR_WORKSPACE: return "workspace is NULL, misaligned or smaller than fa_bwd_workspace_bytes()";
+            return "layout: head-dim stride must be 1 and pointers/strides 16-byte aligned; a dbias must not be broadcast over "
+                   "the keys, and where it is broadcast over batches or heads but not over the query rows, the bias must be too";
+        case FA_ERR_WORKSPACE: return "workspace is NULL, misaligned or smaller than fa_fwd_workspace_bytes() / fa_bwd_args_workspace_bytes()";
         case FA_ERR_UNSUPPORTED: return "combination not built into this library";
         case FA_ERR_LAUNCH: return "HIP kernel launch failed";
         case FA_ERR_TOO_LARGE: return "fa_bwd_noalloc: the problem exceeds FA_NOALLOC_MAX_ROWS";

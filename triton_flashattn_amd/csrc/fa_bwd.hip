@@ -717,8 +717,8 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
     };
     // bias slice (BMI rows x 32 keys) of query block mb -> ring slot.  Chunk c = 64 it + lane of the
     // slice (row c / BCPR, 16-byte chunk c % BCPR) lands at byte 16 c of the slot, i.e. the slot
-    // is the row-major slice.  Rows past M re-read row M - 1 and chunks that start past N re-read
-    // column 0: both are masked where they are used.
+    // is the row-major slice.  Rows past M re-read row M - 1 (masked where they are used) and chunks that start past N
+    // re-read column 0 (a lane is a key: what such a lane forms is not stored).
     auto issue_bias = [&](int mb) {
         if constexpr (TB != 0) {
             const unsigned dst = lds_base + C::OFF_BIAS + (kb * C::RING + (mb - mb_first) % C::RING) * C::BT_BYTES;

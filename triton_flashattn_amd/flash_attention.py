@@ -32,7 +32,8 @@ Beyond the reference (which needs every bias materialized as (B, H, M, N), READM
   * ``AlibiBias(slopes)`` as the bias makes the kernels compute -slope[h] * |i * N / M - j| from the
     indices; the gradient comes back for the slopes;
   * v may have another head dim than q and k (the reference's forward allows it, :98-99; its
-    backward does not, :211): the narrower operands are zero-padded to the wider head dim;
+    backward does not, :211), and both may be other than the kernels': multiples of 8 up to 128 run without copies at the
+    next head dim of the kernels, others are zero-padded to it;
   * gradients that autograd does not ask for are not computed, autocast regions are honoured, and
     ``flash_attention_op`` is the same operator registered with torch.library, for torch.compile.
 """
