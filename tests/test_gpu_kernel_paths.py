@@ -205,14 +205,15 @@ def test_head_dims_below_the_kernels(gpu_device, d_qk, d_v):
             assert a.shape == ref.shape and rel_l2(a, ref) <= 5e-2, (name, M, N, causal, kind)
 
 
-@pytest.mark.parametrize("d", [8, 24, 40, 64, 72, 80, 120, 128])
-def test_infinite_keys_at_head_dims_below_the_kernels(gpu_device, d):
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("d,d_v", [(8, 8), (24, 24), (40, 40), (64, 64), (72, 72), (80, 80), (120, 120), (128, 128), (8, 128), (56, 72)])
+def test_infinite_keys_at_head_dims_below_the_kernels(gpu_device, d, d_v, dtype):
     """A key of -inf in one column, met by positive queries, has scores of -inf and a weight of zero, as at the head dims
     of the kernels: everything but the column of dQ that multiplies it stays finite."""
     g = torch.Generator().manual_seed(d)
     for M, N, causal, kind in [(130, 200, False, None), (97, 333, False, "bool"), (64, 2500, False, None), (150, 150, True, "dense")]:
-        mk = lambda n: torch.randn(2, n, 2, d, generator=g).bfloat16()
-        q, k, v, do = mk(M), mk(N), mk(N), mk(M)
+        mk = lambda n, w=d: torch.randn(2, n, 2, w, generator=g).to(dtype)
+        q, k, v, do = mk(M), mk(N), mk(N, d_v), mk(M, d_v)
         q[..., 0] = q[..., 0].abs() + 0.1
         k[:, 1::3, :, 0] = float("-inf")
         ins = [t.to(gpu_device).requires_grad_(True) for t in (q, k, v)]
@@ -221,7 +222,7 @@ def test_infinite_keys_at_head_dims_below_the_kernels(gpu_device, d):
         if kind == "bool":
             bias = (torch.rand(2, 2, M, N, generator=g) > 0.3).index_fill(3, torch.tensor([0]), True).to(gpu_device)
         elif kind == "dense":
-            bias = torch.randn(2, 2, M, N, generator=g).bfloat16().to(gpu_device)
+            bias = torch.randn(2, 2, M, N, generator=g).to(dtype).to(gpu_device)
         out = flash_attention_fn(*ins, bias, causal)
         dq, dk, dv = torch.autograd.grad(out, ins, do)
         q, k, v = (t.detach() for t in ins)
