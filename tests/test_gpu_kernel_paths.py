@@ -39,6 +39,31 @@ def test_forward_reference_point_of_growing_scores(gpu_device, D, dtype):
         assert err <= 2e-2, (slope, N, causal, bias_kind, err)
 
 
+@pytest.mark.parametrize("kind", [None, "dense", "row"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D,causal", [(32, False), (64, False), (128, True), (256, False)])
+def test_forward_error_where_few_keys_carry_a_row(gpu_device, D, causal, dtype, kind):
+    """Scores of standard deviation 8, where one weight is most of a row: it is 1, which rounds to itself, whenever it
+    raised the reference point, so that the output's own rounding is most of its error (1.13 to 1.15 times it, 1.19 with
+    a running maximum that is raised at 2^8; 1.26 to 1.37 where the point is left behind further)."""
+    g = torch.Generator().manual_seed(D)
+    S, H = 700, 8
+    q, k, v = (torch.randn(2, S, H, D, generator=g).to(gpu_device) for _ in range(3))
+    q, k, v = q.to(dtype), (k * (8 if kind is None else 1)).to(dtype), v.to(dtype)
+    bias = None
+    if kind is not None:
+        bias = (torch.randn((2, H, S, S) if kind == "dense" else (2, H, 1, S), generator=g) * 8).to(dtype).to(gpu_device)
+    with torch.no_grad():
+        out = flash_attention_fn(q, k, v, bias, causal).double()
+    qd, kd, vd = (t.double().transpose(1, 2).contiguous() for t in (q, k, v))
+    s = qd @ kd.transpose(2, 3).contiguous() * D ** -0.5
+    s = s if bias is None else s + bias.double()
+    if causal:
+        s = s.masked_fill(torch.ones(S, S, dtype=torch.bool, device=gpu_device).triu(1), float("-inf"))
+    ref = (s.softmax(-1) @ vd).transpose(1, 2)
+    assert (out - ref).norm() <= 1.22 * (ref.to(dtype).double() - ref).norm()
+
+
 @pytest.mark.parametrize("D", [16, 32, 64, 128, 256])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_forward_of_biases_that_grow_along_the_keys(gpu_device, D, dtype):

@@ -26,12 +26,13 @@
 
 namespace fa {
 
-// Sum of a lane's exponentials of a block (or half of one) beyond which their reference point is raised: far from what overflows the
-// element type of P and the fp32 accumulators, and high, so that scores that grow along the keys (a distance
-// penalty on the way to the diagonal) raise it seldom.  The accumulators hold P V: in bf16 they overflow where such scores
-// meet values of V beyond about 2^95 (2^119 with a limit of 2^8, with which biases that grow would gain nothing over a
-// running maximum: ALiBi at M=1024 N=8192 H=32 D=128 184 us, 173 with this limit, 182 with the maximum).
-template <typename T> constexpr float kRaise = __is_same(T, _Float16) ? 0x1p14f : 0x1p32f;
+// Sum of a lane's exponentials of a block (or half of one) beyond which their reference point is raised to the maximum.
+// No higher: after a raise the largest weight is 1, which rounding to 16 bits leaves as it is, and where few keys carry a row
+// its rounding is most of the error.  Scores of standard deviation 8, D=64: out off by 1.87e-3 of its norm in bf16 and 2.36e-4 in
+// fp16, with limits of 2^32 and 2^14 2.27e-3 and 2.61e-4 (a running maximum raised at 2^8: 1.95e-3, 2.47e-4).  The accumulators
+// keep their range too (values of V up to about 2^119).  Random scores of deviation 1 never reach either limit; biases that
+// grow take the higher ones 4 to 13 % faster (ALiBi at M=1024 N=8192 H=32 D=128 167 -> 182 us, as with a running maximum).
+constexpr float kRaise = 0x1p8f;
 
 // Biases that grow along the keys block after block (a distance penalty: ALiBi, its tensor, slope * key index in a
 // row-broadcast bias).  Taking the exponentials first and again once their sum is over the limit then costs a second set
@@ -42,11 +43,10 @@ template <typename T> constexpr float kRaise = __is_same(T, _Float16) ? 0x1p14f 
 //            branch itself costs more than it saves: it takes 2 to 5 % from the causal kernels of a bias tile up to D = 64
 //            and from those of a tile or a row-broadcast bias at 128 (B=1 H=16 M=N=4096 bf16 tensor 186.5 -> 190.7).
 //   kSum     neither.
-// Forward, us, kSum -> the rule here (B=2 H=16 M=N=2048 or, marked *, B=1 H=16 M=N=4096):
-//   ALiBi causal D=32* 93.2 -> 71.4, D=64* 94.3 -> 82.4, D=128* 120.1 -> 112.8; not causal D=32 60.7 -> 54.0, D=64 72.0 -> 64.1,
-//   D=128 95.7 -> 93.1, M=1024 N=8192 H=32 173 -> 170; as a bf16 tensor D=32 67.1 -> 61.6, fp16 D=64 74.0 -> 67.4, causal
-//   D=256 175 -> 166; slope * key as a row D=32 60.7 -> 56.8, causal B=8 D=64 115.3 -> 107.9.  Biases without a trend lose at most
-//   2 % (row-broadcast not causal D=32 79.3 -> 80.7*, D=64 97.8 -> 99.3*).
+// Forward, us, kSum -> the rule here, both with a limit of 2^32 (B=2 H=16 M=N=2048 or, marked *, B=1 H=16 M=N=4096):
+//   ALiBi causal D=32* 93.2 -> 71.4, D=64* 94.3 -> 82.4, D=128* 120.1 -> 112.8; not causal D=32 60.7 -> 54.0, D=64 72.0 -> 64.1;
+//   as a tensor D=32 67.1 -> 61.6, fp16 D=64 74.0 -> 67.4; slope * key as a row D=32 60.7 -> 56.8.  Biases without a trend lose at
+//   most 2 % (row-broadcast not causal D=32 79.3 -> 80.7*, D=64 97.8 -> 99.3*).
 enum Growth { kSum, kAfter, kRowMax };
 constexpr Growth growth_rule(int bias, int D, bool causal) {
     if (bias == 5) return causal || D <= 64 ? kRowMax : kAfter;
@@ -234,7 +234,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
                 return rs;
             };
             auto settle = [&](const f32x16& x, T8 (&out)[2], float rs) {
-                if (__builtin_amdgcn_ballot_w64(!(rs <= kRaise<T>)) != 0) {
+                if (__builtin_amdgcn_ballot_w64(!(rs <= kRaise)) != 0) {
                     float mx = -INFINITY;
 #pragma unroll
                     for (int i = 0; i < 16; i++) mx = fmaxf(mx, x[i]);
@@ -392,7 +392,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
                     }
                 };
                 exps();
-                if (GROWTH != kRowMax && __builtin_amdgcn_ballot_w64(!(rs <= kRaise<T>)) != 0) {
+                if (GROWTH != kRowMax && __builtin_amdgcn_ballot_w64(!(rs <= kRaise)) != 0) {
                     float mx = -INFINITY;
 #pragma unroll
                     for (int i = part * PL; i < 16; i++) mx = fmaxf(mx, s[i]);
