@@ -1397,6 +1397,9 @@ __global__ __launch_bounds__(LANES) void fa_bwd_slope_reduce_kernel(const BwdPar
     if (lane == 0) reinterpret_cast<float*>(p.dbias)[h] = s;
 }
 
+// fa_bwd_narrow.hip: dK, dV and dBias up to head dim 64
+template <int D> hipError_t launch_bwd_narrow_d(const BwdParams& p, int dtype, int bias, bool causal, int dbias, hipStream_t st);
+
 // dbias: 0 = none, 1 = dense, 2 = reduced in the kernels (see fa_bwd_kernel), 3 = of a shared bias (not here)
 template <typename T, int D> static hipError_t launch_all(const BwdParams& p, int bias, bool causal, int dbias, int stages, hipStream_t st) {
     constexpr int RPB = 256 / (D / 8);
@@ -1468,13 +1471,16 @@ template <typename T, int D> static hipError_t launch_all(const BwdParams& p, in
         if (e != hipSuccess) return e;
     }
     if (stages & 2) {
-#define FA_CASE(BK, DBK)                                                                                      \
-    if (kbias == BK && kdbias == DBK)                                                                          \
-        e = causal ? launch_main<T, D, BK, true, DBK>(p, st) : launch_main<T, D, BK, false, DBK>(p, st);
     // a bias that is the same for every query row is one register per key for this kernel
     // (dbias 3, the gradient of a shared bias, is a kernel of its own: here the bias is only read)
     const int kbias = (p.row_bias_kind != 0 && dbias != 1) ? (p.row_bias_kind == 1 ? 7 : 6) : bias;
     const int kdbias = dbias == 3 ? 0 : dbias;
+    if constexpr (D <= 64) {
+        e = launch_bwd_narrow_d<D>(p, __is_same(T, __bf16), kbias, causal, kdbias, st);
+    } else {
+#define FA_CASE(BK, DBK)                                                                                      \
+    if (kbias == BK && kdbias == DBK)                                                                          \
+        e = causal ? launch_main<T, D, BK, true, DBK>(p, st) : launch_main<T, D, BK, false, DBK>(p, st);
     FA_CASE(0, 0)
     else FA_CASE(6, 0)
     else FA_CASE(6, 2)
@@ -1493,6 +1499,7 @@ template <typename T, int D> static hipError_t launch_all(const BwdParams& p, in
     else FA_CASE(5, 2)
     else return hipErrorInvalidValue;
 #undef FA_CASE
+    }
         if (e != hipSuccess) return e;
         if (dbias == 2) {
             if (bias == 5) {
