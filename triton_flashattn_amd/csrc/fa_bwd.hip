@@ -492,21 +492,15 @@ template <> struct BiasQuad<4> {
 };
 
 // ---------------------------------------------------------------------------------------------
-// OCC2: two work-groups per CU (four waves per SIMD, 128 registers each, half of the LDS): the
-// configuration of the small head dims without a bias tile (no bias, or one kept in a register per
-// key), whose blocks are small enough.
-constexpr bool bwd_occ2(int D, int bias) { return D <= 64 && (bias == 0 || bias == 6 || bias == 7); }
-template <int D, int BIAS, bool OCC2 = false> struct BwdCfg {
+template <int D, int BIAS> struct BwdCfg {
     // waves per role: four pairs of waves on a 128-key tile, two on a 64-key tile for head dim 256,
     // where a wave needs the whole register file of its SIMD (128 accumulator registers and 64 of the
     // resident operand before anything streams)
     static constexpr int WPR = D > 128 ? 2 : 4;
     static constexpr int BN = 32 * WPR, NT = 128 * WPR;
-    static constexpr int LDS_LIMIT = OCC2 ? 81920 : 163840;
-    static constexpr int NSUB = (D <= 64 && BIAS == 0 && !OCC2) ? 2 : 1;  // 32-row sub-blocks of a query block
-    static constexpr int BMI = 32 * NSUB;
-    static constexpr int DP = D < 32 ? 32 : D;
-    static constexpr int DB = DP / 32;
+    static constexpr int LDS_LIMIT = 163840;
+    static constexpr int BMI = 32;                         // rows of a query block
+    static constexpr int DB = D / 32;
     static constexpr int KSTEPS = D / 16;
     static constexpr int CPR = D / 8;
     static constexpr int DSS = BMI + 4;                    // dS^T tile: elements between two keys
@@ -525,7 +519,7 @@ template <int D, int BIAS, bool OCC2 = false> struct BwdCfg {
     // The LSE (delta) values of a block: a copy is 64 lanes wide, so a slot is 64 floats; with 32-row
     // blocks the upper lanes copy the same 32 values again (no lane mask, no branch around the copy).
     static constexpr int STAT_BYTES = 64 * 4;
-    static constexpr int P_BYTES = 4 * NSUB * 64 * 16 * WPR;  // P hand-off: 16 floats per lane per sub-block
+    static constexpr int P_BYTES = 4 * 64 * 16 * WPR;         // P hand-off: 16 floats per lane
     static constexpr int BT_BYTES = BMI * 32 * ES;         // bias slice of one S-wave
     // LDS bytes with copies la blocks ahead: la + 1 dO buffers and bias slots, la + 2 Q buffers and
     // one more if the dK product of a block is deferred by a step (so that it does not wait for
@@ -547,7 +541,7 @@ template <int D, int BIAS, bool OCC2 = false> struct BwdCfg {
     static constexpr int LOOP_BYTES = OFF_BIAS + WPR * RING * BT_BYTES;
     static constexpr int LDS_BYTES = LOOP_BYTES;
     static_assert(LDS_BYTES <= LDS_LIMIT, "LDS budget of the configuration");
-    static constexpr int WAVES_PER_SIMD = OCC2 ? 4 : (WPR == 2 ? 1 : 2);
+    static constexpr int WAVES_PER_SIMD = WPR == 2 ? 1 : 2;
 };
 
 // Work split inside a work-group of 8 waves.  Waves 0-3 ("S-waves") and waves 4-7 ("dP-waves")
@@ -567,20 +561,21 @@ template <int D, int BIAS, bool OCC2 = false> struct BwdCfg {
 // query rows, one fp32 per (batch, head, key), for ALiBi the gradient of the slope, one fp32 per
 // (batch, head, key tile, wave); a second small kernel sums those over the broadcast dimensions.
 template <typename T, int D, int BIAS, bool CAUSAL, int DBIAS>
-__global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT), (BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::WAVES_PER_SIMD)) void fa_bwd_kernel(const BwdParams p) {
+__global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS)>::NT), (BwdCfg<D, tile_kind(BIAS)>::WAVES_PER_SIMD)) void fa_bwd_kernel(const BwdParams p) {
     constexpr int TB = tile_kind(BIAS);  // kind of bias tile that is streamed (none for ALiBi)
-    typedef BwdCfg<D, TB, bwd_occ2(D, BIAS)> C;
+    static_assert(D > 64, "fa_bwd_narrow.hip");
+    typedef BwdCfg<D, TB> C;
     typedef Swz<D> SW;
     typedef typename VecOf<T>::v8 T8;
     typedef typename VecOf<T>::v4 T4;
     typedef typename BiasElem<tile_kind(BIAS)>::type E;
-    constexpr int BN = C::BN, BMI = C::BMI, CPR = C::CPR, DSS = C::DSS, NSUB = C::NSUB;
+    constexpr int BN = C::BN, BMI = C::BMI, CPR = C::CPR, DSS = C::DSS;
     // dBias leaves through the dS tile (16-byte row stores) when it has the element type of dS
     constexpr bool DB_VIA_LDS = DBIAS == 1 && ((BIAS == 2 && __is_same(T, _Float16)) || (BIAS == 3 && __is_same(T, __bf16)));
     // an fp32 dBias leaves through LDS too, as fp32: the dP-wave turns its part of the P hand-off buffer,
     // which it has just read and which is not written again before the next step, into a row-major
     // 32 x 32 tile (4-byte stores, one per element) and stores 16 bytes per lane from there
-    constexpr bool DB_VIA_LDS32 = DBIAS == 1 && BIAS == 4 && BMI == 32;
+    constexpr bool DB_VIA_LDS32 = DBIAS == 1 && BIAS == 4;
 
     __shared__ __align__(16) unsigned char smem[C::LDS_BYTES];
 
@@ -629,7 +624,7 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
     }
     constexpr bool NATURAL = BIAS >= 2 && BIAS != 7;  // the bias term is in natural units (else log2 units)
     unsigned char* ring_lds = smem + C::OFF_BIAS + kb * C::RING * C::BT_BYTES;
-    float* p_lds = reinterpret_cast<float*>(smem + C::OFF_P) + kb * NSUB * 64 * 16;  // + buffer * P_BYTES / 4
+    float* p_lds = reinterpret_cast<float*>(smem + C::OFF_P) + kb * 64 * 16;  // + buffer * P_BYTES / 4
 
     // ---- this wave's 32 keys as B operand (column my_n, k = d): K for an S-wave, V for a dP-wave
     T8 opreg[C::KSTEPS];
@@ -756,10 +751,6 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
     // the last few of a tile) walk the query blocks in order, so their copies keep running block
     // pointers in scalar registers, one 64-bit add per block, and need no clamps; run_start() points
     // them at the first blocks an interior loop issues.
-    // (The kernels that run two work-groups per CU have 128 registers per wave and no room for the
-    // second copy of the loop: they run every step in its general form.  With their operand reads
-    // left to the compiler they fit, and gain 2 % on the causal D = 64 shape: not worth a second form.)
-    constexpr bool IN_LOOPS = !bwd_occ2(D, BIAS);
     const int n_full = M / BMI;  // blocks whose rows all exist
     uint64_t run_rows = 0, run_stat = 0, run_bias = 0;  // Q and LSE (role that issues Q) or dO and delta; bias slices
     unsigned bias_off0 = 0;  // this lane's byte offset in the first bias copy of a block, from the block's first row
@@ -806,22 +797,19 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
     // per-element path for bias rows that cannot be copied in aligned 16-byte chunks
     auto load_bias_scalar = [&](int mb, unsigned char* dst) {
         if constexpr (TB != 0) {
-            // all loads of a 32-row sub-block in flight together (clamped addresses instead of
+            // all loads of the block in flight together (clamped addresses instead of
             // branches; what lies outside the bias is masked where it is used)
             const int m0 = mb * BMI;
             const int nn = my_n < N ? my_n : N - 1;
-#pragma unroll 1
-            for (int sb = 0; sb < NSUB; sb++) {
-                E vals[16];
+            E vals[16];
 #pragma unroll
-                for (int j = 0; j < 16; j++) {
-                    int m = m0 + sb * 32 + 2 * j + g;
-                    m = m < M ? m : M - 1;
-                    vals[j] = bp[(int64_t)m * p.sbias.m + (int64_t)nn * p.sbias.n];
-                }
-#pragma unroll
-                for (int j = 0; j < 16; j++) reinterpret_cast<E*>(dst)[(sb * 32 + 2 * j + g) * 32 + r] = vals[j];
+            for (int j = 0; j < 16; j++) {
+                int m = m0 + 2 * j + g;
+                m = m < M ? m : M - 1;
+                vals[j] = bp[(int64_t)m * p.sbias.m + (int64_t)nn * p.sbias.n];
             }
+#pragma unroll
+            for (int j = 0; j < 16; j++) reinterpret_cast<E*>(dst)[(2 * j + g) * 32 + r] = vals[j];
         }
     };
 
@@ -839,11 +827,9 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
     wait_vmcnt<0>();
     __syncthreads();
 
-    T8 op_cur[NSUB][2];  // P^T (S-wave) or dS^T (dP-wave) of the block whose accumulation is still due
+    T8 op_cur[2];  // P^T (S-wave) or dS^T (dP-wave) of the block whose accumulation is still due
 #pragma unroll
-    for (int sb = 0; sb < NSUB; sb++)
-#pragma unroll
-        for (int kk = 0; kk < 2; kk++) op_cur[sb][kk] = as_vec<T8>(i32x4{0, 0, 0, 0});
+    for (int kk = 0; kk < 2; kk++) op_cur[kk] = as_vec<T8>(i32x4{0, 0, 0, 0});
 
     // A wave issues its instructions in order and only two waves share a SIMD, so every LDS round
     // trip that sits between two dependent pieces of a step is dead time.  A step therefore
@@ -851,47 +837,37 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
     // products and the inputs of the element-wise work, each ahead of work that hides the trip.
     // With D = 256 there is no register room for that and the compiler places the reads.
     constexpr bool PRELOAD = D <= 128;
-    constexpr int NR = NSUB * C::KSTEPS;  // A operands of a row product: 32 rows x 16 of the head dim each
-    constexpr int NA = NSUB * 2 * C::DB;  // A operands of a column product: 32 of the head dim x 16 rows each
+    constexpr int NR = C::KSTEPS;  // A operands of a row product: 32 rows x 16 of the head dim each
+    constexpr int NA = 2 * C::DB;  // A operands of a column product: 32 of the head dim x 16 rows each
     // tiles are named by their LDS byte address (scalar); the two per-lane address constants of
     // Swz cover every operand read of the loop
     const unsigned rows_l = SW::rows_lane(lane), cols_l = SW::cols_lane(lane);
     auto load_rows = [&](unsigned tile, T8 (&a)[NR]) {
         const unsigned base = tile + rows_l;
 #pragma unroll
-        for (int sb = 0; sb < NSUB; sb++)
-#pragma unroll
-            for (int ks = 0; ks < C::KSTEPS; ks++) a[sb * C::KSTEPS + ks] = SW::template row8_at<T8>(base, sb * 32, ks);
+        for (int ks = 0; ks < C::KSTEPS; ks++) a[ks] = SW::template row8_at<T8>(base, 0, ks);
     };
     // sacc = rows(tile) x opreg: S = Q K^T (S-wave) or dP = dO V^T (dP-wave)
-    auto mma_rows = [&](const T8 (&a)[NR], f32x16 (&sacc)[NSUB]) {
+    auto mma_rows = [&](const T8 (&a)[NR], f32x16& sacc) {
 #pragma unroll
-        for (int sb = 0; sb < NSUB; sb++) {
+        for (int i = 0; i < 16; i++) sacc[i] = 0.f;
 #pragma unroll
-            for (int i = 0; i < 16; i++) sacc[sb][i] = 0.f;
-#pragma unroll
-            for (int ks = 0; ks < C::KSTEPS; ks++) sacc[sb] = mfma32(a[sb * C::KSTEPS + ks], opreg[ks], sacc[sb]);
-        }
+        for (int ks = 0; ks < C::KSTEPS; ks++) sacc = mfma32(a[ks], opreg[ks], sacc);
     };
     // the A operands of acc^T += tile^T op are columns of the tile, gathered with ds_read_b64_tr_b16
     auto load_cols = [&](unsigned tile, T8 (&a)[NA]) {
         const unsigned base = tile + cols_l;
 #pragma unroll
-        for (int sb = 0; sb < NSUB; sb++)
+        for (int kk = 0; kk < 2; kk++)
 #pragma unroll
-            for (int kk = 0; kk < 2; kk++)
-#pragma unroll
-                for (int db = 0; db < C::DB; db++)
-                    a[(sb * 2 + kk) * C::DB + db] = SW::template col8_at<T8>(base, sb * 32 + kk * 16, db);
+            for (int db = 0; db < C::DB; db++) a[kk * C::DB + db] = SW::template col8_at<T8>(base, kk * 16, db);
     };
     // acc^T += tile^T op: dV^T += dO^T P (S-wave) or dK^T += Q^T dS (dP-wave)
-    auto mma_cols = [&](const T8 (&a)[NA], const T8 (&op)[NSUB][2]) {
+    auto mma_cols = [&](const T8 (&a)[NA], const T8 (&op)[2]) {
 #pragma unroll
-        for (int sb = 0; sb < NSUB; sb++)
+        for (int kk = 0; kk < 2; kk++)
 #pragma unroll
-            for (int kk = 0; kk < 2; kk++)
-#pragma unroll
-                for (int db = 0; db < C::DB; db++) acc[db] = mfma32(a[(sb * 2 + kk) * C::DB + db], op[sb][kk], acc[db]);
+            for (int db = 0; db < C::DB; db++) acc[db] = mfma32(a[kk * C::DB + db], op[kk], acc[db]);
     };
     // ring slots of a block index that may run one or two blocks below zero at the first steps
     auto q_tile = [&](int mb) { return lds_base + (unsigned)(((mb < 0 ? 0 : mb) % C::NQB) * C::Q_BYTES); };
@@ -913,7 +889,7 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
         // dP-wave has the most vector work), a loss of 5 % with a bias that is only read and of 4 %
         // without one, which keep the plain order.
         constexpr bool S_AHEAD = TB != 0 && C::LA >= 3 && DBIAS == 1;
-        f32x16 sacc[NSUB];
+        f32x16 sacc;
         if constexpr (S_AHEAD) {
             T8 a_rows[NR];
             load_rows(q_tile(mb_first), a_rows);
@@ -923,7 +899,7 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
             // IN: an interior step: blocks t .. t + 2 + LA are whole and in range, block t + 1 needs no mask
             constexpr bool IN = decltype(in_tag)::value;
             const int nb = t + 1;  // the block whose P is produced in this step
-            T8 op_next[NSUB][2];
+            T8 op_next[2];
             // Copies for the steps to come (their buffers were last read one step ago).  With a bias
             // they are issued behind the LDS reads of the step, whose round trip they cover; without
             // one right after the barrier: measured, each way is a few per cent better in its case.
@@ -944,20 +920,18 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
             const unsigned char* bt_lds = ring_lds + ((nb - mb_first) % C::RING) * C::BT_BYTES;
             const float* lse_lds = reinterpret_cast<const float*>(smem + C::OFF_LSE) + (IN ? (unsigned)nb % C::NQB : nb % C::NQB) * (C::STAT_BYTES / 4);
             // inputs of P: LSE of 4 consecutive rows and the bias of those rows at this lane's key
-            f32x4 lse_in[NSUB][4];
-            BiasQuad<BIAS> bias_in[NSUB][4];
+            f32x4 lse_in[4];
+            BiasQuad<BIAS> bias_in[4];
             auto load_p_inputs = [&]() {
 #pragma unroll
-                for (int sb = 0; sb < NSUB; sb++)
-#pragma unroll
-                    for (int q4 = 0; q4 < 4; q4++) {
-                        const int ml0 = sb * 32 + 8 * q4 + 4 * g;  // first of 4 consecutive rows
-                        lse_in[sb][q4] = *reinterpret_cast<const f32x4*>(lse_lds + ml0);
-                        bias_in[sb][q4].load(bt_lds, ml0, r, lane);
-                    }
+                for (int q4 = 0; q4 < 4; q4++) {
+                    const int ml0 = 8 * q4 + 4 * g;  // first of 4 consecutive rows
+                    lse_in[q4] = *reinterpret_cast<const f32x4*>(lse_lds + ml0);
+                    bias_in[q4].load(bt_lds, ml0, r, lane);
+                }
             };
-            // ---- P (flash_attention.py:281-294) of block nb from its scores; register i of sub-block
-            // sb is row m0 + 32 sb + 8 (i/4) + 4 g + i%4, the lane is key my_n.  Blocks that touch a
+            // ---- P (flash_attention.py:281-294) of block nb from its scores; register i
+            // is row m0 + 8 (i/4) + 4 g + i%4, the lane is key my_n.  Blocks that touch a
             // ragged edge or the causal diagonal follow the reference's additive -1e6 arithmetic term
             // by term; interior blocks fold everything into one exponent. ----
             auto make_p = [&](auto&& after_pair) {
@@ -970,43 +944,40 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
                 auto p_step = [&](auto masked_tag) {
                     constexpr bool MASKED = decltype(masked_tag)::value;
 #pragma unroll
-                    for (int sb = 0; sb < NSUB; sb++) {
+                    for (int q4 = 0; q4 < 4; q4++) {
+                        const int ml0 = 8 * q4 + 4 * g;
+                        const f32x4 lse4 = lse_in[q4];
+                        f32x4 p4;
 #pragma unroll
-                        for (int q4 = 0; q4 < 4; q4++) {
-                            const int ml0 = sb * 32 + 8 * q4 + 4 * g;
-                            const f32x4 lse4 = lse_in[sb][q4];
-                            f32x4 p4;
-#pragma unroll
-                            for (int e = 0; e < 4; e++) {
-                                const int i = q4 * 4 + e;
-                                // bool mask: the additive term in log2 units; float bias: natural units
-                                float bv = bias_in[sb][q4].get(e);
-                                if constexpr (BIAS == 5) bv = alibi_bias(neg_slope, ratio, mf0 + (float)(ml0 - 4 * g + e), (float)my_n);
-                                if constexpr (BIAS == 6 || BIAS == 7) bv = row_bv;
-                                float pv;
-                                if constexpr (MASKED) {
-                                    const int m = m0 + ml0 + e;
-                                    float x = __fmul_rn(sacc[sb][i], qk_scale);
-                                    const bool oob = (m >= M) || (my_n >= N);
-                                    float tmask = oob ? kMask : 0.f;
-                                    if (CAUSAL) tmask += (m < my_n) ? kMask : 0.f;
-                                    float add = NATURAL ? __fmul_rn(bv, kLog2e) : bv;
-                                    if (BIAS != 0) add = oob ? kMask : add;  // out-of-range bias reads as masked
-                                    x = __fadd_rn(x, __fadd_rn(tmask, add));
-                                    pv = fast_exp2(x - lse4[e]);
-                                } else {
-                                    // (without a bias the offset is the negated LSE itself: written as 0 - lse it
-                                    // would cost a subtraction per element, +0 - x not being -x)
-                                    const float off = BIAS == 0 ? -lse4[e] : (NATURAL ? __builtin_fmaf(bv, kLog2e, -lse4[e]) : bv - lse4[e]);
-                                    pv = fast_exp2(__builtin_fmaf(sacc[sb][i], qk_scale, off));
-                                }
-                                p4[e] = pv;
-                                op_next[sb][i >> 3][i & 7] = (T)pv;
-                                if (e & 1) after_pair(sb * 8 + (i >> 1));
+                        for (int e = 0; e < 4; e++) {
+                            const int i = q4 * 4 + e;
+                            // bool mask: the additive term in log2 units; float bias: natural units
+                            float bv = bias_in[q4].get(e);
+                            if constexpr (BIAS == 5) bv = alibi_bias(neg_slope, ratio, mf0 + (float)(ml0 - 4 * g + e), (float)my_n);
+                            if constexpr (BIAS == 6 || BIAS == 7) bv = row_bv;
+                            float pv;
+                            if constexpr (MASKED) {
+                                const int m = m0 + ml0 + e;
+                                float x = __fmul_rn(sacc[i], qk_scale);
+                                const bool oob = (m >= M) || (my_n >= N);
+                                float tmask = oob ? kMask : 0.f;
+                                if (CAUSAL) tmask += (m < my_n) ? kMask : 0.f;
+                                float add = NATURAL ? __fmul_rn(bv, kLog2e) : bv;
+                                if (BIAS != 0) add = oob ? kMask : add;  // out-of-range bias reads as masked
+                                x = __fadd_rn(x, __fadd_rn(tmask, add));
+                                pv = fast_exp2(x - lse4[e]);
+                            } else {
+                                // (without a bias the offset is the negated LSE itself: written as 0 - lse it
+                                // would cost a subtraction per element, +0 - x not being -x)
+                                const float off = BIAS == 0 ? -lse4[e] : (NATURAL ? __builtin_fmaf(bv, kLog2e, -lse4[e]) : bv - lse4[e]);
+                                pv = fast_exp2(__builtin_fmaf(sacc[i], qk_scale, off));
                             }
-                            // hand P to the dP-wave of the same keys: same lane, same register order
-                            *reinterpret_cast<f32x4*>(p_out + ((sb * 4 + q4) * 64 + lane) * 4) = p4;
+                            p4[e] = pv;
+                            op_next[i >> 3][i & 7] = (T)pv;
+                            if (e & 1) after_pair(i >> 1);
                         }
+                        // hand P to the dP-wave of the same keys: same lane, same register order
+                        *reinterpret_cast<f32x4*>(p_out + (q4 * 64 + lane) * 4) = p4;
                     }
                 };
                 if constexpr (IN) {
@@ -1052,13 +1023,13 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
                 // kernels of head dim 128 without a bias and with a bias that is only read, a loss of 5 % at
                 // head dim 64 with a bool mask; the same interleaving of the dK product into the dS
                 // arithmetic of the dP-wave costs 1-4 %).
-                constexpr bool FUSE = IN && NSUB == 1 && D == 128;
+                constexpr bool FUSE = IN && D == 128;
                 if constexpr (FUSE) {
                     mma_rows(a_rows, sacc);
                     __builtin_amdgcn_sched_barrier(0);
                     make_p([&](int j) {
                         __builtin_amdgcn_sched_barrier(0);
-                        acc[j % C::DB] = mfma32(a_cols[j], op_cur[0][j / C::DB], acc[j % C::DB]);
+                        acc[j % C::DB] = mfma32(a_cols[j], op_cur[j / C::DB], acc[j % C::DB]);
                         __builtin_amdgcn_sched_barrier(0);
                     });
                 } else {
@@ -1072,9 +1043,7 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
                 }
             }
 #pragma unroll
-            for (int sb = 0; sb < NSUB; sb++)
-#pragma unroll
-                for (int kk = 0; kk < 2; kk++) op_cur[sb][kk] = op_next[sb][kk];
+            for (int kk = 0; kk < 2; kk++) op_cur[kk] = op_next[kk];
             // The barrier publishes the copies that the next step reads.  Copies complete in issue
             // order (Q rows, then the bias slice of the same step).  S_AHEAD: the next step reads the
             // Q rows issued one step ago, so only the bias slice issued behind them and this step's
@@ -1096,19 +1065,16 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
         if (TB != 0 && !BV) t_out = t_in;  // bias element by element: no interior
         t_in = t_in < t_end ? t_in : t_end;
         t_out = t_out < t_in ? t_in : (t_out < t_end ? t_out : t_end);
-        if (!IN_LOOPS) t_in = t_out = t_end;  // one general loop
         // (two passes over ONE copy of the general loop, the interior loop between them)
         int t = mb_first - 1, stop = t_in;
 #pragma unroll 1
-        for (int pass = 0; pass < (IN_LOOPS ? 2 : 1); pass++) {
+        for (int pass = 0; pass < 2; pass++) {
 #pragma unroll 1
             for (; t < stop; t++) s_step(t, std::false_type{});
-            if constexpr (IN_LOOPS) {
-                if (pass == 0 && t_in < t_out) {
-                    run_start(qp, p.sq.s, lsep, t_in + 1 + C::LA, t_in + 1 + C::LA);
+            if (pass == 0 && t_in < t_out) {
+                run_start(qp, p.sq.s, lsep, t_in + 1 + C::LA, t_in + 1 + C::LA);
 #pragma unroll 1
-                    for (; t < t_out; t++) s_step(t, std::true_type{});
-                }
+                for (; t < t_out; t++) s_step(t, std::true_type{});
             }
             stop = t_end;
         }
@@ -1120,7 +1086,6 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
         // dS^T tile of this wave: 32 keys x BMI rows.  A lane writes its 4 consecutive rows of one key
         // with one 8-byte store, and ds_read_b64_tr_b16 hands a lane 4 consecutive keys of one row.
         T* ds_lds = reinterpret_cast<T*>(smem + C::OFF_DS) + kb * 32 * DSS;
-        static_assert(!DB_VIA_LDS || BMI == 32, "the dBias path is laid out for 32-row blocks");
         // lane -> row 16 ((lane/16)%2) + lane%16, keys 8 (lane/32 + 2 it) .. + 7 of the slice
         const int db_row = 16 * ((lane >> 4) & 1) + (lane & 15);
         const int db_src = (8 * (lane >> 5) + ((lane & 15) >> 2)) * DSS + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
@@ -1173,15 +1138,13 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
             const float* delta_lds = reinterpret_cast<const float*>(smem + C::OFF_DELTA) + (IN ? (unsigned)t % C::NDOB : (t < 0 ? 0 : t) % C::NDOB) * (C::STAT_BYTES / 4);
             const float* p_in = p_lds + (t & 1) * (C::P_BYTES / 4);
             T8 a_cols[NA], a_rows[NR];
-            f32x4 del_in[NSUB][4], p_vals[NSUB][4];
+            f32x4 del_in[4], p_vals[4];
             auto load_ds_inputs = [&]() {
 #pragma unroll
-                for (int sb = 0; sb < NSUB; sb++)
-#pragma unroll
-                    for (int q4 = 0; q4 < 4; q4++) {
-                        del_in[sb][q4] = *reinterpret_cast<const f32x4*>(delta_lds + sb * 32 + 8 * q4 + 4 * g);
-                        p_vals[sb][q4] = *reinterpret_cast<const f32x4*>(p_in + ((sb * 4 + q4) * 64 + lane) * 4);
-                    }
+                for (int q4 = 0; q4 < 4; q4++) {
+                    del_in[q4] = *reinterpret_cast<const f32x4*>(delta_lds + 8 * q4 + 4 * g);
+                    p_vals[q4] = *reinterpret_cast<const f32x4*>(p_in + (q4 * 64 + lane) * 4);
+                }
             };
             if constexpr (TB == 0) issue_copies();
             // operands of both products up front: Q(t-1)^T for dK, the rows of dO(t) for dP
@@ -1191,7 +1154,7 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
             if constexpr (TB != 0) issue_copies();  // behind the reads, whose round trip they cover
             if (C::DEFER_DK && (IN || t - 1 >= mb_first)) mma_cols(a_cols, op_cur);  // dK^T += Q(t-1)^T dS(t-1)
             if (live) {
-                f32x16 sacc[NSUB];
+                f32x16 sacc;
                 if constexpr (PRELOAD) {
                     load_ds_inputs();  // land while the products run
                     __builtin_amdgcn_sched_barrier(0);
@@ -1199,41 +1162,38 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
                 mma_rows(a_rows, sacc);
                 if constexpr (!PRELOAD) load_ds_inputs();
                 // ---- dS = P (dP - delta) (flash_attention.py:303-308) ----
+                i32x2 pk_even = {0, 0};
 #pragma unroll
-                for (int sb = 0; sb < NSUB; sb++) {
-                    i32x2 pk_even = {0, 0};
+                for (int q4 = 0; q4 < 4; q4++) {
+                    const int ml0 = 8 * q4 + 4 * g;
+                    const f32x4 del4 = del_in[q4];
+                    const f32x4 p4 = p_vals[q4];
+                    T4 d4;
 #pragma unroll
-                    for (int q4 = 0; q4 < 4; q4++) {
-                        const int ml0 = sb * 32 + 8 * q4 + 4 * g;
-                        const f32x4 del4 = del_in[sb][q4];
-                        const f32x4 p4 = p_vals[sb][q4];
-                        T4 d4;
-#pragma unroll
-                        for (int e = 0; e < 4; e++) {
-                            const int i = q4 * 4 + e;
-                            const float dsv = p4[e] * (sacc[sb][i] - del4[e]);
-                            d4[e] = (T)dsv;
-                            if constexpr (DBIAS == 2) {
-                                // rows past M have P = 0 exactly, hence dS = 0
-                                if constexpr (BIAS == 5)  // d bias / d slope = -|i N / M - j|
-                                    red_acc -= dsv * __builtin_fabsf(__builtin_fmaf((float)(m0 + 4 * g) + (float)(ml0 - 4 * g + e), ratio, -(float)my_n));
-                                else red_acc += dsv;
-                            }
-                            if constexpr (DBIAS == 1 && !DB_VIA_LDS && !DB_VIA_LDS32) {
-                                const int m = m0 + ml0 + e;
-                                if (m < M && my_n < N) dbp[(int64_t)m * p.sdbias.m + (int64_t)my_n * p.sdbias.n] = (E)dsv;
-                            }
-                            // (p_in is this wave's part of the hand-off buffer read at the top of the step)
-                            if constexpr (DB_VIA_LDS32) const_cast<float*>(p_in)[(ml0 + e) * 32 + r] = dsv;
+                    for (int e = 0; e < 4; e++) {
+                        const int i = q4 * 4 + e;
+                        const float dsv = p4[e] * (sacc[i] - del4[e]);
+                        d4[e] = (T)dsv;
+                        if constexpr (DBIAS == 2) {
+                            // rows past M have P = 0 exactly, hence dS = 0
+                            if constexpr (BIAS == 5)  // d bias / d slope = -|i N / M - j|
+                                red_acc -= dsv * __builtin_fabsf(__builtin_fmaf((float)(m0 + 4 * g) + (float)(ml0 - 4 * g + e), ratio, -(float)my_n));
+                            else red_acc += dsv;
                         }
-                        // the operand of the dK product is made of the same packed words that go to the dS
-                        // tile (assembled as integers: element-wise inserts made the compiler convert
-                        // every value a second time, one by one, and merge the halves with permutes)
-                        const i32x2 pk = __builtin_bit_cast(i32x2, d4);
-                        if (q4 & 1) op_cur[sb][q4 >> 1] = __builtin_bit_cast(T8, (i32x4){pk_even[0], pk_even[1], pk[0], pk[1]});
-                        else pk_even = pk;
-                        if constexpr (DB_VIA_LDS) *reinterpret_cast<T4*>(ds_lds + r * DSS + ml0) = d4;
+                        if constexpr (DBIAS == 1 && !DB_VIA_LDS && !DB_VIA_LDS32) {
+                            const int m = m0 + ml0 + e;
+                            if (m < M && my_n < N) dbp[(int64_t)m * p.sdbias.m + (int64_t)my_n * p.sdbias.n] = (E)dsv;
+                        }
+                        // (p_in is this wave's part of the hand-off buffer read at the top of the step)
+                        if constexpr (DB_VIA_LDS32) const_cast<float*>(p_in)[(ml0 + e) * 32 + r] = dsv;
                     }
+                    // the operand of the dK product is made of the same packed words that go to the dS
+                    // tile (assembled as integers: element-wise inserts made the compiler convert
+                    // every value a second time, one by one, and merge the halves with permutes)
+                    const i32x2 pk = __builtin_bit_cast(i32x2, d4);
+                    if (q4 & 1) op_cur[q4 >> 1] = __builtin_bit_cast(T8, (i32x4){pk_even[0], pk_even[1], pk[0], pk[1]});
+                    else pk_even = pk;
+                    if constexpr (DB_VIA_LDS) *reinterpret_cast<T4*>(ds_lds + r * DSS + ml0) = d4;
                 }
                 // ---- dBias rows of this wave's 32 keys, 16 bytes per lane, out of the dS^T tile ----
                 if constexpr (DB_VIA_LDS) {
@@ -1297,19 +1257,16 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
         int t_in = mb_first + 1, t_out = n_full - C::LA;
         t_in = t_in < t_end ? t_in : t_end;
         t_out = t_out < t_in ? t_in : (t_out < t_end ? t_out : t_end);
-        if (!IN_LOOPS) t_in = t_out = t_end;  // one general loop
         // (two passes over ONE copy of the general loop, the interior loop between them)
         int t = mb_first - 1, stop = t_in;
 #pragma unroll 1
-        for (int pass = 0; pass < (IN_LOOPS ? 2 : 1); pass++) {
+        for (int pass = 0; pass < 2; pass++) {
 #pragma unroll 1
             for (; t < stop; t++) dp_step(t, std::false_type{});
-            if constexpr (IN_LOOPS) {
-                if (pass == 0 && t_in < t_out) {
-                    run_start(dop, p.sdo.s, deltap, t_in + C::LA, 0);
+            if (pass == 0 && t_in < t_out) {
+                run_start(dop, p.sdo.s, deltap, t_in + C::LA, 0);
 #pragma unroll 1
-                    for (; t < t_out; t++) dp_step(t, std::true_type{});
-                }
+                for (; t < t_out; t++) dp_step(t, std::true_type{});
             }
             stop = t_end;
         }
@@ -1361,7 +1318,7 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)
 template <typename T, int D, int BIAS, bool CAUSAL, int DBIAS>
 static hipError_t launch_main(const BwdParams& p, hipStream_t st) {
     dim3 grid((unsigned)(p.n_ntiles * p.B * p.H));
-    hipLaunchKernelGGL((fa_bwd_kernel<T, D, BIAS, CAUSAL, DBIAS>), grid, dim3((BwdCfg<D, tile_kind(BIAS), bwd_occ2(D, BIAS)>::NT)), 0, st, p);
+    hipLaunchKernelGGL((fa_bwd_kernel<T, D, BIAS, CAUSAL, DBIAS>), grid, dim3((BwdCfg<D, tile_kind(BIAS)>::NT)), 0, st, p);
     return hipGetLastError();
 }
 
