@@ -109,13 +109,18 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
     }
     if (FROM_DS) bp = reinterpret_cast<const E*>(p.dbias) + (int64_t)b * p.sdbias.b + (int64_t)h * p.sdbias.h + (int64_t)key0 * p.sdbias.n;
 
-    if (ROWB)
-        stage_row_bias(reinterpret_cast<float*>(smem + C::LDS_BYTES), p.bias, p.row_bias_kind,
-                       (int64_t)b * p.sbias.b + (int64_t)h * p.sbias.h + (int64_t)key0 * p.sbias.n, p.sbias.n, N, tid);
+    // The first copies go out before anything is loaded and waited for (as in the forward kernel).
+    const LiveChunks chunks{p.d_qk / 8, p.qk_inv};
+    const unsigned rows_l = SW::rows_lane(lane), cols_l = SW::cols_lane(lane);
+    KeyStream<T, D, stream_kind(BIAS), !FROM_DS> ks_;
+    ks_.init(smem, kp, vp, bp, p.sk.s, p.sv.s, FROM_DS ? p.sdbias.m : p.sbias.m, FROM_DS ? p.sdbias.n : p.sbias.n, M, N,
+             mw, wave, lane, chunks, p.d_v / 8);
+    const bool bias_copies = FROM_DS || (TB != 0 && p.bias_vec);
+    if (bias_copies) ks_.template prologue<true>();
+    else ks_.template prologue<false>();
 
     // Q^T and dO^T as B operands: column my_m, k = d
     const T* dop = reinterpret_cast<const T*>(p.dout) + (int64_t)b * p.sdo.b + (int64_t)h * p.sdo.h;
-    const LiveChunks chunks{p.d_qk / 8, p.qk_inv};
     T8 qreg[C::KSTEPS], doreg[C::KSTEPS];
 #pragma unroll
     for (int ks = 0; ks < C::KSTEPS; ks++) {
@@ -180,10 +185,9 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
 #pragma unroll
         for (int i = 0; i < 16; i++) dq_acc[db][i] = 0.f;
 
-    const unsigned rows_l = SW::rows_lane(lane), cols_l = SW::cols_lane(lane);
-    KeyStream<T, D, stream_kind(BIAS), !FROM_DS> ks_;
-    ks_.init(smem, kp, vp, bp, p.sk.s, p.sv.s, FROM_DS ? p.sdbias.m : p.sbias.m, FROM_DS ? p.sdbias.n : p.sbias.n, M, N,
-             mw, wave, lane, chunks, p.d_v / 8);
+    if (ROWB)
+        stage_row_bias(reinterpret_cast<float*>(smem + C::LDS_BYTES), p.bias, p.row_bias_kind,
+                       (int64_t)b * p.sbias.b + (int64_t)h * p.sbias.h + (int64_t)key0 * p.sbias.n, p.sbias.n, N, tid);
 
     // One step of the K/V stream.  Interior steps (every key in range and visible to every row of
     // the work-group) run with STEP_MASKED = false: no range checks, no mask arithmetic.  BV: the
@@ -352,10 +356,9 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
         // The loads of this lane's rows issued above are the compiler's own.  Left in flight, they would
         // make it wait for "all vector-memory operations" at their first use inside EVERY step of the
         // loops (it cannot know that they land once), and that wait drains the queue of copies issued
-        // steps ahead.  Waiting for them here, before the first copy, keeps the loops free of it.
+        // steps ahead.  Waiting for them here, with the first copies, keeps the loops free of it.
         wait_vmcnt<0>();
-        ks_.template prologue<BV>();
-        if constexpr (TB == 0) split_q();  // (while the first copies are on their way)
+        if constexpr (TB == 0) split_q();
         // the leading fast steps whose copies stay inside the tensors issue them without clamps
         const int n_lean = (BV || TB == 0) ? ks_.lean_steps(n_fast, m0 + BM) : 0;
         int k = 0;
@@ -369,7 +372,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
 #pragma unroll 1
         for (; k < n_steps; k++) kv_step(k, std::true_type{}, bv_tag, std::false_type{});
     };
-    if (FROM_DS || (TB != 0 && p.bias_vec)) run(std::true_type{});
+    if (bias_copies) run(std::true_type{});
     else run(std::false_type{});
 
     // ---- epilogue: dq = dQ * sm_scale (flash_attention.py:644-646) ----

@@ -108,12 +108,18 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
         ratio = (float)p.N / (float)p.M;
     }
 
-    if (ROWB)
-        stage_row_bias(reinterpret_cast<float*>(smem + C::LDS_BYTES), p.bias, p.row_bias_kind,
-                       (int64_t)b * p.sbias.b + (int64_t)h * p.sbias.h + (int64_t)key0 * p.sbias.n, p.sbias.n, N, tid);
+    // The first copies go out before anything is loaded and waited for: a short problem is a chain of memory latencies,
+    // and those of K and V, of Q and of a bias row are one this way (B=32 H=12 M=N=197 D=64 with a padding mask, us per call:
+    // 15.3 -> 14.8; nothing where streams are long).
+    const LiveChunks chunks{p.d_qk / 8, p.qk_inv};
+    const unsigned rows_l = SW::rows_lane(lane), cols_l = SW::cols_lane(lane);
+    KeyStream<T, D, fwd_stream_kind(BIAS)> ks_;
+    ks_.init(smem, kp, vp, bp, p.sk.s, p.sv.s, p.sbias.m, p.sbias.n, M, N, mw, wave, lane, chunks, p.d_v / 8);
+    const bool bias_copies = TB != 0 && p.bias_vec;
+    if (bias_copies) ks_.template prologue<true>();
+    else ks_.template prologue<false>();
 
     // Q^T as B operand: column my_m, k = d
-    const LiveChunks chunks{p.d_qk / 8, p.qk_inv};
     T8 qreg[C::KSTEPS];
 #pragma unroll
     for (int ks = 0; ks < C::KSTEPS; ks++) {
@@ -147,9 +153,9 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
 #pragma unroll
         for (int i = 0; i < 16; i++) o_acc[db][i] = 0.f;
 
-    const unsigned rows_l = SW::rows_lane(lane), cols_l = SW::cols_lane(lane);
-    KeyStream<T, D, fwd_stream_kind(BIAS)> ks_;
-    ks_.init(smem, kp, vp, bp, p.sk.s, p.sv.s, p.sbias.m, p.sbias.n, M, N, mw, wave, lane, chunks, p.d_v / 8);
+    if (ROWB)
+        stage_row_bias(reinterpret_cast<float*>(smem + C::LDS_BYTES), p.bias, p.row_bias_kind,
+                       (int64_t)b * p.sbias.b + (int64_t)h * p.sbias.h + (int64_t)key0 * p.sbias.n, p.sbias.n, N, tid);
 
     // raises the reference point of this row's exponentials to mx (log2 units) where it is lower
     auto raise = [&](float mx) {
@@ -437,10 +443,9 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
         // The loads of this lane's rows issued above are the compiler's own.  Left in flight, they would
         // make it wait for "all vector-memory operations" at their first use inside EVERY step of the
         // loops (it cannot know that they land once), and that wait drains the queue of copies issued
-        // steps ahead.  Waiting for them here, before the first copy, keeps the loops free of it.
+        // steps ahead.  Waiting for them here, with the first copies, keeps the loops free of it.
         wait_vmcnt<0>();
-        ks_.template prologue<BV>();
-        if constexpr (TB == 0) split_q();  // (while the first copies are on their way)
+        if constexpr (TB == 0) split_q();
         // the leading fast steps whose copies stay inside the tensors issue them without clamps
         const int n_lean = (BV || TB == 0) ? ks_.lean_steps(n_fast, m0 + BM) : 0;
         int k = 0;
@@ -454,7 +459,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
 #pragma unroll 1
         for (; k < n_steps; k++) kv_step(k, std::true_type{}, bv_tag, std::false_type{});
     };
-    if (TB != 0 && p.bias_vec) run(std::true_type{});
+    if (bias_copies) run(std::true_type{});
     else run(std::false_type{});
 
     // ---- epilogue (flash_attention.py:188-194) ----
