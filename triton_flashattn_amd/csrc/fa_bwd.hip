@@ -107,6 +107,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
         neg_slope = -reinterpret_cast<const float*>(p.bias)[h];
         ratio = (float)p.N / (float)p.M;
     }
+    const float log2_slope = neg_slope * kLog2e;
     if (FROM_DS) bp = reinterpret_cast<const E*>(p.dbias) + (int64_t)b * p.sdbias.b + (int64_t)h * p.sdbias.h + (int64_t)key0 * p.sdbias.n;
 
     // The first copies go out before anything is loaded and waited for (as in the forward kernel).
@@ -267,6 +268,8 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
             // Masked tiles follow the reference's additive -1e6 arithmetic term by term.
             auto ds_step = [&](auto masked_tag) {
                 constexpr bool MASKED = decltype(masked_tag)::value;
+                const float nf0 = (float)(key0 + n0 + nh + 4 * g);              // ALiBi: the lane's first key,
+                const float dist0 = __builtin_fmaf((float)my_m, ratio, -nf0);  // and the distance to it
 #pragma unroll
                 for (int q4 = 0; q4 < 4; q4++) {
                     const int nl = 8 * q4 + 4 * g;  // first of 4 consecutive keys of the block
@@ -285,10 +288,9 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
                         f32x4 w = *reinterpret_cast<const f32x4*>(b_lds + ks_.b_off(r, nl));
 #pragma unroll
                         for (int e = 0; e < 4; e++) bv[e] = w[e];
-                    } else if constexpr (BIAS == 5) {
+                    } else if constexpr (BIAS == 5 && MASKED) {
 #pragma unroll
-                        for (int e = 0; e < 4; e++)
-                            bv[e] = alibi_bias(neg_slope, ratio, (float)my_m, (float)(key0 + n0 + nh + 4 * g) + (float)(8 * q4 + e));
+                        for (int e = 0; e < 4; e++) bv[e] = alibi_bias(neg_slope, ratio, (float)my_m, nf0 + (float)(8 * q4 + e));
                     } else if constexpr (ROWB) {
                         f32x4 w = *reinterpret_cast<const f32x4*>(row_lds + n0 + nh + nl);
 #pragma unroll
@@ -313,6 +315,9 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
                             pv = fast_exp2(x - lse_i);
                         } else if constexpr (BIAS == 0) {
                             pv = fast_exp2(__builtin_fmaf(s[i], qk_scale, -lse_i));
+                        } else if constexpr (BIAS == 5) {
+                            const float dist = dist0 - (float)(8 * q4 + e);
+                            pv = fast_exp2(__builtin_fmaf(__builtin_fabsf(dist), log2_slope, __builtin_fmaf(s[i], qk_scale, -lse_i)));
                         } else if constexpr (BIAS == 1) {
                             pv = fast_exp2(__builtin_fmaf(s[i], qk_scale, keep[e] ? neg_lse : mask_lse));
                         } else if constexpr (BOOLROW) {
@@ -612,6 +617,7 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS)>::NT), (BwdCfg<D, tile_k
         neg_slope = -reinterpret_cast<const float*>(p.bias)[h];
         ratio = (float)p.N / (float)p.M;
     }
+    const float log2_slope = neg_slope * kLog2e;
     // row-broadcast bias: the term of this lane's key, natural units (6) or 0 / mask value in log2 units (7)
     float row_bv = 0.f;
     if (BIAS == 6 || BIAS == 7) {
@@ -942,7 +948,8 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS)>::NT), (BwdCfg<D, tile_k
                 // (keys past N need no mask: the lane is the key, and nothing of such a lane is stored.  A ragged
                 // last tile so runs interior steps like any other: B=1 H=16 M=N=6001 D=128 0.607 -> 0.540 ms)
                 const bool need_mask = !IN && ((m0 + BMI > M) || (CAUSAL && m0 < n0 + BN - 1));
-                const float mf0 = (float)(m0 + 4 * g);  // ALiBi: first row of this lane's registers, as a float
+                const float mf0 = (float)(m0 + 4 * g);  // ALiBi: first row of this lane's registers, as a float,
+                const float dist0 = __builtin_fmaf(mf0, ratio, -(float)my_n);  // and its distance to the lane's key
                 float* p_out = p_lds + (nb & 1) * (C::P_BYTES / 4);
                 auto p_step = [&](auto masked_tag) {
                     constexpr bool MASKED = decltype(masked_tag)::value;
@@ -972,7 +979,9 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS)>::NT), (BwdCfg<D, tile_k
                             } else {
                                 // (without a bias the offset is the negated LSE itself: written as 0 - lse it
                                 // would cost a subtraction per element, +0 - x not being -x)
-                                const float off = BIAS == 0 ? -lse4[e] : (NATURAL ? __builtin_fmaf(bv, kLog2e, -lse4[e]) : bv - lse4[e]);
+                                const float off = BIAS == 0   ? -lse4[e]
+                                                  : BIAS == 5 ? __builtin_fmaf(__builtin_fabsf(__builtin_fmaf((float)(8 * q4 + e), ratio, dist0)), log2_slope, -lse4[e])
+                                                              : (NATURAL ? __builtin_fmaf(bv, kLog2e, -lse4[e]) : bv - lse4[e]);
                                 pv = fast_exp2(__builtin_fmaf(sacc[i], qk_scale, off));
                             }
                             p4[e] = pv;

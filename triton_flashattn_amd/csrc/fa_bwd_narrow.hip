@@ -156,6 +156,7 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
         neg_slope = -reinterpret_cast<const float*>(p.bias)[h];
         ratio = (float)p.N / (float)p.M;
     }
+    const float log2_slope = neg_slope * kLog2e;
     // row-broadcast bias: the term of this lane's key, natural units (6) or 0 / mask value in log2 units (7)
     float row_bv = 0.f;
     if ((BIAS == 6 || BIAS == 7) && my_n < N) {
@@ -408,7 +409,11 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
                     if (BIAS != 0) add = oob ? kMask : add;  // out-of-range bias reads as masked
                     return fast_exp2(__fadd_rn(__fmul_rn(s, qk_scale), __fadd_rn(tmask, add)) - lse);
                 } else {
-                    const float off = BIAS == 0 ? -lse : (NATURAL ? __builtin_fmaf(bv, kLog2e, -lse) : bv - lse);
+                    float off = BIAS == 0 ? -lse : (NATURAL ? __builtin_fmaf(bv, kLog2e, -lse) : bv - lse);
+                    if constexpr (BIAS == 5) {  // distance of the lane's first row to its key, and from there to row i
+                        const float dist0 = __builtin_fmaf((float)(m0 + 4 * g), ratio, -(float)my_n);
+                        off = __builtin_fmaf(__builtin_fabsf(__builtin_fmaf((float)(8 * (i >> 2) + (i & 3)), ratio, dist0)), log2_slope, -lse);
+                    }
                     return fast_exp2(__builtin_fmaf(s, qk_scale, off));
                 }
             };

@@ -103,9 +103,14 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
     if (TB != 0) bp = reinterpret_cast<const E*>(p.bias) + (int64_t)b * p.sbias.b + (int64_t)h * p.sbias.h + (int64_t)key0 * p.sbias.n;
     // ALiBi: the slope of this head and the position of this lane's query row on the key axis
     float neg_slope = 0.f, ratio = 0.f;
+    // ... and, for unmasked steps, the slope in units of the dot product (its distances reach N)
+    float raw_slope = 0.f;
+    bool raw_ok = true;
     if (BIAS == 5) {
         neg_slope = -reinterpret_cast<const float*>(p.bias)[h];
         ratio = (float)p.N / (float)p.M;
+        raw_slope = neg_slope / p.sm_scale;
+        raw_ok = __builtin_fabsf(raw_slope) * (float)p.N < 1e30f;
     }
 
     // The first copies go out before anything is loaded and waited for: a short problem is a chain of memory latencies,
@@ -313,10 +318,14 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
         auto softmax_step = [&](auto masked_tag) {
             constexpr bool MASKED = decltype(masked_tag)::value;
             // units of s[i] below: raw dot product (no bias), natural (float bias), log2 (MASKED, bool masks)
-            constexpr bool RAW = !MASKED && BIAS == 0;
-            constexpr bool NAT = !MASKED && BIAS >= 2 && !BOOLROW;
+            constexpr bool RAW = !MASKED && (BIAS == 0 || BIAS == 5);
+            constexpr bool NAT = !MASKED && BIAS >= 2 && !BOOLROW && !RAW;
             const float to_log2 = RAW ? qk_scale : (NAT ? kLog2e : 1.f);
             const float mf = (float)my_m, nf0 = (float)(key0 + n0 + nh + 4 * g);  // ALiBi: row and first key as floats
+            // (unmasked: the distance to a key is that to the lane's first less a constant, and the slope goes into one
+            // fused multiply-add: 2 instructions per score, 4 with the bias formed first; with the same in the backward kernels a training
+            // step at M=1024 N=8192 H=32 D=128 718 -> 697 us)
+            const float dist0 = __builtin_fmaf(mf, ratio, -nf0);
 #pragma unroll
             for (int q4 = 0; q4 < 4; q4++) {
                 const int nl = 8 * q4 + 4 * g;            // first of 4 consecutive keys
@@ -335,6 +344,10 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
                     f32x4 w = *reinterpret_cast<const f32x4*>(b_lds + ks_.b_off(r, nl));
 #pragma unroll
                     for (int e = 0; e < 4; e++) bv[e] = w[e];
+                } else if constexpr (BIAS == 5 && RAW) {
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        s[q4 * 4 + e] = __builtin_fmaf(__builtin_fabsf(dist0 - (float)(8 * q4 + e)), raw_slope, s[q4 * 4 + e]);
                 } else if constexpr (BIAS == 5) {
 #pragma unroll
                     for (int e = 0; e < 4; e++) bv[e] = alibi_bias(neg_slope, ratio, mf, nf0 + (float)(8 * q4 + e));
@@ -425,7 +438,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
             // 32 matrix products of a block there costs the registers that the interior loops need)
             softmax_step(std::true_type{});
         } else if constexpr (STEP_MASKED) {
-            if (need_mask || !(qk_scale > 0.f)) softmax_step(std::true_type{});
+            if (need_mask || !(qk_scale > 0.f) || !raw_ok) softmax_step(std::true_type{});
             else softmax_step(std::false_type{});
         } else {
             softmax_step(std::false_type{});
@@ -436,7 +449,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
     int n_fast = N / BK;  // leading steps that need no masks
     if (CAUSAL) n_fast = n_fast < (m0 + 1) / BK ? n_fast : (m0 + 1) / BK;
     if (n_fast > n_steps) n_fast = n_steps;
-    if (!(qk_scale > 0.f)) n_fast = 0;
+    if (!(qk_scale > 0.f) || !raw_ok) n_fast = 0;
 
     auto run = [&](auto bv_tag) {
         constexpr bool BV = decltype(bv_tag)::value;
