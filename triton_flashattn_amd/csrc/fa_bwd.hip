@@ -207,6 +207,88 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
         const unsigned k_tile = ks_.k_addr(k), v_tile = ks_.v_addr(k);  // operand reads by address
         const unsigned char* b_lds = ks_.b_lds(k);
         static_assert(TB == 0 || C::NH == 1, "a bias slot covers one 32-key block");
+        // Interior steps of two blocks (no bias tile), as in the forward kernel: S and dP of block 1 are issued between the
+        // element-wise work of block 0, and the dQ product of block 0 between that of block 1, one fenced slot per two
+        // elements.  Operands are fetched a phase ahead, above head dim 64 one slot ahead.  Same bits; us, one block after
+        // the other -> this: B=4 H=16 S=2048 D=64 causal 65.1 -> 60.9, B=1 H=16 S=6001 D=128 causal 218 -> 206, B=2 H=16
+        // M=N=4096 D=128 362 -> 350.
+        if constexpr (!STEP_MASKED && C::NH == 2 && !FROM_DS) {
+            constexpr int NS = 2 * C::KSTEPS, NP = 2 * C::DB;  // matrix instructions of S and dP, and of dQ, per block
+            constexpr bool AHEAD = D <= 64;
+            constexpr int NSS = AHEAD ? NS : NS / 8, NPS = AHEAD ? NP : NP / 8;  // operands fetched at a time
+            auto fence = []() { __builtin_amdgcn_sched_barrier(0); };
+            T8 ra[AHEAD ? 1 : 2][NSS], ca[AHEAD ? 1 : 2][NPS];
+            f32x16 sc[2], dpc[2];
+            auto load_rows = [&](int nb, int slot) {  // operands slot * NSS .. of S and dP of block nb
+#pragma unroll
+                for (int i = 0; i < NSS; i++) {
+                    const int at = slot * NSS + i;
+                    ra[AHEAD ? 0 : slot & 1][i] = at < C::KSTEPS ? SW::template row8_at<T8>(k_tile + rows_l, nb * 32, at)
+                                                                 : SW::template row8_at<T8>(v_tile + rows_l, nb * 32, at - C::KSTEPS);
+                }
+            };
+            auto load_cols = [&](int nb, int slot) {
+#pragma unroll
+                for (int i = 0; i < NPS; i++) {
+                    const int at = slot * NPS + i;
+                    ca[AHEAD ? 0 : slot & 1][i] = SW::template col8_at<T8>(k_tile + cols_l, nb * 32 + (at / C::DB) * 16, at % C::DB);
+                }
+            };
+            // the matrix instructions of slot j of 8 of S and dP, and of dQ
+            auto mma_s = [&](int nb, int j) {
+                if (!AHEAD && j < 7) load_rows(nb, j + 1);
+#pragma unroll
+                for (int i = j * NS / 8; i < (j + 1) * NS / 8; i++) {
+                    const T8 a = ra[AHEAD ? 0 : j & 1][AHEAD ? i : i - j * NSS];
+                    if (i < C::KSTEPS) sc[nb] = mfma32(a, qreg[i], sc[nb]);
+                    else dpc[nb] = mfma32(a, doreg[i - C::KSTEPS], dpc[nb]);
+                }
+            };
+            auto mma_dq = [&](int nb, const T8 (&ds)[2], int j) {
+                if (!AHEAD && j < 7) load_cols(nb, j + 1);
+#pragma unroll
+                for (int i = j * NP / 8; i < (j + 1) * NP / 8; i++)
+                    dq_acc[i % C::DB] = mfma32(ca[AHEAD ? 0 : j & 1][AHEAD ? i : i - j * NPS], ds[i / C::DB], dq_acc[i % C::DB]);
+            };
+            auto elements = [&](int nb, T8 (&ds)[2], auto&& between) {
+                f32x4 bias4;
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+#pragma unroll
+                    for (int i = 2 * j; i < 2 * j + 2; i++) {
+                        float off = -lse_i;
+                        if constexpr (ROWB) {
+                            if (i % 4 == 0) bias4 = *reinterpret_cast<const f32x4*>(row_lds + n0 + nb * 32 + 2 * i + 4 * g);
+                            off = BOOLROW ? bias4[i & 3] - lse_i : __builtin_fmaf(bias4[i & 3], kLog2e, -lse_i);
+                        }
+                        const float pv = fast_exp2(__builtin_fmaf(sc[nb][i], qk_scale, off));
+                        ds[i >> 3][i & 7] = (T)(pv * (dpc[nb][i] - delta_i));
+                    }
+                    fence();
+                    between(j);
+                    fence();
+                }
+            };
+#pragma unroll
+            for (int nb = 0; nb < 2; nb++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) sc[nb][i] = dpc[nb][i] = 0.f;
+            load_rows(0, 0);
+#pragma unroll
+            for (int j = 0; j < 8; j++) mma_s(0, j);
+            issue_ahead();  // in the shadow of the MFMAs just issued
+            load_rows(1, 0);
+            fence();
+            T8 ds0[2], ds1[2];
+            elements(0, ds0, [&](int j) { mma_s(1, j); });
+            load_cols(0, 0);
+            fence();
+            elements(1, ds1, [&](int j) { mma_dq(0, ds0, j); });
+            load_cols(1, 0);
+#pragma unroll
+            for (int j = 0; j < 8; j++) mma_dq(1, ds1, j);
+            return;
+        }
         // The step is consumed 32 keys at a time, so that only one 32 x 32 score block is live.
 #pragma unroll
         for (int nb = 0; nb < C::NH; nb++) {

@@ -294,16 +294,19 @@ __device__ __forceinline__ float alibi_bias(float neg_slope, float ratio, float 
 __device__ __forceinline__ void stage_row_bias(float* row_lds, const void* bias, int kind, int64_t at0, int64_t stride_n,
                                                int N, int tid) {
     const int n_stage = (N + 63) & ~63;
-    for (int n = tid; n < n_stage; n += 256) {
-        float v = 0.f;
-        if (n < N) {
-            const int64_t at = at0 + (int64_t)n * stride_n;
-            switch (kind) {
-                case 1: v = reinterpret_cast<const unsigned char*>(bias)[at] != 0 ? 0.f : kMask; break;
-                case 2: v = (float)reinterpret_cast<const _Float16*>(bias)[at]; break;
-                case 3: v = (float)reinterpret_cast<const __bf16*>(bias)[at]; break;
-                default: v = reinterpret_cast<const float*>(bias)[at]; break;
-            }
+    for (int n0 = tid; n0 < n_stage; n0 += LOADS * 256) {
+        E v[LOADS];
+#pragma unroll
+        for (int j = 0; j < LOADS; j++) {
+            const int n = n0 + 256 * j;
+            v[j] = at[(int64_t)(n < N ? n : N - 1) * stride_n];
+        }
+#pragma unroll
+        for (int j = 0; j < LOADS; j++) {
+            const int n = n0 + 256 * j;
+            float f = (float)v[j];
+            if (__is_same(E, unsigned char)) f = f != 0.f ? 0.f : kMask;
+            if (n < n_stage) row_lds[n] = n < N ? f : 0.f;
         }
         row_lds[n] = v;
     }
@@ -379,11 +382,12 @@ template <int D, int BIAS> struct StreamCfg {
     __device__ static __forceinline__ int bswz(int row) {
         return ES == 4 ? ((row >> 1) & 7) : (ES == 2 ? ((row >> 2) & 3) : ((row >> 3) & 1));
     }
-    // two work-groups per CU whenever registers and LDS allow it, three with a byte mask up to head dim 64: a step of such
+    // two work-groups per CU whenever registers and LDS allow it, three with a byte mask up to head dim 64 (and without a
+    // tile, where all but the dQ kernels of a row-broadcast bias have the registers anyway): a step of such
     // a kernel is short next to its waits, and three of its rings fit LDS (those of a 16-bit bias do not).  D = 64, us, two
     // -> three: forward B=8 H=12 S=1024 51.7 -> 47.6, B=16 H=8 S=2048 250 -> 238; forward and backward, causal, B=8 H=12
     // S=1024 144.7 -> 140.4.  (Head dims up to 32 stayed below 168 registers on their own: no change.)
-    static constexpr int MIN_BLOCKS = D <= 64 && BIAS == 1 ? 3 : (D <= 128 && LDS_BYTES <= 81920) ? 2 : 1;
+    static constexpr int MIN_BLOCKS = D <= 64 && BIAS <= 1 ? 3 : (D <= 128 && LDS_BYTES <= 81920) ? 2 : 1;
 };
 
 // The copy machinery of the kernels tiled by StreamCfg (forward, dQ): one object per thread.
