@@ -1,9 +1,11 @@
-"""GPU tests of the dK / dV / dBias kernel of head dims up to 64 where its tiles end, against the fp32 oracle with the
-tolerances of the parity tests."""
+"""GPU tests of the dK / dV / dBias kernel of the smaller head dims where its tiles end, and of the kernels of head dim 96,
+against the fp32 oracle with the tolerances of the parity tests."""
 import pytest
 import torch
 
-from test_gpu_parity import check, make_inputs, run_oracle, run_ours
+from oracle.attention_oracle import attention_backward, attention_forward
+from test_gpu_parity import check, make_inputs, rel_l2, run_oracle, run_ours
+from triton_flashattn_amd import AlibiBias, flash_attention_fn
 
 pytestmark = pytest.mark.gpu
 
@@ -19,3 +21,47 @@ def test_edges_of_steps_waves_and_tiles(gpu_device, D, kind):
                                         (64, 64, True), (97, 97, True), (128, 128, True), (200, 200, True), (391, 391, True)]):
         q, k, v, do, bias = make_inputs(gpu_device, 1, M, N, 3, D, torch.bfloat16, kind, seed=10 * i + D, trainable=i % 3 != 2)
         check(run_ours(q, k, v, do, bias, causal), run_oracle(q, k, v, do, bias, causal), str((D, kind, M, N, causal)))
+
+
+@pytest.mark.parametrize("d_qk,d_v", [(96, 96), (72, 88), (96, 64), (8, 96)])
+@pytest.mark.parametrize("kind", [None, "alibi", "row", "boolrow", "dense"])
+def test_head_dims_up_to_96(gpu_device, d_qk, d_v, kind):
+    """Head dims between 64 and 96 run at 96: rows of 192 bytes in LDS, the edges of steps and tiles, keys split between
+    work-groups in both directions, and neighbouring columns that hold NaN."""
+    g = torch.Generator().manual_seed(d_qk + d_v)
+    for B, M, N, causal in [(1, 1, 1, False), (1, 33, 65, False), (2, 64, 128, False), (1, 129, 193, False), (1, 40, 2200, False),
+                            (1, 257, 257, True), (2, 128, 128, True), (1, 391, 391, True)]:
+        if kind == "alibi" and N == 1:
+            continue
+        H = 2
+        wide = lambda n, d: torch.cat([torch.randn(B, n, H, d, generator=g), torch.full((B, n, H, 8), float("nan"))], -1).bfloat16().to(gpu_device)[..., :d]
+        q, k, v, do = (t.requires_grad_(i < 3) for i, t in enumerate((wide(M, d_qk), wide(N, d_qk), wide(N, d_v), wide(M, d_v))))
+        bias, dense, grad_of = None, None, None
+        if kind == "alibi":
+            grad_of = torch.tensor([0.02, 0.3], device=gpu_device).requires_grad_(True)
+            bias = AlibiBias(grad_of)
+            dense = bias.materialize(M, N).detach()
+        elif kind in ("row", "dense"):
+            bias = grad_of = torch.randn(1, H, 1 if kind == "row" else M, N, generator=g).expand(1 if kind == "row" else B, -1, -1, -1)
+            bias = grad_of = bias.bfloat16().contiguous().to(gpu_device).requires_grad_(True)
+            dense = bias.detach()
+        elif kind == "boolrow":
+            bias = dense = (torch.rand(B, 1, 1, N, generator=g) > 0.3).index_fill(3, torch.tensor([0]), True).to(gpu_device)
+        out = flash_attention_fn(q, k, v, bias, causal)
+        grads = torch.autograd.grad(out, [q, k, v] + ([] if grad_of is None else [grad_of]), do)
+        full = None if dense is None else dense.expand(B, H, M, N)
+        o, lse = attention_forward(q.detach(), k.detach(), v.detach(), full, causal)
+        dq, dk, dv, db, _ = attention_backward(do, q.detach(), k.detach(), v.detach(), o, lse, full, causal)
+        assert (out.float() - o).abs().max().item() <= 2e-2, (M, N, causal)
+        for name, a, b in zip("qkv", grads, (dq, dk, dv)):
+            assert rel_l2(a, b) <= 5e-2, (name, M, N, causal)
+        if kind == "dense":
+            assert rel_l2(grads[3], db) <= 5e-2, (M, N)
+        elif kind == "row":
+            # (a sum over M rows of terms that are rounded nowhere but in the products: see the ragged tiles' test)
+            limit = 1e-2 * db.abs().sum((0, 2)).max() + M * B * d_v * 2 ** -22
+            assert (grads[3].float() - db.sum((0, 2), keepdim=True)).abs().max() <= limit, (M, N)
+        elif kind == "alibi":
+            i, j = torch.arange(M, device=gpu_device)[:, None], torch.arange(N, device=gpu_device)[None, :]
+            terms = db * -(i * (N / M) - j).abs()
+            assert (grads[3] - terms.sum((0, 2, 3))).abs().max() <= 1e-2 * terms.abs().sum((0, 2, 3)).max(), (M, N)

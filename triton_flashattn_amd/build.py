@@ -15,10 +15,10 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libfa_mi355.so")
 HOST = os.path.join(HERE, "_torch_host.so")
-HEAD_DIMS = (128, 64, 256, 32, 16)  # longest compiles first
+HEAD_DIMS = (128, 64, 256, 96, 32, 16)  # longest compiles first
 # (source, head dim or None): the kernel files are compiled once per head dimension
 UNITS = [(f, d) for f in ("fa_bwd.hip", "fa_fwd.hip", "fa_bwd_narrow.hip", "fa_bwd_shared.hip") for d in HEAD_DIMS
-         if f != "fa_bwd_narrow.hip" or d <= 64] + [("fa_api.hip", None)]
+         if not (f == "fa_bwd_narrow.hip" and d > 96) and not (f == "fa_bwd_shared.hip" and d == 96)] + [("fa_api.hip", None)]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-munsafe-fp-atomics",

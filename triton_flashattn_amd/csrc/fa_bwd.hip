@@ -151,7 +151,10 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
         // each with fused multiply-adds, adds chunk c to chunk c ^ w for w = D / 16, ..., 2 (both in this
         // lane) and last to chunk c ^ 1 (in the lane of the other g).  The dK/dV kernel reads what is stored.
         const T* op = reinterpret_cast<const T*>(p.o) + (int64_t)b * p.so.b + (int64_t)h * p.so.h;
-        float part[C::KSTEPS];
+        constexpr int NP = D == 96 ? 8 : C::KSTEPS;  // (delta of D = 96 is formed like that of 128, whose last chunks are zero)
+        float part[NP];
+#pragma unroll
+        for (int ks = C::KSTEPS; ks < NP; ks++) part[ks] = 0.f;
 #pragma unroll
         for (int ks = 0; ks < C::KSTEPS; ks++) {
             i32x4 ro = {0, 0, 0, 0};
@@ -163,7 +166,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
             part[ks] = a;
         }
 #pragma unroll
-        for (int hs = C::KSTEPS / 2; hs >= 1; hs >>= 1)
+        for (int hs = NP / 2; hs >= 1; hs >>= 1)
 #pragma unroll
             for (int ks = 0; ks < hs; ks++) part[ks] = part[ks] + part[ks + hs];
         delta_i = part[0] + __shfl_xor(part[0], 32, 64);
@@ -215,23 +218,23 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
         if constexpr (!STEP_MASKED && C::NH == 2 && !FROM_DS) {
             constexpr int NS = 2 * C::KSTEPS, NP = 2 * C::DB;  // matrix instructions of S and dP, and of dQ, per block
             constexpr bool AHEAD = D <= 64;
-            constexpr int NSS = AHEAD ? NS : NS / 8, NPS = AHEAD ? NP : NP / 8;  // operands fetched at a time
+            constexpr int NSS = AHEAD ? NS : (NS + 7) / 8, NPS = AHEAD ? NP : (NP + 7) / 8;  // operands fetched at a time
             auto fence = []() { __builtin_amdgcn_sched_barrier(0); };
             T8 ra[AHEAD ? 1 : 2][NSS], ca[AHEAD ? 1 : 2][NPS];
             f32x16 sc[2], dpc[2];
-            auto load_rows = [&](int nb, int slot) {  // operands slot * NSS .. of S and dP of block nb
+            auto load_rows = [&](int nb, int slot) {  // operands of S and dP of block nb: of slot `slot` of 8, or all
+                const int first = AHEAD ? 0 : slot * NS / 8, last = AHEAD ? NS : (slot + 1) * NS / 8;
 #pragma unroll
-                for (int i = 0; i < NSS; i++) {
-                    const int at = slot * NSS + i;
-                    ra[AHEAD ? 0 : slot & 1][i] = at < C::KSTEPS ? SW::template row8_at<T8>(k_tile + rows_l, nb * 32, at)
+                for (int at = first; at < last; at++) {
+                    ra[AHEAD ? 0 : slot & 1][at - first] = at < C::KSTEPS ? SW::template row8_at<T8>(k_tile + rows_l, nb * 32, at)
                                                                  : SW::template row8_at<T8>(v_tile + rows_l, nb * 32, at - C::KSTEPS);
                 }
             };
             auto load_cols = [&](int nb, int slot) {
+                const int first = AHEAD ? 0 : slot * NP / 8, last = AHEAD ? NP : (slot + 1) * NP / 8;
 #pragma unroll
-                for (int i = 0; i < NPS; i++) {
-                    const int at = slot * NPS + i;
-                    ca[AHEAD ? 0 : slot & 1][i] = SW::template col8_at<T8>(k_tile + cols_l, nb * 32 + (at / C::DB) * 16, at % C::DB);
+                for (int at = first; at < last; at++) {
+                    ca[AHEAD ? 0 : slot & 1][at - first] = SW::template col8_at<T8>(k_tile + cols_l, nb * 32 + (at / C::DB) * 16, at % C::DB);
                 }
             };
             // the matrix instructions of slot j of 8 of S and dP, and of dQ
@@ -239,7 +242,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
                 if (!AHEAD && j < 7) load_rows(nb, j + 1);
 #pragma unroll
                 for (int i = j * NS / 8; i < (j + 1) * NS / 8; i++) {
-                    const T8 a = ra[AHEAD ? 0 : j & 1][AHEAD ? i : i - j * NSS];
+                    const T8 a = ra[AHEAD ? 0 : j & 1][AHEAD ? i : i - j * NS / 8];
                     if (i < C::KSTEPS) sc[nb] = mfma32(a, qreg[i], sc[nb]);
                     else dpc[nb] = mfma32(a, doreg[i - C::KSTEPS], dpc[nb]);
                 }
@@ -248,7 +251,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
                 if (!AHEAD && j < 7) load_cols(nb, j + 1);
 #pragma unroll
                 for (int i = j * NP / 8; i < (j + 1) * NP / 8; i++)
-                    dq_acc[i % C::DB] = mfma32(ca[AHEAD ? 0 : j & 1][AHEAD ? i : i - j * NPS], ds[i / C::DB], dq_acc[i % C::DB]);
+                    dq_acc[i % C::DB] = mfma32(ca[AHEAD ? 0 : j & 1][AHEAD ? i : i - j * NP / 8], ds[i / C::DB], dq_acc[i % C::DB]);
             };
             auto elements = [&](int nb, T8 (&ds)[2], auto&& between) {
                 f32x4 bias4;
@@ -653,7 +656,7 @@ template <int D, int BIAS> struct BwdCfg {
 template <typename T, int D, int BIAS, bool CAUSAL, int DBIAS>
 __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS)>::NT), (BwdCfg<D, tile_kind(BIAS)>::WAVES_PER_SIMD)) void fa_bwd_kernel(const BwdParams p) {
     constexpr int TB = tile_kind(BIAS);  // kind of bias tile that is streamed (none for ALiBi)
-    static_assert(D > 64, "fa_bwd_narrow.hip");
+    static_assert(D > 96, "fa_bwd_narrow.hip");
     typedef BwdCfg<D, TB> C;
     typedef Swz<D> SW;
     typedef typename VecOf<T>::v8 T8;
@@ -1448,12 +1451,13 @@ __global__ __launch_bounds__(LANES) void fa_bwd_slope_reduce_kernel(const BwdPar
     if (lane == 0) reinterpret_cast<float*>(p.dbias)[h] = s;
 }
 
-// fa_bwd_narrow.hip: dK, dV and dBias up to head dim 64
+// fa_bwd_narrow.hip: dK, dV and dBias up to head dim 96
 template <int D> hipError_t launch_bwd_narrow_d(const BwdParams& p, int dtype, int bias, bool causal, int dbias, hipStream_t st);
 
 // dbias: 0 = none, 1 = dense, 2 = reduced in the kernels (see fa_bwd_kernel), 3 = of a shared bias (not here)
 template <typename T, int D> static hipError_t launch_all(const BwdParams& p, int bias, bool causal, int dbias, int stages, hipStream_t st) {
-    constexpr int RPB = 256 / (D / 8);
+    constexpr int PREP_D = D == 96 ? 128 : D;  // (a power of two of chunks per row)
+    constexpr int RPB = 256 / (PREP_D / 8);
     const int64_t rows = (int64_t)p.B * p.H * p.M;
     dim3 rgrid((unsigned)((rows + RPB - 1) / RPB));
     hipError_t e = hipSuccess;
@@ -1513,7 +1517,7 @@ template <typename T, int D> static hipError_t launch_all(const BwdParams& p, in
         return eq;
     };
     if ((stages & 1) && !dq_first) {
-        hipLaunchKernelGGL((fa_bwd_prep_kernel<T, D>), rgrid, dim3(256), 0, st, p);
+        hipLaunchKernelGGL((fa_bwd_prep_kernel<T, PREP_D>), rgrid, dim3(256), 0, st, p);
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
@@ -1526,7 +1530,7 @@ template <typename T, int D> static hipError_t launch_all(const BwdParams& p, in
     // (dbias 3, the gradient of a shared bias, is a kernel of its own: here the bias is only read)
     const int kbias = (p.row_bias_kind != 0 && dbias != 1) ? (p.row_bias_kind == 1 ? 7 : 6) : bias;
     const int kdbias = dbias == 3 ? 0 : dbias;
-    if constexpr (D <= 64) {
+    if constexpr (D <= 96) {
         e = launch_bwd_narrow_d<D>(p, __is_same(T, __bf16), kbias, causal, kdbias, st);
     } else {
 #define FA_CASE(BK, DBK)                                                                                      \
@@ -1570,10 +1574,10 @@ template <typename T, int D> static hipError_t launch_all(const BwdParams& p, in
     return e;
 }
 
-// This file is compiled once per head dimension (-DFA_HEAD_DIM=16 ... 256); each object exports
+// This file is compiled once per head dimension (-DFA_HEAD_DIM=16 ... 256, 96 for those of 128 that are no larger); each object exports
 // launch_bwd_d<FA_HEAD_DIM>.
 #ifndef FA_HEAD_DIM
-#error "compile with -DFA_HEAD_DIM=<16|32|64|128|256>"
+#error "compile with -DFA_HEAD_DIM=<16|32|64|96|128|256>"
 #endif
 template <int D> hipError_t launch_bwd_d(const BwdParams& p, int dtype, int bias, bool causal, int dbias, int stages, hipStream_t st);
 template <> hipError_t launch_bwd_d<FA_HEAD_DIM>(const BwdParams& p, int dtype, int bias, bool causal, int dbias, int stages, hipStream_t st) {

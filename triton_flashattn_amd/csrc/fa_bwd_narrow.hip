@@ -1,4 +1,4 @@
-// dK, dV and dBias for head dims up to 64 (flash_attention.py:237-454).
+// dK, dV and dBias for head dims up to 64, and up to 96 without a bias tile (flash_attention.py:237-454).
 //
 // A work-group of 4 waves owns 128 keys, a wave 32 of them with everything that belongs to them: K and V as operands in
 // registers, the scores, dP, and the accumulators of dK^T and dV^T (128 registers at D = 64).  Query rows stream through
@@ -36,7 +36,7 @@ template <int D, int BIAS> struct NarrowCfg {
     static constexpr int NS = LA + 1;                    // slots of every ring
     static constexpr int ROWS_BYTES = SR * D * 2;        // the Q (or dO) rows of a step, swizzled
     static constexpr int NQD = ROWS_BYTES / 1024;        // 1 KB copies of them
-    static constexpr int QD = NQD >= 4 ? NQD / 4 : 1;    // of which each wave issues this many
+    static constexpr int QD = (NQD + 3) / 4;             // of which each wave issues this many
     static constexpr int STAT_BYTES = 64 * 4;            // LSE (or delta) of a step: a copy is 64 lanes wide
     static constexpr int EPC = ES > 0 ? 16 / ES : 8;     // bias elements per 16-byte chunk
     static constexpr int BCPR = 2 * ES;                  // 16-byte chunks per bias row of 32 keys
@@ -74,7 +74,7 @@ template <> struct BiasBlock<1> {
     __device__ __forceinline__ void load(unsigned slice, int lane) {
         typedef i32x2 __attribute__((address_space(3))) * lds_ptr;
         const int row = ((lane & 15) >> 1), first = 4 * (lane >> 5) + (row & 3) + 8 * (row >> 2);
-        const unsigned at = slice + (unsigned)(first * 32 + 16 * ((lane >> 4) & 1) + 8 * (lane & 1));
+        const unsigned at = formed_here(slice + (unsigned)(first * 32 + 16 * ((lane >> 4) & 1) + 8 * (lane & 1)));
         w[0] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_ptr)(uintptr_t)at);
         w[1] = __builtin_amdgcn_ds_read_tr8_b64_v2i32((lds_ptr)(uintptr_t)(at + 16 * 32));
     }
@@ -83,8 +83,9 @@ template <> struct BiasBlock<1> {
 template <typename V4> struct BiasBlock16 {
     i16x4 raw[4];
     __device__ __forceinline__ void load(unsigned slice, int lane) {
+        const unsigned at = formed_here(slice + 2u * (unsigned)tr_offset(lane, 4 * (lane >> 5), 0, 32));
 #pragma unroll
-        for (int q4 = 0; q4 < 4; q4++) raw[q4] = lds_read_tr4_at(slice + 2u * (unsigned)tr_offset(lane, 8 * q4 + 4 * (lane >> 5), 0, 32));
+        for (int q4 = 0; q4 < 4; q4++) raw[q4] = lds_read_tr4_at(at + 512 * q4);
     }
     __device__ __forceinline__ float get(int i) const { return (float)__builtin_bit_cast(V4, raw[i >> 2])[i & 3]; }
 };
@@ -322,10 +323,10 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
     // ---- where dBias goes.  16 bits: through a dS^T tile of the wave (8-byte stores of 4 rows of a key,
     // ds_read_b64_tr_b16 hands a lane 8 keys of a row).  fp32: over the bias values just read, whose place a lane's dS
     // takes, and out row by row.  Either way 16 bytes per lane. ----
-    E* ds_lds = reinterpret_cast<E*>(smem + C::OFF_DS + wave * C::DS_BYTES);
+    const unsigned ds_tile = lds_base + C::OFF_DS + (unsigned)wave * C::DS_BYTES;
     // lane -> row 16 ((lane/16)%2) + lane%16, keys 8 (lane/32 + 2 it) .. + 7 of the slice
     const int db_row = 16 * ((lane >> 4) & 1) + (lane & 15);
-    const int db_src = (8 * g + ((lane & 15) >> 2)) * C::DSS + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+    const int db_src = 2 * ((8 * g + ((lane & 15) >> 2)) * C::DSS + 16 * ((lane >> 4) & 1) + 4 * (lane & 3));  // (bytes)
     // fp32: lane -> row 8 it + lane / 8, keys 4 (lane % 8) .. + 3, it = 0 .. 3
     const int db32_row = lane >> 3, db32_key = 4 * (lane & 7);
     // rows of whole aligned chunks leave through unconditional buffer stores (chunks outside the tensor get an offset
@@ -425,9 +426,10 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
             };
             auto store_dbias = [&](int nb, int m0) {
                 if constexpr (DB16) {
+                    const unsigned at = formed_here(ds_tile + (unsigned)db_src);
 #pragma unroll
                     for (int it = 0; it < 2; it++) {
-                        const i16x4 lo = lds_read_tr4(ds_lds + db_src + it * 16 * C::DSS), hi = lds_read_tr4(ds_lds + db_src + it * 16 * C::DSS + 4 * C::DSS);
+                        const i16x4 lo = lds_read_tr4_at(at + it * 32 * C::DSS), hi = lds_read_tr4_at(at + it * 32 * C::DSS + 8 * C::DSS);
                         typedef short i16x8 __attribute__((ext_vector_type(8)));
                         const i32x4 v = __builtin_bit_cast(i32x4, (i16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
                         const int m = m0 + db_row, nn = nw + 8 * (g + 2 * it);
@@ -606,6 +608,8 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
                 }
                 if constexpr (DB16) {
                     typedef typename VecOf<E>::v4 E4;
+                    typedef E4 __attribute__((address_space(3))) * lds_ptr;
+                    const unsigned at = formed_here(ds_tile + (unsigned)(2 * (r * C::DSS + 4 * g)));
 #pragma unroll
                     for (int q4 = 0; q4 < 4; q4++) {
                         E4 d4;
@@ -614,7 +618,7 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
                             if constexpr (__is_same(T, E)) d4[e] = ds[q4 >> 1][(q4 & 1) * 4 + e];
                             else d4[e] = (E)dp[q4 * 4 + e];
                         }
-                        *reinterpret_cast<E4*>(ds_lds + r * C::DSS + 8 * q4 + 4 * g) = d4;
+                        *(lds_ptr)(uintptr_t)(at + 16 * q4) = d4;
                     }
                 }
                 if constexpr (DB32) {
@@ -698,10 +702,10 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
     }
 }
 
-// This file is compiled once per head dimension (-DFA_HEAD_DIM=16, 32, 64); each object exports
+// This file is compiled once per head dimension (-DFA_HEAD_DIM=16, 32, 64, 96); each object exports
 // launch_bwd_narrow_d<FA_HEAD_DIM>.  bias: 0 ... 7, dbias: 0, 1 or 2, as the kernel takes them.
 #ifndef FA_HEAD_DIM
-#error "compile with -DFA_HEAD_DIM=<16|32|64>"
+#error "compile with -DFA_HEAD_DIM=<16|32|64|96>"
 #endif
 template <typename T, int BIAS, int DBIAS> static hipError_t launch_one(const BwdParams& p, bool causal, hipStream_t st) {
     const dim3 grid((unsigned)(p.n_ntiles * p.B * p.H));
@@ -713,6 +717,13 @@ template <typename T> static hipError_t launch_typed(const BwdParams& p, int bia
 #define FA_CASE(B, DB) \
     if (bias == B && dbias == DB) return launch_one<T, B, DB>(p, causal, st);
     FA_CASE(0, 0)
+    FA_CASE(5, 0)
+    FA_CASE(5, 2)
+    FA_CASE(6, 0)
+    FA_CASE(6, 2)
+    FA_CASE(7, 0)
+#if FA_HEAD_DIM <= 64
+    // (at 96 there are no registers for a bias tile: fa_bwd_kernel at 128 takes those)
     FA_CASE(1, 0)
     FA_CASE(2, 0)
     FA_CASE(2, 1)
@@ -723,11 +734,7 @@ template <typename T> static hipError_t launch_typed(const BwdParams& p, int bia
     FA_CASE(4, 0)
     FA_CASE(4, 1)
     FA_CASE(4, 2)
-    FA_CASE(5, 0)
-    FA_CASE(5, 2)
-    FA_CASE(6, 0)
-    FA_CASE(6, 2)
-    FA_CASE(7, 0)
+#endif
 #undef FA_CASE
     return hipErrorInvalidValue;
 }

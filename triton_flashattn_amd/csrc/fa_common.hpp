@@ -110,6 +110,8 @@ __device__ __forceinline__ i16x4 lds_read_tr4_at(unsigned addr) {
 // stride: the address of a lane's chunk is (tile + L) ^ step + rows, with ONE per-lane constant
 // L per access pattern (rows_lane for row operands, cols_lane for column gathers), a
 // compile-time `step`, and a compile-time row term that goes into the offset field of the read.
+// (D = 96 has rows of three times 64 bytes: its swizzle moves chunks within 64 bytes, so that the 32 rows of an operand and
+// the 8 of a gather still meet every bank alike, and `step` beyond 64 bytes goes into the offset field too.)
 // A kernel so keeps two address constants per lane instead of one per read.
 template <int D> struct Swz {
     static constexpr int CPR = D / 8;  // chunks per row
@@ -117,7 +119,7 @@ template <int D> struct Swz {
     __device__ static __forceinline__ int f(int row) {
         if (CPR >= 16) return ((row & 3) << 2) | ((row >> 2) & 3);
         if (CPR == 8) return (((row >> 1) & 1) << 2) | ((row >> 2) & 3);
-        if (CPR == 4) return (row >> 2) & 3;
+        if (CPR == 4 || CPR == 12) return (row >> 2) & 3;
         return (row >> 3) & 1;
     }
     __device__ static __forceinline__ int off(int row, int col) {
@@ -141,6 +143,8 @@ template <int D> struct Swz {
         return (unsigned)(r * RB + 16 * (g ^ f(r)));
     }
     template <typename V8> __device__ static __forceinline__ V8 row8_at(unsigned tile_plus_l, int rows, int ks) {
+        if constexpr (CPR == 12)  // (rows of 192 bytes: the swizzle stays within 64 of them, the others are an addition)
+            return __builtin_bit_cast(V8, lds_read16_at((tile_plus_l ^ (unsigned)(32 * (ks & 1))) + (unsigned)(rows * RB + 64 * (ks >> 1))));
         return __builtin_bit_cast(V8, lds_read16_at((tile_plus_l ^ (unsigned)(32 * ks)) + (unsigned)(rows * RB)));
     }
     // Column operand (what col8 returns) for head-dim block db (32 wide) and rows row0 .. row0 + 15,
@@ -149,14 +153,14 @@ template <int D> struct Swz {
     __device__ static __forceinline__ unsigned cols_lane(int lane) {
         const int g = lane >> 5, s = lane & 15;
         const int rl = 4 * g + (s >> 2);
-        const int col = (((lane >> 4) & 1) * 16 + (s & 3) * 4) & (D - 1);
+        const int col = (((lane >> 4) & 1) * 16 + (s & 3) * 4) & (D < 32 ? D - 1 : 31);
         return (unsigned)(rl * RB + 16 * ((col >> 3) ^ f(rl)) + 2 * (col & 7));
     }
     template <typename V8> __device__ static __forceinline__ V8 col8_at(unsigned tile_plus_l, int row0, int db) {
         constexpr unsigned H = CPR == 2 ? 16u : 32u;  // f(row + 8) ^ f(row), as a byte offset
-        const unsigned x = (unsigned)((64 * db) & (RB - 1));
-        i16x4 lo = lds_read_tr4_at((tile_plus_l ^ x) + (unsigned)(row0 * RB));
-        i16x4 hi = lds_read_tr4_at((tile_plus_l ^ x ^ H) + (unsigned)((row0 + 8) * RB));
+        const unsigned x = CPR == 12 ? 0u : (unsigned)((64 * db) & (RB - 1)), y = CPR == 12 ? (unsigned)(64 * db) : 0u;
+        i16x4 lo = lds_read_tr4_at((tile_plus_l ^ x) + (unsigned)(row0 * RB) + y);
+        i16x4 hi = lds_read_tr4_at((tile_plus_l ^ x ^ H) + (unsigned)((row0 + 8) * RB) + y);
         typedef short i16x8 __attribute__((ext_vector_type(8)));
         return __builtin_bit_cast(V8, (i16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
     }
@@ -379,7 +383,7 @@ template <int D, int BIAS> struct StreamCfg {
     static constexpr int EPC = ES > 0 ? 16 / ES : 8; // bias elements per 16-byte chunk
     static constexpr int STEP_BYTES = BK * D * 2;    // K (or V) rows of one step, unpadded, swizzled
     static constexpr int NKD = STEP_BYTES / 1024;    // 1 KB copies per K (or V) step
-    static constexpr int KD = NKD >= 4 ? NKD / 4 : 1;  // of which each wave issues this many
+    static constexpr int KD = (NKD + 3) / 4;         // of which each wave issues this many
     static constexpr int NKV = LA + 1;               // K/V ring slots
     static constexpr int O_BYTES = BM * OS * 2;
     static constexpr int KV_BYTES = 2 * NKV * STEP_BYTES;
@@ -637,7 +641,7 @@ template <typename T, int D, int BIAS, bool WITH_V = true> struct KeyStream {
             // unaligned bias rows or non-unit key stride: one element per lane, 16 rows per lane,
             // RB loads in flight together (clamped addresses instead of branches; what lies outside
             // the bias is masked where it is used)
-            if constexpr (D >= 128 && C::ES == 4) {
+            if constexpr (D > 64 && C::ES == 4) {
                 // (no register to spare in this variant: one row at a time)
                 if (lane < 32) {
 #pragma unroll 1
@@ -649,7 +653,7 @@ template <typename T, int D, int BIAS, bool WITH_V = true> struct KeyStream {
                     }
                 }
             } else {
-                constexpr int RB = D >= 128 ? 4 : (D == 64 && BIAS == 1 ? 8 : 16);  // as many as the registers of the kernel allow (16: 190 at D = 64)
+                constexpr int RB = D > 64 ? 4 : (D == 64 && BIAS == 1 ? 8 : 16);  // as many as the registers of the kernel allow (16: 190 at D = 64)
                 const int key = lane & 31;
                 int n = k * C::BK + key;
                 n = n < N ? n : N - 1;

@@ -599,10 +599,10 @@ template <typename T, int D> static hipError_t launch_bias(const FwdParams& p, i
     return hipErrorInvalidValue;
 }
 
-// This file is compiled once per head dimension (-DFA_HEAD_DIM=16 ... 256); each object exports
+// This file is compiled once per head dimension (-DFA_HEAD_DIM=16 ... 256, 96 for those of 128 that are no larger); each object exports
 // launch_fwd_d<FA_HEAD_DIM>.  dtype: 0 = fp16, 1 = bf16.  The caller has validated every argument.
 #ifndef FA_HEAD_DIM
-#error "compile with -DFA_HEAD_DIM=<16|32|64|128|256>"
+#error "compile with -DFA_HEAD_DIM=<16|32|64|96|128|256>"
 #endif
 template <int D> hipError_t launch_fwd_d(const FwdParams& p, int dtype, int bias, bool causal, hipStream_t st);
 template <> hipError_t launch_fwd_d<FA_HEAD_DIM>(const FwdParams& p, int dtype, int bias, bool causal, hipStream_t st) {
