@@ -33,6 +33,8 @@ constexpr float kMask = -1.0e6f;  // additive mask term, in log2 units
 template <typename T> struct VecOf;
 template <> struct VecOf<__bf16> { typedef bf16x8 v8; typedef bf16x4 v4; };
 template <> struct VecOf<_Float16> { typedef f16x8 v8; typedef f16x4 v4; };
+template <> struct VecOf<float> { typedef f32x4 v4; };  // (types of a bias; named, not used, where another one is streamed)
+template <> struct VecOf<unsigned char> { typedef unsigned char v4 __attribute__((ext_vector_type(4))); };
 
 __device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
@@ -368,11 +370,15 @@ struct LiveChunks {
 // keys, K/V in a ring of 3 slots (two steps ahead), the bias in a ring of 4 slots per wave (three
 // steps ahead).  Without: steps of 64 keys, K/V double buffered (one step ahead), which halves the
 // number of barriers.
-template <int D, int BIAS> struct StreamCfg {
-    static constexpr int NH = BIAS == 0 ? 2 : 1;     // 32-key blocks per step
+// The forward's byte masks and 16-bit biases up to head dim 64 (WIDE): steps of 64 keys too, double buffered like K and V
+// (forward, us, 32 -> 64: causal, bf16 bias, B=2 H=16 S=2048 D=64 42.7 -> 38.6, byte mask B=4 H=16 S=1024 D=32 25.9 -> 20.9,
+// B=8 H=12 S=1024 D=64 34.9 -> 33.6; the dQ kernel, with a third product between the same exponentials, loses 1 to 2 %).
+template <int D, int BIAS, bool WIDE = false> struct StreamCfg {
+    static constexpr bool WIDE_TILE = WIDE && D <= 64 && BIAS >= 1 && BIAS <= 3;
+    static constexpr int NH = BIAS == 0 || WIDE_TILE ? 2 : 1;  // 32-key blocks per step
     // steps the K/V copies run ahead (an fp32 bias: shallower rings, so that two work-groups fit a
     // CU: measured 27 % faster in the forward than one work-group with the deeper rings)
-    static constexpr int LA = (BIAS == 0 || BIAS == 4) ? 1 : 2;
+    static constexpr int LA = (BIAS == 0 || BIAS == 4 || WIDE_TILE) ? 1 : 2;
     static constexpr int BM = 128, BK = 32 * NH, NT = 256;
     static constexpr int DP = D < 32 ? 32 : D;       // head dim padded to one 32-wide MFMA block
     static constexpr int OS = DP + 8;                // O staging row stride (elements)
@@ -389,9 +395,11 @@ template <int D, int BIAS> struct StreamCfg {
     static constexpr int KV_BYTES = 2 * NKV * STEP_BYTES;
     static constexpr int BCPR = 2 * ES;              // 16-byte chunks per bias row of 32 keys
     static constexpr int BROW = 32 * ES;             // bytes per bias row of a slot
-    static constexpr int BSLOT = 32 * BROW;          // one wave's bias slice of one step
+    static constexpr int BBLOCK = 32 * BROW;         // one wave's bias slice of one 32-key block
+    static constexpr int BSLOT = NH * BBLOCK;        // ... of one step
     static constexpr int BCH = BSLOT / 1024;         // 1 KB copies per bias slice
-    static constexpr int NBS = BIAS == 4 ? 3 : 4;    // bias ring slots per wave
+    static constexpr int BPB = BBLOCK / 1024 > 0 ? BBLOCK / 1024 : 1;  // ... of them per block
+    static constexpr int NBS = WIDE_TILE ? 2 : BIAS == 4 ? 3 : 4;  // bias ring slots per wave
     static constexpr int BIAS_BYTES = 4 * NBS * BSLOT;
     // (the output tile is staged over the K/V slots and, where it is larger, into the bias rings
     // behind them: all of them are dead by then)
@@ -413,8 +421,8 @@ template <int D, int BIAS> struct StreamCfg {
 // Completion of the copies is counted by hand: they complete in issue order and every wave issues
 // the same number every step, also past the last step (clamped rows, never used).
 // WITH_V = false leaves the V rows out (a kernel that only needs K).
-template <typename T, int D, int BIAS, bool WITH_V = true> struct KeyStream {
-    typedef StreamCfg<D, BIAS> C;
+template <typename T, int D, int BIAS, bool WITH_V = true, bool WIDE = false> struct KeyStream {
+    typedef StreamCfg<D, BIAS, WIDE> C;
     typedef Swz<D> SW;
     typedef typename BiasElem<BIAS>::type E;
     unsigned char* smem;      // K slots, then V slots, then the bias rings of the four waves
@@ -537,10 +545,10 @@ template <typename T, int D, int BIAS, bool WITH_V = true> struct KeyStream {
             const uint64_t base = uniform_ptr(bp);
 #pragma unroll
             for (int it = 0; it < C::BCH; it++) {
-                const int c = it * 64 + lane;
+                const int c = (it % C::BPB) * 64 + lane;
                 const int row = c / C::BCPR;
                 int m = mw + row;
-                int n = k * C::BK + ((c % C::BCPR) ^ C::bswz(row)) * C::EPC;
+                int n = k * C::BK + it / C::BPB * 32 + ((c % C::BCPR) ^ C::bswz(row)) * C::EPC;
                 m = m < M ? m : M - 1;
                 n = n < N ? n : 0;
                 // a (batch, head) slice that takes this path is smaller than 2 GiB
@@ -557,7 +565,8 @@ template <typename T, int D, int BIAS, bool WITH_V = true> struct KeyStream {
             run_b = uniform_ptr(reinterpret_cast<const unsigned char*>(bp) + ((int64_t)mw * sbm + (int64_t)k_b * C::BK) * C::ES);
             // (2-byte elements: a copy covers 16 rows and the chunk order depends on (row / 4) % 4;
             // 1-byte elements: one copy per slice)
-            static_assert(C::ES == 4 || C::ES == 2 || C::BCH == 1, "chunk order repeats from copy to copy");
+            static_assert(C::ES == 4 || C::ES == 2 || C::BPB == 1, "chunk order repeats from copy to copy");
+            static_assert(C::ES != 4 || C::NH == 1, "one offset per copy of a block");
 #pragma unroll
             for (int it = 0; it < NBOFF; it++) {
                 const int c = it * 64 + lane;
@@ -596,7 +605,7 @@ template <typename T, int D, int BIAS, bool WITH_V = true> struct KeyStream {
 #pragma unroll
             for (int it = 0; it < C::BCH; it++) {
                 const unsigned off = C::ES == 4 ? lean_boff[it < NBOFF ? it : 0]
-                                                : lean_boff[0] + (unsigned)(it * (64 / C::BCPR) * (int)sbm * C::ES);
+                                                : lean_boff[0] + (unsigned)((it % C::BPB) * (64 / C::BCPR) * (int)sbm * C::ES + it / C::BPB * 32 * C::ES);
                 lds_copy16(run_b, off, dst + it * 1024);
             }
             run_b += C::BK * C::ES;
@@ -631,11 +640,12 @@ template <typename T, int D, int BIAS, bool WITH_V = true> struct KeyStream {
     // Top of step k: wait for its K/V rows (and with them its bias slice, issued earlier) and
     // publish them.  The slots that step k - 1 read are free from here on.
     template <bool BV> __device__ __forceinline__ void begin_step(int k) {
-        static_assert(BIAS == 0 || C::LA < C::NBS - 1, "the bias slice of a step must be issued before its K/V rows");
+        static_assert(BIAS == 0 || C::LA <= C::NBS - 1, "the bias slice of a step must be issued in time");
+        constexpr bool EARLY = C::LA < C::NBS - 1;  // the bias slice of a step is issued before its K/V rows
         constexpr int OPS = (WITH_V ? 2 : 1) * C::KD + (BV ? C::BCH : 0);  // copies per wave per step
         // K/V of this step were issued LA steps ago; the bias copies issued right after them and
         // the copies of the steps since may still be in flight
-        wait_vmcnt<(BV ? C::BCH : 0) + OPS*(C::LA - 1)>();
+        wait_vmcnt<(BV && EARLY ? C::BCH : 0) + OPS*(C::LA - 1)>();
         lds_barrier();
         if constexpr (C::ES != 0 && !BV) {
             // unaligned bias rows or non-unit key stride: one element per lane, 16 rows per lane,
@@ -655,10 +665,11 @@ template <typename T, int D, int BIAS, bool WITH_V = true> struct KeyStream {
             } else {
                 constexpr int RB = D > 64 ? 4 : (D == 64 && BIAS == 1 ? 8 : 16);  // as many as the registers of the kernel allow (16: 190 at D = 64)
                 const int key = lane & 31;
-                int n = k * C::BK + key;
-                n = n < N ? n : N - 1;
 #pragma unroll 1
-                for (int j0 = 0; j0 < 16; j0 += RB) {
+                for (int jb = 0; jb < 16 * C::NH; jb += RB) {
+                    const int j0 = jb % 16, nb = jb / 16;
+                    int n = k * C::BK + nb * 32 + key;
+                    n = n < N ? n : N - 1;
                     E vals[RB];
 #pragma unroll
                     for (int j = 0; j < RB; j++) {
@@ -668,7 +679,7 @@ template <typename T, int D, int BIAS, bool WITH_V = true> struct KeyStream {
                     }
 #pragma unroll
                     for (int j = 0; j < RB; j++)
-                        *reinterpret_cast<E*>(b_lds(k) + b_off(2 * (j0 + j) + (lane >> 5), key)) = vals[j];
+                        *reinterpret_cast<E*>(b_lds(k) + nb * C::BBLOCK + b_off(2 * (j0 + j) + (lane >> 5), key)) = vals[j];
                 }
             }
         }

@@ -54,15 +54,15 @@ constexpr Growth growth_rule(int bias, int D, bool causal) {
     return (tile && D <= 64 && !causal) || (bias == 6 && D <= 64) || ((tile || bias == 6) && D > 128) ? kAfter : kSum;
 }
 
-// The K/V stream of a row-broadcast bias (kinds 6, 7) is tiled like that of ALiBi, in steps of 32
-// keys: the bias values of a block need the registers that 64-key steps spend on a second block of
-// scores.
-constexpr int fwd_stream_kind(int bias) { return bias >= 5 ? 6 : bias; }
+// The K/V stream of a row-broadcast bias (kinds 6, 7) is tiled like that without a bias up to head dim 64 (so that it takes
+// the steps, and the bits, of the same mask written out), above like that of ALiBi, in steps of 32 keys: the bias values of a
+// block need the registers that 64-key steps spend on a second block of scores.
+constexpr int fwd_stream_kind(int bias, int D) { return bias >= 6 && D <= 64 ? 0 : bias >= 5 ? 6 : bias; }
 
 template <typename T, int D, int BIAS, bool CAUSAL>
-__global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOCKS)) void fa_fwd_kernel(const FwdParams p) {
+__global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>::MIN_BLOCKS)) void fa_fwd_kernel(const FwdParams p) {
     constexpr int TB = tile_kind(BIAS);  // kind of bias tile that is streamed (none for ALiBi)
-    typedef StreamCfg<D, fwd_stream_kind(BIAS)> C;
+    typedef StreamCfg<D, fwd_stream_kind(BIAS, D), true> C;
     typedef Swz<D> SW;
     typedef typename VecOf<T>::v8 T8;
     typedef typename VecOf<T>::v4 T4;
@@ -119,7 +119,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
     // wait for the lane's own loads would be one for all of them (byte mask, B=8 H=12 S=1024 D=64: dQ 40.5 -> 42.7).
     const LiveChunks chunks{p.d_qk / 8, p.qk_inv};
     const unsigned rows_l = SW::rows_lane(lane), cols_l = SW::cols_lane(lane);
-    KeyStream<T, D, fwd_stream_kind(BIAS)> ks_;
+    KeyStream<T, D, fwd_stream_kind(BIAS, D), true, true> ks_;
     ks_.init(smem, kp, vp, bp, p.sk.s, p.sv.s, p.sbias.m, p.sbias.n, M, N, mw, wave, lane, chunks, p.d_v / 8);
     const bool bias_copies = TB != 0 && p.bias_vec;
     if constexpr (TB == 0) ks_.template prologue<false>();
@@ -188,9 +188,8 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
         const int n0 = k * BK;
         ks_.template begin_step<BV>(k);
         const unsigned k_rows = ks_.k_addr(k) + rows_l, v_cols = ks_.v_addr(k) + cols_l;  // operand reads by address
-        const unsigned char* b_lds = ks_.b_lds(k);
-        static_assert(TB == 0 || C::NH == 1, "a bias slot covers one 32-key block");
-        // Interior steps of two blocks (no bias): the matrix instructions of one block are issued between
+        const unsigned char* b_slot = ks_.b_lds(k);
+        // Interior steps of two blocks: the matrix instructions of one block are issued between
         // the exponentials of the other, S of block 1 under the exponentials of block 0 and the PV product
         // of block 0 under those of block 1, one fenced slot per two score elements.  Their LDS operands are
         // fetched a phase ahead; head dim 256 has no registers for that and fetches them one slot ahead.  (Bound by
@@ -201,6 +200,9 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
             constexpr int NS = C::KSTEPS, NP = 2 * C::DB;  // matrix instructions of S and of PV per block
             constexpr bool AHEAD = D <= 128;
             constexpr int NSS = AHEAD ? NS : NS / 8, NPS = AHEAD ? NP : NP / 8;  // operands fetched at a time
+            // units of the scores once their bias is in: raw dot product without one, log2 with a mask, else natural
+            constexpr bool LOG2 = TB == 1 || BOOLROW, RAW = TB == 0 && !ROWB;
+            const float to_log2 = RAW ? qk_scale : LOG2 ? 1.f : kLog2e;
             T8 ka[2][NSS], va[2][NPS];
             f32x16 sc[2];
             auto load_k = [&](int nb, int slot) {  // operands slot * NSS .. of S of block nb
@@ -236,7 +238,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
 #pragma unroll
                     for (int e = 0; e < 2; e++) {
                         const int i = 2 * j + e;
-                        const float pv = fast_exp2(__builtin_fmaf(x[i], qk_scale, -m_i));
+                        const float pv = LOG2 ? fast_exp2(x[i] - m_i) : fast_exp2(__builtin_fmaf(x[i], to_log2, -m_i));
                         rs += pv;
                         out[i >> 3][i & 7] = (T)pv;
                     }
@@ -249,10 +251,47 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
                     float mx = -INFINITY;
 #pragma unroll
                     for (int i = 0; i < 16; i++) mx = fmaxf(mx, x[i]);
-                    raise(pair_max(mx) * qk_scale);
+                    raise(pair_max(mx) * to_log2);
                     rs = exps(x, out, [](int) {});
+                    if (GROWTH == kAfter) rising = k > 0;
                 }
                 l_i += rs;
+            };
+            auto add_bias = [&](f32x16& x, int nb) {
+                if constexpr (ROWB) {
+#pragma unroll
+                    for (int q4 = 0; q4 < 4; q4++) {
+                        const f32x4 w = *reinterpret_cast<const f32x4*>(row_lds + n0 + nb * 32 + 8 * q4 + 4 * g);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) x[q4 * 4 + e] = x[q4 * 4 + e] * (LOG2 ? qk_scale : p.sm_scale) + w[e];
+                    }
+                } else if constexpr (TB != 0) {
+#pragma unroll
+                    for (int q4 = 0; q4 < 4; q4++) {
+                        const unsigned char* at = b_slot + nb * C::BBLOCK + ks_.b_off(r, 8 * q4 + 4 * g);
+                        if constexpr (TB == 1) {
+                            const unsigned int w = *reinterpret_cast<const unsigned int*>(at);
+#pragma unroll
+                            for (int e = 0; e < 4; e++) {
+                                const int i = q4 * 4 + e;
+                                x[i] = ((w >> (8 * e)) & 0xffu) != 0 ? x[i] * qk_scale : x[i] * qk_scale + kMask;
+                            }
+                        } else {
+                            const typename VecOf<E>::v4 hv = *reinterpret_cast<const typename VecOf<E>::v4*>(at);
+#pragma unroll
+                            for (int e = 0; e < 4; e++) x[q4 * 4 + e] = x[q4 * 4 + e] * p.sm_scale + (float)hv[e];
+                        }
+                    }
+                }
+            };
+            auto look_ahead = [&](const f32x16& x) {
+                float mx = -INFINITY;
+#pragma unroll
+                for (int i = 0; i < 16; i++) mx = fmaxf(mx, x[i]);
+                mx = pair_max(mx) * to_log2;
+                const bool higher = __builtin_amdgcn_ballot_w64(mx > m_i + 8.f) != 0;
+                if (higher) raise(mx);
+                if (GROWTH == kAfter) rising = higher;
             };
             load_k(0, 0);
             if (AHEAD) load_k(1, 0);
@@ -265,6 +304,8 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
             issue_ahead();  // in the shadow of the MFMAs just issued
             if (!AHEAD) load_k(1, 0);
             if (AHEAD) load_v(0, 0);
+            add_bias(sc[0], 0);
+            if (GROWTH != kSum && rising) look_ahead(sc[0]);
             __builtin_amdgcn_sched_barrier(0);
             T8 p0[2], p1[2];
             float rs = exps(sc[0], p0, [&](int j) {
@@ -274,11 +315,20 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
             });
             if (!AHEAD) load_v(0, 0);
             settle(sc[0], p0, rs);
-            rs = exps(sc[1], p1, [&](int j) {
-                __builtin_amdgcn_sched_barrier(0);
-                mma_pv(0, p0, j);
-                __builtin_amdgcn_sched_barrier(0);
-            });
+            add_bias(sc[1], 1);
+            if (GROWTH != kSum && rising) {
+                // (the point may be raised here: what block 0 adds, relative to the one it had, must be in O before)
+#pragma unroll
+                for (int j = 0; j < 8; j++) mma_pv(0, p0, j);
+                look_ahead(sc[1]);
+                rs = exps(sc[1], p1, [](int) {});
+            } else {
+                rs = exps(sc[1], p1, [&](int j) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    mma_pv(0, p0, j);
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+            }
             load_v(1, 0);
             settle(sc[1], p1, rs);
 #pragma unroll
@@ -288,6 +338,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS)>::MIN_BLOC
 #pragma unroll
         for (int nb = 0; nb < C::NH; nb++) {
         const int nh = nb * 32;  // first key of this block inside the step
+        const unsigned char* b_lds = b_slot + nb * C::BBLOCK;
         __builtin_amdgcn_sched_barrier(0);  // keep the blocks apart
         // blocks entirely above this wave's diagonal or past the last key contribute nothing
         if (STEP_MASKED && ((CAUSAL && n0 + nh > mw + 31) || n0 + nh >= N)) {
