@@ -65,3 +65,38 @@ def test_head_dims_up_to_96(gpu_device, d_qk, d_v, kind):
             i, j = torch.arange(M, device=gpu_device)[:, None], torch.arange(N, device=gpu_device)[None, :]
             terms = db * -(i * (N / M) - j).abs()
             assert (grads[3] - terms.sum((0, 2, 3))).abs().max() <= 1e-2 * terms.abs().sum((0, 2, 3)).max(), (M, N)
+
+
+@pytest.mark.parametrize("kind", [None, "bool", "bf16", "f32", "alibi", "row"])
+def test_tiles_of_64_keys_at_head_dim_128(gpu_device, kind):
+    """Few query rows at head dim 128 take 64-key tiles: around the line (512 rows, 1024 with a causal mask), key counts
+    around a tile and a wave, and the slope and row gradients that are summed per tile."""
+    g = torch.Generator().manual_seed(7)
+    H = 2
+    for M, N, causal in [(1, 63, False), (33, 64, False), (100, 65, False), (512, 97, False), (513, 130, False), (96, 333, False),
+                         (64, 64, True), (161, 161, True), (1000, 1000, True), (1025, 1025, True)]:
+        q, k, v, do, bias = make_inputs(gpu_device, 1, M, N, H, 128, torch.bfloat16, kind if kind in ("bool", "bf16", "f32") else None,
+                                        seed=M, trainable=False)
+        if kind in (None, "bool", "bf16", "f32"):
+            check(run_ours(q, k, v, do, bias, causal), run_oracle(q, k, v, do, bias, causal), str((kind, M, N, causal)))
+            continue
+        if kind == "alibi":
+            grad_of = torch.tensor([0.02, 0.3], device=gpu_device).requires_grad_(True)
+            bias = AlibiBias(grad_of)
+            dense = bias.materialize(M, N).detach()
+        else:
+            bias = grad_of = torch.randn(1, H, 1, N, generator=g).bfloat16().to(gpu_device).requires_grad_(True)
+            dense = bias.detach()
+        ins = [t.requires_grad_(True) for t in (q, k, v)]
+        grads = torch.autograd.grad(flash_attention_fn(*ins, bias, causal), ins + [grad_of], do)
+        ref = run_oracle(q.detach(), k.detach(), v.detach(), do, dense.expand(1, H, M, N), causal)
+        for name, a in zip(("dq", "dk", "dv"), grads):
+            assert rel_l2(a, ref[name]) <= 5e-2, (name, M, N, causal)
+        db = ref["dbias"]
+        if kind == "row":
+            limit = 1e-2 * db.abs().sum((0, 2)).max() + M * 128 * 2 ** -22
+            assert (grads[3].float() - db.sum((0, 2), keepdim=True)).abs().max() <= limit, (M, N)
+        else:
+            i, j = torch.arange(M, device=gpu_device)[:, None], torch.arange(N, device=gpu_device)[None, :]
+            terms = db * -(i * (N / M) - j).abs()
+            assert (grads[3] - terms.sum((0, 2, 3))).abs().max() <= 1e-2 * terms.abs().sum((0, 2, 3)).max(), (M, N)

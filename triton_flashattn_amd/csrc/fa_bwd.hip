@@ -585,13 +585,15 @@ template <> struct BiasQuad<4> {
 };
 
 // ---------------------------------------------------------------------------------------------
-template <int D, int BIAS> struct BwdCfg {
-    // waves per role: four pairs of waves on a 128-key tile, two on a 64-key tile for head dim 256,
-    // where a wave needs the whole register file of its SIMD (128 accumulator registers and 64 of the
-    // resident operand before anything streams)
-    static constexpr int WPR = D > 128 ? 2 : 4;
+// W, waves per role: four pairs of waves on a 128-key tile; two on a 64-key tile for head dim 256, where a wave needs the
+// whole register file of its SIMD (128 accumulator registers and 64 of the resident operand before anything streams), and for
+// few query rows at 128, where two such work-groups share a CU (short_rows below).
+constexpr int bwd_waves(int D) { return D > 128 ? 2 : 4; }
+template <int D, int BIAS, int W = bwd_waves(D)> struct BwdCfg {
+    static constexpr int WPR = W;
+    static constexpr bool HALF = D <= 128 && W == 2;  // half of a CU's LDS
     static constexpr int BN = 32 * WPR, NT = 128 * WPR;
-    static constexpr int LDS_LIMIT = 163840;
+    static constexpr int LDS_LIMIT = HALF ? 81920 : 163840;
     static constexpr int BMI = 32;                         // rows of a query block
     static constexpr int DB = D / 32;
     static constexpr int KSTEPS = D / 16;
@@ -620,7 +622,7 @@ template <int D, int BIAS> struct BwdCfg {
     static constexpr int lds_total(int la, int defer) {
         return (2 * la + 3 + defer) * (Q_BYTES + STAT_BYTES) + DS_BYTES + 2 * P_BYTES + WPR * (la + 1) * BT_BYTES;
     }
-    static constexpr int LA = D > 128 ? 1 : (lds_total(3, 1) <= LDS_LIMIT ? 3 : 2);
+    static constexpr int LA = D > 128 ? 1 : HALF ? (lds_total(2, 1) <= LDS_LIMIT ? 2 : 1) : (lds_total(3, 1) <= LDS_LIMIT ? 3 : 2);
     static constexpr bool DEFER_DK = D <= 128 && lds_total(LA, 1) <= LDS_LIMIT;
     static constexpr int NDOB = LA + 1;                    // dO (+delta) buffers
     static constexpr int RING = LA + 1;                    // bias slots per S-wave
@@ -634,7 +636,7 @@ template <int D, int BIAS> struct BwdCfg {
     static constexpr int LOOP_BYTES = OFF_BIAS + WPR * RING * BT_BYTES;
     static constexpr int LDS_BYTES = LOOP_BYTES;
     static_assert(LDS_BYTES <= LDS_LIMIT, "LDS budget of the configuration");
-    static constexpr int WAVES_PER_SIMD = WPR == 2 ? 1 : 2;
+    static constexpr int WAVES_PER_SIMD = D > 128 ? 1 : 2;
 };
 
 // Work split inside a work-group of 8 waves.  Waves 0-3 ("S-waves") and waves 4-7 ("dP-waves")
@@ -653,11 +655,11 @@ template <int D, int BIAS> struct BwdCfg {
 // (flash_attention.py:307-308); 2 = reduced in the kernel: for a float bias the sums of dS over the
 // query rows, one fp32 per (batch, head, key), for ALiBi the gradient of the slope, one fp32 per
 // (batch, head, key tile, wave); a second small kernel sums those over the broadcast dimensions.
-template <typename T, int D, int BIAS, bool CAUSAL, int DBIAS>
-__global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS)>::NT), (BwdCfg<D, tile_kind(BIAS)>::WAVES_PER_SIMD)) void fa_bwd_kernel(const BwdParams p) {
+template <typename T, int D, int BIAS, bool CAUSAL, int DBIAS, int W>
+__global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, tile_kind(BIAS), W>::WAVES_PER_SIMD)) void fa_bwd_kernel(const BwdParams p) {
     constexpr int TB = tile_kind(BIAS);  // kind of bias tile that is streamed (none for ALiBi)
     static_assert(D > 96, "fa_bwd_narrow.hip");
-    typedef BwdCfg<D, TB> C;
+    typedef BwdCfg<D, TB, W> C;
     typedef Swz<D> SW;
     typedef typename VecOf<T>::v8 T8;
     typedef typename VecOf<T>::v4 T4;
@@ -1412,10 +1414,22 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS)>::NT), (BwdCfg<D, tile_k
 }
 
 // ---------------------------------------------------------------------------------------------
-template <typename T, int D, int BIAS, bool CAUSAL, int DBIAS>
+// Few query rows at head dim 128: tiles of 64 keys, two work-groups to a CU.  What a tile costs beyond its steps (its operands,
+// its first copies, two steps of skew, its stores: about 16 us) is then spent next to the steps of another one.  us, 128 -> 64
+// keys: no bias B=8 H=12 S=512 53.0 -> 44.7, M=256 N=4096 H=32 83.3 -> 76.0; causal S=1024 95.7 -> 85.1, with a byte mask 108.6 ->
+// 97.5, causal B=2 H=8 S=512 24.1 -> 17.3.  With more rows the second reading of Q and dO costs as much (B=4 H=16 S=2048 289 ->
+// 293, byte mask B=2 H=16 S=1024 51.6 -> 52.6), and where dBias is written the shallow rings cost more (M=N=4096 712 -> 928).
+constexpr bool short_rows(int M, bool causal) { return M <= 512 || (causal && M <= 1024); }
+constexpr bool short_rows_built(int bias, int dbias) { return dbias == 0 || (dbias == 2 && bias >= 5); }
+
+template <typename T, int D, int BIAS, bool CAUSAL, int DBIAS, int W = bwd_waves(D)>
 static hipError_t launch_main(const BwdParams& p, hipStream_t st) {
+    // (the host has put 64-key tiles into p: short_rows)
+    if constexpr (D == 128 && W == 4 && short_rows_built(BIAS, DBIAS)) {
+        if (p.waves_per_role == 2) return launch_main<T, D, BIAS, CAUSAL, DBIAS, 2>(p, st);
+    }
     dim3 grid((unsigned)(p.n_ntiles * p.B * p.H));
-    hipLaunchKernelGGL((fa_bwd_kernel<T, D, BIAS, CAUSAL, DBIAS>), grid, dim3((BwdCfg<D, tile_kind(BIAS)>::NT)), 0, st, p);
+    hipLaunchKernelGGL((fa_bwd_kernel<T, D, BIAS, CAUSAL, DBIAS, W>), grid, dim3((BwdCfg<D, tile_kind(BIAS), W>::NT)), 0, st, p);
     return hipGetLastError();
 }
 
@@ -1530,12 +1544,17 @@ template <typename T, int D> static hipError_t launch_all(const BwdParams& p, in
     // (dbias 3, the gradient of a shared bias, is a kernel of its own: here the bias is only read)
     const int kbias = (p.row_bias_kind != 0 && dbias != 1) ? (p.row_bias_kind == 1 ? 7 : 6) : bias;
     const int kdbias = dbias == 3 ? 0 : dbias;
+    BwdParams pk = p;
+    if (D == 128 && short_rows_built(kbias, kdbias) && short_rows(p.M, causal)) {
+        pk.n_ntiles = (p.N + 63) / 64;
+        pk.waves_per_role = 2;
+    }
     if constexpr (D <= 96) {
         e = launch_bwd_narrow_d<D>(p, __is_same(T, __bf16), kbias, causal, kdbias, st);
     } else {
 #define FA_CASE(BK, DBK)                                                                                      \
     if (kbias == BK && kdbias == DBK)                                                                          \
-        e = causal ? launch_main<T, D, BK, true, DBK>(p, st) : launch_main<T, D, BK, false, DBK>(p, st);
+        e = causal ? launch_main<T, D, BK, true, DBK>(pk, st) : launch_main<T, D, BK, false, DBK>(pk, st);
     FA_CASE(0, 0)
     else FA_CASE(6, 0)
     else FA_CASE(6, 2)
@@ -1558,7 +1577,7 @@ template <typename T, int D> static hipError_t launch_all(const BwdParams& p, in
         if (e != hipSuccess) return e;
         if (dbias == 2) {
             if (bias == 5) {
-                hipLaunchKernelGGL((fa_bwd_slope_reduce_kernel<64>), dim3((unsigned)p.H), dim3(64), 0, st, p);
+                hipLaunchKernelGGL((fa_bwd_slope_reduce_kernel<64>), dim3((unsigned)p.H), dim3(64), 0, st, pk);
             } else {
                 const int64_t outs = (int64_t)(p.sdbias.b == 0 ? 1 : p.B) * (p.sdbias.h == 0 ? 1 : p.H) * p.N;
                 dim3 g((unsigned)((outs + 255) / 256));
