@@ -7,7 +7,8 @@
 // (flash_attention.py:699-704), which become fp32 multiplies inside the kernels.
 //
 //   fa_bwd_prep_kernel   delta[b,h,m] = sum_d o * do                  (flash_attention.py:215-227)
-//   fa_bwd_kernel        dK, dV, dBias of 128 keys per work-group     (flash_attention.py:237-454)
+//   fa_bwd_kernel        dK, dV, dBias of 128 (or 64) keys per work-group, head dims 128 and 256 (flash_attention.py:237-454;
+//                        fa_bwd_narrow.hip holds the kernel of the smaller ones)
 //   fa_bwd_dq_kernel     dQ of 128 query rows per work-group          (flash_attention.py:458-646)
 #include <type_traits>
 
