@@ -101,6 +101,30 @@ def test_fully_masked_rows_causal_follow_a_reference_schedule(gpu_device):
     assert (o[:, live].float() - ref[:, live]).abs().max().item() <= OUT_ATOL
 
 
+# ---------------------------------------------------------------- rows masked by a float bias
+def _padded_rows_case(dev, M, N, H, D, rows, kind, seed, trainable):
+    """Query rows that a float bias of -1e9 masks throughout, as a mask of padded rows does, and whose upstream gradient is
+    zero: their log-sum-exp is about -1.4e9, far below the additive -1.0e6 of a mask."""
+    q, k, v, do, bias = make_inputs(dev, 1, M, N, H, D, torch.bfloat16, kind, seed=seed, trainable=False)
+    bias[:, :, rows, :] = -1.0e9
+    do[:, rows] = 0.0
+    return q, k, v, do, bias.requires_grad_(trainable)
+
+
+@pytest.mark.parametrize("D", [16, 32, 64, 80, 128, 256])
+@pytest.mark.parametrize("kind", ["bf16", "f32"])
+def test_nothing_of_a_masked_last_row_reaches_the_rows_past_it(gpu_device, D, kind):
+    """The dK / dV kernels read the last row again in place of the rows past the end of its block.  The probabilities of
+    these are zero whatever its log-sum-exp is."""
+    for M, N in ((33, 64), (97, 128), (513, 64), (705, 64)):
+        for trainable in (False, True):
+            case = _padded_rows_case(gpu_device, M, N, 2, D, [M - 1], kind, M + D, trainable)
+            ours, ref = run_ours(*case, False), run_oracle(*case, False)
+            for n in ("out", "dq", "dk", "dv"):
+                assert torch.isfinite(ours[n].float()).all(), (n, M, N, trainable)
+            check(ours, ref, str((M, N, trainable)))
+
+
 # ---------------------------------------------------------------- non-positive scales
 @pytest.mark.parametrize("sm_scale", [-0.1, 0.0])
 @pytest.mark.parametrize("bias_kind", [None, "bool", "bf16"])

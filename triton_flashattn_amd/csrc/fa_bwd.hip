@@ -1028,9 +1028,9 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
                 }
             };
             // ---- P (flash_attention.py:281-294) of block nb from its scores; register i
-            // is row m0 + 8 (i/4) + 4 g + i%4, the lane is key my_n.  Blocks that touch a
-            // ragged edge or the causal diagonal follow the reference's additive -1e6 arithmetic term
-            // by term; interior blocks fold everything into one exponent. ----
+            // is row m0 + 8 (i/4) + 4 g + i%4, the lane is key my_n.  Blocks that touch the
+            // last rows or the causal diagonal follow the reference's additive -1e6 arithmetic term
+            // by term, and rows past M have none; interior blocks fold everything into one exponent. ----
             auto make_p = [&](auto&& after_pair) {
                 const int m0 = nb * BMI;
                 // (keys past N need no mask: the lane is the key, and nothing of such a lane is stored.  A ragged
@@ -1056,14 +1056,10 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
                             float pv;
                             if constexpr (MASKED) {
                                 const int m = m0 + ml0 + e;
-                                float x = __fmul_rn(sacc[i], qk_scale);
-                                const bool oob = (m >= M) || (my_n >= N);
-                                float tmask = oob ? kMask : 0.f;
-                                if (CAUSAL) tmask += (m < my_n) ? kMask : 0.f;
-                                float add = NATURAL ? __fmul_rn(bv, kLog2e) : bv;
-                                if (BIAS != 0) add = oob ? kMask : add;  // out-of-range bias reads as masked
-                                x = __fadd_rn(x, __fadd_rn(tmask, add));
-                                pv = fast_exp2(x - lse4[e]);
+                                const float tmask = CAUSAL && m < my_n ? kMask : 0.f;
+                                const float add = NATURAL ? __fmul_rn(bv, kLog2e) : bv;
+                                pv = fast_exp2(__fadd_rn(__fmul_rn(sacc[i], qk_scale), __fadd_rn(tmask, add)) - lse4[e]);
+                                pv = m < M ? pv : 0.f;  // (not an additive term: the LSE read again may lie below any)
                             } else {
                                 // (without a bias the offset is the negated LSE itself: written as 0 - lse it
                                 // would cost a subtraction per element, +0 - x not being -x)

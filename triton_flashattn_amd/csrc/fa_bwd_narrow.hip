@@ -210,7 +210,7 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
 
     // ---- global -> LDS copies of a step: Q and dO rows, LSE and delta, this wave's bias slice.  Copy ci fills bytes
     // [1024 ci, 1024 ci + 1024) of a swizzled slot; every wave issues the same number in every step, completion is counted
-    // (they complete in issue order).  Rows past M re-read the last row: their P is exactly zero. ----
+    // (they complete in issue order).  Rows past M re-read the last row: p_value gives them zero. ----
     unsigned cq_off[C::QD], cdo_off[C::QD];
     int c_idx[C::QD];
 #pragma unroll
@@ -394,8 +394,9 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
             auto load_delta = [&](int nb) { return stat[C::STAT_BYTES / 4 + nb * 32 + 8 * ((lane & 15) >> 2) + 4 * g + (lane & 3)]; };
             auto load_lse = [&](int nb, int q4) { return *reinterpret_cast<const f32x4*>(stat + nb * 32 + 8 * q4 + 4 * g); };
             // ---- P (flash_attention.py:281-294); register i is row m0 + 8 (i/4) + 4 g + i%4, the lane is key my_n.  Blocks
-            // that touch a ragged edge or the causal diagonal follow the reference's additive -1.0e6 arithmetic term by
-            // term; the others fold everything into one exponent.  (Keys past N need no mask: nothing of them is stored.) ----
+            // that touch the last rows or the causal diagonal follow the reference's additive -1.0e6 arithmetic term by
+            // term, and rows past M have none; the others fold everything into one exponent.  (Keys past N need no mask:
+            // nothing of them is stored.) ----
             auto p_value = [&](auto mk_tag, int m0, int i, float s, float lse, const BiasBlock<BIAS>& bias) {
                 constexpr bool MK = decltype(mk_tag)::value;
                 float bv = bias.get(i);
@@ -403,12 +404,10 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
                 if constexpr (BIAS == 6 || BIAS == 7) bv = row_bv;
                 if constexpr (MK) {
                     const int m = m0 + 8 * (i >> 2) + 4 * g + (i & 3);
-                    const bool oob = m >= M || my_n >= N;
-                    float tmask = oob ? kMask : 0.f;
-                    if (CAUSAL) tmask += m < my_n ? kMask : 0.f;
-                    float add = NATURAL ? __fmul_rn(bv, kLog2e) : bv;
-                    if (BIAS != 0) add = oob ? kMask : add;  // out-of-range bias reads as masked
-                    return fast_exp2(__fadd_rn(__fmul_rn(s, qk_scale), __fadd_rn(tmask, add)) - lse);
+                    const float tmask = CAUSAL && m < my_n ? kMask : 0.f;
+                    const float add = NATURAL ? __fmul_rn(bv, kLog2e) : bv;
+                    const float pv = fast_exp2(__fadd_rn(__fmul_rn(s, qk_scale), __fadd_rn(tmask, add)) - lse);
+                    return m < M ? pv : 0.f;  // (not an additive term: the LSE read again may lie below any)
                 } else {
                     float off = BIAS == 0 ? -lse : (NATURAL ? __builtin_fmaf(bv, kLog2e, -lse) : bv - lse);
                     if constexpr (BIAS == 5) {  // distance of the lane's first row to its key, and from there to row i
