@@ -125,6 +125,35 @@ def test_nothing_of_a_masked_last_row_reaches_the_rows_past_it(gpu_device, D, ki
             check(ours, ref, str((M, N, trainable)))
 
 
+@pytest.mark.parametrize("D", [16, 32, 64, 80, 128, 256])
+@pytest.mark.parametrize("kind", ["bf16", "f32", "row"])
+def test_nothing_of_the_keys_past_the_end_reaches_a_masked_row(gpu_device, D, kind):
+    """A last step of keys that is not whole reads the last key again in place of those past the end.  Their weights are
+    zero also in a row whose scores all lie far below the mask term.  Rows of zeros with a bias of -2^22, whose product
+    with log2 e is exact in every order: the output is the mean of v.  Few rows against many keys split the keys."""
+    for M, N, causal in ((70, 77, False), (33, 1, False), (5, 1000, False), (161, 161, True), (97, 321, False)):
+        if causal and kind == "row":
+            continue
+        # (causal: the hidden keys of a row are masked by 1.0e6 alone, so only the last row has none but masked ones)
+        rows = [M - 1] if causal or M < 34 else [0, 33, M - 1]
+        q, k, v, do, bias = _padded_rows_case(gpu_device, M, N, 2, D, rows, "bf16" if kind == "row" else kind, M + D, False)
+        where = (slice(None), rows) if kind != "row" else (slice(None), slice(None), 1)   # "row": every row of one head
+        q[where], do[where] = 0.0, 0.0
+        if kind == "row":
+            bias = bias[:, :, 1:2].clone()
+            bias[:, 1] = -2.0 ** 22
+        else:
+            bias[:, :, rows] = -2.0 ** 22
+        bias.requires_grad_(kind != "row")
+        full = bias.detach().expand(1, 2, M, N)
+        ours, ref = run_ours(q, k, v, do, bias, causal), run_oracle(q, k, v, do, full, causal)
+        assert (ref["out"] - v.float().mean(1, keepdim=True))[where].abs().max().item() < 1e-5
+        check(ours, ref, str((M, N, causal)))
+        if D != 80:   # (the launcher takes the kernels' head dims)
+            _, lse = _flash_attn_fwd(q, k, v, bias.detach(), causal, D ** -0.5)
+            assert torch.allclose(lse, ref["lse2"], atol=3e-3, rtol=2e-7), (M, N, causal)   # one fp32 step at 6e6
+
+
 # ---------------------------------------------------------------- non-positive scales
 @pytest.mark.parametrize("sm_scale", [-0.1, 0.0])
 @pytest.mark.parametrize("bias_kind", [None, "bool", "bf16"])

@@ -350,7 +350,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
             if (nb == 0) issue_ahead();  // in the shadow of the MFMAs just issued
 
             // ---- P = 2^(S*scale + bias - LSE), dS = P (dP - delta) (flash_attention.py:497-517).
-            // Masked tiles follow the reference's additive -1e6 arithmetic term by term.
+            // Masked tiles follow the reference's additive -1e6 arithmetic term by term; keys past N have P = 0.
             auto ds_step = [&](auto masked_tag) {
                 constexpr bool MASKED = decltype(masked_tag)::value;
                 const float nf0 = (float)(key0 + n0 + nh + 4 * g);              // ALiBi: the lane's first key,
@@ -386,18 +386,14 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
                         const int i = q4 * 4 + e;
                         float pv;
                         if constexpr (MASKED) {
-                            float x = __fmul_rn(s[i], qk_scale);
                             const int n = n0 + nh + nl + e;
-                            const bool oob = (n >= N) || (my_m >= M);
-                            float t = oob ? kMask : 0.f;
-                            if (CAUSAL) t += (my_m < n) ? kMask : 0.f;
+                            const float t = CAUSAL && my_m < n ? kMask : 0.f;
                             float add = 0.f;
                             if (BIAS == 1) add = keep[e] ? 0.f : kMask;
                             if (BOOLROW) add = bv[e];
                             if (BIAS >= 2 && !BOOLROW) add = __fmul_rn(bv[e], kLog2e);
-                            if (BIAS != 0) add = oob ? kMask : add;  // out-of-range bias reads as masked
-                            x = __fadd_rn(x, __fadd_rn(t, add));
-                            pv = fast_exp2(x - lse_i);
+                            pv = fast_exp2(__fadd_rn(__fmul_rn(s[i], qk_scale), __fadd_rn(t, add)) - lse_i);
+                            pv = n < N ? pv : 0.f;  // (not an additive term: the LSE may lie below any)
                         } else if constexpr (BIAS == 0) {
                             pv = fast_exp2(__builtin_fmaf(s[i], qk_scale, -lse_i));
                         } else if constexpr (BIAS == 5) {

@@ -29,6 +29,7 @@ template <bool V> struct BoolTag { static constexpr bool value = V; };  // a com
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kMask = -1.0e6f;  // additive mask term, in log2 units
+constexpr float kLowest = -3.402823466e38f;  // score of a key that does not exist
 
 template <typename T> struct VecOf;
 template <> struct VecOf<__bf16> { typedef bf16x8 v8; typedef bf16x4 v4; };

@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
     const float qk_scale = p.sm_scale * kLog2e;
     // (the lowest number, not -inf: keys whose bias is -inf then have exponentials of 0 also where no other key has been
     // seen yet, as in a share of the keys that is padding from end to end)
-    float m_i = -3.402823466e38f, l_i = 0.f;
+    float m_i = kLowest, l_i = 0.f;
     constexpr Growth GROWTH = growth_rule(BIAS, D, CAUSAL);
     bool rising = GROWTH == kRowMax;  // (the same in every lane) the next block's maximum is formed before its exponentials
     f32x16 o_acc[C::DB];
@@ -359,8 +359,8 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
 
         // ---- online softmax step.  `masked` steps (ragged edge, causal diagonal) and a
         // non-positive scale follow the reference's arithmetic term by term: scaled score,
-        // plus additive -1e6 terms in log2 units, plus bias (flash_attention.py:39-53).  Interior
-        // steps skip the mask terms and fold the scale into the exponent.
+        // plus additive -1e6 terms in log2 units, plus bias (flash_attention.py:39-53); keys past N get the lowest
+        // number.  Interior steps skip the mask terms and fold the scale into the exponent.
         // The reference point m_i of the exponentials is arbitrary (out = acc / l and LSE = m + log2 l do
         // not depend on it), so no running maximum is kept: the exponentials are taken against the m_i at
         // hand, and only when the sum of a lane's 8 or 16 of them exceeds kRaise (as at the first keys, where m_i is
@@ -414,14 +414,13 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
                         if constexpr (MASKED) {
                             x = __fmul_rn(s[i], qk_scale);
                             const int n = n0 + nh + nl + e;
-                            float t = (n >= N) ? kMask : 0.f;
-                            if (CAUSAL) t += (my_m < n) ? kMask : 0.f;
+                            const float t = CAUSAL && my_m < n ? kMask : 0.f;
                             float add = 0.f;
                             if (BIAS == 1) add = keep[e] ? 0.f : kMask;
                             if (BOOLROW) add = bv[e];
                             if (BIAS >= 2 && !BOOLROW) add = __fmul_rn(bv[e], kLog2e);
-                            if (BIAS != 0) add = (n >= N) ? kMask : add;  // out-of-range bias reads as masked
                             x = __fadd_rn(x, __fadd_rn(t, add));
+                            x = n < N ? x : kLowest;  // (not an additive term: a float bias may mask a whole row below any)
                         } else if constexpr (BIAS == 1) {
                             x = keep[e] ? s[i] * qk_scale : s[i] * qk_scale + kMask;
                         } else if constexpr (BOOLROW) {
