@@ -476,7 +476,7 @@ int bwd_enqueue(const fa_bwd_args* a, int d_qk, int d_v, void* stream, int stage
     k.n_ntiles = (p.N + bn - 1) / bn;
     k.waves_per_role = bn / 32;
     k.n_mtiles = (p.M + fa::fwd_block_m() - 1) / fa::fwd_block_m();
-    k.causal = p.causal != 0; k.bias_kind = p.bias_dtype; k.shared_splits = splits;
+    k.causal = p.causal != 0; k.bias_kind = p.bias_dtype; k.shared_splits = splits; k.cus = compute_units();
     if (db_mode == 3) {
         k.shared_tiles = (int)shared_tiles(a);
         k.bias_quads = bias_quads_ok(a->bias, a->bias_strides, p) ? 1 : 0;

@@ -8,7 +8,7 @@
 //
 //   fa_bwd_prep_kernel   delta[b,h,m] = sum_d o * do                  (flash_attention.py:215-227)
 //   fa_bwd_kernel        dK, dV, dBias of 128 (or 64) keys per work-group, head dims 128 and 256 (flash_attention.py:237-454;
-//                        fa_bwd_narrow.hip holds the kernel of the smaller ones)
+//                        fa_bwd_narrow.hip holds the kernel of the smaller ones, but for the biases of pair_of_waves)
 //   fa_bwd_dq_kernel     dQ of 128 query rows per work-group          (flash_attention.py:458-646)
 #include <type_traits>
 
@@ -586,13 +586,17 @@ template <> struct BiasQuad<4> {
 // whole register file of its SIMD (128 accumulator registers and 64 of the resident operand before anything streams), and for
 // few query rows at 128, where two such work-groups share a CU (short_rows below).
 constexpr int bwd_waves(int D) { return D > 128 ? 2 : 4; }
+// Biases that this kernel takes up to head dim 64, by the rule of pair_of_waves: fp32 tiles, and a dBias of q's type
+template <typename T> constexpr bool pair_built(int D, int bias, int dbias) {
+    return (bias == 4 && dbias == 1 && D <= 64) || (D == 64 && ((bias == 4 && dbias == 0) || (bias == (__is_same(T, _Float16) ? 2 : 3) && dbias == 1)));
+}
 template <int D, int BIAS, int W = bwd_waves(D)> struct BwdCfg {
     static constexpr int WPR = W;
     static constexpr bool HALF = D <= 128 && W == 2;  // half of a CU's LDS
     static constexpr int BN = 32 * WPR, NT = 128 * WPR;
     static constexpr int LDS_LIMIT = HALF ? 81920 : 163840;
     static constexpr int BMI = 32;                         // rows of a query block
-    static constexpr int DB = D / 32;
+    static constexpr int DB = D < 32 ? 1 : D / 32;
     static constexpr int KSTEPS = D / 16;
     static constexpr int CPR = D / 8;
     static constexpr int DSS = BMI + 4;                    // dS^T tile: elements between two keys
@@ -655,7 +659,7 @@ template <int D, int BIAS, int W = bwd_waves(D)> struct BwdCfg {
 template <typename T, int D, int BIAS, bool CAUSAL, int DBIAS, int W>
 __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, tile_kind(BIAS), W>::WAVES_PER_SIMD)) void fa_bwd_kernel(const BwdParams p) {
     constexpr int TB = tile_kind(BIAS);  // kind of bias tile that is streamed (none for ALiBi)
-    static_assert(D > 96, "fa_bwd_narrow.hip");
+    static_assert(D > 96 || pair_built<T>(D, BIAS, DBIAS), "fa_bwd_narrow.hip");
     typedef BwdCfg<D, TB, W> C;
     typedef Swz<D> SW;
     typedef typename VecOf<T>::v8 T8;
@@ -1415,6 +1419,25 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
 constexpr bool short_rows(int M, bool causal) { return M <= 512 || (causal && M <= 1024); }
 constexpr bool short_rows_built(int bias, int dbias) { return dbias == 0 || (dbias == 2 && bias >= 5); }
 
+// Up to head dim 64: which of the kernels takes a float tile.  A pair of waves keeps two waves per SIMD and the bias of three
+// blocks in flight where a CU gets one tile only, and streams an fp32 bias and its gradient at the copy rate with one tile per
+// CU (two of fa_bwd_narrow.hip read and write twice as many rows at a time: 4.6 TB/s).  us, one wave -> pair, D = 64:
+//   one tile to a CU: fp32 read M=N=1024 H=32 37 -> 33, M=N=2048 H=8 62 -> 50; bf16 and dBias M=N=1500 H=8 57 -> 51, M=N=577 B=2
+//     H=8 27 -> 24, 512 rows the same; at 256 tiles of 2048 rows 73 -> 82.  Below 512 rows the ends of a tile count for more
+//     (fp32 read B=2 H=4 M=N=77 7 -> 8) but for fp32 and dBias, causal, whose tiles are few steps long: B=4 H=8 S=197 17 -> 16.
+//   more, fp32 and dBias, not causal: B=2 H=16 M=N=2016 224 -> 206, M=N=3000 562 -> 528, 256 rows 139 -> 164; causal, where
+//     long tiles are paired with short ones, B=2 H=16 M=N=2048 193 -> 230.
+//   D = 32, fp32 and dBias, not causal, more than one tile to a CU: M=N=2016 214 -> 197, M=N=4096 791 -> 728; with one the same.
+// (measured at 256 CUs, B=1 where none is given)
+static bool pair_of_waves(const BwdParams& p, int D, int bias, int dbias, bool causal) {
+    const int64_t tiles = (int64_t)p.n_ntiles * p.B * p.H;
+    const bool fp32_dbias = bias == 4 && dbias == 1;
+    if (fp32_dbias && !causal && p.M > 512 && (D == 64 || tiles > p.cus)) return true;
+    if (D != 64 || tiles > p.cus) return false;
+    if (p.M < 512) return fp32_dbias && causal;
+    return bias == 4 || tiles < p.cus || p.M < 2048;
+}
+
 template <typename T, int D, int BIAS, bool CAUSAL, int DBIAS, int W = bwd_waves(D)>
 static hipError_t launch_main(const BwdParams& p, hipStream_t st) {
     // (the host has put 64-key tiles into p: short_rows)
@@ -1543,7 +1566,19 @@ template <typename T, int D> static hipError_t launch_all(const BwdParams& p, in
         pk.waves_per_role = 2;
     }
     if constexpr (D <= 96) {
-        e = launch_bwd_narrow_d<D>(p, __is_same(T, __bf16), kbias, causal, kdbias, st);
+        bool pair = false;
+        if constexpr (D <= 64) {
+            pair = pair_built<T>(D, kbias, kdbias) && pair_of_waves(p, D, kbias, kdbias, causal);
+#define FA_CASE(BK, DBK)                                                                                      \
+    if constexpr (pair_built<T>(D, BK, DBK))                                                                   \
+        if (pair && kbias == BK && kdbias == DBK)                                                              \
+            e = causal ? launch_main<T, D, BK, true, DBK>(p, st) : launch_main<T, D, BK, false, DBK>(p, st);
+            FA_CASE(4, 1)
+            FA_CASE(4, 0)
+            FA_CASE(DS_BIAS, 1)
+#undef FA_CASE
+        }
+        if (!pair) e = launch_bwd_narrow_d<D>(p, __is_same(T, __bf16), kbias, causal, kdbias, st);
     } else {
 #define FA_CASE(BK, DBK)                                                                                      \
     if (kbias == BK && kdbias == DBK)                                                                          \

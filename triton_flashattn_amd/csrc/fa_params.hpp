@@ -80,6 +80,7 @@ struct BwdParams {
     int bias_quads, dbias_quads;  // ... four consecutive elements of its rows / of its gradient's may be accessed at once
     int shared_tiles;   // ... tiles of its gradient, over all slices
     int shared_splits;  // ... work-groups that share the (batch, head) pairs of a tile (1: it stores the gradient itself)
+    int cus;            // compute units of the device, for the rules that ask how many tiles one of them gets
     int dq_makes_delta; // the dQ kernel runs before the dK/dV kernel and forms delta itself (and stores it),
                         // in place of fa_bwd_prep_kernel and bit for bit like it
 };
