@@ -5,6 +5,7 @@ import torch
 
 from oracle.attention_oracle import attention_backward, attention_forward
 from test_gpu_parity import check, make_inputs, rel_l2, run_oracle, run_ours
+from test_gpu_parity_edges import _launch_directly
 from triton_flashattn_amd import AlibiBias, flash_attention_fn
 
 pytestmark = pytest.mark.gpu
@@ -113,3 +114,19 @@ def test_float_biases_that_a_pair_of_waves_takes(gpu_device, D, kind):
         for trainable in (True, False):
             q, k, v, do, bias = make_inputs(gpu_device, 1, M, N, H, D, torch.bfloat16, kind, seed=M + D, trainable=trainable)
             check(run_ours(q, k, v, do, bias, causal), run_oracle(q, k, v, do, bias, causal), str((D, kind, M, N, H, causal, trainable)))
+
+
+@pytest.mark.parametrize("D", [16, 32, 64])
+@pytest.mark.parametrize("kind", ["bf16", "f16", "f32"])
+def test_bias_and_gradient_rows_that_allow_no_aligned_accesses(gpu_device, D, kind):
+    """Straight to the kernels, rows of an odd number of keys, dense (element by element) and with a padded pitch (16 bytes at
+    a time), the bias and its gradient each in either."""
+    for i, (M, N, causal) in enumerate([(70, 197, False), (131, 131, True), (33, 5, False), (300, 129, False)]):
+        q, k, v, do, bias = make_inputs(gpu_device, 2, M, N, 2, D, torch.bfloat16, kind, seed=D + i, trainable=False)
+        ref = run_oracle(q, k, v, do, bias, causal)
+        wide = torch.full((2, 2, M, -(-N // 8) * 8), float("nan"), dtype=bias.dtype, device=gpu_device)
+        wide[..., :N] = bias
+        for b in (bias, wide[..., :N]):
+            for out in (torch.empty_like(bias), torch.empty_like(wide)[..., :N]):
+                res = _launch_directly(q, k, v, do, b, out, causal)
+                check(res, ref, str((D, kind, M, N, causal, b.stride(2), out.stride(2))))

@@ -586,9 +586,9 @@ template <> struct BiasQuad<4> {
 // whole register file of its SIMD (128 accumulator registers and 64 of the resident operand before anything streams), and for
 // few query rows at 128, where two such work-groups share a CU (short_rows below).
 constexpr int bwd_waves(int D) { return D > 128 ? 2 : 4; }
-// Biases that this kernel takes up to head dim 64, by the rule of pair_of_waves: fp32 tiles, and a dBias of q's type
-template <typename T> constexpr bool pair_built(int D, int bias, int dbias) {
-    return (bias == 4 && dbias == 1 && D <= 64) || (D == 64 && ((bias == 4 && dbias == 0) || (bias == (__is_same(T, _Float16) ? 2 : 3) && dbias == 1)));
+// Biases that this kernel takes up to head dim 64, by the rule of pair_of_waves
+constexpr bool pair_built(int D, int bias, int dbias) {
+    return D <= 64 && ((bias >= 2 && bias <= 4 && dbias == 1) || (bias == 4 && dbias == 0));
 }
 template <int D, int BIAS, int W = bwd_waves(D)> struct BwdCfg {
     static constexpr int WPR = W;
@@ -659,7 +659,7 @@ template <int D, int BIAS, int W = bwd_waves(D)> struct BwdCfg {
 template <typename T, int D, int BIAS, bool CAUSAL, int DBIAS, int W>
 __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, tile_kind(BIAS), W>::WAVES_PER_SIMD)) void fa_bwd_kernel(const BwdParams p) {
     constexpr int TB = tile_kind(BIAS);  // kind of bias tile that is streamed (none for ALiBi)
-    static_assert(D > 96 || pair_built<T>(D, BIAS, DBIAS), "fa_bwd_narrow.hip");
+    static_assert(D > 96 || pair_built(D, BIAS, DBIAS), "fa_bwd_narrow.hip");
     typedef BwdCfg<D, TB, W> C;
     typedef Swz<D> SW;
     typedef typename VecOf<T>::v8 T8;
@@ -1428,8 +1428,14 @@ constexpr bool short_rows_built(int bias, int dbias) { return dbias == 0 || (dbi
 //   more, fp32 and dBias, not causal: B=2 H=16 M=N=2016 224 -> 206, M=N=3000 562 -> 528, 256 rows 139 -> 164; causal, where
 //     long tiles are paired with short ones, B=2 H=16 M=N=2048 193 -> 230.
 //   D = 32, fp32 and dBias, not causal, more than one tile to a CU: M=N=2016 214 -> 197, M=N=4096 791 -> 728; with one the same.
+//   a dBias of the other 16-bit type: always one wave (M=N=1024 H=32 48 -> 37).
+// Rows of a dBias or its bias that allow no aligned 16-byte accesses: always a pair, whose stores go out of registers, 32 keys
+// of a row each, and which has 16 loads of a lane in flight, not 8 (fp32 dBias B=2 H=8 M=N=577 57 -> 38, bf16 q and fp16 dBias
+// B=2 H=16 M=N=1023 131 -> 59); an fp32 bias of such rows that is only read too (M=N=1023 68 -> 55).
 // (measured at 256 CUs, B=1 where none is given)
-static bool pair_of_waves(const BwdParams& p, int D, int bias, int dbias, bool causal) {
+static bool pair_of_waves(const BwdParams& p, int D, int bias, int dbias, bool own_type, bool causal) {
+    if (!p.bias_vec || (dbias == 1 && !p.dbias_vec)) return true;
+    if (bias != 4 && !own_type) return false;
     const int64_t tiles = (int64_t)p.n_ntiles * p.B * p.H;
     const bool fp32_dbias = bias == 4 && dbias == 1;
     if (fp32_dbias && !causal && p.M > 512 && (D == 64 || tiles > p.cus)) return true;
@@ -1568,14 +1574,14 @@ template <typename T, int D> static hipError_t launch_all(const BwdParams& p, in
     if constexpr (D <= 96) {
         bool pair = false;
         if constexpr (D <= 64) {
-            pair = pair_built<T>(D, kbias, kdbias) && pair_of_waves(p, D, kbias, kdbias, causal);
+            pair = pair_built(D, kbias, kdbias) && pair_of_waves(p, D, kbias, kdbias, kbias == DS_BIAS, causal);
 #define FA_CASE(BK, DBK)                                                                                      \
-    if constexpr (pair_built<T>(D, BK, DBK))                                                                   \
-        if (pair && kbias == BK && kdbias == DBK)                                                              \
-            e = causal ? launch_main<T, D, BK, true, DBK>(p, st) : launch_main<T, D, BK, false, DBK>(p, st);
+    if (pair && kbias == BK && kdbias == DBK)                                                                  \
+        e = causal ? launch_main<T, D, BK, true, DBK>(p, st) : launch_main<T, D, BK, false, DBK>(p, st);
+            FA_CASE(2, 1)
+            FA_CASE(3, 1)
             FA_CASE(4, 1)
             FA_CASE(4, 0)
-            FA_CASE(DS_BIAS, 1)
 #undef FA_CASE
         }
         if (!pair) e = launch_bwd_narrow_d<D>(p, __is_same(T, __bf16), kbias, causal, kdbias, st);

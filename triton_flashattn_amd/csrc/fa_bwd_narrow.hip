@@ -114,8 +114,9 @@ __device__ __forceinline__ float row_bcast(float x, int i) {
     return row_bcast<15>(x);
 }
 
-// DBIAS as in fa_bwd_kernel: 0 = the bias is not trainable; 1 = dBias is written densely; 2 = reduced: the sums of dS over
-// the query rows, or (ALiBi) the slope's gradient, one fp32 per (batch, head, key tile, wave).
+// DBIAS as in fa_bwd_kernel: 0 = the bias is not trainable; 1 = dBias is written densely (rows of both that allow aligned
+// 16-byte accesses: fa_bwd_kernel takes the others); 2 = reduced: the sums of dS over the query rows, or (ALiBi) the slope's
+// gradient, one fp32 per (batch, head, key tile, wave).
 template <typename T, int D, int BIAS, bool CAUSAL, int DBIAS>
 __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) void fa_bwd_narrow_kernel(const BwdParams p) {
     constexpr int TB = tile_kind(BIAS);
@@ -191,19 +192,18 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
     // causal: steps that end above the first key of this tile see none of its keys
     const int t0 = CAUSAL ? n0 / SR : 0, t_end = (M + SR - 1) / SR;
     const bool bias_vec = TB != 0 && p.bias_vec;
-    const bool dbias_vec = DBIAS == 1 && p.dbias_vec;
 
     // rows above the diagonal block of a wave are not visited and owe zeros to dBias
     if (DBIAS == 1 && CAUSAL) {
         const int rows_skipped = nw < M ? nw : M;
         for (int c = lane; c < rows_skipped * C::BCPR; c += 64) {
             const int m = c / C::BCPR, nn = nw + (c % C::BCPR) * C::EPC;
-            E* dst = dbp + (int64_t)m * p.sdbias.m + (int64_t)nn * p.sdbias.n;
-            if (dbias_vec && nn + C::EPC <= N) {
+            E* dst = dbp + (int64_t)m * p.sdbias.m + nn;
+            if (nn + C::EPC <= N) {
                 gst16(dst, i32x4{0, 0, 0, 0});
             } else {
                 for (int e = 0; e < C::EPC; e++)
-                    if (nn + e < N) dst[(int64_t)e * p.sdbias.n] = (E)0.f;
+                    if (nn + e < N) dst[e] = (E)0.f;
             }
         }
     }
@@ -331,7 +331,7 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
     const int db32_row = lane >> 3, db32_key = 4 * (lane & 7);
     // rows of whole aligned chunks leave through unconditional buffer stores (chunks outside the tensor get an offset
     // outside the view), so that the loop has no branch around its stores and can count them
-    const bool db_fast = dbias_vec && (N % C::EPC == 0);
+    const bool db_fast = DBIAS == 1 && N % C::EPC == 0;
     __amdgpu_buffer_rsrc_t db_rsrc = make_buffer(nullptr, 0);
     int db_off[2] = {0, 0};
     const int db_row_bytes = DBIAS == 1 ? (int)p.sdbias.m * C::ES : 0;
@@ -435,13 +435,13 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
                         if constexpr (DB_FAST) {
                             buf_store16(db_rsrc, v, !MASKED || m < M ? db_off[it] + m0 * db_row_bytes : (int)0x80000000);
                         } else if (m < M && nn < N) {
-                            E* dst = dbp + (int64_t)m * p.sdbias.m + (int64_t)nn * p.sdbias.n;
-                            if (dbias_vec && nn + 8 <= N) {
+                            E* dst = dbp + (int64_t)m * p.sdbias.m + nn;
+                            if (nn + 8 <= N) {
                                 gst16(dst, v);
                             } else {
 #pragma unroll
                                 for (int e = 0; e < 8; e++)
-                                    if (nn + e < N) dst[(int64_t)e * p.sdbias.n] = __builtin_bit_cast(E, (short)(v[e >> 1] >> (16 * (e & 1))));
+                                    if (nn + e < N) dst[e] = __builtin_bit_cast(E, (short)(v[e >> 1] >> (16 * (e & 1))));
                             }
                         }
                     }
@@ -456,13 +456,13 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
                         if constexpr (DB_FAST) {
                             buf_store16(db_rsrc, __builtin_bit_cast(i32x4, w), !MASKED || m < M ? db_off[0] + (m0 + 8 * it) * db_row_bytes : (int)0x80000000);
                         } else if (m < M && nn < N) {
-                            float* dst = reinterpret_cast<float*>(dbp) + (int64_t)m * p.sdbias.m + (int64_t)nn * p.sdbias.n;
-                            if (dbias_vec && nn + 4 <= N) {
+                            float* dst = reinterpret_cast<float*>(dbp) + (int64_t)m * p.sdbias.m + nn;
+                            if (nn + 4 <= N) {
                                 gst16(dst, __builtin_bit_cast(i32x4, w));
                             } else {
 #pragma unroll
                                 for (int e = 0; e < 4; e++)
-                                    if (nn + e < N) dst[(int64_t)e * p.sdbias.n] = w[e];
+                                    if (nn + e < N) dst[e] = w[e];
                             }
                         }
                     }
@@ -658,9 +658,8 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
         wait_vmcnt<0>();  // nothing may land in LDS once the work-group is gone
     };
     if constexpr (DBIAS == 1) {
-        if (bias_vec && db_fast) run(std::true_type{}, std::true_type{});
-        else if (bias_vec) run(std::true_type{}, std::false_type{});
-        else run(std::false_type{}, std::false_type{});
+        if (db_fast) run(std::true_type{}, std::true_type{});
+        else run(std::true_type{}, std::false_type{});
     } else if constexpr (TB != 0) {
         if (bias_vec) run(std::true_type{}, std::false_type{});
         else run(std::false_type{}, std::false_type{});
@@ -739,6 +738,7 @@ template <typename T> static hipError_t launch_typed(const BwdParams& p, int bia
 }
 template <int D> hipError_t launch_bwd_narrow_d(const BwdParams& p, int dtype, int bias, bool causal, int dbias, hipStream_t st);
 template <> hipError_t launch_bwd_narrow_d<FA_HEAD_DIM>(const BwdParams& p, int dtype, int bias, bool causal, int dbias, hipStream_t st) {
+    if (dbias == 1 && !(p.bias_vec && p.dbias_vec)) return hipErrorInvalidValue;  // (fa_bwd_kernel's)
     return dtype == 0 ? launch_typed<_Float16>(p, bias, causal, dbias, st) : launch_typed<__bf16>(p, bias, causal, dbias, st);
 }
 
