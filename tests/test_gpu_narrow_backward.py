@@ -130,3 +130,11 @@ def test_bias_and_gradient_rows_that_allow_no_aligned_accesses(gpu_device, D, ki
             for out in (torch.empty_like(bias), torch.empty_like(wide)[..., :N]):
                 res = _launch_directly(q, k, v, do, b, out, causal)
                 check(res, ref, str((D, kind, M, N, causal, b.stride(2), out.stride(2))))
+
+
+def test_tiles_of_64_or_128_keys_with_an_fp32_bias(gpu_device):
+    """An fp32 bias that is only read at head dim 128, in few and in many tiles, around the lines between 64 and 128 keys."""
+    for M, N, H, causal in [(320, 65, 520, False), (321, 65, 520, False), (513, 65, 2, False), (512, 130, 260, False),
+                            (321, 321, 350, True), (320, 320, 350, True), (1000, 1000, 2, True)]:
+        q, k, v, do, bias = make_inputs(gpu_device, 1, M, N, H, 128, torch.bfloat16, "f32", seed=M, trainable=False)
+        check(run_ours(q, k, v, do, bias, causal), run_oracle(q, k, v, do, bias, causal), str((M, N, H, causal)))

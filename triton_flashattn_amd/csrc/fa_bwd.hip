@@ -1414,9 +1414,16 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
 // Few query rows at head dim 128: tiles of 64 keys, two work-groups to a CU.  What a tile costs beyond its steps (its operands,
 // its first copies, two steps of skew, its stores: about 16 us) is then spent next to the steps of another one.  us, 128 -> 64
 // keys: no bias B=8 H=12 S=512 53.0 -> 44.7, M=256 N=4096 H=32 83.3 -> 76.0; causal S=1024 95.7 -> 85.1, with a byte mask 108.6 ->
-// 97.5, causal B=2 H=8 S=512 24.1 -> 17.3.  With more rows the second reading of Q and dO costs as much (B=4 H=16 S=2048 289 ->
-// 293, byte mask B=2 H=16 S=1024 51.6 -> 52.6), and where dBias is written the shallow rings cost more (M=N=4096 712 -> 928).
-constexpr bool short_rows(int M, bool causal) { return M <= 512 || (causal && M <= 1024); }
+// 97.5, causal B=2 H=8 S=512 24.1 -> 17.3; read-only bf16 bias B=8 H=12 S=512 54.9 -> 45.2, B=64 491 -> 496.  With more rows the
+// second reading of Q and dO costs as much (B=4 H=16 S=2048 289 -> 293, byte mask B=2 H=16 S=1024 51.6 -> 52.6), and where dBias is
+// written the shallow rings cost more (M=N=4096 712 -> 928).  An fp32 bias is copied one step ahead only in these rings, which costs
+// more where a CU has many tiles, whose reads overlap anyway: B=8 H=12 S=512 56 -> 47, B=64 H=16 S=512 493 -> 513, causal 432 -> 460;
+// causal B=8 H=12 S=1024 115 -> 112, B=32 H=16 565 -> 642.  Up to 320 rows in any number: M=N=257 B=32 H=16 135 -> 117, M=256 N=8192
+// H=32 196 -> 190.
+static bool short_rows(const BwdParams& p, int bias, bool causal) {
+    if (bias == 4 && (int64_t)((p.N + 127) / 128) * p.B * p.H > (causal ? 4 : 2) * (int64_t)p.cus) return p.M <= 320;
+    return p.M <= 512 || (causal && p.M <= 1024);
+}
 constexpr bool short_rows_built(int bias, int dbias) { return dbias == 0 || (dbias == 2 && bias >= 5); }
 
 // Up to head dim 64: which of the kernels takes a float tile.  A pair of waves keeps two waves per SIMD and the bias of three
@@ -1567,7 +1574,7 @@ template <typename T, int D> static hipError_t launch_all(const BwdParams& p, in
     const int kbias = (p.row_bias_kind != 0 && dbias != 1) ? (p.row_bias_kind == 1 ? 7 : 6) : bias;
     const int kdbias = dbias == 3 ? 0 : dbias;
     BwdParams pk = p;
-    if (D == 128 && short_rows_built(kbias, kdbias) && short_rows(p.M, causal)) {
+    if (D == 128 && short_rows_built(kbias, kdbias) && short_rows(p, kbias, causal)) {
         pk.n_ntiles = (p.N + 63) / 64;
         pk.waves_per_role = 2;
     }
