@@ -10,6 +10,52 @@ from triton_flashattn_amd import AlibiBias, flash_attention_fn
 
 pytestmark = pytest.mark.gpu
 
+# Largest error of a gradient that is summed inside the kernels over the sum of its terms' magnitudes, against 64 bits and
+# with the kernel's own output in delta, so that nothing but fp32 sums and exponentials is left: 2.0e-7 over head dims 32 to
+# 128 and 33 to 1100 rows; four times that.
+SUM_RTOL = 8e-7
+
+
+def dscores(q, k, v, do, out, dense, causal):
+    """dS (B, H, M, N) of the output that the kernels returned, in 64 bits."""
+    q, k, v, out = (t.detach() for t in (q, k, v, out))
+    _, lse = attention_forward(q, k, v, dense, causal, dtype=torch.float64)
+    return attention_backward(do, q, k, v, out, lse, dense, causal, dtype=torch.float64)[3]
+
+
+def add_trend(v, do, causal):
+    """Adds to the first column of v a slope over the keys and to that of do its counterpart over the rows, so that the terms
+    of a slope's gradient do not cancel between rows or tiles: a tile that is lost shows."""
+    M, N = do.shape[1], v.shape[1]
+    i, j = (torch.arange(n, device=v.device)[None, :, None] / n for n in (M, N))
+    v[..., 0] += 6.0 * j
+    do[..., 0] += 6.0 if causal else 6.0 - 12.0 * i
+
+
+def check_slope_gradient(got, ds, causal, tag):
+    """The gradient of ALiBi slopes, the sum of -|i N / M - j| dS per head; no 32 keys of a wave may be lost in it."""
+    M, N = ds.shape[2:]
+    i, j = torch.arange(M, device=ds.device)[:, None], torch.arange(N, device=ds.device)[None, :]
+    terms = ds * -(i * (N / M) - j).abs()
+    limit = SUM_RTOL * terms.abs().sum((0, 2, 3))
+    for first in range(0, N, 32):
+        # (causal: the last key alone is seen by the last row alone, at distance 0)
+        if not (causal and first == N - 1):
+            assert (terms[..., first:first + 32].sum((0, 2, 3)).abs() > limit).all(), ("a loss of 32 keys would not show", tag, first)
+    assert ((got - terms.sum((0, 2, 3))).abs() <= limit).all(), (tag, got, terms.sum((0, 2, 3)))
+
+
+def check_row_gradient(got, ds, tag):
+    """The gradient of a (1, H, 1, N) bias, the sum of dS over batches and rows, key by key: rounded to the bias's type and off
+    by the limit of the sum (and by the rounding of dP - delta where that vanishes)."""
+    want, size = ds.sum((0, 2)), ds.abs().sum((0, 2))
+    limit = torch.finfo(got.dtype).eps / 2 * want.abs() + SUM_RTOL * size + ds.shape[0] * ds.shape[2] * 2.0 ** -22
+    for first in range(0, ds.shape[3], 32):
+        if ds.shape[3] > 1:
+            part = slice(first, first + 32)
+            assert (want[:, part].abs() > 2 * limit[:, part]).any(), ("a loss of 32 keys would not show", tag, first)
+    assert ((got[0, :, 0].double() - want).abs() <= limit).all(), tag
+
 
 @pytest.mark.parametrize("D", [16, 32, 64])
 @pytest.mark.parametrize("kind", [None, "bool", "bf16", "f16", "f32"])
@@ -138,3 +184,22 @@ def test_tiles_of_64_or_128_keys_with_an_fp32_bias(gpu_device):
                             (321, 321, 350, True), (320, 320, 350, True), (1000, 1000, 2, True)]:
         q, k, v, do, bias = make_inputs(gpu_device, 1, M, N, H, 128, torch.bfloat16, "f32", seed=M, trainable=False)
         check(run_ours(q, k, v, do, bias, causal), run_oracle(q, k, v, do, bias, causal), str((M, N, H, causal)))
+
+
+def test_alibi_of_long_tiles_at_head_dim_96(gpu_device):
+    """dK, dV and the slope gradient of ALiBi at head dims up to 96 around the line between the kernels of 96 and 128: 1024
+    rows, and more tiles than there are CUs."""
+    for M, N, H, causal, d in [(1024, 130, 1, False, 96), (1025, 130, 2, False, 72), (1100, 1100, 1, True, 96), (1030, 130, 130, False, 88)]:
+        g = torch.Generator().manual_seed(M)
+        q, k, v, do = (torch.randn(1, n, H, d, generator=g) for n in (M, N, N, M))
+        add_trend(v, do, causal)
+        q, k, v, do = (t.bfloat16().to(gpu_device) for t in (q, k, v, do))
+        slopes = torch.linspace(0.01, 0.002, H, device=gpu_device).requires_grad_(True)
+        dense = AlibiBias(slopes).materialize(M, N).detach()
+        ins = [t.requires_grad_(True) for t in (q, k, v)]
+        out = flash_attention_fn(*ins, AlibiBias(slopes), causal)
+        grads = torch.autograd.grad(out, ins + [slopes], do)
+        ref = run_oracle(q.detach(), k.detach(), v.detach(), do, dense, causal)
+        for name, a in zip(("dq", "dk", "dv"), grads):
+            assert rel_l2(a, ref[name]) <= 5e-2, (name, M, N, causal)
+        check_slope_gradient(grads[3], dscores(q, k, v, do, out, dense, causal), causal, (M, N))

@@ -46,7 +46,18 @@ static hipError_t launch_fwd(const FwdParams& p, int D, int dtype, int bias, boo
 }
 static hipError_t launch_bwd(const BwdParams& p, int D, int dtype, int bias, bool causal, int dbias, int stages, hipStream_t st) {
     const bool bias_tile = bias >= 1 && bias <= 4 && !(p.row_bias_kind != 0 && dbias != 1);
-    switch (bias_tile ? D : tight_head_dim(D, p.d_qk, p.d_v)) {
+    const int kernel_dim = bias_tile ? D : tight_head_dim(D, p.d_qk, p.d_v);
+    // ALiBi at 96: dK / dV of long tiles, one to a CU, by the pair of waves of 128, whose distances and slope gradient one wave
+    // has to form beside everything else (us, at 96 -> at 128: M=N=2048 H=8 62 -> 59, with the gradient 69 -> 63, M=N=4096 H=4 129 ->
+    // 114; at 1024 rows, H=32, 2 % the other way, at two tiles to a CU 26 %)
+    if (kernel_dim == 96 && bias == 5 && (stages & 2) && p.M > 1024 && (int64_t)p.n_ntiles * p.B * p.H <= p.cus) {
+        if (stages & 5) {
+            const hipError_t e = launch_bwd_d<96>(p, dtype, bias, causal, dbias, stages & ~2, st);
+            if (e != hipSuccess) return e;
+        }
+        return launch_bwd_d<128>(p, dtype, bias, causal, dbias, 2, st);
+    }
+    switch (kernel_dim) {
         case 16: return launch_bwd_d<16>(p, dtype, bias, causal, dbias, stages, st);
         case 32: return launch_bwd_d<32>(p, dtype, bias, causal, dbias, stages, st);
         case 64: return launch_bwd_d<64>(p, dtype, bias, causal, dbias, stages, st);
