@@ -214,8 +214,9 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
         // element-wise work of block 0, and the dQ product of block 0 between that of block 1, one fenced slot per two
         // elements.  Operands are fetched a phase ahead, above head dim 64 one slot ahead.  Same bits; us, one block after
         // the other -> this: B=4 H=16 S=2048 D=64 causal 65.1 -> 60.9, B=1 H=16 S=6001 D=128 causal 218 -> 206, B=2 H=16
-        // M=N=4096 D=128 362 -> 350.
-        if constexpr (!STEP_MASKED && C::NH == 2 && !FROM_DS) {
+        // M=N=4096 D=128 362 -> 350.  Not with a staged bias row up to head dim 64, whose reads between the fences it waits for:
+        // B=2 H=8 M=N=577 D=32 11.0 -> 11.9, B=4 H=16 S=2048 D=64 causal 63 -> 65.
+        if constexpr (!STEP_MASKED && C::NH == 2 && !FROM_DS && !(ROWB && D <= 64)) {
             constexpr int NS = 2 * C::KSTEPS, NP = 2 * C::DB;  // matrix instructions of S and dP, and of dQ, per block
             constexpr bool AHEAD = D <= 64;
             constexpr int NSS = AHEAD ? NS : (NS + 7) / 8, NPS = AHEAD ? NP : (NP + 7) / 8;  // operands fetched at a time
