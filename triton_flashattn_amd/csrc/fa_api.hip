@@ -233,11 +233,13 @@ int compute_units() {
 }
 
 // Keys of a query tile split between work-groups when the query tiles alone leave the GPU half empty
-// (fewer than two work-groups per CU): as many splits as it takes to get there, each with at least 16
-// steps of the K/V stream.  A few short tiles (at most one per four CUs, at most 256 query rows) go down
+// (fewer than two work-groups per CU): as many splits as it takes to get there, each with at least 1024 keys, or
+// 512 with a bias, whose steps cost more (D=64, byte mask, B=1 H=8 M=512 N=2048, shares of 512 / of 1024 keys: forward
+// 19 / 25 us, dQ 19 / 27; bf16 tile 18 / 23 and 18 / 24; bf16 row 17 / 21 and 18 / 23; B=1 H=16 M=N=1024, a
+// row: forward 19 / 17, dQ 20 / 20).  A few short tiles (at most one per four CUs, at most 256 query rows) go down
 // to shares of 256 keys: their shares of the output are small next to the keys that they have read, and without
 // that a token decoded against a long cache runs on a handful of CUs.  Beyond 32 shares the merge costs more than the
-// last of them bring.  One query row, D = 128, us per call, at most 4 shares of at least 16 steps / this rule / 64 shares
+// last of them bring.  One query row, D = 128, us per call, at most 4 shares of at least 1024 / this rule / 64 shares
 // allowed: B=1 H=8 N=1024 19.2 / 11.9 / 11.9, N=4096 22.8 / 15.4 / 15.4, N=16384 87 / 30 / 38.  Where the line lies: 256 keys
 // at 256 tiles (B=16 H=16 N=700 D=64) 16.0 -> 18.5, at 1024 rows (B=2 H=8 M=N=1024 D=64) 14.8 -> 18.2.
 // The answer depends on the current device (its CU
@@ -250,14 +252,14 @@ FwdSplit fwd_split(const fa_problem& p) {
     const int64_t wgs = (int64_t)((p.M + fa::fwd_block_m() - 1) / fa::fwd_block_m()) * p.B * p.H;
     const int64_t full = 2 * (int64_t)compute_units();
     if (wgs >= full) return {1, 0};
-    const int bk = p.bias_dtype == FA_BIAS_NONE ? 64 : 32;  // keys per step of the forward kernel
-    const int n_steps = (p.N + bk - 1) / bk;
+    const int unit = p.bias_dtype == FA_BIAS_NONE ? 64 : 32;  // keys are dealt in these
+    const int n_units = (p.N + unit - 1) / unit;
     int s = (int)(full / wgs);
     s = s > 32 ? 32 : s;
-    const int min_steps = p.M <= 256 && 8 * wgs <= full ? 256 / bk : 16;
-    while (s > 1 && n_steps / s < min_steps) s--;
+    const int min_units = p.M <= 256 && 8 * wgs <= full ? 256 / unit : 16;
+    while (s > 1 && n_units / s < min_units) s--;
     if (s <= 1) return {1, 0};
-    const int keys = ((n_steps + s - 1) / s * bk + 63) / 64 * 64;  // whole steps of either kernel tiling
+    const int keys = ((n_units + s - 1) / s * unit + 63) / 64 * 64;  // whole steps of every kernel tiling
     return {(p.N + keys - 1) / keys, keys};                        // (rounded up, they may need fewer shares: none is empty)
 }
 
