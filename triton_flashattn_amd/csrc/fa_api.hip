@@ -1,5 +1,6 @@
 // C ABI of libfa_mi355.so (declared in include/fa_mi355.h): argument validation and dispatch.
-// Host code only; the kernels live in fa_fwd.hip and fa_bwd.hip.
+// Host code only; the kernels live in fa_fwd.hip, fa_bwd.hip, fa_bwd_narrow.hip (dK, dV and dBias of the small head dims) and
+// fa_bwd_shared.hip (the gradient of a shared bias).
 #include <hip/hip_runtime.h>
 
 #include <atomic>
@@ -12,21 +13,27 @@
 #include "fa_params.hpp"
 
 namespace fa {
-// one object file per head dimension defines these (fa_fwd.hip, fa_bwd.hip with -DFA_HEAD_DIM)
+// one object file per head dimension defines these (fa_fwd.hip, fa_bwd.hip, fa_bwd_shared.hip with -DFA_HEAD_DIM)
 template <int D> hipError_t launch_fwd_d(const FwdParams& p, int dtype, int bias, bool causal, hipStream_t st);
 template <int D> hipError_t launch_bwd_d(const BwdParams& p, int dtype, int bias, bool causal, int dbias, int stages, hipStream_t st);
 template <int D> hipError_t launch_bwd_shared_d(const BwdParams& p, int dtype, hipStream_t st);
 #define FA_DECLARE_D(D)                                                                                         \
     template <> hipError_t launch_fwd_d<D>(const FwdParams& p, int dtype, int bias, bool causal, hipStream_t st); \
-    template <> hipError_t launch_bwd_d<D>(const BwdParams& p, int dtype, int bias, bool causal, int dbias, int stages, hipStream_t st); \
-    template <> hipError_t launch_bwd_shared_d<D>(const BwdParams& p, int dtype, hipStream_t st);
+    template <> hipError_t launch_bwd_d<D>(const BwdParams& p, int dtype, int bias, bool causal, int dbias, int stages, hipStream_t st);
+#define FA_DECLARE_SHARED_D(D) template <> hipError_t launch_bwd_shared_d<D>(const BwdParams& p, int dtype, hipStream_t st);
 FA_DECLARE_D(16)
 FA_DECLARE_D(32)
 FA_DECLARE_D(64)
-FA_DECLARE_D(128)
 FA_DECLARE_D(96)
+FA_DECLARE_D(128)
 FA_DECLARE_D(256)
+FA_DECLARE_SHARED_D(16)
+FA_DECLARE_SHARED_D(32)
+FA_DECLARE_SHARED_D(64)
+FA_DECLARE_SHARED_D(128)
+FA_DECLARE_SHARED_D(256)
 #undef FA_DECLARE_D
+#undef FA_DECLARE_SHARED_D
 
 // Head dims of a D = 128 problem that fit 96: three quarters of the products, copies and LDS, and the dK / dV kernel of the
 // small head dims where no bias tile is streamed.  Forward / backward, us, at 128 -> at 96: B=2 H=16 M=N=4096 D=96 250 / 829 ->

@@ -1523,12 +1523,16 @@ template <typename T, int D> static hipError_t launch_all(const BwdParams& p, in
         pq.dq_makes_delta = makes_delta ? 1 : 0;
         if (from_ds && pq.dq_splits < 4) pq.dq_splits = 1;
         dim3 qgrid((unsigned)(pq.n_mtiles * pq.dq_splits * pq.B * pq.H));
-        if (from_ds && bias == DS_BIAS) {
-            if (causal) hipLaunchKernelGGL((fa_bwd_dq_kernel<T, D, DS_BIAS, true, true>), qgrid, dim3(256), 0, st, pq);
-            else hipLaunchKernelGGL((fa_bwd_dq_kernel<T, D, DS_BIAS, false, true>), qgrid, dim3(256), 0, st, pq);
-        } else if (from_ds && bias == 4) {
-            if (causal) hipLaunchKernelGGL((fa_bwd_dq_kernel<T, D, 4, true, true>), qgrid, dim3(256), 0, st, pq);
-            else hipLaunchKernelGGL((fa_bwd_dq_kernel<T, D, 4, false, true>), qgrid, dim3(256), 0, st, pq);
+        if (from_ds) {
+            if constexpr (D == 96) {
+                return hipErrorInvalidValue;  // (a dense dBias runs at 128)
+            } else if (bias == DS_BIAS) {
+                if (causal) hipLaunchKernelGGL((fa_bwd_dq_kernel<T, D, DS_BIAS, true, true>), qgrid, dim3(256), 0, st, pq);
+                else hipLaunchKernelGGL((fa_bwd_dq_kernel<T, D, DS_BIAS, false, true>), qgrid, dim3(256), 0, st, pq);
+            } else {
+                if (causal) hipLaunchKernelGGL((fa_bwd_dq_kernel<T, D, 4, true, true>), qgrid, dim3(256), 0, st, pq);
+                else hipLaunchKernelGGL((fa_bwd_dq_kernel<T, D, 4, false, true>), qgrid, dim3(256), 0, st, pq);
+            }
         } else {
 #define FA_CASE(BK)                                                                                               \
     case BK:                                                                                                      \

@@ -125,20 +125,6 @@ template <int D> struct Swz {
         if (CPR == 4 || CPR == 12) return (row >> 2) & 3;
         return (row >> 3) & 1;
     }
-    __device__ static __forceinline__ int off(int row, int col) {
-        return row * D + ((((col >> 3) ^ f(row)) << 3) | (col & 7));
-    }
-    // 8 k-slots gathered down column col0 + lane%32: rows row0 + 4g + {0..3}, row0 + 8 + 4g + {0..3}
-    template <typename V8, typename T>
-    __device__ static __forceinline__ V8 col8(const T* tile, int lane, int row0, int col0) {
-        const int g = lane >> 5, s = lane & 15;
-        const int row = row0 + 4 * g + (s >> 2);
-        const int col = (col0 + ((lane >> 4) & 1) * 16 + (s & 3) * 4) & (D - 1);
-        i16x4 lo = lds_read_tr4(tile + off(row, col));
-        i16x4 hi = lds_read_tr4(tile + off(row + 8, col));
-        typedef short i16x8 __attribute__((ext_vector_type(8)));
-        return __builtin_bit_cast(V8, (i16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-    }
     // Row operand: lane l reads row (rows + l%32), head-dim elements 16 ks + 8 (l/32) .. + 7.
     // rows_lane(lane) is L; `rows` is a multiple of 32 known at compile time.
     __device__ static __forceinline__ unsigned rows_lane(int lane) {
@@ -150,7 +136,7 @@ template <int D> struct Swz {
             return __builtin_bit_cast(V8, lds_read16_at((tile_plus_l ^ (unsigned)(32 * (ks & 1))) + (unsigned)(rows * RB + 64 * (ks >> 1))));
         return __builtin_bit_cast(V8, lds_read16_at((tile_plus_l ^ (unsigned)(32 * ks)) + (unsigned)(rows * RB)));
     }
-    // Column operand (what col8 returns) for head-dim block db (32 wide) and rows row0 .. row0 + 15,
+    // Column operand: 8 k-slots gathered down a column of head-dim block db (32 wide) in rows row0 .. row0 + 15,
     // row0 a multiple of 16 known at compile time.  The second gather sits 8 rows further down,
     // where the swizzle differs by one fixed bit.
     __device__ static __forceinline__ unsigned cols_lane(int lane) {
