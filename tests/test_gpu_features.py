@@ -117,18 +117,21 @@ def test_row_broadcast_bias_never_becomes_dense(gpu_device):
 @pytest.mark.parametrize("kind", ["bool", "f16", "bf16", "f32"])
 def test_row_broadcast_bias_is_staged_once_per_work_group(gpu_device, D, kind):
     """The forward and dQ kernels keep a bias without a row dimension as an fp32 row in LDS (up to
-    4096 keys per work-group): every element kind, ragged and causal shapes, a strided row, a row that
-    is split between work-groups, one that is too long for LDS (dense path through the zero stride),
-    and a batch whose keys are all masked."""
+    4096 keys per work-group): every element kind, ragged and causal shapes, a strided row, rows that
+    are split between work-groups (also of more than 4096 keys), rows that are too long for LDS (causal, whose keys are
+    not split: dense path through the zero stride), and a batch whose keys are all masked."""
     bdt = {"bool": torch.bool, "f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}[kind]
     cases = [  # B, M, N, H, causal, key stride of the bias row
         (2, 300, 333, 3, False, 1), (2, 333, 333, 2, True, 1), (1, 130, 1000, 2, False, 2),
-        (1, 64, 4096, 2, False, 1), (1, 40, 4200, 1, False, 1), (1, 96, 6000, 2, False, 1)]
+        (1, 64, 4096, 2, False, 1), (1, 40, 4200, 1, False, 1), (1, 96, 6000, 2, False, 1),
+        (1, 4200, 4200, 1, True, 1), (1, 4133, 4133, 1, True, 1), (1, 4104, 4104, 1, True, 2)]
     for i, (B, M, N, H, causal, step) in enumerate(cases):
         q, k, v, do, _ = make_inputs(gpu_device, B, M, N, H, D, torch.bfloat16 if i % 2 else torch.float16, None, seed=7 * D + i)
         g = torch.Generator().manual_seed(100 + i)
         if kind == "bool":
             row = torch.rand(B, 1, 1, N * step, generator=g) < 0.7
+            if M > 4096:
+                row[..., 0] = True  # (a causal row without a visible key has no defined result: see the parity edges' test of them)
             if B > 1:
                 row[1] = False  # every key of batch 1 masked: uniform attention (flash_attention.py:49-53)
             bias = row.to(gpu_device)[..., ::step]
