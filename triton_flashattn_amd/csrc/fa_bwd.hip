@@ -111,14 +111,12 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
     const float log2_slope = neg_slope * kLog2e;
     if (FROM_DS) bp = reinterpret_cast<const E*>(p.dbias) + (int64_t)b * p.sdbias.b + (int64_t)h * p.sdbias.h + (int64_t)key0 * p.sdbias.n;
 
-    // Where a bias row is staged the first copies go out before anything is loaded and waited for (as in the forward kernel).
     const LiveChunks chunks{p.d_qk / 8, p.qk_inv};
     const unsigned rows_l = SW::rows_lane(lane), cols_l = SW::cols_lane(lane);
     KeyStream<T, D, stream_kind(BIAS), !FROM_DS> ks_;
     ks_.init(smem, kp, vp, bp, p.sk.s, p.sv.s, FROM_DS ? p.sdbias.m : p.sbias.m, FROM_DS ? p.sdbias.n : p.sbias.n, M, N,
              mw, wave, lane, chunks, p.d_v / 8);
     const bool bias_copies = FROM_DS || (TB != 0 && p.bias_vec);
-    if constexpr (ROWB) ks_.template prologue<false>();
 
     // Q^T and dO^T as B operands: column my_m, k = d
     const T* dop = reinterpret_cast<const T*>(p.dout) + (int64_t)b * p.sdo.b + (int64_t)h * p.sdo.h;
@@ -445,7 +443,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
         // loops (it cannot know that they land once), and that wait drains the queue of copies issued
         // steps ahead.  Waiting for them here keeps the loops free of it.
         wait_vmcnt<0>();
-        if constexpr (!ROWB) ks_.template prologue<BV>();
+        ks_.template prologue<BV>();
         if constexpr (TB == 0) split_q();  // (while the first copies are on their way)
         // the leading fast steps whose copies stay inside the tensors issue them without clamps
         const int n_lean = (BV || TB == 0) ? ks_.lean_steps(n_fast, m0 + BM) : 0;

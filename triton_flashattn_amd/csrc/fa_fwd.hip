@@ -113,15 +113,11 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
         raw_ok = __builtin_fabsf(raw_slope) * (float)p.N < 1e30f;
     }
 
-    // Where a bias row is staged the first copies go out before anything is loaded and waited for: the latencies of K and V, of
-    // Q and of the row are one this way (B=32 H=12 M=N=197 D=64 with a padding mask, us per call: 15.3 -> 14.8).  Elsewhere the
-    // wait for Q would become one for all of them (no bias, B=8 H=16 S=512 D=64: 15.4 -> 15.9).
     const LiveChunks chunks{p.d_qk / 8, p.qk_inv};
     const unsigned rows_l = SW::rows_lane(lane), cols_l = SW::cols_lane(lane);
     KeyStream<T, D, fwd_stream_kind(BIAS, D), true, true> ks_;
     ks_.init(smem, kp, vp, bp, p.sk.s, p.sv.s, p.sbias.m, p.sbias.n, M, N, mw, wave, lane, chunks, p.d_v / 8);
     const bool bias_copies = TB != 0 && p.bias_vec;
-    if constexpr (ROWB) ks_.template prologue<false>();
 
     // Q^T as B operand: column my_m, k = d
     T8 qreg[C::KSTEPS];
@@ -507,7 +503,9 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
         // loops (it cannot know that they land once), and that wait drains the queue of copies issued
         // steps ahead.  Waiting for them here keeps the loops free of it.
         wait_vmcnt<0>();
-        if constexpr (!ROWB) ks_.template prologue<BV>();
+        // (After the wait and not before the loads, where it would be one for the first copies too.  B=32 H=12 M=N=197 D=64, us
+        // per call, after / before: padding mask 13.45 / 13.96; no bias, B=8 H=16 S=512 15.4 / 15.9.)
+        ks_.template prologue<BV>();
         if constexpr (TB == 0) split_q();  // (while the first copies are on their way)
         // the leading fast steps whose copies stay inside the tensors issue them without clamps
         const int n_lean = (BV || TB == 0) ? ks_.lean_steps(n_fast, m0 + BM) : 0;
