@@ -1430,10 +1430,14 @@ constexpr bool short_rows_built(int bias, int dbias) { return dbias == 0 || (dbi
 // CU (two of fa_bwd_narrow.hip read and write twice as many rows at a time: 4.6 TB/s).  us, one wave -> pair, D = 64:
 //   one tile to a CU: fp32 read M=N=1024 H=32 37 -> 33, M=N=2048 H=8 62 -> 50; bf16 and dBias M=N=1500 H=8 57 -> 51, M=N=577 B=2
 //     H=8 27 -> 24, 512 rows the same; at 256 tiles of 2048 rows 73 -> 82.  Below 512 rows the ends of a tile count for more
-//     (fp32 read B=2 H=4 M=N=77 7 -> 8) but for fp32 and dBias, causal, whose tiles are few steps long: B=4 H=8 S=197 17 -> 16.
-//   more, fp32 and dBias, not causal: B=2 H=16 M=N=2016 224 -> 206, M=N=3000 562 -> 528, 256 rows 139 -> 164; causal, where
-//     long tiles are paired with short ones, B=2 H=16 M=N=2048 193 -> 230.
-//   D = 32, fp32 and dBias, not causal, more than one tile to a CU: M=N=2016 214 -> 197, M=N=4096 791 -> 728; with one the same.
+//     (fp32 read B=2 H=4 M=N=77 7 -> 8) but for fp32 and dBias, causal, whose tiles are few steps long: B=4 H=8 S=197 17 -> 16.  Long
+//     ones of these that leave few CUs idle end up waiting for memory (with the delta pass: S=1500, 156 tiles 67 -> 61, 192 the
+//     same, 216 91 -> 95, S=2000, 192 tiles 105 -> 109).
+//   more, fp32 and dBias, not causal, any D: pairs of long tiles, whose last round of one to a CU is nearly full (with the delta
+//     pass: M=N=2016 H=32 233 -> 218, D=32 222 -> 207, M=1280 N=1024 H=64 D=32 144 -> 140, 1.75 rounds the same, 1.25 or 2.5
+//     rounds 122 -> 125 and 202 -> 209; 1024 rows, two rounds, 126 -> 128; M=600 N=1000 H=40 52 -> 63); where they are very
+//     long the last round, then alone with the memory, matters less (M=N=4096, 1.5 rounds 343 -> 334, M=4096 N=512, 2.5 rounds 637
+//     -> 613; M=2048 N=1024, 2.5 rounds 305 -> 308).  Causal, where long tiles are paired with short ones, B=2 H=16 M=N=2048 193 -> 230.
 //   a dBias of the other 16-bit type: always one wave (M=N=1024 H=32 48 -> 37).
 // Rows of a dBias or its bias that allow no aligned 16-byte accesses: always a pair, whose stores go out of registers, 32 keys
 // of a row each, and which has 16 loads of a lane in flight, not 8 (fp32 dBias B=2 H=8 M=N=577 57 -> 38, bf16 q and fp16 dBias
@@ -1444,9 +1448,14 @@ static bool pair_of_waves(const BwdParams& p, int D, int bias, int dbias, bool o
     if (bias != 4 && !own_type) return false;
     const int64_t tiles = (int64_t)p.n_ntiles * p.B * p.H;
     const bool fp32_dbias = bias == 4 && dbias == 1;
-    if (fp32_dbias && !causal && p.M > 512 && (D == 64 || tiles > p.cus)) return true;
-    if (D != 64 || tiles > p.cus) return false;
+    if (tiles > p.cus) {
+        if (!fp32_dbias || causal) return false;
+        const int64_t last = tiles % p.cus;
+        return (p.M >= 1280 && (last == 0 || 4 * last >= 3 * (int64_t)p.cus)) || (p.M > 2048 && 2 * tiles >= 3 * (int64_t)p.cus);
+    }
+    if (D != 64) return false;
     if (p.M < 512) return fp32_dbias && causal;
+    if (fp32_dbias && causal && p.M >= 1500 && 4 * tiles >= 3 * (int64_t)p.cus) return false;
     return bias == 4 || tiles < p.cus || p.M < 2048;
 }
 
