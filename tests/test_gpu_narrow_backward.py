@@ -202,13 +202,14 @@ def test_tiles_of_64_keys_at_head_dim_128(gpu_device, kind):
 
 
 @pytest.mark.parametrize("D", [16, 32, 64])
-@pytest.mark.parametrize("kind", ["bf16", "f32"])
-def test_float_biases_that_a_pair_of_waves_takes(gpu_device, D, kind):
-    """Up to head dim 64 float biases of at least 512 rows go to the kernel of two waves per 32 keys, an fp32 one with a
+@pytest.mark.parametrize("kind", ["bool", "bf16", "f32"])
+def test_biases_that_a_pair_of_waves_takes(gpu_device, D, kind):
+    """Up to head dim 64 biases of at least 512 (masks 1500, head dim 16 1025) rows go to the kernel of two waves per 32 keys, an fp32 one with a
     gradient also in whole rounds of as many tiles as there are CUs and, causal, with fewer rows: around the lines, with ragged rows and keys,
     rows of the bias that are whole chunks and rows that are not."""
     for M, N, H, causal in [(511, 130, 2, False), (512, 97, 2, False), (513, 264, 2, False), (640, 33, 1, False),
-                            (545, 136, 140, False), (1281, 130, 256, False), (1280, 33, 300, False), (2049, 65, 400, False), (1, 1, 2, True), (33, 33, 2, True), (200, 200, 2, True), (512, 512, 2, True), (577, 577, 2, True), (650, 650, 1, True), (1500, 1500, 16, True)]:
+                            (545, 136, 140, False), (1281, 130, 256, False), (1280, 33, 300, False), (2049, 65, 400, False), (1499, 70, 2, False), (1500, 264, 2, False), (1525, 130, 1, False),
+                            (1025, 264, 20, False), (1, 1, 2, True), (33, 33, 2, True), (200, 200, 2, True), (512, 512, 2, True), (577, 577, 2, True), (650, 650, 1, True), (1500, 1500, 16, True)]:
         for trainable in (True, False):
             q, k, v, do, bias = make_inputs(gpu_device, 1, M, N, H, D, torch.bfloat16, kind, seed=M + D, trainable=trainable)
             check(run_ours(q, k, v, do, bias, causal), run_oracle(q, k, v, do, bias, causal), str((D, kind, M, N, H, causal, trainable)))

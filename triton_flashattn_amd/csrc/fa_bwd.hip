@@ -587,7 +587,7 @@ template <> struct BiasQuad<4> {
 constexpr int bwd_waves(int D) { return D > 128 ? 2 : 4; }
 // Biases that this kernel takes up to head dim 64, by the rule of pair_of_waves
 constexpr bool pair_built(int D, int bias, int dbias) {
-    return D <= 64 && ((bias >= 2 && bias <= 4 && dbias == 1) || (bias == 4 && dbias == 0));
+    return (D <= 64 && ((bias >= 2 && bias <= 4 && dbias == 1) || (bias == 4 && dbias == 0))) || (D == 64 && bias == 1 && dbias == 0);
 }
 template <int D, int BIAS, int W = bwd_waves(D)> struct BwdCfg {
     static constexpr int WPR = W;
@@ -1425,7 +1425,7 @@ static bool short_rows(const BwdParams& p, int bias, bool causal) {
 }
 constexpr bool short_rows_built(int bias, int dbias) { return dbias == 0 || (dbias == 2 && bias >= 5); }
 
-// Up to head dim 64: which of the kernels takes a float tile.  A pair of waves keeps two waves per SIMD and the bias of three
+// Up to head dim 64: which of the kernels takes a bias tile.  A pair of waves keeps two waves per SIMD and the bias of three
 // blocks in flight where a CU gets one tile only, and streams an fp32 bias and its gradient at the copy rate with one tile per
 // CU (two of fa_bwd_narrow.hip read and write twice as many rows at a time: 4.6 TB/s).  us, one wave -> pair, D = 64:
 //   one tile to a CU: fp32 read M=N=1024 H=32 37 -> 33, M=N=2048 H=8 62 -> 50; bf16 and dBias M=N=1500 H=8 57 -> 51, M=N=577 B=2
@@ -1438,20 +1438,30 @@ constexpr bool short_rows_built(int bias, int dbias) { return dbias == 0 || (dbi
 //     rounds 122 -> 125 and 202 -> 209; 1024 rows, two rounds, 126 -> 128; M=600 N=1000 H=40 52 -> 63); where they are very
 //     long the last round, then alone with the memory, matters less (M=N=4096, 1.5 rounds 343 -> 334, M=4096 N=512, 2.5 rounds 637
 //     -> 613; M=2048 N=1024, 2.5 rounds 305 -> 308).  Causal, where long tiles are paired with short ones, B=2 H=16 M=N=2048 193 -> 230.
+//   D = 16, one tile to a CU (with the delta pass, N=512, us): more than 1024 rows in 51 tiles and more, fp32 read, H=32 M=2304 60 ->
+//     53 (32 tiles of 1088 rows 29 -> 30), and 16 bits and dBias where most CUs are idle, H=16 M=2304 57 -> 53 (128 tiles of 4096
+//     rows 106 -> 130); fp32 and dBias the same either way.  At D = 32 none gains 5 %.
+//   a byte mask, not causal, one tile to a CU of 1500 rows and more (N=512, H=16): M=1536 46.2 -> 44.5, M=4096 108 -> 101, 1088 rows
+//     35.0 -> 34.5; causal S=2000 57.6 -> 58.7.
 //   a dBias of the other 16-bit type: always one wave (M=N=1024 H=32 48 -> 37).
 // Rows of a dBias or its bias that allow no aligned 16-byte accesses: always a pair, whose stores go out of registers, 32 keys
 // of a row each, and which has 16 loads of a lane in flight, not 8 (fp32 dBias B=2 H=8 M=N=577 57 -> 38, bf16 q and fp16 dBias
 // B=2 H=16 M=N=1023 131 -> 59); an fp32 bias of such rows that is only read too (M=N=1023 68 -> 55).
 // (measured at 256 CUs, B=1 where none is given)
 static bool pair_of_waves(const BwdParams& p, int D, int bias, int dbias, bool own_type, bool causal) {
+    const int64_t tiles = (int64_t)p.n_ntiles * p.B * p.H;
+    if (bias == 1) return !causal && p.bias_vec && p.M >= 1500 && tiles <= p.cus;
     if (!p.bias_vec || (dbias == 1 && !p.dbias_vec)) return true;
     if (bias != 4 && !own_type) return false;
-    const int64_t tiles = (int64_t)p.n_ntiles * p.B * p.H;
     const bool fp32_dbias = bias == 4 && dbias == 1;
     if (tiles > p.cus) {
         if (!fp32_dbias || causal) return false;
         const int64_t last = tiles % p.cus;
         return (p.M >= 1280 && (last == 0 || 4 * last >= 3 * (int64_t)p.cus)) || (p.M > 2048 && 2 * tiles >= 3 * (int64_t)p.cus);
+    }
+    if (D == 16) {
+        const bool long_tiles = !causal && p.M > 1024 && 5 * tiles >= p.cus;
+        return long_tiles && !fp32_dbias && (bias == 4 ? 4 * tiles <= 3 * (int64_t)p.cus : 8 * tiles <= 3 * (int64_t)p.cus);
     }
     if (D != 64) return false;
     if (p.M < 512) return fp32_dbias && causal;
@@ -1594,6 +1604,7 @@ template <typename T, int D> static hipError_t launch_all(const BwdParams& p, in
         bool pair = false;
         if constexpr (D <= 64) {
             pair = pair_built(D, kbias, kdbias) && pair_of_waves(p, D, kbias, kdbias, kbias == DS_BIAS, causal);
+            if (pair) e = hipErrorInvalidValue;  // (until one of these has it)
 #define FA_CASE(BK, DBK)                                                                                      \
     if (pair && kbias == BK && kdbias == DBK)                                                                  \
         e = causal ? launch_main<T, D, BK, true, DBK>(p, st) : launch_main<T, D, BK, false, DBK>(p, st);
@@ -1602,6 +1613,9 @@ template <typename T, int D> static hipError_t launch_all(const BwdParams& p, in
             FA_CASE(4, 1)
             FA_CASE(4, 0)
 #undef FA_CASE
+            if constexpr (D == 64) {
+                if (pair && kbias == 1) e = launch_main<T, D, 1, false, 0>(p, st);
+            }
         }
         if (!pair) e = launch_bwd_narrow_d<D>(p, __is_same(T, __bf16), kbias, causal, kdbias, st);
     } else {
