@@ -1115,9 +1115,8 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
                 // Interior steps: the scores first, then the dV product (its operands do not depend on this
                 // step) one MFMA at a time between the exponentials of two score elements, so that the wave
                 // has vector work to issue while its matrix instructions execute (measured 2-3 % on the
-                // kernels of head dim 128 without a bias and with a bias that is only read, a loss of 5 % at
-                // head dim 64 with a bool mask; the same interleaving of the dK product into the dS
-                // arithmetic of the dP-wave costs 1-4 %).
+                // kernels of head dim 128 without a bias and with a bias that is only read; the same interleaving of
+                // the dK product into the dS arithmetic of the dP-wave costs 1-4 %).
                 constexpr bool FUSE = IN && D == 128;
                 if constexpr (FUSE) {
                     mma_rows(a_rows, sacc);
@@ -1413,7 +1412,9 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
 // Few query rows at head dim 128: tiles of 64 keys, two work-groups to a CU.  What a tile costs beyond its steps (its operands,
 // its first copies, two steps of skew, its stores: about 16 us) is then spent next to the steps of another one.  us, 128 -> 64
 // keys: no bias B=8 H=12 S=512 53.0 -> 44.7, M=256 N=4096 H=32 83.3 -> 76.0; causal S=1024 95.7 -> 85.1, with a byte mask 108.6 ->
-// 97.5, causal B=2 H=8 S=512 24.1 -> 17.3; read-only bf16 bias B=8 H=12 S=512 54.9 -> 45.2, B=64 491 -> 496.  With more rows the
+// 97.5, causal B=2 H=8 S=512 24.1 -> 17.3; read-only bf16 bias B=8 H=12 S=512 54.9 -> 45.2, B=64 491 -> 496.  (With the delta pass:) padding
+// mask B=8 H=12 S=512 59.5 -> 53.1, B=64 H=16 498 -> 482, causal B=32 H=16 S=1024 575 -> 550; bf16 row and its gradient 63.3 -> 56.5, 517 ->
+// 496, 617 -> 570; a trainable table for all batches 61.4 -> 53.4, 503 -> 496, 590 -> 545.  With more rows the
 // second reading of Q and dO costs as much (B=4 H=16 S=2048 289 -> 293, byte mask B=2 H=16 S=1024 51.6 -> 52.6), and where dBias is
 // written the shallow rings cost more (M=N=4096 712 -> 928).  An fp32 bias is copied one step ahead only in these rings, which costs
 // more where a CU has many tiles, whose reads overlap anyway: B=8 H=12 S=512 56 -> 47, B=64 H=16 S=512 493 -> 513, causal 432 -> 460;

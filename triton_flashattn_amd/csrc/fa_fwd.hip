@@ -5,20 +5,20 @@
 // the kernel as an fp32 multiply.
 //
 // Work split.  One work-group (4 waves) owns 128 query rows of one (batch, head); each wave
-// owns 32 of them for the whole kernel.  Keys/values are streamed through LDS in steps of 32
-// (with a bias) or 64 keys, consumed 32 at a time.
+// owns 32 of them for the whole kernel.  Keys/values are streamed through LDS in steps of 64 keys (32 with an
+// fp32 bias or ALiBi, and above head dim 64 with any bias: StreamCfg, fwd_stream_kind), consumed 32 at a time.
 // Scores are computed TRANSPOSED, S^T = K Q^T, so that in the MFMA accumulator a lane holds one
 // query row (column l%32 of S^T) and 16 of the 32 keys: the row maximum and row sum of the online
-// softmax are then per-lane loops plus a single exchange with lane l^32, the running maximum, the
+// softmax are then per-lane loops plus a single exchange with lane l^32, the reference point of the exponentials, the
 // running sum and the rescale factor are one scalar per lane, and P^T is already laid out as the
 // B operand of O^T += V^T P^T.  V^T is gathered from the row-major V rows with
 // ds_read_b64_tr_b16.
 //
-// Memory -> LDS.  The K and V rows of a step (ring of 3 slots issued two steps ahead; double
-// buffered and one step ahead without a bias) and the bias slice of each wave (32 rows x 32 keys,
-// ring of 4 wave-private slots, issued three steps ahead) arrive through direct global -> LDS copies that the compiler does not see; their
-// completion is counted by hand (copies complete in issue order and every step issues the same
-// number).  The bias is a pure HBM stream: only a queue this deep keeps enough bytes in flight.
+// Memory -> LDS.  The K and V rows of a step (double buffered, one step ahead, where a step has 64 keys or the bias is in fp32; else a
+// ring of 3 slots, two ahead) and the bias slice of each wave (32 rows x 32 or 64 keys, a wave-private ring: of 4 slots,
+// three steps ahead, 3 in fp32, 2 where a step has 64 keys) arrive through direct global -> LDS copies that the compiler
+// does not see; their completion is counted by hand (copies complete in issue order and every step issues the same number).
+// The bias is a pure HBM stream: a queue of 96 (64) keys a row keeps enough bytes in flight.
 #include <type_traits>
 
 #include "fa_common.hpp"
