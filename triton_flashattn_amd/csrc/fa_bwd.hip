@@ -1057,8 +1057,10 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
                                 const int m = m0 + ml0 + e;
                                 const float tmask = CAUSAL && m < my_n ? kMask : 0.f;
                                 const float add = NATURAL ? __fmul_rn(bv, kLog2e) : bv;
-                                pv = fast_exp2(__fadd_rn(__fmul_rn(sacc[i], qk_scale), __fadd_rn(tmask, add)) - lse4[e]);
-                                pv = m < M ? pv : 0.f;  // (not an additive term: the LSE read again may lie below any)
+                                // (no row, no weight.  Not an additive term: the LSE read again may lie below any; and selected here, not
+                                // behind the exponential, which took 2 to 3 % where dBias leaves element by element)
+                                const float lse = m < M ? lse4[e] : __builtin_inff();
+                                pv = fast_exp2(__fadd_rn(__fmul_rn(sacc[i], qk_scale), __fadd_rn(tmask, add)) - lse);
                             } else {
                                 // (without a bias the offset is the negated LSE itself: written as 0 - lse it
                                 // would cost a subtraction per element, +0 - x not being -x)
