@@ -73,7 +73,12 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
     constexpr bool BOOLROW = BIAS == 7;  // ... a bool mask: the row holds 0 or the mask term, in log2 units
     static_assert(!(FROM_DS && ROWB), "a row-broadcast bias has no dense dS");
 
-    __shared__ __align__(1024) unsigned char smem[C::LDS_BYTES + (ROWB ? kRowBiasKeys * 4 : 0)];
+    // Q and dO rows come through LDS (WaveRows).  A place for dO beside that of Q where it costs no work-group on a CU; else one
+    // after the other.
+    typedef WaveRows<T, D> WR;
+    constexpr bool STAGED = C::STAGE != C::kNowhere && !FROM_DS;
+    constexpr bool BESIDE = STAGED && !ROWB && (C::LDS_BYTES + 4 * WR::BYTES) * C::MIN_BLOCKS <= 163840;
+    __shared__ __align__(1024) unsigned char smem[C::LDS_BYTES + (ROWB ? kRowBiasKeys * 4 : 0) + (BESIDE ? 4 * WR::BYTES : 0)];
     const float* row_lds = reinterpret_cast<const float*>(smem + C::LDS_BYTES);
 
     const int tid = threadIdx.x;
@@ -113,22 +118,26 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
 
     const LiveChunks chunks{p.d_qk / 8, p.qk_inv};
     const unsigned rows_l = SW::rows_lane(lane), cols_l = SW::cols_lane(lane);
-    KeyStream<T, D, stream_kind(BIAS), !FROM_DS> ks_;
+    typedef KeyStream<T, D, stream_kind(BIAS), !FROM_DS> KS;
+    KS ks_;
     ks_.init(smem, kp, vp, bp, p.sk.s, p.sv.s, FROM_DS ? p.sdbias.m : p.sbias.m, FROM_DS ? p.sdbias.n : p.sbias.n, M, N,
              mw, wave, lane, chunks, p.d_v / 8);
     const bool bias_copies = FROM_DS || (TB != 0 && p.bias_vec);
 
     // Q^T and dO^T as B operands: column my_m, k = d
     const T* dop = reinterpret_cast<const T*>(p.dout) + (int64_t)b * p.sdo.b + (int64_t)h * p.sdo.h;
+    const T* outp = reinterpret_cast<const T*>(p.o) + (int64_t)b * p.so.b + (int64_t)h * p.so.h;
     T8 qreg[C::KSTEPS], doreg[C::KSTEPS];
+    if constexpr (!STAGED) {
 #pragma unroll
-    for (int ks = 0; ks < C::KSTEPS; ks++) {
-        i32x4 rq = {0, 0, 0, 0}, rd = {0, 0, 0, 0};
-        const int d = ks * 16 + 8 * g;
-        if (!FROM_DS && my_m < M) rq = gld16(qp + (int64_t)my_m * p.sq.s + (D <= 128 ? chunks.wrap(2 * ks + g) * 8 : d));
-        if (!FROM_DS && my_m < M && d < p.d_v) rd = gld16(dop + (int64_t)my_m * p.sdo.s + d);
-        qreg[ks] = as_vec<T8>(rq);
-        doreg[ks] = as_vec<T8>(rd);
+        for (int ks = 0; ks < C::KSTEPS; ks++) {
+            i32x4 rq = {0, 0, 0, 0}, rd = {0, 0, 0, 0};
+            const int d = ks * 16 + 8 * g;
+            if (!FROM_DS && my_m < M) rq = gld16(qp + (int64_t)my_m * p.sq.s + (D <= 128 ? chunks.wrap(2 * ks + g) * 8 : d));
+            if (!FROM_DS && my_m < M && d < p.d_v) rd = gld16(dop + (int64_t)my_m * p.sdo.s + d);
+            qreg[ks] = as_vec<T8>(rq);
+            doreg[ks] = as_vec<T8>(rd);
+        }
     }
     auto split_q = [&]() {
         if (D <= 128 && !FROM_DS && p.d_qk < D) {
@@ -136,39 +145,84 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
             for (int ks = 0; ks < C::KSTEPS; ks++) qreg[ks] = chunks.part(qreg[ks], 2 * ks + g, C::CPR);
         }
     };
-    if constexpr (TB != 0) split_q();  // (kernels of a bias tile have no registers for it later)
     // LSE (log2 units) and delta of this lane's query row
     float lse_i = 0.f, delta_i = 0.f;
     if (!FROM_DS && my_m < M) {
         lse_i = p.lse[((int64_t)b * p.H + h) * M + my_m];
         if (!p.dq_makes_delta) delta_i = p.delta[((int64_t)b * p.H + h) * M + my_m];
     }
-    if (!FROM_DS && p.dq_makes_delta) {
-        // This kernel runs first and forms delta = sum_d o * do itself (flash_attention.py:215-227), in the
-        // order of fa_bwd_prep_kernel: this lane holds the chunks 2 ks + g of its row (dO^T above), sums
-        // each with fused multiply-adds, adds chunk c to chunk c ^ w for w = D / 16, ..., 2 (both in this
-        // lane) and last to chunk c ^ 1 (in the lane of the other g).  The dK/dV kernel reads what is stored.
-        const T* op = reinterpret_cast<const T*>(p.o) + (int64_t)b * p.so.b + (int64_t)h * p.so.h;
-        constexpr int NP = D == 96 ? 8 : C::KSTEPS;  // (delta of D = 96 is formed like that of 128, whose last chunks are zero)
-        float part[NP];
+    // Where this kernel runs first it forms delta = sum_d o * do itself (flash_attention.py:215-227), bit for bit as
+    // fa_bwd_prep_kernel does: a chunk of 8 by fused multiply-adds, then chunk c with chunk c ^ w for w = D / 16, ..., 1.  The
+    // dK/dV kernel reads what is stored.
+    // O in the order of a WaveRows tile: chunk c = 64 it + l of the 32 rows to lane l, which finds dO's beside it in LDS
+    constexpr bool O_AS_TILE = STAGED && D != 96;
+    i32x4 o_raw[O_AS_TILE ? WR::COPIES : 1];
+    auto o_chunk = [&](int it, int& row, int& src) {
+        row = (it * 64 + lane) / CPR;
+        src = ((it * 64 + lane) % CPR) ^ SW::f(row);
+    };
+    auto load_o = [&]() {
+        if constexpr (O_AS_TILE) {
 #pragma unroll
-        for (int ks = C::KSTEPS; ks < NP; ks++) part[ks] = 0.f;
-#pragma unroll
-        for (int ks = 0; ks < C::KSTEPS; ks++) {
-            i32x4 ro = {0, 0, 0, 0};
-            if (my_m < M && ks * 16 + 8 * g < p.d_v) ro = gld16(op + (int64_t)my_m * p.so.s + ks * 16 + 8 * g);
-            const T8 ov = as_vec<T8>(ro);
-            float a = 0.f;
-#pragma unroll
-            for (int e = 0; e < 8; e++) a = __builtin_fmaf((float)ov[e], (float)doreg[ks][e], a);
-            part[ks] = a;
+            for (int it = 0; it < WR::COPIES; it++) {
+                int row, src;
+                o_chunk(it, row, src);
+                const int m = mw + row < M ? mw + row : M - 1;
+                o_raw[it] = i32x4{0, 0, 0, 0};
+                if (p.dq_makes_delta && src * 8 < p.d_v) o_raw[it] = gld16(outp + (int64_t)m * p.so.s + src * 8);
+            }
         }
+    };
+    auto make_delta = [&](unsigned do_tile) {
+        if (!p.dq_makes_delta) return;
+        if constexpr (O_AS_TILE) {
+            constexpr int RPI = 64 / CPR;  // rows of a copy
+            float sum[WR::COPIES];
 #pragma unroll
-        for (int hs = NP / 2; hs >= 1; hs >>= 1)
+            for (int it = 0; it < WR::COPIES; it++) {
+                int row, src;
+                o_chunk(it, row, src);
+                const T8 ov = as_vec<T8>(o_raw[it]), dv = as_vec<T8>(lds_read16_at(do_tile + 1024 * it + 16 * lane));
+                float a = 0.f;
 #pragma unroll
-            for (int ks = 0; ks < hs; ks++) part[ks] = part[ks] + part[ks + hs];
-        delta_i = part[0] + __shfl_xor(part[0], 32, 64);
+                for (int e = 0; e < 8; e++) a = __builtin_fmaf((float)ov[e], (float)dv[e], a);
+                sum[it] = src * 8 < p.d_v ? a : 0.f;
+            }
+#pragma unroll
+            for (int w = CPR / 2; w >= 1; w >>= 1)
+#pragma unroll
+                for (int it = 0; it < WR::COPIES; it++) sum[it] += __shfl_xor(sum[it], w, 64);
+#pragma unroll
+            for (int it = 0; it < WR::COPIES; it++) {
+                const float x = __shfl(sum[it], r % RPI * CPR, 64);
+                if (r / RPI == it) delta_i = x;
+            }
+        } else {
+            constexpr int NP = D == 96 ? 8 : C::KSTEPS;  // (delta of D = 96 is formed like that of 128, whose last chunks are zero)
+            float part[NP];
+#pragma unroll
+            for (int ks = C::KSTEPS; ks < NP; ks++) part[ks] = 0.f;
+#pragma unroll
+            for (int ks = 0; ks < C::KSTEPS; ks++) {
+                i32x4 ro = {0, 0, 0, 0};
+                if (my_m < M && ks * 16 + 8 * g < p.d_v) ro = gld16(outp + (int64_t)my_m * p.so.s + ks * 16 + 8 * g);
+                const T8 ov = as_vec<T8>(ro);
+                float a = 0.f;
+#pragma unroll
+                for (int e = 0; e < 8; e++) a = __builtin_fmaf((float)ov[e], (float)doreg[ks][e], a);
+                part[ks] = a;
+            }
+#pragma unroll
+            for (int hs = NP / 2; hs >= 1; hs >>= 1)
+#pragma unroll
+                for (int ks = 0; ks < hs; ks++) part[ks] = part[ks] + part[ks + hs];
+            delta_i = part[0] + __shfl_xor(part[0], 32, 64);
+        }
         if (g == 0 && my_m < M && split == 0) p.delta[((int64_t)b * p.H + h) * M + my_m] = delta_i;
+    };
+    if constexpr (!STAGED && !FROM_DS) {
+        if constexpr (TB != 0) split_q();  // (kernels of a bias tile have no registers for it later)
+        make_delta(0);
     }
 
     int n_steps = (N + BK - 1) / BK;
@@ -186,10 +240,6 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
     for (int db = 0; db < C::DB; db++)
 #pragma unroll
         for (int i = 0; i < 16; i++) dq_acc[db][i] = 0.f;
-
-    if (ROWB)
-        stage_row_bias(reinterpret_cast<float*>(smem + C::LDS_BYTES), p.bias, p.row_bias_kind,
-                       (int64_t)b * p.sbias.b + (int64_t)h * p.sbias.h + (int64_t)key0 * p.sbias.n, p.sbias.n, N, tid);
 
     // One step of the K/V stream.  Interior steps (every key in range and visible to every row of
     // the work-group) run with STEP_MASKED = false: no range checks, no mask arithmetic.  BV: the
@@ -438,13 +488,58 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
     if (!(qk_scale > 0.f)) n_fast = 0;
     auto run = [&](auto bv_tag) {
         constexpr bool BV = decltype(bv_tag)::value;
+        auto stage_row = [&]() {
+            if (ROWB)
+                stage_row_bias(reinterpret_cast<float*>(smem + C::LDS_BYTES), p.bias, p.row_bias_kind,
+                               (int64_t)b * p.sbias.b + (int64_t)h * p.sbias.h + (int64_t)key0 * p.sbias.n, p.sbias.n, N, tid);
+        };
+        if constexpr (STAGED) {
+            constexpr bool FIRST_KV = C::STAGE != C::kOwnRing;  // the first copies of the stream need not wait for the rows
+            constexpr int PRO = FIRST_KV ? KS::template prologue_copies<BV>() : 0;
+            const unsigned q_tile = ks_.stage_addr(), do_tile = BESIDE ? ks_.lds_kv + C::LDS_BYTES + ks_.wave_s * WR::BYTES : q_tile;
+            auto copy = [&](bool is_q) {
+                const unsigned saved_m0 = lds_copy_begin();
+                if (is_q) WR::issue(qp, p.sq.s, mw, M, q_tile, lane, [&](int c) { return D <= 128 ? chunks.wrap(c) : c; });
+                else WR::issue(dop, p.sdo.s, mw, M, do_tile, lane, [&](int c) { return live_chunk(c, p.d_v / 8); });
+                lds_copy_end(saved_m0);
+            };
+            load_o();
+            copy(true);
+            if constexpr (BESIDE) copy(false);
+            if constexpr (FIRST_KV) ks_.template prologue<BV>();
+            WR::template arrived<PRO + (BESIDE ? WR::COPIES : 0)>();
+#pragma unroll
+            for (int ks = 0; ks < C::KSTEPS; ks++) qreg[ks] = SW::template row8_at<T8>(q_tile + rows_l, 0, ks);
+            if constexpr (!BESIDE) {
+                WR::done();
+                copy(false);
+                WR::template arrived<0>();
+            } else {
+                WR::template arrived<PRO>();
+            }
+#pragma unroll
+            for (int ks = 0; ks < C::KSTEPS; ks++) {
+                const i32x4 x = as_raw(SW::template row8_at<T8>(do_tile + rows_l, 0, ks));
+                doreg[ks] = as_vec<T8>(ks * 16 + 8 * g < p.d_v ? x : i32x4{0, 0, 0, 0});
+            }
+            split_q();
+            make_delta(do_tile);
+            if constexpr (!FIRST_KV) {
+                WR::done();
+                ks_.template prologue<BV>();
+            }
+            stage_row();
+        }
         // The loads of this lane's rows issued above are the compiler's own.  Left in flight, they would
         // make it wait for "all vector-memory operations" at their first use inside EVERY step of the
         // loops (it cannot know that they land once), and that wait drains the queue of copies issued
         // steps ahead.  Waiting for them here keeps the loops free of it.
         wait_vmcnt<0>();
-        ks_.template prologue<BV>();
-        if constexpr (TB == 0) split_q();  // (while the first copies are on their way)
+        if constexpr (!STAGED) {
+            stage_row();
+            ks_.template prologue<BV>();
+            if constexpr (TB == 0 && !FROM_DS) split_q();  // (while the first copies are on their way)
+        }
         // the leading fast steps whose copies stay inside the tensors issue them without clamps
         const int n_lean = (BV || TB == 0) ? ks_.lean_steps(n_fast, m0 + BM) : 0;
         int k = 0;
@@ -495,11 +590,14 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
             *reinterpret_cast<T4*>(o_lds + r * OS + db * 32 + 8 * q4 + 4 * g) = pk;
         }
     }
-    __syncthreads();
     T* op = reinterpret_cast<T*>(p.dq) + (int64_t)b * p.sdq.b + (int64_t)h * p.sdq.h;
-    for (int c = lane; c < 32 * CPR; c += 64) {
-        int row = c / CPR, ch = c % CPR;
-        if (mw + row < M && ch * 8 < p.d_qk) gst16(op + (int64_t)(mw + row) * p.sdq.s + ch * 8, lds_read16(o_lds + row * OS + ch * 8));
+    i32x4 out[WR::COPIES];  // (a wave's own rows: no barrier; all reads in flight together)
+#pragma unroll
+    for (int it = 0; it < WR::COPIES; it++) out[it] = lds_read16(o_lds + (it * 64 + lane) / CPR * OS + (it * 64 + lane) % CPR * 8);
+#pragma unroll
+    for (int it = 0; it < WR::COPIES; it++) {
+        const int row = (it * 64 + lane) / CPR, ch = (it * 64 + lane) % CPR;
+        if (mw + row < M && ch * 8 < p.d_qk) gst16(op + (int64_t)(mw + row) * p.sdq.s + ch * 8, out[it]);
     }
 }
 

@@ -326,6 +326,41 @@ __device__ __forceinline__ void stage_row_bias(float* row_lds, const void* bias,
 // zeros there), or makes columns of the result that are not stored.
 __device__ __forceinline__ int live_chunk(int chunk, int chunks) { return chunk < chunks ? chunk : 0; }
 
+// 32 rows of a (seq, D) tensor that one wave needs as an operand, lane = row: by direct copies of whole kilobytes into a
+// swizzled tile of the wave's own and from there by row8_at.  Loaded straight into the operand's layout, 16 bytes of a row to
+// a lane, every load touches 32 cache lines, a fourth or an eighth of each, and those of the waves of a CU (96 to 192 KB) do
+// not all stay in its 32 KB of L1 until the loads of the other parts come.  dQ kernel (Q, dO and O), us, before -> after: B=8
+// H=12 S=512 D=128 34.1 -> 31.3, causal S=1024 with a byte mask 75 -> 69, B=32 H=12 S=197 D=64 21.5 -> 19.7, B=8 H=16 S=257
+// D=80 20.1 -> 18.2, B=4 H=16 S=2048 D=64 causal 61.4 -> 60.5.
+template <typename T, int D> struct WaveRows {
+    static constexpr int COPIES = D / 16, BYTES = 64 * D;
+    // between lds_copy_begin() and lds_copy_end(); rows past n_rows are the last row again; chunk(c) is the chunk of a row that
+    // stands in for chunk c (head dims below D)
+    template <typename F>
+    __device__ static __forceinline__ void issue(const T* base, int64_t stride, int row0, int n_rows, unsigned dst, int lane, F&& chunk) {
+        const int first = row0 < n_rows ? row0 : n_rows - 1;
+        const uint64_t at = uniform_ptr(base + (int64_t)first * stride);
+#pragma unroll
+        for (int i = 0; i < COPIES; i++) {
+            const int c = i * 64 + lane;
+            int row = c / Swz<D>::CPR;
+            const int src = (c % Swz<D>::CPR) ^ Swz<D>::f(row);
+            row = row < n_rows - 1 - first ? row : n_rows - 1 - first;
+            lds_copy16(at, (unsigned)(row * (int)stride * 2 + chunk(src) * 16), dst + 1024 * i);
+        }
+    }
+    // all but the wave's last `LATER` copies have landed: the rows may be read
+    template <int LATER> __device__ static __forceinline__ void arrived() {
+        wait_vmcnt<LATER>();
+        asm volatile("" : : : "memory");
+    }
+    // the rows have been read: copies may take their place
+    __device__ static __forceinline__ void done() {
+        __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));  // lgkmcnt(0)
+        asm volatile("" : : : "memory");
+    }
+};
+
 // S = K Q^T of the forward and the dQ kernel is formed differently: a key may hold infinities (scores of -inf, weights of
 // zero), and 0 * inf would make all of its row NaN.  Chunk c behind the end of a K row is its chunk c mod `live`, and what
 // meets it is a number of the sign of Q there (0 for 0) instead of zero, so that no product has a value or a sign that the
@@ -390,7 +425,17 @@ template <int D, int BIAS, bool WIDE = false> struct StreamCfg {
     static constexpr int BIAS_BYTES = 4 * NBS * BSLOT;
     // (the output tile is staged over the K/V slots and, where it is larger, into the bias rings
     // behind them: all of them are dead by then)
-    static constexpr int LDS_BYTES = KV_BYTES + BIAS_BYTES > O_BYTES ? KV_BYTES + BIAS_BYTES : O_BYTES;
+    static constexpr int LOOP_BYTES = KV_BYTES + BIAS_BYTES > O_BYTES ? KV_BYTES + BIAS_BYTES : O_BYTES;
+    // Where the rows of a wave (WaveRows) stand before the first step: in the ring slots that the first copies leave free
+    // (half of one to a wave, or for waves 2 and 3 behind everything else), behind everything else, or in the wave's own ring
+    // of bias slots, whose first copies then wait for them.  (Bias tiles at head dim 256: nowhere.)
+    enum Stage { kHalfSlots, kOwnRing, kBehind, kSlotsAndBehind, kNowhere };
+    static constexpr Stage STAGE = NH == 2                          ? kHalfSlots
+                                   : D > 128                        ? kNowhere
+                                   : ES == 0                        ? kBehind
+                                   : NBS * BSLOT >= 64 * D          ? kOwnRing
+                                                                    : kSlotsAndBehind;
+    static constexpr int LDS_BYTES = LOOP_BYTES + (STAGE == kBehind ? 256 * D : STAGE == kSlotsAndBehind ? 128 * D : 0);
     // 16-byte chunk c of bias row `row` is stored at chunk c ^ bswz(row): rows that share LDS banks
     // get different chunk orders
     __device__ static __forceinline__ int bswz(int row) {
@@ -402,7 +447,8 @@ template <int D, int BIAS, bool WIDE = false> struct StreamCfg {
     // a kernel is short next to its waits, and three of its rings fit LDS (those of a 16-bit bias do not).  D = 64, us, two
     // -> three: forward B=8 H=12 S=1024 51.7 -> 47.6, B=16 H=8 S=2048 250 -> 238; forward and backward, causal, B=8 H=12
     // S=1024 144.7 -> 140.4.  (Head dims up to 32 stayed below 168 registers on their own: no change.)
-    static constexpr int MIN_BLOCKS = D <= 64 && BIAS <= 1 ? 3 : (D <= 128 && LDS_BYTES <= 81920) ? 2 : 1;
+    static constexpr int MIN_BLOCKS = D <= 64 && BIAS <= 1 ? 3 : (D <= 128 && LOOP_BYTES <= 81920) ? 2 : 1;
+    static_assert(LDS_BYTES * MIN_BLOCKS <= 163840, "LDS of a CU");
 };
 
 // The copy machinery of the kernels tiled by StreamCfg (forward, dQ): one object per thread.
@@ -481,6 +527,17 @@ template <typename T, int D, int BIAS, bool WITH_V = true, bool WIDE = false> st
     // the K and V slots by LDS byte address (scalar), for the operand reads by address of Swz
     __device__ __forceinline__ unsigned k_addr(int k) const { return lds_kv + (unsigned)((k % C::NKV) * C::STEP_BYTES); }
     __device__ __forceinline__ unsigned v_addr(int k) const { return lds_kv + (unsigned)((C::NKV + k % C::NKV) * C::STEP_BYTES); }
+    // LDS address of the place for 32 rows of this wave before the first step (WaveRows)
+    __device__ __forceinline__ unsigned stage_addr() const {
+        constexpr unsigned R = 64 * D;  // (bytes of 32 rows)
+        const unsigned k_free = lds_kv + C::LA * C::STEP_BYTES, v_free = lds_kv + (C::NKV + C::LA) * C::STEP_BYTES;
+        if constexpr (C::STAGE == C::kHalfSlots) return (wave_s < 2 ? k_free : v_free) + (unsigned)(wave_s & 1) * R;
+        else if constexpr (C::STAGE == C::kOwnRing) return lds_bias;
+        else if constexpr (C::STAGE == C::kBehind) return lds_kv + C::LOOP_BYTES + (unsigned)wave_s * R;
+        else return wave_s == 0 ? k_free : wave_s == 1 ? v_free : lds_kv + C::LOOP_BYTES + (unsigned)(wave_s - 2) * R;
+    }
+    // copies of a wave in prologue()
+    template <bool BV> static constexpr int prologue_copies() { return C::LA * (WITH_V ? 2 : 1) * C::KD + (BV ? (C::NBS - 1) * C::BCH : 0); }
     // byte offset of bias (row, key .. key + 3) inside a slot
     __device__ static __forceinline__ int b_off(int row, int key) {
         const int byte = key * C::ES;
