@@ -770,7 +770,7 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
     // 32 x 32 tile (4-byte stores, one per element) and stores 16 bytes per lane from there
     constexpr bool DB_VIA_LDS32 = DBIAS == 1 && BIAS == 4;
 
-    __shared__ __align__(16) unsigned char smem[C::LDS_BYTES];
+    __shared__ __align__(1024) unsigned char smem[C::LDS_BYTES];
 
     const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63;
@@ -820,9 +820,16 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
     unsigned char* ring_lds = smem + C::OFF_BIAS + kb * C::RING * C::BT_BYTES;
     float* p_lds = reinterpret_cast<float*>(smem + C::OFF_P) + kb * 64 * 16;  // + buffer * P_BYTES / 4
 
-    // ---- this wave's 32 keys as B operand (column my_n, k = d): K for an S-wave, V for a dP-wave
+    // ---- this wave's 32 keys as B operand (column my_n, k = d): K for an S-wave, V for a dP-wave.  Up to head dim 128 they come
+    // through LDS with the first copies (WaveRows): K through the hand-off buffers, V through the Q and dO slots that those
+    // copies leave free.  A tile spent 14 000 clocks before its first step and 6 000 after its last one, a quarter of it at 1024
+    // rows.  With this and the way back at the end, us, before -> after, D = 128: B=8 H=12 S=512 44.9 -> 38.5, with dBias 63.5 ->
+    // 58, S=1024 causal with a byte mask 95.6 -> 87.6, H=32 M=1024 N=8192 with dBias 552 -> 528, M=N=4096 843 -> 833; the way
+    // back alone, D = 256 B=4 H=8 S=1024 104.5 -> 99.4. ----
+    typedef WaveRows<T, D> WR;
+    constexpr bool STAGED = D <= 128;
     T8 opreg[C::KSTEPS];
-    {
+    if constexpr (!STAGED) {
         const T* src = s_wave ? kp + (int64_t)my_n * p.sk.s : vp + (int64_t)my_n * p.sv.s;
 #pragma unroll
         for (int ks = 0; ks < C::KSTEPS; ks++) {
@@ -1007,9 +1014,22 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
         }
     };
 
-    // ---- prologue: the first LA blocks of Q and LA - 1 blocks of dO ----
+    // ---- prologue: this wave's keys, the first LA blocks of Q and LA - 1 blocks of dO ----
+    unsigned op_tile = 0;
+    if constexpr (STAGED) {
+        constexpr int FREE_Q = C::NQB - C::LA;  // Q slots without a block yet, and two of dO
+        static_assert(2 * C::P_BYTES >= C::WPR * WR::BYTES && FREE_Q + 2 >= C::WPR && C::Q_BYTES == WR::BYTES, "room for the keys");
+        if (s_wave) op_tile = lds_base + C::OFF_P + (unsigned)kb * WR::BYTES;
+        else if (kb < FREE_Q) op_tile = lds_base + (unsigned)((mb_first + C::LA + kb) % C::NQB) * C::Q_BYTES;
+        else op_tile = lds_base + C::OFF_DO + (unsigned)((mb_first + C::LA - 1 + kb - FREE_Q) % C::NDOB) * C::Q_BYTES;
+        op_tile = __builtin_amdgcn_readfirstlane(op_tile);
+    }
     {
         const unsigned saved_m0 = lds_copy_begin();
+        if constexpr (STAGED) {
+            const int chunks = (s_wave ? p.d_qk : p.d_v) / 8;
+            WR::issue(s_wave ? kp : vp, s_wave ? p.sk.s : p.sv.s, nw, N, op_tile, lane, [&](int c) { return live_chunk(c, chunks); });
+        }
 #pragma unroll 1
         for (int i = 0; i < C::LA; i++) {
             if (s_wave == Q_BY_S) issue_q(mb_first + i);
@@ -1018,7 +1038,14 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
         }
         lds_copy_end(saved_m0);
     }
-    wait_vmcnt<0>();
+    WR::template arrived<0>();
+    if constexpr (STAGED) {  // (of a key past the end, the last one again: nothing of such a lane is stored)
+#pragma unroll
+        for (int ks = 0; ks < C::KSTEPS; ks++) {
+            const i32x4 x = as_raw(SW::template row8_at<T8>(op_tile + SW::rows_lane(lane), 0, ks));
+            opreg[ks] = as_vec<T8>(ks * 16 + 8 * g < (s_wave ? p.d_qk : p.d_v) ? x : i32x4{0, 0, 0, 0});
+        }
+    }
     __syncthreads();
 
     T8 op_cur[2];  // P^T (S-wave) or dS^T (dP-wave) of the block whose accumulation is still due
@@ -1487,25 +1514,13 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
         }
     }
     // ---- dV (S-wave) or dK (dP-wave) of this wave's 32 keys (flash_attention.py:449-454) ----
-    if (my_n < N) {
-        T* dst = s_wave ? reinterpret_cast<T*>(p.dv) + (int64_t)b * p.sdv.b + (int64_t)h * p.sdv.h + (int64_t)my_n * p.sdv.s
-                        : reinterpret_cast<T*>(p.dk) + (int64_t)b * p.sdk.b + (int64_t)h * p.sdk.h + (int64_t)my_n * p.sdk.s;
-        const float out_scale = s_wave ? 1.f : p.sm_scale;
-        const int d_out = s_wave ? p.d_v : p.d_qk;
-#pragma unroll
-        for (int db = 0; db < C::DB; db++) {
-#pragma unroll
-            for (int q4 = 0; q4 < 4; q4++) {
-                const int d = db * 32 + 8 * q4 + 4 * g;
-                if (d < d_out) {
-                    T4 o4;
-#pragma unroll
-                    for (int e = 0; e < 4; e++) o4[e] = (T)(acc[db][q4 * 4 + e] * out_scale);
-                    *reinterpret_cast<T4*>(dst + d) = o4;
-                }
-            }
-        }
-    }
+    wait_vmcnt<0>();
+    lds_barrier();  // (the rings are dead and no copy is in flight)
+    static_assert(2 * C::WPR * WR::BYTES <= C::LDS_BYTES, "room for the way back");
+    T* dst = s_wave ? reinterpret_cast<T*>(p.dv) + (int64_t)b * p.sdv.b + (int64_t)h * p.sdv.h
+                    : reinterpret_cast<T*>(p.dk) + (int64_t)b * p.sdk.b + (int64_t)h * p.sdk.h;
+    const unsigned own = lds_base + (unsigned)__builtin_amdgcn_readfirstlane(wave) * WR::BYTES;
+    WR::store(acc, s_wave ? 1.f : p.sm_scale, own, dst, s_wave ? p.sdv.s : p.sdk.s, nw, N, s_wave ? p.d_v : p.d_qk, lane);
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -354,6 +354,38 @@ template <typename T, int D> struct WaveRows {
         wait_vmcnt<LATER>();
         asm volatile("" : : : "memory");
     }
+    // The way back: 32 rows that lie in accumulators, lane = row, registers = head dim (acc[d / 32], C layout), through `lds` (64 D
+    // bytes that are the wave's own) to memory, 16 bytes to a lane and whole rows at a time.  Straight from the registers, 8
+    // bytes of a row to a lane, every store touches 32 cache lines: 4 000 clocks at the end of a tile of 128 keys.
+    // (fa_bwd_kernel has the figures.)
+    template <int DB>
+    __device__ static __forceinline__ void store(const f32x16 (&acc)[DB], float scale, unsigned lds, T* base, int64_t stride, int row0,
+                                                 int n_rows, int d_live, int lane) {
+        typedef typename VecOf<T>::v4 T4;
+        typedef T4 __attribute__((address_space(3))) * lds_ptr;
+        constexpr int CPR = Swz<D>::CPR;
+        asm volatile("" : "+v"(lane));  // (what is formed of it here is not kept in registers from the first copies on)
+        const int r = lane & 31, g = lane >> 5;
+        const unsigned at = lds + (unsigned)(r * Swz<D>::RB + 8 * g);
+#pragma unroll
+        for (int db = 0; db < DB; db++)
+#pragma unroll
+            for (int q4 = 0; q4 < 4; q4++) {
+                if (db * 32 + 8 * q4 >= D) continue;
+                T4 x;
+#pragma unroll
+                for (int e = 0; e < 4; e++) x[e] = (T)(acc[db][q4 * 4 + e] * scale);
+                *(lds_ptr)(uintptr_t)(at + 16u * (unsigned)((db * 4 + q4) ^ Swz<D>::f(r))) = x;
+            }
+        i32x4 out[COPIES];  // (the wave's own rows: no barrier)
+#pragma unroll
+        for (int i = 0; i < COPIES; i++) out[i] = lds_read16_at(lds + 1024u * i + 16u * (unsigned)lane);
+#pragma unroll
+        for (int i = 0; i < COPIES; i++) {
+            const int row = (i * 64 + lane) / CPR, c = ((i * 64 + lane) % CPR) ^ Swz<D>::f(row);
+            if (row0 + row < n_rows && c * 8 < d_live) gst16(base + (int64_t)(row0 + row) * stride + c * 8, out[i]);
+        }
+    }
     // the rows have been read: copies may take their place
     __device__ static __forceinline__ void done() {
         __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));  // lgkmcnt(0)
