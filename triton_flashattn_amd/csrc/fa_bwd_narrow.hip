@@ -49,7 +49,14 @@ template <int D, int BIAS> struct NarrowCfg {
     static constexpr int OFF_STAT = 2 * NS * ROWS_BYTES;
     static constexpr int OFF_BIAS = OFF_STAT + NS * 2 * STAT_BYTES;
     static constexpr int OFF_DS = OFF_BIAS + NS * 4 * BSLOT;
-    static constexpr int LDS_BYTES = OFF_DS + 4 * DS_BYTES;
+    static constexpr int LOOP_BYTES = OFF_DS + 4 * DS_BYTES;
+    // Where the K and V rows of a wave stand before the first step (WaveRows): in the slots that the first copies leave free, of
+    // Q and dO rows, half a slot to a wave, or in the wave's own bias slot; else behind everything else.  (V beside an fp32
+    // bias at D = 64: nowhere, there the lanes load it.)
+    enum Stage { kHalfSlots, kBiasSlot, kBehind, kNowhere };
+    static constexpr Stage K_STAGE = ES == 4 ? kBiasSlot : kHalfSlots;
+    static constexpr Stage V_STAGE = ES == 4 ? (128 * D <= BSLOT ? kBiasSlot : kNowhere) : 64 * D <= BSLOT ? kBiasSlot : kBehind;
+    static constexpr int LDS_BYTES = LOOP_BYTES + (V_STAGE == kBehind ? 256 * D : 0);
     static constexpr int MIN_BLOCKS = D <= 32 && ES <= 1 ? 3 : 2;  // work-groups per CU
     static_assert(LDS_BYTES * MIN_BLOCKS <= 163840, "LDS of a CU");
 };
@@ -171,16 +178,20 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
         }
     }
 
-    // K and V of this wave's keys as B operands (column my_n, k = d)
+    // K and V of this wave's keys as B operands (column my_n, k = d), through LDS with the first copies (WaveRows).  With this and
+    // the way back at the end, us, before -> after: padding mask B=32 H=12 S=197 D=64 25.6 -> 21.9, with an fp32 table 31.1 ->
+    // 27.6, B=8 H=16 S=257 D=80 22.1 -> 19.3, B=4 H=16 S=2048 D=64 causal 81.6 -> 78.2, B=4 H=32 M=N=4096 1105 -> 1078.
+    typedef WaveRows<T, D> WR;
+    constexpr bool V_STAGED = C::V_STAGE != C::kNowhere;
     T8 kreg[C::KSTEPS], vreg[C::KSTEPS];
+    if constexpr (!V_STAGED) {
 #pragma unroll
-    for (int ks = 0; ks < C::KSTEPS; ks++) {
-        i32x4 rk = {0, 0, 0, 0}, rv = {0, 0, 0, 0};
-        const int d = ks * 16 + 8 * g;
-        if (my_n < N && d < p.d_qk) rk = gld16(kp + (int64_t)my_n * p.sk.s + d);
-        if (my_n < N && d < p.d_v) rv = gld16(vp + (int64_t)my_n * p.sv.s + d);
-        kreg[ks] = as_vec<T8>(rk);
-        vreg[ks] = as_vec<T8>(rv);
+        for (int ks = 0; ks < C::KSTEPS; ks++) {
+            i32x4 rv = {0, 0, 0, 0};
+            const int d = ks * 16 + 8 * g;
+            if (my_n < N && d < p.d_v) rv = gld16(vp + (int64_t)my_n * p.sv.s + d);
+            vreg[ks] = as_vec<T8>(rv);
+        }
     }
     f32x16 dk[C::DB], dv[C::DB];  // dK^T, dV^T: rows = head dim, column = my_n
 #pragma unroll
@@ -356,13 +367,32 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
         constexpr bool DB_FAST = decltype(fast_tag)::value;
         constexpr int OPS = 2 * C::QD + 1 + (BV ? C::BCH : 0);  // copies per wave and step
         {
+            const unsigned free_slot = slot_of(t0 + LA);
+            const unsigned half_slot = lds_base + (wave < 2 ? 0u : (unsigned)C::OFF_DO) + free_slot * C::ROWS_BYTES + (unsigned)(wave & 1) * WR::BYTES;
+            const unsigned bias_slot = bias_dst + free_slot * 4 * C::BSLOT;
+            const unsigned k_tile = C::K_STAGE == C::kBiasSlot ? bias_slot : half_slot;
+            const unsigned v_tile = C::V_STAGE == C::kBehind ? lds_base + C::LOOP_BYTES + (unsigned)wave * WR::BYTES
+                                                             : bias_slot + (C::K_STAGE == C::kBiasSlot ? WR::BYTES : 0);
             const unsigned saved_m0 = lds_copy_begin();
+            WR::issue(kp, p.sk.s, nw, N, k_tile, lane, [&](int c) { return live_chunk(c, p.d_qk / 8); });
+            if constexpr (V_STAGED) WR::issue(vp, p.sv.s, nw, N, v_tile, lane, [&](int c) { return live_chunk(c, p.d_v / 8); });
 #pragma unroll
             for (int i = 0; i < LA; i++) issue(t0 + i, BV);
             lds_copy_end(saved_m0);
+            // (the compiler's own loads, too: left in flight, it would wait for everything in every step)
+            WR::template arrived<0>();
+            // (of a key past the end the last one again: nothing of such a lane is stored)
+#pragma unroll
+            for (int ks = 0; ks < C::KSTEPS; ks++) {
+                const int d = ks * 16 + 8 * g;
+                const i32x4 rk = as_raw(SW::template row8_at<T8>(k_tile + rows_l, 0, ks));
+                kreg[ks] = as_vec<T8>(d < p.d_qk ? rk : i32x4{0, 0, 0, 0});
+                if constexpr (V_STAGED) {
+                    const i32x4 rv = as_raw(SW::template row8_at<T8>(v_tile + rows_l, 0, ks));
+                    vreg[ks] = as_vec<T8>(d < p.d_v ? rv : i32x4{0, 0, 0, 0});
+                }
+            }
         }
-        // (the row loads above are the compiler's own: left in flight, it would wait for everything in every step)
-        wait_vmcnt<0>();
         int whole = 0;  // steps since one that may have stored less than STORES
 
         auto step = [&](int t, auto masked_tag, auto lean_tag) {
@@ -679,25 +709,13 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
         if (g == 0 && my_n < N) p.partials[(int64_t)bh * N + my_n] = s;
     }
     // ---- dV and dK of this wave's keys (flash_attention.py:449-454) ----
-    if (my_n < N) {
-        T* dvp = reinterpret_cast<T*>(p.dv) + (int64_t)b * p.sdv.b + (int64_t)h * p.sdv.h + (int64_t)my_n * p.sdv.s;
-        T* dkp = reinterpret_cast<T*>(p.dk) + (int64_t)b * p.sdk.b + (int64_t)h * p.sdk.h + (int64_t)my_n * p.sdk.s;
-#pragma unroll
-        for (int db = 0; db < C::DB; db++) {
-#pragma unroll
-            for (int q4 = 0; q4 < 4; q4++) {
-                const int d = db * 32 + 8 * q4 + 4 * g;
-                T4 v4, k4;
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    v4[e] = (T)dv[db][q4 * 4 + e];
-                    k4[e] = (T)(dk[db][q4 * 4 + e] * p.sm_scale);
-                }
-                if (d < p.d_v) *reinterpret_cast<T4*>(dvp + d) = v4;
-                if (d < p.d_qk) *reinterpret_cast<T4*>(dkp + d) = k4;
-            }
-        }
-    }
+    lds_barrier();  // (the rings are dead and no copy is in flight)
+    static_assert(8 * WR::BYTES <= C::LDS_BYTES, "room for the way back");
+    const unsigned own = lds_base + 2u * (unsigned)wave * WR::BYTES;
+    T* dvp = reinterpret_cast<T*>(p.dv) + (int64_t)b * p.sdv.b + (int64_t)h * p.sdv.h;
+    T* dkp = reinterpret_cast<T*>(p.dk) + (int64_t)b * p.sdk.b + (int64_t)h * p.sdk.h;
+    WR::store(dv, 1.f, own, dvp, p.sdv.s, nw, N, p.d_v, lane);
+    WR::store(dk, p.sm_scale, own + WR::BYTES, dkp, p.sdk.s, nw, N, p.d_qk, lane);
 }
 
 // This file is compiled once per head dimension (-DFA_HEAD_DIM=16, 32, 64, 96); each object exports

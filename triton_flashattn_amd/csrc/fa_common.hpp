@@ -338,6 +338,7 @@ template <typename T, int D> struct WaveRows {
     // stands in for chunk c (head dims below D)
     template <typename F>
     __device__ static __forceinline__ void issue(const T* base, int64_t stride, int row0, int n_rows, unsigned dst, int lane, F&& chunk) {
+        asm volatile("" : "+v"(lane));  // (nothing formed of it here is kept in registers for later)
         const int first = row0 < n_rows ? row0 : n_rows - 1;
         const uint64_t at = uniform_ptr(base + (int64_t)first * stride);
 #pragma unroll
