@@ -72,8 +72,8 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
     constexpr bool ROWB = BIAS >= 6;     // the same bias for every query row, kept as an fp32 row in LDS
     constexpr bool BOOLROW = BIAS == 7;  // ... a bool mask: the row holds 0 or the mask term, in log2 units
 
-    __shared__ __align__(1024) unsigned char smem[C::LDS_BYTES + (ROWB ? kRowBiasKeys * 4 : 0)];
-    const float* row_lds = reinterpret_cast<const float*>(smem + C::LDS_BYTES);
+    __shared__ __align__(1024) unsigned char smem[C::LOOP_BYTES + (ROWB ? kRowBiasKeys * 4 : 0)];
+    const float* row_lds = reinterpret_cast<const float*>(smem + C::LOOP_BYTES);
 
     const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63;
@@ -115,17 +115,25 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
 
     const LiveChunks chunks{p.d_qk / 8, p.qk_inv};
     const unsigned rows_l = SW::rows_lane(lane), cols_l = SW::cols_lane(lane);
-    KeyStream<T, D, fwd_stream_kind(BIAS, D), true, true> ks_;
+    typedef KeyStream<T, D, fwd_stream_kind(BIAS, D), true, true> KS;
+    KS ks_;
     ks_.init(smem, kp, vp, bp, p.sk.s, p.sv.s, p.sbias.m, p.sbias.n, M, N, mw, wave, lane, chunks, p.d_v / 8);
     const bool bias_copies = TB != 0 && p.bias_vec;
 
     // Q^T as B operand: column my_m, k = d
+    // Without a bias, from head dim 96 on, through LDS with the first K/V rows (WaveRows; us: B=8 H=12 S=512 D=128 23.6 -> 22.4,
+    // B=8 H=16 S=257 D=80 14.0 -> 13.5).  At 64 it is the same (197, 512 and 2048 rows), and so with a staged row (padding mask
+    // B=32 H=12 S=197 15.4 / 15.3) or a tile, whose first copies would have to wait for the rows (fp32 table there 20.4 / 20.8).
+    typedef WaveRows<T, D> WR;
+    constexpr bool STAGED = BIAS == 0 && D >= 96;
     T8 qreg[C::KSTEPS];
+    if constexpr (!STAGED) {
 #pragma unroll
-    for (int ks = 0; ks < C::KSTEPS; ks++) {
-        i32x4 raw = {0, 0, 0, 0};
-        if (my_m < M) raw = gld16(qp + (int64_t)my_m * p.sq.s + (D <= 128 ? chunks.wrap(2 * ks + g) : 2 * ks + g) * 8);
-        qreg[ks] = as_vec<T8>(raw);
+        for (int ks = 0; ks < C::KSTEPS; ks++) {
+            i32x4 raw = {0, 0, 0, 0};
+            if (my_m < M) raw = gld16(qp + (int64_t)my_m * p.sq.s + (D <= 128 ? chunks.wrap(2 * ks + g) : 2 * ks + g) * 8);
+            qreg[ks] = as_vec<T8>(raw);
+        }
     }
     auto split_q = [&]() {
         if (D <= 128 && p.d_qk < D) {
@@ -133,7 +141,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
             for (int ks = 0; ks < C::KSTEPS; ks++) qreg[ks] = chunks.part(qreg[ks], 2 * ks + g, C::CPR);
         }
     };
-    if constexpr (TB != 0) split_q();  // (kernels of a bias tile have no registers for it later)
+    if constexpr (!STAGED && TB != 0) split_q();  // (kernels of a bias tile have no registers for it later)
 
     int n_steps = (N + BK - 1) / BK;
     if (CAUSAL) {
@@ -153,9 +161,11 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
 #pragma unroll
         for (int i = 0; i < 16; i++) o_acc[db][i] = 0.f;
 
-    if (ROWB)
-        stage_row_bias(reinterpret_cast<float*>(smem + C::LDS_BYTES), p.bias, p.row_bias_kind,
-                       (int64_t)b * p.sbias.b + (int64_t)h * p.sbias.h + (int64_t)key0 * p.sbias.n, p.sbias.n, N, tid);
+    auto stage_row = [&]() {
+        if (ROWB)
+            stage_row_bias(reinterpret_cast<float*>(smem + C::LOOP_BYTES), p.bias, p.row_bias_kind,
+                           (int64_t)b * p.sbias.b + (int64_t)h * p.sbias.h + (int64_t)key0 * p.sbias.n, p.sbias.n, N, tid);
+    };
 
     // raises the reference point of this row's exponentials to mx (log2 units) where it is lower
     auto raise = [&](float mx) {
@@ -498,15 +508,28 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
 
     auto run = [&](auto bv_tag) {
         constexpr bool BV = decltype(bv_tag)::value;
-        // The loads of this lane's rows issued above are the compiler's own.  Left in flight, they would
-        // make it wait for "all vector-memory operations" at their first use inside EVERY step of the
-        // loops (it cannot know that they land once), and that wait drains the queue of copies issued
-        // steps ahead.  Waiting for them here keeps the loops free of it.
-        wait_vmcnt<0>();
-        // (After the wait and not before the loads, where it would be one for the first copies too.  B=32 H=12 M=N=197 D=64, us
-        // per call, after / before: padding mask 13.45 / 13.96; no bias, B=8 H=16 S=512 15.4 / 15.9.)
-        ks_.template prologue<BV>();
-        if constexpr (TB == 0) split_q();  // (while the first copies are on their way)
+        if constexpr (STAGED) {
+            const unsigned q_tile = ks_.stage_addr();
+            const unsigned saved_m0 = lds_copy_begin();
+            WR::issue(qp, p.sq.s, mw, M, q_tile, lane, [&](int c) { return D <= 128 ? chunks.wrap(c) : c; });
+            lds_copy_end(saved_m0);
+            ks_.template prologue<BV>();
+            WR::template arrived<KS::template prologue_copies<BV>()>();
+#pragma unroll
+            for (int ks = 0; ks < C::KSTEPS; ks++) qreg[ks] = SW::template row8_at<T8>(q_tile + rows_l, 0, ks);
+            split_q();
+        } else {
+            stage_row();
+            // The loads of this lane's rows issued above are the compiler's own.  Left in flight, they would
+            // make it wait for "all vector-memory operations" at their first use inside EVERY step of the
+            // loops (it cannot know that they land once), and that wait drains the queue of copies issued
+            // steps ahead.  Waiting for them here keeps the loops free of it.
+            wait_vmcnt<0>();
+            // (After the wait and not before the loads, where it would be one for the first copies too.  B=32 H=12 M=N=197 D=64, us
+            // per call, after / before: padding mask 13.45 / 13.96; no bias, B=8 H=16 S=512 15.4 / 15.9.)
+            ks_.template prologue<BV>();
+            if constexpr (TB == 0) split_q();  // (while the first copies are on their way)
+        }
         // the leading fast steps whose copies stay inside the tensors issue them without clamps
         const int n_lean = (BV || TB == 0) ? ks_.lean_steps(n_fast, m0 + BM) : 0;
         int k = 0;
@@ -569,11 +592,16 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
             *reinterpret_cast<T4*>(o_lds + r * OS + db * 32 + 8 * q4 + 4 * g) = pk;
         }
     }
-    __syncthreads();
     T* op = reinterpret_cast<T*>(p.o) + (int64_t)b * p.so.b + (int64_t)h * p.so.h;
-    for (int c = lane; c < 32 * CPR; c += 64) {
-        int row = c / CPR, ch = c % CPR;
-        if (mw + row < M && ch * 8 < p.d_v) gst16(op + (int64_t)(mw + row) * p.so.s + ch * 8, lds_read16(o_lds + row * OS + ch * 8));
+    int lane_late = lane;  // (as above)
+    asm volatile("" : "+v"(lane_late));
+    i32x4 out[WR::COPIES];  // (a wave's own rows: no barrier; all reads in flight together)
+#pragma unroll
+    for (int it = 0; it < WR::COPIES; it++) out[it] = lds_read16(o_lds + (it * 64 + lane_late) / CPR * OS + (it * 64 + lane_late) % CPR * 8);
+#pragma unroll
+    for (int it = 0; it < WR::COPIES; it++) {
+        const int row = (it * 64 + lane_late) / CPR, ch = (it * 64 + lane_late) % CPR;
+        if (mw + row < M && ch * 8 < p.d_v) gst16(op + (int64_t)(mw + row) * p.so.s + ch * 8, out[it]);
     }
 }
 
