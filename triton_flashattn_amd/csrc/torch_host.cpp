@@ -68,8 +68,11 @@ bool bias_rows_ok(const Tensor& b) {
     return last * es + padded <= (int64_t)b.storage().nbytes();
 }
 
+// rows that start at multiples of 16 bytes, from 512 bytes on at whole cache lines (_empty_padded_rows in flash_attention.py)
 Tensor empty_padded_rows(at::IntArrayRef shape, const at::TensorOptions& opt) {
-    const int64_t per = 16 / (int64_t)opt.dtype().itemsize(), n = shape[3], n_pad = (n + per - 1) / per * per;
+    const int64_t es = (int64_t)opt.dtype().itemsize(), n = shape[3];
+    const bool lines = n * es % 16 != 0 && n * es >= 512 && shape[2] * (n * es + 128) < (int64_t)1 << 31;
+    const int64_t per = (lines ? 128 : 16) / es, n_pad = (n + per - 1) / per * per;
     if (n_pad == n) return at::empty(shape, opt);
     return at::empty({shape[0], shape[1], shape[2], n_pad}, opt).narrow(3, 0, n);
 }
