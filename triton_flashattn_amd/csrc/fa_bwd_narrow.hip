@@ -341,8 +341,10 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
     // fp32: lane -> row 8 it + lane / 8, keys 4 (lane % 8) .. + 3, it = 0 .. 3
     const int db32_row = lane >> 3, db32_key = 4 * (lane & 7);
     // rows of whole aligned chunks leave through unconditional buffer stores (chunks outside the tensor get an offset
-    // outside the view), so that the loop has no branch around its stores and can count them
-    const bool db_fast = DBIAS == 1 && N % C::EPC == 0;
+    // outside the view), so that the loop has no branch around its stores and can count them.  (16 bits: of rows that end inside a
+    // chunk, all but the wave that holds the last keys; B=2 H=12 M=N=1001 D=32 34.6 -> 33.3 us.  fp32 there 48.4 -> 49.2, and the
+    // pair of waves gains nothing: D=64 bf16 38.4 / 38.5, fp32 47.5 / 50.)
+    const bool db_fast = DBIAS == 1 && (N % C::EPC == 0 || (DB16 && nw + 32 <= N));
     __amdgpu_buffer_rsrc_t db_rsrc = make_buffer(nullptr, 0);
     int db_off[2] = {0, 0};
     const int db_row_bytes = DBIAS == 1 ? (int)p.sdbias.m * C::ES : 0;

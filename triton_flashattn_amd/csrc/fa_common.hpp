@@ -516,10 +516,11 @@ template <typename T, int D, int BIAS, bool WITH_V = true, bool WIDE = false> st
     // the keys with running 64-bit addresses in scalar registers, one add per step: the K and V rows
     // of the next step to copy, and this wave's bias rows at the first key of the next slice to copy.
     uint64_t run_k, run_v, run_b;
-    // byte offset of this lane's chunk in bias copy `it`: with 1- and 2-byte elements the copies of a
-    // slice are whole groups of rows apart with the same chunk order, so one offset and a stride do
-    static constexpr int NBOFF = C::ES == 4 ? C::BCH : 1;
-    unsigned lean_boff[NBOFF];
+    // byte offset of this lane's chunk in copy `it` of a bias block, rows past M clamped to the last one.  (Formed from one offset
+    // and a stride, which has no clamp, the work-group with the last rows had no lean steps, and the grid waited for it.  us, dQ:
+    // byte mask B=8 H=12 M=N=1001 D=128 100 -> 92, dS B=2 H=12 M=N=1000 D=128 17.5 -> 15.8, D=64 13.4 -> 11.7; forward: bf16 B=4
+    // H=12 M=N=577 D=128 25.3 -> 23.2, fp32 B=4 H=16 M=N=1000 D=128 73.5 -> 71.2.)
+    unsigned lean_boff[C::BPB];
     // chunk index of copy i of this wave (scalar)
     __device__ __forceinline__ int copy_idx(int i) const { return LEAN ? (wave_s * C::KD + i) % C::NKD : c_idx[i]; }
 
@@ -640,21 +641,18 @@ template <typename T, int D, int BIAS, bool WITH_V = true, bool WIDE = false> st
         run_v = uniform_ptr(vp + (int64_t)k_kv * C::BK * sv);
         run_b = 0;
         if constexpr (C::ES != 0) {
-            run_b = uniform_ptr(reinterpret_cast<const unsigned char*>(bp) + ((int64_t)mw * sbm + (int64_t)k_b * C::BK) * C::ES);
-            // (2-byte elements: a copy covers 16 rows and the chunk order depends on (row / 4) % 4;
-            // 1-byte elements: one copy per slice)
-            static_assert(C::ES == 4 || C::ES == 2 || C::BPB == 1, "chunk order repeats from copy to copy");
-            static_assert(C::ES != 4 || C::NH == 1, "one offset per copy of a block");
+            const int first = mw < M ? mw : M - 1;
+            run_b = uniform_ptr(reinterpret_cast<const unsigned char*>(bp) + ((int64_t)first * sbm + (int64_t)k_b * C::BK) * C::ES);
 #pragma unroll
-            for (int it = 0; it < NBOFF; it++) {
+            for (int it = 0; it < C::BPB; it++) {
                 const int c = it * 64 + lane;
-                const int row = c / C::BCPR;
-                lean_boff[it] = (unsigned)(((int64_t)row * sbm + ((c % C::BCPR) ^ C::bswz(row)) * C::EPC) * C::ES);
+                const int row = c / C::BCPR, at = row < M - first ? row : M - 1 - first;
+                lean_boff[it] = (unsigned)(((int64_t)at * sbm + ((c % C::BCPR) ^ C::bswz(row)) * C::EPC) * C::ES);
             }
         }
     }
-    // issue_ahead for a step whose copies (K/V rows of step k + LA, bias slice of step k + NBS - 1, all
-    // 32 rows of this wave) lie wholly inside the tensors; run_start() was called for the first such step
+    // issue_ahead for a step whose copies (K/V rows of step k + LA, keys of the bias slice of step k + NBS - 1) lie
+    // wholly inside the tensors; run_start() was called for the first such step
     template <bool BV> __device__ __forceinline__ void issue_ahead_lean(int k) {
         const unsigned saved_m0 = lds_copy_begin();
         settle_ptrs(run_k, run_v, run_b);
@@ -682,20 +680,16 @@ template <typename T, int D, int BIAS, bool WITH_V = true, bool WIDE = false> st
             const unsigned dst = lds_bias + (unsigned)((k + C::NBS - 1) % C::NBS) * C::BSLOT;
 #pragma unroll
             for (int it = 0; it < C::BCH; it++) {
-                const unsigned off = C::ES == 4 ? lean_boff[it < NBOFF ? it : 0]
-                                                : lean_boff[0] + (unsigned)((it % C::BPB) * (64 / C::BCPR) * (int)sbm * C::ES + it / C::BPB * 32 * C::ES);
-                lds_copy16(run_b, off, dst + it * 1024);
+                lds_copy16(run_b, lean_boff[it % C::BPB] + (unsigned)(it / C::BPB * 32 * C::ES), dst + it * 1024);
             }
             run_b += C::BK * C::ES;
         }
         lds_copy_end(saved_m0);
     }
-    // lean steps a kernel may run from step 0: those whose copies stay inside N keys (and, with a bias, whose
-    // work-group has all of its rows), at most `limit`
-    __device__ __forceinline__ int lean_steps(int limit, int wg_rows_end) const {
+    // lean steps a kernel may run from step 0: those whose copies stay inside N keys, at most `limit`
+    __device__ __forceinline__ int lean_steps(int limit) const {
         constexpr int AHEAD = (C::ES != 0 && C::NBS - 1 > C::LA) ? C::NBS - 1 : C::LA;
         int n = N / C::BK - AHEAD;
-        if (C::ES != 0 && wg_rows_end > M) n = 0;
         n = n < limit ? n : limit;
         return n < 0 ? 0 : n;
     }

@@ -531,7 +531,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
             if constexpr (TB == 0) split_q();  // (while the first copies are on their way)
         }
         // the leading fast steps whose copies stay inside the tensors issue them without clamps
-        const int n_lean = (BV || TB == 0) ? ks_.lean_steps(n_fast, m0 + BM) : 0;
+        const int n_lean = (BV || TB == 0) ? ks_.lean_steps(n_fast) : 0;
         int k = 0;
         if (n_lean > 0) {
             ks_.run_start(C::LA, C::NBS - 1);
