@@ -26,7 +26,8 @@
  * the bytes behind the last key of EVERY row, up to the end of its 16-byte chunk, are read (never
  * written), the last row of the last (batch, head) slice included: the caller guarantees that the
  * chunk holding the last element of the tensor lies inside the allocation (a row-strided view whose
- * last row ends the allocation does not qualify and must be copied to a padded pitch first).  With FA_MI355_VERBOSE set in the
+ * last row ends the allocation does not qualify and must be copied to a padded pitch first).  An fp32 bias with unit N
+ * stride that misses it is read 4 bytes to a lane up to head dim 64, by copies too and nothing behind a row.  With FA_MI355_VERBOSE set in the
  * environment the library says on stderr, once per process, when a bias or dbias misses that path
  * and is read or written element by element (several times slower).
  */

@@ -195,6 +195,15 @@ bool bias_vec_ok(const void* ptr, const int64_t s[4], const fa_problem& p) {
     return true;
 }
 
+// How the kernels fetch the rows of a bias: 1 in aligned 16-byte chunks; 2 (fp32, head dims up to 64) 4 bytes to a lane, whatever
+// multiple of 4 bytes a row starts at; 0 element by element.
+int bias_rows(const void* ptr, const int64_t s[4], const fa_problem& p) {
+    if (bias_vec_ok(ptr, s, p)) return 1;
+    if (p.bias_dtype != FA_BIAS_F32 || p.D > 64 || (p.N > 1 && s[3] != 1) || reinterpret_cast<uintptr_t>(ptr) % 4 != 0) return 0;
+    // (offsets from the first row of a (batch, head) slice are formed in 32 bits)
+    return s[2] >= 0 && ((int64_t)(p.M - 1) * s[2] + p.N) * 4 < (1ll << 31) ? 2 : 0;
+}
+
 // rows of bias or dbias may be accessed four elements at a time, at multiples of four
 bool bias_quads_ok(const void* ptr, const int64_t s[4], const fa_problem& p) {
     const int es = bias_elem_size(p.bias_dtype);
@@ -375,7 +384,7 @@ int fa_fwd_dims(const fa_fwd_args* a, int d_qk, int d_v, void* stream) {
     k.d_qk = d_qk; k.d_v = d_v; k.qk_inv = (256 + d_qk / 8 - 1) / (d_qk / 8);
     if (a->bias && p.bias_dtype != FA_BIAS_ALIBI) {
         k.sbias = s4(a->bias_strides);
-        k.bias_vec = bias_vec_ok(a->bias, a->bias_strides, p) ? 1 : 0;
+        k.bias_vec = bias_rows(a->bias, a->bias_strides, p);
         if (!k.bias_vec) note_slow_bias("bias", a->bias, a->bias_strides, p);
     }
     k.n_mtiles = (p.M + fa::fwd_block_m() - 1) / fa::fwd_block_m();
@@ -478,7 +487,7 @@ int bwd_enqueue(const fa_bwd_args* a, int d_qk, int d_v, void* stream, int stage
     k.sdo = s3(a->do_strides); k.sdq = s3(a->dq_strides); k.sdk = s3(a->dk_strides); k.sdv = s3(a->dv_strides);
     if (a->bias && p.bias_dtype != FA_BIAS_ALIBI) {
         k.sbias = s4(a->bias_strides);
-        k.bias_vec = bias_vec_ok(a->bias, a->bias_strides, p) ? 1 : 0;
+        k.bias_vec = bias_rows(a->bias, a->bias_strides, p);
     }
     // a bias that does not depend on the query row: the dK/dV kernel keeps it in one register per key
     if (a->bias && p.bias_dtype >= FA_BIAS_BOOL && p.bias_dtype <= FA_BIAS_F32 && (p.M == 1 || a->bias_strides[2] == 0))

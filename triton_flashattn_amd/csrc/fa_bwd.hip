@@ -122,7 +122,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
     KS ks_;
     ks_.init(smem, kp, vp, bp, p.sk.s, p.sv.s, FROM_DS ? p.sdbias.m : p.sbias.m, FROM_DS ? p.sdbias.n : p.sbias.n, M, N,
              mw, wave, lane, chunks, p.d_v / 8);
-    const bool bias_copies = FROM_DS || (TB != 0 && p.bias_vec);
+    constexpr bool BY_DWORD = BIAS == 4 && D <= 64 && !FROM_DS;
 
     // Q^T and dO^T as B operands: column my_m, k = d
     const T* dop = reinterpret_cast<const T*>(p.dout) + (int64_t)b * p.sdo.b + (int64_t)h * p.sdo.h;
@@ -247,7 +247,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
     // LEAN: the copies of the step need no clamps (KeyStream::issue_ahead_lean).
     auto kv_step = [&](int k, auto step_tag, auto bv_tag, auto lean_tag) {
         constexpr bool STEP_MASKED = decltype(step_tag)::value;
-        constexpr bool BV = decltype(bv_tag)::value;
+        constexpr int BV = decltype(bv_tag)::value;
         constexpr bool LEAN = decltype(lean_tag)::value;
         auto issue_ahead = [&]() {
             if constexpr (LEAN) ks_.template issue_ahead_lean<BV>(k);
@@ -487,7 +487,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
     // ragged last tile was the longest of a causal grid: B=1 H=16 M=N=6001 D=128 0.298 -> 0.218 ms)
     if (!(qk_scale > 0.f)) n_fast = 0;
     auto run = [&](auto bv_tag) {
-        constexpr bool BV = decltype(bv_tag)::value;
+        constexpr int BV = decltype(bv_tag)::value;
         auto stage_row = [&]() {
             if (ROWB)
                 stage_row_bias(reinterpret_cast<float*>(smem + C::LDS_BYTES), p.bias, p.row_bias_kind,
@@ -541,10 +541,10 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
             if constexpr (TB == 0 && !FROM_DS) split_q();  // (while the first copies are on their way)
         }
         // the leading fast steps whose copies stay inside the tensors issue them without clamps
-        const int n_lean = (BV || TB == 0) ? ks_.lean_steps(n_fast) : 0;
+        const int n_lean = (BV != kByElement || TB == 0) ? ks_.lean_steps(n_fast) : 0;
         int k = 0;
         if (n_lean > 0) {
-            ks_.run_start(C::LA, C::NBS - 1);
+            ks_.template run_start<BV>(C::LA, C::NBS - 1);
 #pragma unroll 1
             for (; k < n_lean; k++) kv_step(k, std::false_type{}, bv_tag, std::true_type{});
         }
@@ -553,8 +553,20 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
 #pragma unroll 1
         for (; k < n_steps; k++) kv_step(k, std::true_type{}, bv_tag, std::false_type{});
     };
-    if (bias_copies) run(std::true_type{});
-    else run(std::false_type{});
+    if constexpr (FROM_DS) {
+        run(RowsTag<kByChunk>{});
+    } else if constexpr (TB == 0) {
+        run(RowsTag<kByElement>{});
+    } else {
+        if constexpr (BY_DWORD) {
+            if (p.bias_vec == kByChunk) run(RowsTag<kByChunk>{});
+            else if (p.bias_vec == kByDword) run(RowsTag<kByDword>{});
+            else run(RowsTag<kByElement>{});
+        } else {
+            if (p.bias_vec == kByChunk) run(RowsTag<kByChunk>{});
+            else run(RowsTag<kByElement>{});
+        }
+    }
 
     // ---- epilogue: dq = dQ * sm_scale (flash_attention.py:644-646) ----
     ks_.drain();  // K/V slots are dead and no copy is in flight: reuse their LDS for the output tile
@@ -850,6 +862,7 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
     const int n_mblocks = (M + BMI - 1) / BMI;
     // causal: query blocks that end above the first key of this tile see none of its keys
     const int mb_first = CAUSAL ? (n0 / BMI) : 0;
+    constexpr bool BY_DWORD = BIAS == 4 && D <= 64;
     const bool bias_vec = TB != 0 && p.bias_vec;
     const bool dbias_vec = DBIAS == 1 && p.dbias_vec;
 
@@ -917,10 +930,19 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
     // slice (row c / BCPR, 16-byte chunk c % BCPR) lands at byte 16 c of the slot, i.e. the slot
     // is the row-major slice.  Rows past M re-read row M - 1 (masked where they are used) and chunks that start past N
     // re-read column 0 (a lane is a key: what such a lane forms is not stored).
-    auto issue_bias = [&](int mb) {
+    auto issue_bias = [&](int mb, auto bv_tag) {
         if constexpr (TB != 0) {
             const unsigned dst = lds_base + C::OFF_BIAS + (kb * C::RING + (mb - mb_first) % C::RING) * C::BT_BYTES;
             const uint64_t base = uniform_ptr(bp);
+            if constexpr (decltype(bv_tag)::value == kByDword) {
+#pragma unroll
+                for (int it = 0; it < 16; it++) {
+                    int m = mb * BMI + 2 * it + g;
+                    m = m < M ? m : M - 1;
+                    lds_copy4(base, (unsigned)(((int64_t)m * p.sbias.m + (my_n < N ? my_n : N - 1)) * 4), dst + it * 256);
+                }
+                return;
+            }
 #pragma unroll
             for (int it = 0; it < C::BCH; it++) {
                 const int c = it * 64 + lane;
@@ -959,6 +981,7 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
         int nn = nw + (lane % C::BCPR) * C::EPC;
         nn = nn < N ? nn : 0;
         bias_off0 = (unsigned)(((int64_t)(lane / C::BCPR) * p.sbias.m + nn) * C::ES);
+        if (BY_DWORD && p.bias_vec == kByDword) bias_off0 = (unsigned)(((int64_t)g * p.sbias.m + (my_n < N ? my_n : N - 1)) * 4);
     }
     auto run_start = [&](const T* rows, int64_t row_stride, const float* stat, int mb, int mb_bias) {
         run_rows = uniform_ptr(rows + (int64_t)mb * BMI * row_stride);
@@ -986,12 +1009,16 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
         const unsigned slot = (unsigned)mb % C::NDOB;
         issue_next_rows(p.sdo.s, cdo_off, lds_base + C::OFF_DO + slot * C::Q_BYTES, lds_base + C::OFF_DELTA + slot * C::STAT_BYTES);
     };
-    auto issue_next_bias = [&](int mb) {
+    auto issue_next_bias = [&](int mb, auto bv_tag) {
         if constexpr (TB != 0) {
+            constexpr int N_COPIES = decltype(bv_tag)::value == kByDword ? 16 : C::BCH;
             const unsigned dst = lds_base + C::OFF_BIAS + (kb * C::RING + (unsigned)(mb - mb_first) % C::RING) * C::BT_BYTES;
-            const unsigned rows_step = (unsigned)((64 / C::BCPR) * (int)p.sbias.m * C::ES);  // the rows one copy covers
+            const unsigned rows_step = (unsigned)(BMI / N_COPIES * (int)p.sbias.m * C::ES);  // the rows one copy covers
 #pragma unroll
-            for (int it = 0; it < C::BCH; it++) lds_copy16(run_bias, bias_off0 + it * rows_step, dst + it * 1024);
+            for (int it = 0; it < N_COPIES; it++) {
+                if constexpr (N_COPIES == C::BCH) lds_copy16(run_bias, bias_off0 + it * rows_step, dst + it * 1024);
+                else lds_copy4(run_bias, bias_off0 + it * rows_step, dst + it * 256);
+            }
             run_bias += (uint64_t)(BMI * C::ES) * (uint64_t)p.sbias.m;
         }
     };
@@ -1033,7 +1060,12 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
 #pragma unroll 1
         for (int i = 0; i < C::LA; i++) {
             if (s_wave == Q_BY_S) issue_q(mb_first + i);
-            if (s_wave && TB != 0 && bias_vec) issue_bias(mb_first + i);
+            if constexpr (BY_DWORD) {
+                if (s_wave && p.bias_vec == kByDword) issue_bias(mb_first + i, RowsTag<kByDword>{});
+                else if (s_wave && bias_vec) issue_bias(mb_first + i, RowsTag<kByChunk>{});
+            } else {
+                if (s_wave && TB != 0 && bias_vec) issue_bias(mb_first + i, RowsTag<kByChunk>{});
+            }
             if (s_wave == DO_BY_S && i < C::LA - 1) issue_do(mb_first + i);
         }
         lds_copy_end(saved_m0);
@@ -1100,8 +1132,9 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
     if (s_wave) {
         // ================================ S-wave ================================
         auto s_loop = [&](auto bv_tag) {
-        constexpr bool BV = decltype(bv_tag)::value;                    // bias slices come by copy
-        constexpr int OPS = (BV ? C::BCH : 0) + ((Q_BY_S ? 1 : 0) + (DO_BY_S ? 1 : 0)) * (C::QD + 1);  // copies per step
+        constexpr int BV = decltype(bv_tag)::value;                    // bias slices come by copy
+        constexpr int BIAS_COPIES = BV == kByElement ? 0 : BV == kByDword ? 16 : C::BCH;
+        constexpr int OPS = BIAS_COPIES + ((Q_BY_S ? 1 : 0) + (DO_BY_S ? 1 : 0)) * (C::QD + 1);  // copies per step
         // S_AHEAD: the scores of a block are formed at the END of the step before the one that turns
         // them into P, so that a step of this role opens with vector work (exponentials) while the
         // partner wave on the same SIMD opens with matrix products, and closes with matrix products
@@ -1129,11 +1162,11 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
                 if constexpr (IN) {
                     settle_ptrs(run_rows, run_stat, run_bias);
                     if constexpr (Q_BY_S) issue_next_q(nb + C::LA);
-                    if constexpr (BV) issue_next_bias(nb + C::LA);
+                    if constexpr (BV != kByElement) issue_next_bias(nb + C::LA, bv_tag);
                     if constexpr (DO_BY_S) issue_next_do(t + C::LA);
                 } else {
                     if constexpr (Q_BY_S) issue_q(nb + C::LA);
-                    if constexpr (BV) issue_bias(nb + C::LA);
+                    if constexpr (BV != kByElement) issue_bias(nb + C::LA, bv_tag);
                     if constexpr (DO_BY_S) issue_do(t + C::LA);
                 }
                 lds_copy_end(saved_m0);
@@ -1209,7 +1242,7 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
                     else p_step(std::false_type{});
                 }
             };
-            if constexpr (TB != 0 && !BV) {
+            if constexpr (TB != 0 && BV == kByElement) {
                 if (nb < n_mblocks) load_bias_scalar(nb, ring_lds + ((nb - mb_first) % C::RING) * C::BT_BYTES);
             }
             if constexpr (S_AHEAD) {
@@ -1273,7 +1306,7 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
             // barrier (it sinks matrix instructions below it where it can): measured 3 % faster at head
             // dim 128 without a bias, slower or equal everywhere else, so only there.
             if constexpr (BIAS == 0 && D == 128) __builtin_amdgcn_sched_barrier(0);
-            if constexpr (S_AHEAD) wait_vmcnt<(BV ? C::BCH : 0) + OPS*(C::LA - 2)>();
+            if constexpr (S_AHEAD) wait_vmcnt<BIAS_COPIES + OPS*(C::LA - 2)>();
             else wait_vmcnt<OPS*(C::LA - 1)>();
             lds_barrier();
         };
@@ -1283,7 +1316,7 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
         const int t_end = n_mblocks + 1;
         int t_in = mb_first, t_out = n_full - C::LA - 1;
         if (CAUSAL) t_in = (n0 + BN - 1 + BMI - 1) / BMI - 1 > t_in ? (n0 + BN - 1 + BMI - 1) / BMI - 1 : t_in;
-        if (TB != 0 && !BV) t_out = t_in;  // bias element by element: no interior
+        if (TB != 0 && BV == kByElement) t_out = t_in;  // bias element by element: no interior
         t_in = t_in < t_end ? t_in : t_end;
         t_out = t_out < t_in ? t_in : (t_out < t_end ? t_out : t_end);
         // (two passes over ONE copy of the general loop, the interior loop between them)
@@ -1300,8 +1333,14 @@ __global__ __launch_bounds__((BwdCfg<D, tile_kind(BIAS), W>::NT), (BwdCfg<D, til
             stop = t_end;
         }
         };
-        if (TB != 0 && bias_vec) s_loop(std::true_type{});
-        else s_loop(std::false_type{});
+        if constexpr (BY_DWORD) {
+            if (p.bias_vec == kByDword) s_loop(RowsTag<kByDword>{});
+            else if (bias_vec) s_loop(RowsTag<kByChunk>{});
+            else s_loop(RowsTag<kByElement>{});
+        } else {
+            if (TB != 0 && bias_vec) s_loop(RowsTag<kByChunk>{});
+            else s_loop(RowsTag<kByElement>{});
+        }
     } else {
         // ================================ dP-wave ================================
         // dS^T tile of this wave: 32 keys x BMI rows.  A lane writes its 4 consecutive rows of one key

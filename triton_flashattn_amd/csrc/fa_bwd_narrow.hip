@@ -107,6 +107,19 @@ template <> struct BiasBlock<4> {
     }
 };
 
+// The same with the values in registers before they are used (an fp32 bias only: the others' are after load()).
+template <int BIAS> struct BiasAhead : BiasBlock<BIAS> {
+    __device__ __forceinline__ void fetch(const BiasBlock<BIAS>& from) { *static_cast<BiasBlock<BIAS>*>(this) = from; }
+};
+template <> struct BiasAhead<4> {
+    float v[16];
+    __device__ __forceinline__ void fetch(const BiasBlock<4>& from) {
+#pragma unroll
+        for (int i = 0; i < 16; i++) v[i] = from.get(i);
+    }
+    __device__ __forceinline__ float get(int i) const { return v[i]; }
+};
+
 // Value that lane 16 (l / 16) + i holds, for lane l: a modifier of the instruction that uses it, no instruction of its own.
 template <int I> __device__ __forceinline__ float row_bcast(float x) {
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x150 + I, 0xf, 0xf, true));
@@ -202,7 +215,7 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
     const float qk_scale = p.sm_scale * kLog2e;
     // causal: steps that end above the first key of this tile see none of its keys
     const int t0 = CAUSAL ? n0 / SR : 0, t_end = (M + SR - 1) / SR;
-    const bool bias_vec = TB != 0 && p.bias_vec;
+    constexpr bool BY_DWORD = TB == 4;
 
     // rows above the diagonal block of a wave are not visited and owe zeros to dBias
     if (DBIAS == 1 && CAUSAL) {
@@ -235,7 +248,8 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
     const unsigned stat_dst = lds_base + C::OFF_STAT + (unsigned)(wave >> 1) * C::STAT_BYTES;
     const unsigned bias_dst = lds_base + C::OFF_BIAS + (unsigned)wave * C::BSLOT;
     auto slot_of = [&](int t) { return (unsigned)t % C::NS; };
-    auto issue = [&](int t, bool bias_copy) {
+    auto issue = [&](int t, auto bv_tag) {
+        constexpr int BV = decltype(bv_tag)::value;
         const unsigned slot = slot_of(t);
         const int m0 = t * SR < M ? t * SR : M - 1;  // a step past the end is the last row over and over
         const uint64_t qb = uniform_ptr(qp + (int64_t)m0 * p.sq.s), dob = uniform_ptr(dop + (int64_t)m0 * p.sdo.s);
@@ -260,7 +274,15 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
         m = m < M ? m : M - 1;
         lds_copy4(uniform_ptr(statp), (unsigned)m * 4u, stat_dst + slot * 2 * C::STAT_BYTES);
         if constexpr (TB != 0) {
-            if (bias_copy) {
+            if constexpr (BV == kByDword) {
+                const uint64_t base = uniform_ptr(bp);
+#pragma unroll
+                for (int it = 0; it < 16; it++) {
+                    int mb = t * SR + 2 * it + g;
+                    mb = mb < M ? mb : M - 1;
+                    lds_copy4(base, (unsigned)(((int64_t)mb * p.sbias.m + (my_n < N ? my_n : N - 1)) * 4), bias_dst + slot * 4 * C::BSLOT + it * 256);
+                }
+            } else if constexpr (BV == kByChunk) {
                 const uint64_t base = uniform_ptr(bp);
 #pragma unroll
                 for (int it = 0; it < C::BCH; it++) {
@@ -281,6 +303,7 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
         int nn = nw + (lane % C::BCPR) * C::EPC;
         nn = nn < N ? nn : 0;
         bias_off0 = (unsigned)(((int64_t)(lane / C::BCPR) * p.sbias.m + nn) * C::ES);
+        if (BY_DWORD && p.bias_vec == kByDword) bias_off0 = (unsigned)(((int64_t)g * p.sbias.m + (my_n < N ? my_n : N - 1)) * 4);
     }
     auto run_start = [&](int t) {
         run_q = uniform_ptr(qp + (int64_t)t * SR * p.sq.s);
@@ -288,7 +311,7 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
         run_stat = uniform_ptr(statp + (int64_t)t * SR);
         if constexpr (TB != 0) run_bias = uniform_ptr(bp + (int64_t)t * SR * p.sbias.m);
     };
-    auto issue_next = [&](int t) {
+    auto issue_next = [&](int t, auto bv_tag) {
         settle_ptrs(run_q, run_do, run_stat);
         if constexpr (TB != 0) run_bias = uniform_ptr(reinterpret_cast<const void*>(run_bias));
         const unsigned slot = slot_of(t);
@@ -304,9 +327,13 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
         run_do += (uint64_t)(SR * 2) * (uint64_t)p.sdo.s;
         run_stat += SR * 4;
         if constexpr (TB != 0) {
-            const unsigned rows_step = (unsigned)((64 / C::BCPR) * (int)p.sbias.m * C::ES);  // the rows one copy covers
+            constexpr int N_COPIES = decltype(bv_tag)::value == kByDword ? 16 : C::BCH;
+            const unsigned rows_step = (unsigned)(SR / N_COPIES * (int)p.sbias.m * C::ES);  // the rows one copy covers
 #pragma unroll
-            for (int it = 0; it < C::BCH; it++) lds_copy16(run_bias, bias_off0 + it * rows_step, bias_dst + slot * 4 * C::BSLOT + it * 1024);
+            for (int it = 0; it < N_COPIES; it++) {
+                if constexpr (N_COPIES == C::BCH) lds_copy16(run_bias, bias_off0 + it * rows_step, bias_dst + slot * 4 * C::BSLOT + it * 1024);
+                else lds_copy4(run_bias, bias_off0 + it * rows_step, bias_dst + slot * 4 * C::BSLOT + it * 256);
+            }
             run_bias += (uint64_t)(SR * C::ES) * (uint64_t)p.sbias.m;
         }
     };
@@ -365,9 +392,9 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
     const unsigned rows_l = SW::rows_lane(lane), cols_l = SW::cols_lane(lane);
 
     auto run = [&](auto bv_tag, auto fast_tag) {
-        constexpr bool BV = decltype(bv_tag)::value;         // bias slices come by copy
+        constexpr int BV = decltype(bv_tag)::value;          // how bias slices come (BiasRows)
         constexpr bool DB_FAST = decltype(fast_tag)::value;
-        constexpr int OPS = 2 * C::QD + 1 + (BV ? C::BCH : 0);  // copies per wave and step
+        constexpr int OPS = 2 * C::QD + 1 + (BV == kByElement ? 0 : BV == kByDword ? 16 : C::BCH);  // copies per wave and step
         {
             const unsigned free_slot = slot_of(t0 + LA);
             const unsigned half_slot = lds_base + (wave < 2 ? 0u : (unsigned)C::OFF_DO) + free_slot * C::ROWS_BYTES + (unsigned)(wave & 1) * WR::BYTES;
@@ -379,7 +406,7 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
             WR::issue(kp, p.sk.s, nw, N, k_tile, lane, [&](int c) { return live_chunk(c, p.d_qk / 8); });
             if constexpr (V_STAGED) WR::issue(vp, p.sv.s, nw, N, v_tile, lane, [&](int c) { return live_chunk(c, p.d_v / 8); });
 #pragma unroll
-            for (int i = 0; i < LA; i++) issue(t0 + i, BV);
+            for (int i = 0; i < LA; i++) issue(t0 + i, bv_tag);
             lds_copy_end(saved_m0);
             // (the compiler's own loads, too: left in flight, it would wait for everything in every step)
             WR::template arrived<0>();
@@ -410,13 +437,13 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
             lds_barrier();
             {
                 const unsigned saved_m0 = lds_copy_begin();
-                if constexpr (LEAN) issue_next(t + LA);
-                else issue(t + LA, BV);
+                if constexpr (LEAN) issue_next(t + LA, bv_tag);
+                else issue(t + LA, bv_tag);
                 lds_copy_end(saved_m0);
             }
             whole = MASKED ? 0 : whole + 1;
             if (MASKED && !live) return;
-            if constexpr (TB != 0 && !BV) load_bias_scalar(t);
+            if constexpr (TB != 0 && BV == kByElement) load_bias_scalar(t);
             const unsigned slot = slot_of(t);
             const unsigned q_tile = lds_base + slot * C::ROWS_BYTES, do_tile = q_tile + C::OFF_DO;
             const float* stat = reinterpret_cast<const float*>(smem + C::OFF_STAT + slot * 2 * C::STAT_BYTES);
@@ -429,7 +456,7 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
             // that touch the last rows or the causal diagonal follow the reference's additive -1.0e6 arithmetic term by
             // term, and rows past M have none; the others fold everything into one exponent.  (Keys past N need no mask:
             // nothing of them is stored.) ----
-            auto p_value = [&](auto mk_tag, int m0, int i, float s, float lse, const BiasBlock<BIAS>& bias) {
+            auto p_value = [&](auto mk_tag, int m0, int i, float s, float lse, const auto& bias) {
                 constexpr bool MK = decltype(mk_tag)::value;
                 float bv = bias.get(i);
                 if constexpr (BIAS == 5) bv = alibi_bias(neg_slope, ratio, (float)(m0 + 4 * g) + (float)(8 * (i >> 2) + (i & 3)), (float)my_n);
@@ -605,25 +632,67 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
                 __builtin_amdgcn_sched_barrier(0);  // keep the blocks apart
                 if (MASKED && ((CAUSAL && m0 + 31 < nw) || m0 >= M)) continue;
                 const bool need_mask = MASKED && (m0 + 32 > M || (CAUSAL && m0 < nw + 31));
+                // Up to head dim 32 there are registers for everything that a block reads from LDS, fetched ahead of where it is
+                // used: operands of the first two products, then, under them, LSE, bias and the operands of the other two.  Left to
+                // the compiler, each read waited for the one before it in some of these kernels.  us, before -> after: D=32, fp32 and
+                // dBias B=2 H=12 M=N=1024 39.1 -> 36.2, B=8 154.8 -> 141.2; bf16 and dBias B=2 30.7 -> 29.5, causal H=8 28.0 -> 26.6;
+                // fp32 read B=16 H=8 M=N=256 10.6 -> 10.2; D=16, fp32 and dBias 38.0 -> 36.5.
+                constexpr bool AHEAD = D <= 32 && C::MIN_BLOCKS == 2;
+                constexpr bool BIAS_AHEAD = AHEAD || (D == 64 && TB == 4 && DBIAS == 0);  // (16 registers)
+                constexpr int NP = 2 * C::DB;
+                auto fence = [&]() {
+                    if constexpr (AHEAD) __builtin_amdgcn_sched_barrier(0);
+                };
+                T8 q_op[C::KSTEPS], do_op[C::KSTEPS], do_col[NP], q_col[NP];
+                f32x4 lse_ahead[4];
+                BiasBlock<BIAS> bias;
+                BiasAhead<BIAS> bias_ahead;
                 const float del = load_delta(nb);
                 f32x16 s, dp;
 #pragma unroll
                 for (int i = 0; i < 16; i++) s[i] = dp[i] = 0.f;
+                if constexpr (AHEAD) {
 #pragma unroll
-                for (int ks = 0; ks < C::KSTEPS; ks++) s = mfma32(SW::template row8_at<T8>(q_tile + rows_l, nb * 32, ks), kreg[ks], s);
+                    for (int ks = 0; ks < C::KSTEPS; ks++) q_op[ks] = SW::template row8_at<T8>(q_tile + rows_l, nb * 32, ks);
 #pragma unroll
-                for (int ks = 0; ks < C::KSTEPS; ks++) dp = mfma32(SW::template row8_at<T8>(do_tile + rows_l, nb * 32, ks), vreg[ks], dp);
-                BiasBlock<BIAS> bias;
-                bias.load(b_tile + nb * C::BBLOCK, lane);
+                    for (int ks = 0; ks < C::KSTEPS; ks++) do_op[ks] = SW::template row8_at<T8>(do_tile + rows_l, nb * 32, ks);
+                    fence();
+#pragma unroll
+                    for (int ks = 0; ks < C::KSTEPS; ks++) s = mfma32(q_op[ks], kreg[ks], s);
+#pragma unroll
+                    for (int ks = 0; ks < C::KSTEPS; ks++) dp = mfma32(do_op[ks], vreg[ks], dp);
+#pragma unroll
+                    for (int q4 = 0; q4 < 4; q4++) lse_ahead[q4] = load_lse(nb, q4);
+                    bias.load(b_tile + nb * C::BBLOCK, lane);
+                    bias_ahead.fetch(bias);
+#pragma unroll
+                    for (int i = 0; i < NP; i++) {
+                        do_col[i] = SW::template col8_at<T8>(do_tile + cols_l, nb * 32 + (i / C::DB) * 16, i % C::DB);
+                        q_col[i] = SW::template col8_at<T8>(q_tile + cols_l, nb * 32 + (i / C::DB) * 16, i % C::DB);
+                    }
+                    fence();
+                } else {
+#pragma unroll
+                    for (int ks = 0; ks < C::KSTEPS; ks++) s = mfma32(SW::template row8_at<T8>(q_tile + rows_l, nb * 32, ks), kreg[ks], s);
+#pragma unroll
+                    for (int ks = 0; ks < C::KSTEPS; ks++) dp = mfma32(SW::template row8_at<T8>(do_tile + rows_l, nb * 32, ks), vreg[ks], dp);
+                    bias.load(b_tile + nb * C::BBLOCK, lane);
+                    if constexpr (BIAS_AHEAD) {
+                        bias_ahead.fetch(bias);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
                 T8 pb[2], ds[2];
                 auto elements = [&](auto mk_tag) {
 #pragma unroll
                     for (int q4 = 0; q4 < 4; q4++) {
-                        const f32x4 lse = load_lse(nb, q4);
+                        const f32x4 lse = AHEAD ? lse_ahead[q4] : load_lse(nb, q4);
 #pragma unroll
                         for (int e = 0; e < 4; e++) {
                             const int i = q4 * 4 + e;
-                            const float pv = p_value(mk_tag, m0, i, s[i], lse[e], bias);
+                            float pv;
+                            if constexpr (BIAS_AHEAD) pv = p_value(mk_tag, m0, i, s[i], lse[e], bias_ahead);
+                            else pv = p_value(mk_tag, m0, i, s[i], lse[e], bias);
                             pb[i >> 3][i & 7] = (T)pv;
                             dp[i] = pv * (dp[i] - row_bcast(del, i));  // dS (flash_attention.py:303-308)
                             ds[i >> 3][i & 7] = (T)dp[i];
@@ -662,8 +731,12 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
                 for (int kk = 0; kk < 2; kk++)
 #pragma unroll
                     for (int db = 0; db < C::DB; db++) {
-                        dv[db] = mfma32(SW::template col8_at<T8>(do_tile + cols_l, nb * 32 + kk * 16, db), pb[kk], dv[db]);
-                        dk[db] = mfma32(SW::template col8_at<T8>(q_tile + cols_l, nb * 32 + kk * 16, db), ds[kk], dk[db]);
+                        if constexpr (!AHEAD) {
+                            do_col[kk * C::DB + db] = SW::template col8_at<T8>(do_tile + cols_l, nb * 32 + kk * 16, db);
+                            q_col[kk * C::DB + db] = SW::template col8_at<T8>(q_tile + cols_l, nb * 32 + kk * 16, db);
+                        }
+                        dv[db] = mfma32(do_col[kk * C::DB + db], pb[kk], dv[db]);
+                        dk[db] = mfma32(q_col[kk * C::DB + db], ds[kk], dk[db]);
                     }
             }
         };
@@ -673,7 +746,7 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
         int t_in = CAUSAL ? (n0 + BN - 1 + SR - 1) / SR : t0;
         t_in = t_in < t_end ? t_in : t_end;
         int t_out = M / SR - LA;
-        if ((TB != 0 && !BV) || !live || t_out < t_in) t_out = t_in;
+        if ((TB != 0 && BV == kByElement) || !live || t_out < t_in) t_out = t_in;
         // (two passes over ONE copy of the general loop, the others between them)
         int t = t0, stop = t_in;
 #pragma unroll 1
@@ -689,14 +762,30 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
         }
         wait_vmcnt<0>();  // nothing may land in LDS once the work-group is gone
     };
+    auto run_rows = [&](auto fast_tag) {
+        if constexpr (TB == 0) {
+            run(RowsTag<kByElement>{}, fast_tag);
+        } else {
+            if constexpr (BY_DWORD && DBIAS == 1) {
+                if (p.bias_vec == kByDword) run(RowsTag<kByDword>{}, fast_tag);
+                else run(RowsTag<kByChunk>{}, fast_tag);
+            } else if constexpr (DBIAS == 1) {
+                run(RowsTag<kByChunk>{}, fast_tag);
+            } else if constexpr (BY_DWORD) {
+                if (p.bias_vec == kByChunk) run(RowsTag<kByChunk>{}, fast_tag);
+                else if (p.bias_vec == kByDword) run(RowsTag<kByDword>{}, fast_tag);
+                else run(RowsTag<kByElement>{}, fast_tag);
+            } else {
+                if (p.bias_vec == kByChunk) run(RowsTag<kByChunk>{}, fast_tag);
+                else run(RowsTag<kByElement>{}, fast_tag);
+            }
+        }
+    };
     if constexpr (DBIAS == 1) {
-        if (db_fast) run(std::true_type{}, std::true_type{});
-        else run(std::true_type{}, std::false_type{});
-    } else if constexpr (TB != 0) {
-        if (bias_vec) run(std::true_type{}, std::false_type{});
-        else run(std::false_type{}, std::false_type{});
+        if (db_fast) run_rows(std::true_type{});
+        else run_rows(std::false_type{});
     } else {
-        run(std::false_type{}, std::false_type{});
+        run_rows(std::false_type{});
     }
 
     if constexpr (DBIAS == 2 && BIAS == 5) {

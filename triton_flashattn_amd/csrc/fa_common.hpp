@@ -27,6 +27,11 @@ typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 
 template <bool V> struct BoolTag { static constexpr bool value = V; };  // a compile-time flag as an argument
 
+// How the rows of a bias tile reach LDS (bias_vec of the parameters): one element at a time through registers, or by direct copies
+// of aligned 16-byte chunks, or, fp32 rows at any multiple of 4 bytes, by direct copies of 4 bytes to a lane.
+enum BiasRows { kByElement = 0, kByChunk = 1, kByDword = 2 };
+template <int V> struct RowsTag { static constexpr int value = V; };
+
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kMask = -1.0e6f;  // additive mask term, in log2 units
 constexpr float kLowest = -3.402823466e38f;  // score of a key that does not exist
@@ -570,8 +575,9 @@ template <typename T, int D, int BIAS, bool WITH_V = true, bool WIDE = false> st
         else if constexpr (C::STAGE == C::kBehind) return lds_kv + C::LOOP_BYTES + (unsigned)wave_s * R;
         else return wave_s == 0 ? k_free : wave_s == 1 ? v_free : lds_kv + C::LOOP_BYTES + (unsigned)(wave_s - 2) * R;
     }
-    // copies of a wave in prologue()
-    template <bool BV> static constexpr int prologue_copies() { return C::LA * (WITH_V ? 2 : 1) * C::KD + (BV ? (C::NBS - 1) * C::BCH : 0); }
+    // BV: how the bias rows come (BiasRows).  Copies of a bias slice, and of a wave in prologue()
+    template <int BV> static constexpr int bias_copies() { return BV == kByElement ? 0 : BV == kByDword ? 4 * C::BCH : C::BCH; }
+    template <int BV> static constexpr int prologue_copies() { return C::LA * (WITH_V ? 2 : 1) * C::KD + (C::NBS - 1) * bias_copies<BV>(); }
     // byte offset of bias (row, key .. key + 3) inside a slot
     __device__ static __forceinline__ int b_off(int row, int key) {
         const int byte = key * C::ES;
@@ -618,10 +624,21 @@ template <typename T, int D, int BIAS, bool WITH_V = true, bool WIDE = false> st
     // 64 it + lane of the slot (row c / BCPR, LDS chunk c % BCPR) holds chunk (c % BCPR) ^ bswz(row)
     // of the row.  Rows past M re-read row M - 1 (never stored) and chunks that start past N
     // re-read column 0 (masked).
-    __device__ __forceinline__ void issue_bias(int k) {
+    // kByDword: copy `it` fills rows 2 it and 2 it + 1 of the same layout, a lane one element of them.
+    template <int BV> __device__ __forceinline__ void issue_bias(int k) {
         if constexpr (C::ES != 0) {
             const unsigned dst = lds_bias + (k % C::NBS) * C::BSLOT;
             const uint64_t base = uniform_ptr(bp);
+            if constexpr (BV == kByDword) {
+#pragma unroll
+                for (int it = 0; it < 16; it++) {
+                    int m = mw + 2 * it + (lane >> 5), n = k * C::BK + ((lane & 31) ^ (4 * (it & 7)));
+                    m = m < M ? m : M - 1;
+                    n = n < N ? n : N - 1;
+                    lds_copy4(base, (unsigned)(((int64_t)m * sbm + n) * 4), dst + it * 256);
+                }
+                return;
+            }
 #pragma unroll
             for (int it = 0; it < C::BCH; it++) {
                 const int c = (it % C::BPB) * 64 + lane;
@@ -636,7 +653,7 @@ template <typename T, int D, int BIAS, bool WITH_V = true, bool WIDE = false> st
         }
     }
     // Points the running addresses at K/V step `k_kv` and bias slice `k_b` (the next ones a lean step issues).
-    __device__ __forceinline__ void run_start(int k_kv, int k_b) {
+    template <int BV> __device__ __forceinline__ void run_start(int k_kv, int k_b) {
         run_k = uniform_ptr(kp + (int64_t)k_kv * C::BK * sk);
         run_v = uniform_ptr(vp + (int64_t)k_kv * C::BK * sv);
         run_b = 0;
@@ -653,7 +670,7 @@ template <typename T, int D, int BIAS, bool WITH_V = true, bool WIDE = false> st
     }
     // issue_ahead for a step whose copies (K/V rows of step k + LA, keys of the bias slice of step k + NBS - 1) lie
     // wholly inside the tensors; run_start() was called for the first such step
-    template <bool BV> __device__ __forceinline__ void issue_ahead_lean(int k) {
+    template <int BV> __device__ __forceinline__ void issue_ahead_lean(int k) {
         const unsigned saved_m0 = lds_copy_begin();
         settle_ptrs(run_k, run_v, run_b);
         const unsigned k_dst = lds_kv + (unsigned)((k + C::LA) % C::NKV) * C::STEP_BYTES;
@@ -676,10 +693,20 @@ template <typename T, int D, int BIAS, bool WITH_V = true, bool WIDE = false> st
         }
         run_k += (uint64_t)(C::BK * 2) * (uint64_t)sk;
         run_v += (uint64_t)(C::BK * 2) * (uint64_t)sv;
-        if constexpr (BV && C::ES != 0) {
+        if constexpr (BV != kByElement && C::ES != 0) {
             const unsigned dst = lds_bias + (unsigned)((k + C::NBS - 1) % C::NBS) * C::BSLOT;
+            if constexpr (BV == kByDword) {
+                int lane_here = lane;  // (nothing of this is kept in registers across the loops)
+                asm volatile("" : "+v"(lane_here));
+                const int first = mw < M ? mw : M - 1, last = M - 1 - first;
 #pragma unroll
-            for (int it = 0; it < C::BCH; it++) {
+                for (int it = 0; it < 16; it++) {
+                    const int row = 2 * it + (lane_here >> 5);
+                    lds_copy4(run_b, (unsigned)(((row < last ? row : last) * (int)sbm + ((lane_here & 31) ^ (4 * (it & 7)))) * 4), dst + it * 256);
+                }
+            }
+#pragma unroll
+            for (int it = 0; it < (BV == kByDword ? 0 : C::BCH); it++) {
                 lds_copy16(run_b, lean_boff[it % C::BPB] + (unsigned)(it / C::BPB * 32 * C::ES), dst + it * 1024);
             }
             run_b += C::BK * C::ES;
@@ -696,30 +723,30 @@ template <typename T, int D, int BIAS, bool WITH_V = true, bool WIDE = false> st
     // Before the first step, in the order the steps assume: the first bias slices, then K/V of a
     // step followed by the bias slice issued in the same step.  BV: the bias slices come by copy.
     // k0: the first step of the stream (0 unless the keys are split between work-groups)
-    template <bool BV> __device__ __forceinline__ void prologue(int k0 = 0) {
+    template <int BV> __device__ __forceinline__ void prologue(int k0 = 0) {
         const unsigned saved_m0 = lds_copy_begin();
-        if constexpr (BV) {
+        if constexpr (BV != kByElement) {
 #pragma unroll
-            for (int i = 0; i < C::NBS - 1 - C::LA; i++) issue_bias(k0 + i);
+            for (int i = 0; i < C::NBS - 1 - C::LA; i++) issue_bias<BV>(k0 + i);
         }
 #pragma unroll
         for (int i = 0; i < C::LA; i++) {
             issue_kv(k0 + i);
-            if constexpr (BV) issue_bias(k0 + C::NBS - 1 - C::LA + i);
+            if constexpr (BV != kByElement) issue_bias<BV>(k0 + C::NBS - 1 - C::LA + i);
         }
         lds_copy_end(saved_m0);
     }
     // Top of step k: wait for its K/V rows (and with them its bias slice, issued earlier) and
     // publish them.  The slots that step k - 1 read are free from here on.
-    template <bool BV> __device__ __forceinline__ void begin_step(int k) {
+    template <int BV> __device__ __forceinline__ void begin_step(int k) {
         static_assert(BIAS == 0 || C::LA <= C::NBS - 1, "the bias slice of a step must be issued in time");
         constexpr bool EARLY = C::LA < C::NBS - 1;  // the bias slice of a step is issued before its K/V rows
-        constexpr int OPS = (WITH_V ? 2 : 1) * C::KD + (BV ? C::BCH : 0);  // copies per wave per step
+        constexpr int OPS = (WITH_V ? 2 : 1) * C::KD + bias_copies<BV>();  // copies per wave per step
         // K/V of this step were issued LA steps ago; the bias copies issued right after them and
         // the copies of the steps since may still be in flight
-        wait_vmcnt<(BV && EARLY ? C::BCH : 0) + OPS*(C::LA - 1)>();
+        wait_vmcnt<(EARLY ? bias_copies<BV>() : 0) + OPS*(C::LA - 1)>();
         lds_barrier();
-        if constexpr (C::ES != 0 && !BV) {
+        if constexpr (C::ES != 0 && BV == kByElement) {
             // unaligned bias rows or non-unit key stride: one element per lane, 16 rows per lane,
             // RB loads in flight together (clamped addresses instead of branches; what lies outside
             // the bias is masked where it is used)
@@ -760,10 +787,10 @@ template <typename T, int D, int BIAS, bool WITH_V = true, bool WIDE = false> st
     // left.  Issuing a copy holds the wave while the copies of the other waves drain through the
     // CU's 64 bytes/clock copy path, so the best place is right behind a batch of MFMAs, whose
     // execution then hides it; right after the barrier all waves would queue up at once.
-    template <bool BV> __device__ __forceinline__ void issue_ahead(int k) {
+    template <int BV> __device__ __forceinline__ void issue_ahead(int k) {
         const unsigned saved_m0 = lds_copy_begin();
         issue_kv(k + C::LA);
-        if constexpr (BV) issue_bias(k + C::NBS - 1);
+        if constexpr (BV != kByElement) issue_bias<BV>(k + C::NBS - 1);
         lds_copy_end(saved_m0);
     }
     // After the last step: nothing may land in LDS that is about to be reused.

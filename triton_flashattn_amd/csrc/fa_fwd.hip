@@ -71,6 +71,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
 
     constexpr bool ROWB = BIAS >= 6;     // the same bias for every query row, kept as an fp32 row in LDS
     constexpr bool BOOLROW = BIAS == 7;  // ... a bool mask: the row holds 0 or the mask term, in log2 units
+    constexpr bool BY_DWORD = BIAS == 4 && D <= 64;
 
     __shared__ __align__(1024) unsigned char smem[C::LOOP_BYTES + (ROWB ? kRowBiasKeys * 4 : 0)];
     const float* row_lds = reinterpret_cast<const float*>(smem + C::LOOP_BYTES);
@@ -118,7 +119,6 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
     typedef KeyStream<T, D, fwd_stream_kind(BIAS, D), true, true> KS;
     KS ks_;
     ks_.init(smem, kp, vp, bp, p.sk.s, p.sv.s, p.sbias.m, p.sbias.n, M, N, mw, wave, lane, chunks, p.d_v / 8);
-    const bool bias_copies = TB != 0 && p.bias_vec;
 
     // Q^T as B operand: column my_m, k = d
     // Without a bias, from head dim 96 on, through LDS with the first K/V rows (WaveRows; us: B=8 H=12 S=512 D=128 23.6 -> 22.4,
@@ -127,14 +127,15 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
     typedef WaveRows<T, D> WR;
     constexpr bool STAGED = BIAS == 0 && D >= 96;
     T8 qreg[C::KSTEPS];
-    if constexpr (!STAGED) {
+    auto load_q = [&]() {
 #pragma unroll
         for (int ks = 0; ks < C::KSTEPS; ks++) {
             i32x4 raw = {0, 0, 0, 0};
             if (my_m < M) raw = gld16(qp + (int64_t)my_m * p.sq.s + (D <= 128 ? chunks.wrap(2 * ks + g) : 2 * ks + g) * 8);
             qreg[ks] = as_vec<T8>(raw);
         }
-    }
+    };
+    if (!STAGED || M <= 32) load_q();
     auto split_q = [&]() {
         if (D <= 128 && p.d_qk < D) {
 #pragma unroll
@@ -184,7 +185,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
     // LEAN: the copies of the step need no clamps (KeyStream::issue_ahead_lean).
     auto kv_step = [&](int k, auto step_tag, auto bv_tag, auto lean_tag) {
         constexpr bool STEP_MASKED = decltype(step_tag)::value;
-        constexpr bool BV = decltype(bv_tag)::value;
+        constexpr int BV = decltype(bv_tag)::value;
         constexpr bool LEAN = decltype(lean_tag)::value;
         auto issue_ahead = [&]() {
             if constexpr (LEAN) ks_.template issue_ahead_lean<BV>(k);
@@ -507,16 +508,21 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
     if (!(qk_scale > 0.f) || !raw_ok) n_fast = 0;
 
     auto run = [&](auto bv_tag) {
-        constexpr bool BV = decltype(bv_tag)::value;
+        constexpr int BV = decltype(bv_tag)::value;
         if constexpr (STAGED) {
-            const unsigned q_tile = ks_.stage_addr();
-            const unsigned saved_m0 = lds_copy_begin();
-            WR::issue(qp, p.sq.s, mw, M, q_tile, lane, [&](int c) { return D <= 128 ? chunks.wrap(c) : c; });
-            lds_copy_end(saved_m0);
-            ks_.template prologue<BV>();
-            WR::template arrived<KS::template prologue_copies<BV>()>();
+            if (M > 32) {
+                const unsigned q_tile = ks_.stage_addr();
+                const unsigned saved_m0 = lds_copy_begin();
+                WR::issue(qp, p.sq.s, mw, M, q_tile, lane, [&](int c) { return D <= 128 ? chunks.wrap(c) : c; });
+                lds_copy_end(saved_m0);
+                ks_.template prologue<BV>();
+                WR::template arrived<KS::template prologue_copies<BV>()>();
 #pragma unroll
-            for (int ks = 0; ks < C::KSTEPS; ks++) qreg[ks] = SW::template row8_at<T8>(q_tile + rows_l, 0, ks);
+                for (int ks = 0; ks < C::KSTEPS; ks++) qreg[ks] = SW::template row8_at<T8>(q_tile + rows_l, 0, ks);
+            } else {  // (a token or a few: 32 copies of the same rows cost a decode step at B=8 H=16 N=4097 1 %)
+                wait_vmcnt<0>();
+                ks_.template prologue<BV>();
+            }
             split_q();
         } else {
             stage_row();
@@ -531,10 +537,10 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
             if constexpr (TB == 0) split_q();  // (while the first copies are on their way)
         }
         // the leading fast steps whose copies stay inside the tensors issue them without clamps
-        const int n_lean = (BV || TB == 0) ? ks_.lean_steps(n_fast) : 0;
+        const int n_lean = (BV != kByElement || TB == 0) ? ks_.lean_steps(n_fast) : 0;
         int k = 0;
         if (n_lean > 0) {
-            ks_.run_start(C::LA, C::NBS - 1);
+            ks_.template run_start<BV>(C::LA, C::NBS - 1);
 #pragma unroll 1
             for (; k < n_lean; k++) kv_step(k, std::false_type{}, bv_tag, std::true_type{});
         }
@@ -543,8 +549,18 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
 #pragma unroll 1
         for (; k < n_steps; k++) kv_step(k, std::true_type{}, bv_tag, std::false_type{});
     };
-    if (bias_copies) run(std::true_type{});
-    else run(std::false_type{});
+    if constexpr (TB == 0) {
+        run(RowsTag<kByElement>{});
+    } else {
+        if constexpr (BY_DWORD) {
+            if (p.bias_vec == kByChunk) run(RowsTag<kByChunk>{});
+            else if (p.bias_vec == kByDword) run(RowsTag<kByDword>{});
+            else run(RowsTag<kByElement>{});
+        } else {
+            if (p.bias_vec == kByChunk) run(RowsTag<kByChunk>{});
+            else run(RowsTag<kByElement>{});
+        }
+    }
 
     // ---- epilogue (flash_attention.py:188-194) ----
     const float l_tot = pair_sum(l_i);

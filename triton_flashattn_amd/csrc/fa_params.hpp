@@ -30,7 +30,7 @@ struct FwdParams {
     Strides4 sbias;
     int B, H, M, N;
     float sm_scale;
-    int bias_vec;  // bias rows may be read with aligned 16-byte loads
+    int bias_vec;  // how bias rows may be read: 0 by element, 1 in aligned 16-byte chunks, 2 (fp32) by dword (BiasRows)
     int n_mtiles;
     // Keys split between n_splits work-groups per query tile (1 = no split): split s takes
     // keys_per_split keys (a multiple of the kernel's step) and writes its output, in fp32,
@@ -67,7 +67,7 @@ struct BwdParams {
     int n_ntiles;   // key tiles of the dK/dV kernel
     int waves_per_role;  // 32-key blocks per key tile of the dK/dV kernel
     int n_mtiles;   // query tiles of the dQ kernel
-    int bias_vec;   // bias rows may be read with aligned 16-byte loads
+    int bias_vec;   // how bias rows may be read: 0 by element, 1 in aligned 16-byte chunks, 2 (fp32) by dword (BiasRows)
     int dbias_vec;  // dbias rows may be written with aligned 16-byte stores
     // dQ kernel: keys split between dq_splits work-groups per query tile (1 = no split), each over
     // dq_keys_per_split keys, their shares of dq in fp32 in part_dq (dq_splits, B*H, M, D);

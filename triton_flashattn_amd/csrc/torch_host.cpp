@@ -68,6 +68,12 @@ bool bias_rows_ok(const Tensor& b) {
     return last * es + padded <= (int64_t)b.storage().nbytes();
 }
 
+// ... or 4 bytes at a time (_bias_dwords_ok), which pays where every (batch, head) pair has its own (_bias_kernel_layout)
+bool bias_dwords_ok(const Tensor& b, int D) {
+    return b.scalar_type() == at::kFloat && D <= 64 && (b.size(3) == 1 || b.stride(3) == 1) && b.stride(2) >= 0 &&
+           ((b.size(2) - 1) * b.stride(2) + b.size(3)) * 4 < (int64_t)1 << 31;
+}
+
 // rows that start at multiples of 16 bytes, from 512 bytes on at whole cache lines (_empty_padded_rows in flash_attention.py)
 Tensor empty_padded_rows(at::IntArrayRef shape, const at::TensorOptions& opt) {
     const int64_t es = (int64_t)opt.dtype().itemsize(), n = shape[3];
@@ -387,7 +393,7 @@ py::object attention(py::handle q_, py::handle k_, py::handle v_, py::handle bia
                 for (int i = 0; i < bias.dim(); i++) shape[4 - bias.dim() + i] = bias.size(i);
                 bias4 = bias.reshape(at::IntArrayRef(shape, 4));
             }
-            if (!bias_rows_ok(bias4)) {
+            if (!bias_rows_ok(bias4) && !(bias4.size(0) * bias4.size(1) == B * H && bias_dwords_ok(bias4, D))) {
                 Tensor padded = empty_padded_rows(bias4.sizes(), bias4.options());
                 padded.copy_(bias4);
                 bias4 = padded;

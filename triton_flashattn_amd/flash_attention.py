@@ -326,11 +326,21 @@ def _empty_padded_rows(shape, dtype, device):
     return torch.empty(tuple(shape[:-1]) + (n_pad,), dtype=dtype, device=device)[..., :shape[-1]]
 
 
-def _bias_kernel_layout(b):
-    """b, or a copy with padded rows when the kernels would have to read b element by element (an odd
+def _bias_dwords_ok(b, D):
+    """Whether the kernels of head dim D can fetch the rows of a 4-D bias 4 bytes at a time (the rule of the C ABI):
+    fp32 with unit key stride, head dims up to 64, (batch, head) slices below 2 GiB."""
+    return (b.dtype == torch.float32 and D <= 64 and (b.shape[3] == 1 or b.stride(3) == 1) and b.stride(2) >= 0
+            and ((b.shape[2] - 1) * b.stride(2) + b.shape[3]) * 4 < 1 << 31)
+
+
+def _bias_kernel_layout(b, D=_HEAD_DIMS[-1], pairs=0):
+    """b, or a copy with padded rows when the kernels of head dim D would have to read b element by element (an odd
     number of keys, a misaligned view): one pass over the bias instead of a several times slower
-    forward and backward."""
-    if _bias_rows_ok(b):
+    forward and backward.  An fp32 bias of its own for each of the `pairs` (batch, head) pairs is fetched 4 bytes at a time
+    instead: the kernels lose less by that than the copy takes (training step, kernels, us, copy / in place: B=2 H=12
+    D=64 M=N=1001 139 / 107, 3001 1239 / 912, B=4 H=8 M=400 N=401 62 / 56), but not where many pairs read one table (32 batches,
+    12 heads, M=N=197 103 / 114)."""
+    if _bias_rows_ok(b) or (b.shape[0] * b.shape[1] == pairs and _bias_dwords_ok(b, D)):
         return b
     out = _empty_padded_rows(b.shape, b.dtype, b.device)
     out.copy_(b)
@@ -440,7 +450,7 @@ class FlashAttentionFn(torch.autograd.Function):
             bias = AlibiBias(alibi_slopes)
         bias = _check_bias(bias, q, k)
         if isinstance(bias, torch.Tensor):
-            bias = _bias_kernel_layout(bias)
+            bias = _bias_kernel_layout(bias, max(q.shape[-1], v.shape[-1]), q.shape[0] * q.shape[2])
         _check_causal(causal, q.shape[1], k.shape[1])
         sm_scale = (q.shape[-1] ** -0.5) if sm_scale is None else sm_scale
         is_bias = bias is not None
@@ -516,7 +526,7 @@ class FlashAttentionQKVPackedFn(torch.autograd.Function):
             bias = AlibiBias(alibi_slopes)
         bias = _check_bias(bias, q, k)
         if isinstance(bias, torch.Tensor):
-            bias = _bias_kernel_layout(bias)
+            bias = _bias_kernel_layout(bias, qkv.shape[-1], q.shape[0] * q.shape[2])
         sm_scale = (qkv.shape[-1] ** -0.5) if sm_scale is None else sm_scale
         is_bias = bias is not None
         alibi = isinstance(bias, AlibiBias)
@@ -617,7 +627,7 @@ def _op_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, bias: Optional[to
         raise ValueError("flash_attention_op needs v with the head dim of q")
     bias = _check_bias(bias, q, k)
     if bias is not None:
-        bias = _bias_kernel_layout(bias)
+        bias = _bias_kernel_layout(bias, q.shape[-1], q.shape[0] * q.shape[2])
     _check_causal(causal, q.shape[1], k.shape[1])
     return _flash_attn_fwd(q, k, v, bias, causal, sm_scale)
 
@@ -636,7 +646,7 @@ def _op_bwd(do: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     b4 = _check_bias(bias, q, k)
     if b4 is not None:
-        b4 = _bias_kernel_layout(b4)
+        b4 = _bias_kernel_layout(b4, q.shape[-1], B * H)
     dbias = _bias_grad_like(b4, B, H, M, k.shape[1]) if bias_grad else None
     _flash_attn_bwd(do, q, k, v, o, b4, causal, sm_scale, lse, dq, dk, dv, dbias)
     # an operator cannot return None: no bias gradient is an empty tensor
