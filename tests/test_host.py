@@ -346,6 +346,27 @@ def test_padded_bias_rows_must_end_inside_the_storage():
     assert fa_mod._bias_rows_ok(exact[:, :, ::2, :])
 
 
+@pytest.mark.parametrize("rows,cols,keep", [(7, 50, 50), (7, 51, 50), (5, 30, 30), (4, 62, 61), (3, 8, 5)])
+def test_fp32_rows_that_end_behind_the_storage_are_copied(rows, cols, keep):
+    """The C ABI sees pointer and strides, not the storage: an fp32 view that it would fetch in 16-byte chunks, the last of
+    them behind the storage, is copied also where fp32 rows are otherwise read in place, 4 bytes at a time.  What stays in place
+    is fetched in chunks inside the storage or not in chunks at all."""
+    for lead in range(4):
+        for step in (1, 2, 3, 4):
+            b = torch.zeros(1, 1, rows, cols + lead)[:, :, ::step, lead:lead + keep]
+            out = fa_mod._bias_kernel_layout(b, 64, 1)
+            es, padded = 4, -(-keep * 4 // 16) * 16
+            by_chunks = b.data_ptr() % 16 == 0 and (b.shape[2] == 1 or b.stride(2) * es % 16 == 0) and (
+                keep * es == padded or b.stride(2) * es >= padded)
+            end = (b.storage_offset() + (b.shape[2] - 1) * b.stride(2)) * es + padded
+            if b.shape[2] > 1 and by_chunks and end > b.untyped_storage().nbytes():
+                assert out is not b and torch.equal(out, b) and fa_mod._bias_rows_ok(out), (lead, step)
+            else:
+                assert out is b, (lead, step)
+    view = torch.zeros(1, 1, 7, 50)[:, :, ::2]   # 400 bytes between rows of 200; the last row ends the storage
+    assert not fa_mod._bias_rows_ok(view) and fa_mod._bias_kernel_layout(view, 64, 1) is not view
+
+
 def test_hip_backend_checks_shapes_before_launching():
     """The launchers may be called directly (as in the reference): tensors that disagree with the extents
     taken from q and k are refused, not read out of bounds."""

@@ -52,26 +52,33 @@ int bias_kind(const Tensor& b) {
     }
 }
 
-// whether the kernels can fetch the rows of a 4-D bias in aligned 16-byte chunks (_bias_rows_ok in flash_attention.py)
-bool bias_rows_ok(const Tensor& b) {
+int64_t padded_row(const Tensor& b) { return (b.size(3) * b.element_size() + 15) / 16 * 16; }  // bytes
+
+// whether the C ABI, going by pointer and strides, fetches the rows of a 4-D bias in aligned 16-byte chunks
+// (_bias_chunks_chosen in flash_attention.py)
+bool bias_chunks_chosen(const Tensor& b) {
     const int64_t es = b.element_size(), n = b.size(3);
-    if (b.size(2) == 1 || b.stride(2) == 0) return true;
     if ((n > 1 && b.stride(3) != 1) || reinterpret_cast<uintptr_t>(b.data_ptr()) % 16 != 0) return false;
-    int64_t last = b.storage_offset();
-    for (int i = 0; i < 3; i++) {
+    for (int i = 0; i < 3; i++)
         if (b.size(i) > 1 && (b.stride(i) * es) % 16 != 0) return false;
-        last += (b.size(i) - 1) * b.stride(i);
-    }
-    const int64_t padded = (n * es + 15) / 16 * 16;
-    if (n * es == padded) return true;
-    if (b.stride(2) * es < padded) return false;
-    return last * es + padded <= (int64_t)b.storage().nbytes();
+    return n * es == padded_row(b) || b.stride(2) * es >= padded_row(b);
+}
+
+// ... and may: no chunk ends behind the storage (_bias_rows_ok)
+bool bias_rows_ok(const Tensor& b) {
+    if (b.size(2) == 1 || b.stride(2) == 0) return true;
+    if (!bias_chunks_chosen(b)) return false;
+    const int64_t es = b.element_size();
+    if (b.size(3) * es == padded_row(b)) return true;
+    int64_t last = b.storage_offset();
+    for (int i = 0; i < 3; i++) last += (b.size(i) - 1) * b.stride(i);
+    return last * es + padded_row(b) <= (int64_t)b.storage().nbytes();
 }
 
 // ... or 4 bytes at a time (_bias_dwords_ok), which pays where every (batch, head) pair has its own (_bias_kernel_layout)
 bool bias_dwords_ok(const Tensor& b, int D) {
     return b.scalar_type() == at::kFloat && D <= 64 && (b.size(3) == 1 || b.stride(3) == 1) && b.stride(2) >= 0 &&
-           ((b.size(2) - 1) * b.stride(2) + b.size(3)) * 4 < (int64_t)1 << 31;
+           ((b.size(2) - 1) * b.stride(2) + b.size(3)) * 4 < (int64_t)1 << 31 && !bias_chunks_chosen(b);
 }
 
 // rows that start at multiples of 16 bytes, from 512 bytes on at whole cache lines (_empty_padded_rows in flash_attention.py)

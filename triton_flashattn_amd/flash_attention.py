@@ -289,22 +289,30 @@ def _check_bias(bias, q, k):
     return b4
 
 
-def _bias_rows_ok(b):
-    """Whether the kernels can fetch the rows of a 4-D bias in aligned 16-byte chunks (the rule of the
-    C ABI): unit key stride, aligned base and strides, and rows that are whole chunks or whose stride
-    covers their last chunk.  A bias without a row dimension is read once per work-group, any layout."""
+def _bias_chunks_chosen(b):
+    """Whether the C ABI fetches the rows of a 4-D bias in aligned 16-byte chunks, going by pointer and strides, which is all
+    it sees: unit key stride, aligned base and strides, and rows that are whole chunks or whose stride covers their last
+    chunk."""
     es, N = b.element_size(), b.shape[3]
-    if b.shape[2] == 1 or b.stride(2) == 0:
-        return True
     if (N > 1 and b.stride(3) != 1) or b.data_ptr() % 16 != 0:
         return False
     if any(b.shape[i] > 1 and (b.stride(i) * es) % 16 != 0 for i in range(3)):
         return False
     padded = -(-N * es // 16) * 16
+    return N * es == padded or b.stride(2) * es >= padded
+
+
+def _bias_rows_ok(b):
+    """Whether the kernels can fetch the rows of a 4-D bias in aligned 16-byte chunks: the C ABI chooses that, and every
+    chunk lies inside the storage.  A bias without a row dimension is read once per work-group, any layout."""
+    es, N = b.element_size(), b.shape[3]
+    if b.shape[2] == 1 or b.stride(2) == 0:
+        return True
+    if not _bias_chunks_chosen(b):
+        return False
+    padded = -(-N * es // 16) * 16
     if N * es == padded:
         return True
-    if b.stride(2) * es < padded:
-        return False
     # rows that end inside a 16-byte chunk are fetched to the end of that chunk: the chunk of the very
     # last row must still lie inside the tensor's storage (true for a column slice of a wider tensor,
     # not for a view whose last row ends the allocation)
@@ -327,10 +335,11 @@ def _empty_padded_rows(shape, dtype, device):
 
 
 def _bias_dwords_ok(b, D):
-    """Whether the kernels of head dim D can fetch the rows of a 4-D bias 4 bytes at a time (the rule of the C ABI):
-    fp32 with unit key stride, head dims up to 64, (batch, head) slices below 2 GiB."""
+    """Whether the kernels of head dim D fetch the rows of a 4-D bias 4 bytes at a time (the rule of the C ABI): fp32 with
+    unit key stride, head dims up to 64, (batch, head) slices below 2 GiB, and rows that they would not fetch in 16-byte
+    chunks (which may reach past the storage: _bias_rows_ok)."""
     return (b.dtype == torch.float32 and D <= 64 and (b.shape[3] == 1 or b.stride(3) == 1) and b.stride(2) >= 0
-            and ((b.shape[2] - 1) * b.stride(2) + b.shape[3]) * 4 < 1 << 31)
+            and ((b.shape[2] - 1) * b.stride(2) + b.shape[3]) * 4 < 1 << 31 and not _bias_chunks_chosen(b))
 
 
 def _bias_kernel_layout(b, D=_HEAD_DIMS[-1], pairs=0):
