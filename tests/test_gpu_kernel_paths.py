@@ -348,6 +348,25 @@ def test_host_path_with_hooks_views_and_transforms(gpu_device):
         torch.func.vmap(lambda x: call(*one) * x)(rnd(3, 1))
 
 
+def test_ragged_fp32_bias_written_to_before_the_backward(gpu_device):
+    """A bias whose rows the kernels do not fetch in 16-byte chunks is copied where a backward may follow: the gradients are
+    those of the bias that the forward saw, also of a tensor that autograd would not save."""
+    g = torch.Generator().manual_seed(3)
+    q, k, v, do = (torch.randn(2, 75, 2, 64, generator=g).bfloat16().to(gpu_device) for _ in range(4))
+    bias = torch.randn(2, 2, 75, 75, generator=g).to(gpu_device)
+    with torch.inference_mode():
+        inference = bias.clone()
+    ins = [t.requires_grad_(True) for t in (q, k, v)]
+    want = torch.autograd.grad(flash_attention_fn(*ins, bias), ins, do)
+    for b in (inference, bias):
+        out = flash_attention_fn(*ins, b)
+        assert "AttentionNode" in out.grad_fn.name()
+        if b is bias:
+            bias.zero_()
+        for x, y in zip(torch.autograd.grad(out, ins, do), want):
+            assert torch.equal(x, y)
+
+
 def test_host_path_raises_what_the_launchers_raise(gpu_device):
     """A problem that the library refuses (2^28 keys, as views of one: nothing is allocated or launched) is a
     NativeLibraryError, in the forward and in the backward, which meets it through a hook; no memory is an OutOfMemoryError."""

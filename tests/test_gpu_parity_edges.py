@@ -309,19 +309,25 @@ def test_bias_rows_that_are_not_whole_chunks(gpu_device, D, kind):
 def test_fp32_bias_rows_at_any_multiple_of_four_bytes(gpu_device, D, causal):
     """fp32 rows that start anywhere are copied 4 bytes to a lane into the layout that 16-byte copies give: the results of
     every kernel (read only and dense gradient; one wave and, from 512 rows on at D = 64, a pair) are those of the same bias
-    in aligned rows, bit for bit.  With head 0 for all (a stride of 0) straight to the kernels."""
+    in aligned rows, bit for bit.  Straight to the kernels, also with head 0 for all (a stride of 0), and through the public
+    function without gradients, which reads such rows in place."""
     for i, (B, H, M, N) in enumerate([(2, 2, 70, 197), (1, 3, 131, 131), (2, 1, 1, 33), (1, 2, 257, 67), (1, 2, 577, 577), (3, 2, 33, 31)]):
         if causal and M != N:
             continue
         q, k, v, do, bias = make_inputs(gpu_device, B, M, N, H, D, torch.bfloat16, "f32", seed=5 * D + i, trainable=False)
-        aligned = torch.zeros(bias.shape[:3] + (-(-N // 4) * 4,), device=gpu_device)[..., :N]
+        padded = lambda: torch.zeros(bias.shape[:3] + (-(-N // 4) * 4,), device=gpu_device)[..., :N]
+        aligned = padded()
         aligned.copy_(bias)
         odd = torch.zeros(bias.numel() + 1, device=gpu_device)[1:].view(bias.shape)  # dense rows behind a misaligned start
         odd.copy_(bias)
         assert fa_mod._bias_dwords_ok(odd, D) and (M == 1 or not fa_mod._bias_rows_ok(odd))
         assert fa_mod._bias_kernel_layout(odd, D, B * H) is odd
+        with torch.no_grad():
+            outs = [flash_attention_fn(q, k, v, t, causal) for t in (aligned, odd)]
+        assert torch.equal(*outs), ("public", B, H, M, N)
         for trainable in (False, True):
-            res = [run_ours(q, k, v, do, t.detach().requires_grad_(trainable), causal) for t in (aligned, odd)]
+            res = [_launch_directly(q, k, v, do, t, padded() if trainable else None, causal) for t in (aligned, odd)]
+            assert torch.equal(res[0]["out"], outs[0])
             for name in ("out", "dq", "dk", "dv") + (("dbias",) if trainable else ()):
                 assert torch.equal(res[0][name], res[1][name]), (name, B, H, M, N, trainable)
         res = [_launch_directly(q, k, v, do, t[:, :1].expand(B, H, M, N), None, causal) for t in (aligned, odd)]

@@ -367,6 +367,39 @@ def test_fp32_rows_that_end_behind_the_storage_are_copied(rows, cols, keep):
     assert not fa_mod._bias_rows_ok(view) and fa_mod._bias_kernel_layout(view, 64, 1) is not view
 
 
+@pytest.mark.parametrize("bias_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("packed", [False, True])
+def test_ragged_bias_written_to_between_forward_and_backward(oracle_backend, bias_dtype, packed):
+    """Rows that no kernel could fetch in 16-byte chunks are copied in a forward with gradients: the backward works on that
+    copy, whatever has become of the caller's tensor (a buffer that is filled again, an inference tensor).  Without
+    gradients fp32 rows are read where they are."""
+    q, k, v = _qkv(M=6, N=6)
+    do = torch.randn_like(q)
+    make = lambda: torch.arange(2 * 2 * 6 * 6).view(2, 2, 6, 6).sin().to(bias_dtype)
+    with torch.inference_mode():
+        inference = make()
+    def call(bias, leaves):
+        return flash_attention_qkvpacked_fn(leaves[0], bias) if packed else flash_attention_fn(*leaves, bias)
+    def leaves():
+        src = [torch.stack((q, k, v), 2)] if packed else [q, k, v]
+        return [t.clone().requires_grad_(True) for t in src]
+    x = leaves()
+    want = torch.autograd.grad(call(make(), x), x, do)
+    for bias in (make(), inference):
+        x = leaves()
+        out = call(bias, x)
+        if bias is not inference:
+            bias.zero_()
+        for a, b in zip(torch.autograd.grad(out, x, do), want):
+            assert torch.equal(a, b)
+    if bias_dtype is torch.float32:
+        bias = make()
+        oracle_backend.calls.clear()
+        with torch.no_grad():
+            call(bias, [t.detach() for t in leaves()])
+        assert oracle_backend.calls[-1][2] == bias.stride()
+
+
 def test_hip_backend_checks_shapes_before_launching():
     """The launchers may be called directly (as in the reference): tensors that disagree with the extents
     taken from q and k are refused, not read out of bounds."""

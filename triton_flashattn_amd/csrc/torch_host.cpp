@@ -75,7 +75,8 @@ bool bias_rows_ok(const Tensor& b) {
     return last * es + padded_row(b) <= (int64_t)b.storage().nbytes();
 }
 
-// ... or 4 bytes at a time (_bias_dwords_ok), which pays where every (batch, head) pair has its own (_bias_kernel_layout)
+// ... or 4 bytes at a time (_bias_dwords_ok), which pays where every (batch, head) pair has its own and no backward may follow
+// (_bias_kernel_layout)
 bool bias_dwords_ok(const Tensor& b, int D) {
     return b.scalar_type() == at::kFloat && D <= 64 && (b.size(3) == 1 || b.stride(3) == 1) && b.stride(2) >= 0 &&
            ((b.size(2) - 1) * b.stride(2) + b.size(3)) * 4 < (int64_t)1 << 31 && !bias_chunks_chosen(b);
@@ -387,6 +388,10 @@ py::object attention(py::handle q_, py::handle k_, py::handle v_, py::handle bia
     if (slopes.defined() && (slopes.dim() != 1 || slopes.size(0) != H || slopes.scalar_type() != at::kFloat)) return py::none();
     const double sm_scale = scale_.is_none() ? std::pow((double)d_qk, -0.5) : PyFloat_AsDouble(scale_.ptr());
 
+    const bool grad = at::GradMode::is_enabled() &&
+                      (q.requires_grad() || (k.defined() && (k.requires_grad() || v.requires_grad())) ||
+                       (bias.defined() && bias.requires_grad()) || (slopes.defined() && slopes.requires_grad()));
+
     py::gil_scoped_release no_gil;
     Tensor out;
     {
@@ -400,16 +405,13 @@ py::object attention(py::handle q_, py::handle k_, py::handle v_, py::handle bia
                 for (int i = 0; i < bias.dim(); i++) shape[4 - bias.dim() + i] = bias.size(i);
                 bias4 = bias.reshape(at::IntArrayRef(shape, 4));
             }
-            if (!bias_rows_ok(bias4) && !(bias4.size(0) * bias4.size(1) == B * H && bias_dwords_ok(bias4, D))) {
+            if (!bias_rows_ok(bias4) && (grad || bias4.size(0) * bias4.size(1) != B * H || !bias_dwords_ok(bias4, D))) {
                 Tensor padded = empty_padded_rows(bias4.sizes(), bias4.options());
                 padded.copy_(bias4);
                 bias4 = padded;
             }
         }
     }
-    const bool grad = at::GradMode::is_enabled() &&
-                      (q.requires_grad() || (k.defined() && (k.requires_grad() || v.requires_grad())) ||
-                       (bias.defined() && bias.requires_grad()) || (slopes.defined() && slopes.requires_grad()));
     if (grad) {
         out = AttentionNode::apply(q, maybe(k), maybe(v), maybe(bias), maybe(slopes), KernelBias{bias4}, causal, sm_scale);
     } else {

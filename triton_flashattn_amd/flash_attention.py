@@ -346,9 +346,11 @@ def _bias_kernel_layout(b, D=_HEAD_DIMS[-1], pairs=0):
     """b, or a copy with padded rows when the kernels of head dim D would have to read b element by element (an odd
     number of keys, a misaligned view): one pass over the bias instead of a several times slower
     forward and backward.  An fp32 bias of its own for each of the `pairs` (batch, head) pairs is fetched 4 bytes at a time
-    instead: the kernels lose less by that than the copy takes (training step, kernels, us, copy / in place: B=2 H=12
-    D=64 M=N=1001 139 / 107, 3001 1239 / 912, B=4 H=8 M=400 N=401 62 / 56), but not where many pairs read one table (32 batches,
-    12 heads, M=N=197 103 / 114)."""
+    instead: the kernels lose less by that than the copy takes (forward, kernels, us, copy / in place: B=2 H=12 D=64 M=N=1001
+    60 / 33, 3001 559 / 250, B=4 H=8 M=400 N=401 26 / 18, B=4 H=4 M=N=129 12.0 / 9.7; D=32, 1001 59 / 29), but not where many
+    pairs read one table (a training step, 32 batches, 12 heads, M=N=197 103 / 114).  The autograd functions give pairs = 0
+    where a backward may follow: it works on the bias of its forward, whatever the caller has written to it since, and on one
+    that autograd would not save (an inference tensor), which takes the copy."""
     if _bias_rows_ok(b) or (b.shape[0] * b.shape[1] == pairs and _bias_dwords_ok(b, D)):
         return b
     out = _empty_padded_rows(b.shape, b.dtype, b.device)
@@ -459,7 +461,8 @@ class FlashAttentionFn(torch.autograd.Function):
             bias = AlibiBias(alibi_slopes)
         bias = _check_bias(bias, q, k)
         if isinstance(bias, torch.Tensor):
-            bias = _bias_kernel_layout(bias, max(q.shape[-1], v.shape[-1]), q.shape[0] * q.shape[2])
+            pairs = 0 if any(ctx.needs_input_grad) else q.shape[0] * q.shape[2]
+            bias = _bias_kernel_layout(bias, max(q.shape[-1], v.shape[-1]), pairs)
         _check_causal(causal, q.shape[1], k.shape[1])
         sm_scale = (q.shape[-1] ** -0.5) if sm_scale is None else sm_scale
         is_bias = bias is not None
@@ -535,7 +538,7 @@ class FlashAttentionQKVPackedFn(torch.autograd.Function):
             bias = AlibiBias(alibi_slopes)
         bias = _check_bias(bias, q, k)
         if isinstance(bias, torch.Tensor):
-            bias = _bias_kernel_layout(bias, qkv.shape[-1], q.shape[0] * q.shape[2])
+            bias = _bias_kernel_layout(bias, qkv.shape[-1], 0 if any(ctx.needs_input_grad) else q.shape[0] * q.shape[2])
         sm_scale = (qkv.shape[-1] ** -0.5) if sm_scale is None else sm_scale
         is_bias = bias is not None
         alibi = isinstance(bias, AlibiBias)
