@@ -603,7 +603,8 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
         }
     }
     T* op = reinterpret_cast<T*>(p.dq) + (int64_t)b * p.sdq.b + (int64_t)h * p.sdq.h;
-    i32x4 out[WR::COPIES];  // (a wave's own rows: no barrier; all reads in flight together)
+    lds_wave_order();  // (a wave's own rows: no barrier)
+    i32x4 out[WR::COPIES];  // (all reads in flight together)
 #pragma unroll
     for (int it = 0; it < WR::COPIES; it++) out[it] = lds_read16(o_lds + (it * 64 + lane) / CPR * OS + (it * 64 + lane) % CPR * 8);
 #pragma unroll

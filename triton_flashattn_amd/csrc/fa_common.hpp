@@ -83,6 +83,14 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// What the lanes of a wave wrote to LDS before is there for all of its lanes behind.  (The hardware executes the LDS accesses of
+// a wave in order; this tells the compiler, and costs no instruction.)
+__device__ __forceinline__ void lds_wave_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // ---- LDS access ---------------------------------------------------------------------------
 __device__ __forceinline__ i32x4 lds_read16(const void* p) { return *reinterpret_cast<const i32x4*>(p); }
 
@@ -383,7 +391,8 @@ template <typename T, int D> struct WaveRows {
                 for (int e = 0; e < 4; e++) x[e] = (T)(acc[db][q4 * 4 + e] * scale);
                 *(lds_ptr)(uintptr_t)(at + 16u * (unsigned)((db * 4 + q4) ^ Swz<D>::f(r))) = x;
             }
-        i32x4 out[COPIES];  // (the wave's own rows: no barrier)
+        lds_wave_order();  // (the wave's own rows: no barrier)
+        i32x4 out[COPIES];
 #pragma unroll
         for (int i = 0; i < COPIES; i++) out[i] = lds_read16_at(lds + 1024u * i + 16u * (unsigned)lane);
 #pragma unroll

@@ -611,7 +611,8 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
     T* op = reinterpret_cast<T*>(p.o) + (int64_t)b * p.so.b + (int64_t)h * p.so.h;
     int lane_late = lane;  // (as above)
     asm volatile("" : "+v"(lane_late));
-    i32x4 out[WR::COPIES];  // (a wave's own rows: no barrier; all reads in flight together)
+    lds_wave_order();  // (a wave's own rows: no barrier)
+    i32x4 out[WR::COPIES];  // (all reads in flight together)
 #pragma unroll
     for (int it = 0; it < WR::COPIES; it++) out[it] = lds_read16(o_lds + (it * 64 + lane_late) / CPR * OS + (it * 64 + lane_late) % CPR * 8);
 #pragma unroll
