@@ -603,13 +603,20 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
         }
     }
     T* op = reinterpret_cast<T*>(p.dq) + (int64_t)b * p.sdq.b + (int64_t)h * p.sdq.h;
+    // Nothing formed of the lane here is kept in registers through the loops.  (It was, up to 60 of them, some of those that the
+    // loops need: D=256 from dS B=2 H=4 S=1024 22.5 -> 20.8 us, B=2 H=16 S=2048 108 -> 102, no bias B=4 H=4 S=512 32.4 -> 31, from
+    // fp32 dS D=32 B=2 H=8 S=1024 17.1 -> 16.3, causal row mask D=64 there 25.3 -> 22.8.  The kernels of a row up to D=32 had them
+    // to spare, and there the loop of causal ones lost its order with them: 18 -> 21.)
+    int lane_late = lane;
+    if constexpr (!(ROWB && D <= 32)) asm volatile("" : "+v"(lane_late));
     lds_wave_order();  // (a wave's own rows: no barrier)
     i32x4 out[WR::COPIES];  // (all reads in flight together)
 #pragma unroll
-    for (int it = 0; it < WR::COPIES; it++) out[it] = lds_read16(o_lds + (it * 64 + lane) / CPR * OS + (it * 64 + lane) % CPR * 8);
+    for (int it = 0; it < WR::COPIES; it++)
+        out[it] = lds_read16(o_lds + (it * 64 + lane_late) / CPR * OS + (it * 64 + lane_late) % CPR * 8);
 #pragma unroll
     for (int it = 0; it < WR::COPIES; it++) {
-        const int row = (it * 64 + lane) / CPR, ch = (it * 64 + lane) % CPR;
+        const int row = (it * 64 + lane_late) / CPR, ch = (it * 64 + lane_late) % CPR;
         if (mw + row < M && ch * 8 < p.d_qk) gst16(op + (int64_t)(mw + row) * p.sdq.s + ch * 8, out[it]);
     }
 }
