@@ -77,7 +77,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
     // after the other.
     typedef WaveRows<T, D> WR;
     constexpr bool STAGED = C::STAGE != C::kNowhere && !FROM_DS;
-    constexpr bool BESIDE = STAGED && !ROWB && (C::LDS_BYTES + 4 * WR::BYTES) * C::MIN_BLOCKS <= 163840;
+    constexpr bool BESIDE = STAGED && !ROWB && (C::LDS_BYTES + 4 * WR::BYTES) * C::ROOM <= 163840;
     __shared__ __align__(1024) unsigned char smem[C::LDS_BYTES + (ROWB ? kRowBiasKeys * 4 : 0) + (BESIDE ? 4 * WR::BYTES : 0)];
     const float* row_lds = reinterpret_cast<const float*>(smem + C::LDS_BYTES);
 

@@ -482,6 +482,10 @@ template <int D, int BIAS, bool WIDE = false> struct StreamCfg {
                                    : ES == 0                        ? kBehind
                                    : NBS * BSLOT >= 64 * D          ? kOwnRing
                                                                     : kSlotsAndBehind;
+    // Work-groups on a CU that such a place must leave room for: three up to head dim 64 where the loops do, which the registers
+    // of most of those kernels allow (dQ, us, D=64 ALiBi, two / three: H=96 S=1024 54 / 51, causal 41 / 36; D=16 with an fp32 tile
+    // B=8 H=12 S=1024 108 / 95).
+    static constexpr int ROOM = D <= 64 && 3 * LOOP_BYTES <= 163840 ? 3 : D <= 128 && LOOP_BYTES <= 81920 ? 2 : 1;
     static constexpr int LDS_BYTES = LOOP_BYTES + (STAGE == kBehind ? 256 * D : STAGE == kSlotsAndBehind ? 128 * D : 0);
     // 16-byte chunk c of bias row `row` is stored at chunk c ^ bswz(row): rows that share LDS banks
     // get different chunk orders
@@ -495,7 +499,7 @@ template <int D, int BIAS, bool WIDE = false> struct StreamCfg {
     // -> three: forward B=8 H=12 S=1024 51.7 -> 47.6, B=16 H=8 S=2048 250 -> 238; forward and backward, causal, B=8 H=12
     // S=1024 144.7 -> 140.4.  (Head dims up to 32 stayed below 168 registers on their own: no change.)
     static constexpr int MIN_BLOCKS = D <= 64 && BIAS <= 1 ? 3 : (D <= 128 && LOOP_BYTES <= 81920) ? 2 : 1;
-    static_assert(LDS_BYTES * MIN_BLOCKS <= 163840, "LDS of a CU");
+    static_assert(MIN_BLOCKS <= ROOM && LDS_BYTES * ROOM <= 163840, "LDS of a CU");
 };
 
 // The copy machinery of the kernels tiled by StreamCfg (forward, dQ): one object per thread.
