@@ -73,13 +73,14 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
     constexpr bool BOOLROW = BIAS == 7;  // ... a bool mask: the row holds 0 or the mask term, in log2 units
     static_assert(!(FROM_DS && ROWB), "a row-broadcast bias has no dense dS");
 
-    // Q and dO rows come through LDS (WaveRows).  A place for dO beside that of Q where it costs no work-group on a CU; else one
-    // after the other.
+    // Q and dO rows come through LDS (WaveRows) where StreamCfg has a place for them.  A place for dO beside that of Q where it
+    // costs no work-group on a CU; else one after the other.
     typedef WaveRows<T, D> WR;
     constexpr bool STAGED = C::STAGE != C::kNowhere && !FROM_DS;
     constexpr bool BESIDE = STAGED && !ROWB && (C::LDS_BYTES + 4 * WR::BYTES) * C::ROOM <= 163840;
-    __shared__ __align__(1024) unsigned char smem[C::LDS_BYTES + (ROWB ? kRowBiasKeys * 4 : 0) + (BESIDE ? 4 * WR::BYTES : 0)];
-    const float* row_lds = reinterpret_cast<const float*>(smem + C::LDS_BYTES);
+    constexpr int LDS_BYTES = STAGED ? C::LDS_BYTES : C::LOOP_BYTES;
+    __shared__ __align__(1024) unsigned char smem[LDS_BYTES + (ROWB ? kRowBiasKeys * 4 : 0) + (BESIDE ? 4 * WR::BYTES : 0)];
+    const float* row_lds = reinterpret_cast<const float*>(smem + LDS_BYTES);
 
     const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63;
@@ -490,13 +491,13 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
         constexpr int BV = decltype(bv_tag)::value;
         auto stage_row = [&]() {
             if (ROWB)
-                stage_row_bias(reinterpret_cast<float*>(smem + C::LDS_BYTES), p.bias, p.row_bias_kind,
+                stage_row_bias(reinterpret_cast<float*>(smem + LDS_BYTES), p.bias, p.row_bias_kind,
                                (int64_t)b * p.sbias.b + (int64_t)h * p.sbias.h + (int64_t)key0 * p.sbias.n, p.sbias.n, N, tid);
         };
         if constexpr (STAGED) {
             constexpr bool FIRST_KV = C::STAGE != C::kOwnRing;  // the first copies of the stream need not wait for the rows
             constexpr int PRO = FIRST_KV ? KS::template prologue_copies<BV>() : 0;
-            const unsigned q_tile = ks_.stage_addr(), do_tile = BESIDE ? ks_.lds_kv + C::LDS_BYTES + ks_.wave_s * WR::BYTES : q_tile;
+            const unsigned q_tile = ks_.stage_addr(), do_tile = BESIDE ? ks_.lds_kv + LDS_BYTES + ks_.wave_s * WR::BYTES : q_tile;
             auto copy = [&](bool is_q) {
                 const unsigned saved_m0 = lds_copy_begin();
                 if (is_q) WR::issue(qp, p.sq.s, mw, M, q_tile, lane, [&](int c) { return D <= 128 ? chunks.wrap(c) : c; });

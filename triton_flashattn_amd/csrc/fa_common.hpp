@@ -475,11 +475,16 @@ template <int D, int BIAS, bool WIDE = false> struct StreamCfg {
     static constexpr int LOOP_BYTES = KV_BYTES + BIAS_BYTES > O_BYTES ? KV_BYTES + BIAS_BYTES : O_BYTES;
     // Where the rows of a wave (WaveRows) stand before the first step: in the ring slots that the first copies leave free
     // (half of one to a wave, or for waves 2 and 3 behind everything else), behind everything else, or in the wave's own ring
-    // of bias slots, whose first copies then wait for them.  (Bias tiles at head dim 256: nowhere.)
+    // of bias slots, whose first copies then wait for them.  Bias tiles at head dim 256: nowhere.  fp32 tiles up to 64, whose
+    // slices are the longest of those first copies: behind everything else at 64, where that is free, and nowhere below, where
+    // rows are so short that the lanes' own loads take less (dQ, us, own ring / here: D=64 B=8 H=12 S=256 12.9 / 12.6; D=32
+    // S=256 causal 11.8 / 11.2, S=128 7.6 / 7.2; D=16 32 x 12 pairs of 192 rows 16.8 / 16.4, B=8 H=12 S=256 10.3 / 9.5).
     enum Stage { kHalfSlots, kOwnRing, kBehind, kSlotsAndBehind, kNowhere };
     static constexpr Stage STAGE = NH == 2                          ? kHalfSlots
                                    : D > 128                        ? kNowhere
                                    : ES == 0                        ? kBehind
+                                   : ES == 4 && D <= 32             ? kNowhere
+                                   : ES == 4 && D == 64             ? kBehind
                                    : NBS * BSLOT >= 64 * D          ? kOwnRing
                                                                     : kSlotsAndBehind;
     // Work-groups on a CU that such a place must leave room for: three up to head dim 64 where the loops do, which the registers
