@@ -609,16 +609,26 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
         }
     }
     T* op = reinterpret_cast<T*>(p.o) + (int64_t)b * p.so.b + (int64_t)h * p.so.h;
-    int lane_late = lane;  // (as above)
-    asm volatile("" : "+v"(lane_late));
     lds_wave_order();  // (a wave's own rows: no barrier)
-    i32x4 out[WR::COPIES];  // (all reads in flight together)
+    if constexpr (BIAS == 5 && CAUSAL && D == 64) {
+        // (One read after the other.  With all of them in flight the compiler turned the order of this kernel's LOOPS: every LDS
+        // read waited for by itself, us, H=16 S=1024 21.5 / 23.9, S=2048 39.4 / 44.6, H=64 62.7 / 63.0.)
+        for (int c = lane; c < 32 * CPR; c += 64) {
+            const int row = c / CPR, ch = c % CPR;
+            if (mw + row < M && ch * 8 < p.d_v) gst16(op + (int64_t)(mw + row) * p.so.s + ch * 8, lds_read16(o_lds + row * OS + ch * 8));
+        }
+    } else {
+        int lane_late = lane;  // (nothing formed of it here is kept in registers from the first copies on)
+        asm volatile("" : "+v"(lane_late));
+        i32x4 out[WR::COPIES];  // (all reads in flight together)
 #pragma unroll
-    for (int it = 0; it < WR::COPIES; it++) out[it] = lds_read16(o_lds + (it * 64 + lane_late) / CPR * OS + (it * 64 + lane_late) % CPR * 8);
+        for (int it = 0; it < WR::COPIES; it++)
+            out[it] = lds_read16(o_lds + (it * 64 + lane_late) / CPR * OS + (it * 64 + lane_late) % CPR * 8);
 #pragma unroll
-    for (int it = 0; it < WR::COPIES; it++) {
-        const int row = (it * 64 + lane_late) / CPR, ch = (it * 64 + lane_late) % CPR;
-        if (mw + row < M && ch * 8 < p.d_v) gst16(op + (int64_t)(mw + row) * p.so.s + ch * 8, out[it]);
+        for (int it = 0; it < WR::COPIES; it++) {
+            const int row = (it * 64 + lane_late) / CPR, ch = (it * 64 + lane_late) % CPR;
+            if (mw + row < M && ch * 8 < p.d_v) gst16(op + (int64_t)(mw + row) * p.so.s + ch * 8, out[it]);
+        }
     }
 }
 
