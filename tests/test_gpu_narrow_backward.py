@@ -218,17 +218,20 @@ def test_biases_that_a_pair_of_waves_takes(gpu_device, D, kind):
 @pytest.mark.parametrize("D", [16, 32, 64])
 @pytest.mark.parametrize("kind", ["bf16", "f16", "f32"])
 def test_bias_and_gradient_rows_that_allow_no_aligned_accesses(gpu_device, D, kind):
-    """Straight to the kernels, rows of an odd number of keys, dense (element by element) and with a padded pitch (16 bytes at
-    a time), the bias and its gradient each in either."""
+    """Straight to the kernels, rows of an odd number of keys, dense (fp32: read 4 bytes to a lane; else, and the gradient,
+    element by element), with a padded pitch (16 bytes at a time) and, the bias, every second column of a wider tensor
+    (element by element), the gradient dense, with a padded pitch, or none."""
     for i, (M, N, causal) in enumerate([(70, 197, False), (131, 131, True), (33, 5, False), (300, 129, False)]):
         q, k, v, do, bias = make_inputs(gpu_device, 2, M, N, 2, D, torch.bfloat16, kind, seed=D + i, trainable=False)
         ref = run_oracle(q, k, v, do, bias, causal)
         wide = torch.full((2, 2, M, -(-N // 8) * 8), float("nan"), dtype=bias.dtype, device=gpu_device)
         wide[..., :N] = bias
-        for b in (bias, wide[..., :N]):
-            for out in (torch.empty_like(bias), torch.empty_like(wide)[..., :N]):
+        apart = torch.full((2, 2, M, 2 * N), float("nan"), dtype=bias.dtype, device=gpu_device)
+        apart[..., ::2] = bias
+        for b in (bias, wide[..., :N], apart[..., ::2]):
+            for out in (torch.empty_like(bias), torch.empty_like(wide)[..., :N], None):
                 res = _launch_directly(q, k, v, do, b, out, causal)
-                check(res, ref, str((D, kind, M, N, causal, b.stride(2), out.stride(2))))
+                check(res, ref, str((D, kind, M, N, causal, b.stride(), None if out is None else out.stride())))
 
 
 def test_tiles_of_64_or_128_keys_with_an_fp32_bias(gpu_device):

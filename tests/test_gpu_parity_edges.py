@@ -268,11 +268,12 @@ def _launch_directly(q, k, v, do, bias, dbias, causal):
 @pytest.mark.parametrize("D", [32, 128])
 @pytest.mark.parametrize("kind", ["bool", "f16", "bf16", "f32"])
 def test_bias_rows_that_are_not_whole_chunks(gpu_device, D, kind):
-    """A number of keys that is no multiple of 16 bytes, three ways: through the public function
+    """A number of keys that is no multiple of 16 bytes, four ways: through the public function
     (which copies such a bias into rows with a padded pitch), straight to the kernels as a dense
-    tensor (read and written element by element) and straight to the kernels as a column slice of a
-    wider tensor (16-byte copies that run into the columns behind the slice: those hold NaN for the
-    bias and must not be touched in dbias)."""
+    tensor (read 4 bytes to a lane where it is fp32 and the head dim at most 64, else element by element,
+    and written element by element), as every second column of a wider tensor (read and written element
+    by element whatever its type) and as a column slice of a wider tensor (16-byte copies that run into the
+    columns behind the slice: those hold NaN for the bias and must not be touched in dbias)."""
     bdt = {"bool": torch.bool, "f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}[kind]
     for i, (B, M, N, H, causal) in enumerate([(2, 70, 197, 2, False), (1, 131, 131, 3, True), (1, 257, 67, 1, False)]):
         dtype = torch.float16 if kind == "f16" else torch.bfloat16
@@ -288,9 +289,17 @@ def test_bias_rows_that_are_not_whole_chunks(gpu_device, D, kind):
         check(ours, ref, "public %s D%d case %d" % (kind, D, i))
         if trainable:
             assert ours["dbias"].shape == bias.shape and ours["dbias"].dtype == bdt
-        # dense rows, element by element
+        # dense rows
         dbias = torch.empty_like(bias) if trainable else None
         check(_launch_directly(q, k, v, do, bias, dbias, causal), ref, "dense %s D%d case %d" % (kind, D, i))
+        # element by element: a key stride of 2, of the bias alone and of its gradient too
+        apart = torch.full((B, H, M, 2 * N), float("nan") if trainable else 1, dtype=bdt, device=gpu_device)
+        apart[..., ::2] = bias
+        dapart = torch.full((B, H, M, 2 * N), 7.0, dtype=bdt, device=gpu_device) if trainable else None
+        for out in (None, torch.empty_like(bias), dapart[..., ::2]) if trainable else (None,):
+            res = _launch_directly(q, k, v, do, apart[..., ::2], out, causal)
+            check(res, ref, "apart %s D%d case %d" % (kind, D, i))
+        assert not trainable or (dapart[..., 1::2] == 7.0).all(), "the columns between those of dbias were written"
         # a column slice of a wider tensor
         per = 16 // bias.element_size()
         width = -(-N // per) * per + per * (i % 2)   # rows start at multiples of 16 bytes and own their last chunk
