@@ -121,28 +121,25 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
     ks_.init(smem, kp, vp, bp, p.sk.s, p.sv.s, p.sbias.m, p.sbias.n, M, N, mw, wave, lane, chunks, p.d_v / 8);
 
     // Q^T as B operand: column my_m, k = d
-    // Without a bias, from head dim 96 on, through LDS with the first K/V rows (WaveRows; us: B=8 H=12 S=512 D=128 23.6 -> 22.4,
-    // B=8 H=16 S=257 D=80 14.0 -> 13.5).  At 64 it is the same (197, 512 and 2048 rows), and so with a staged row (padding mask
-    // B=32 H=12 S=197 15.4 / 15.3) or a tile, whose first copies would have to wait for the rows (fp32 table there 20.4 / 20.8).
+    // (Rows through LDS, as in the dQ kernel, lose as much as they gain in this one, which needs them once and has its K and V
+    // copies to wait for anyway.  us, the lanes' own loads / LDS, no bias: D=128 B=16 H=12 S=197 16.5 / 15.8, B=32 S=192 21.0 /
+    // 21.4, causal 21.2 / 22.4, B=12 H=16 S=577 causal 36.4 / 38.3, H=16 S=2000 causal 36.1 / 37.0; D=256 H=32 S=1001 44.0 / 46.8,
+    // B=12 H=16 S=577 116.5 / 120; D=80 B=4 H=8 S=512 12.4 / 13.2, B=16 H=12 S=197 14.0 / 13.3.)
     typedef WaveRows<T, D> WR;
-    constexpr bool STAGED = BIAS == 0 && D >= 96;
     T8 qreg[C::KSTEPS];
-    auto load_q = [&]() {
 #pragma unroll
-        for (int ks = 0; ks < C::KSTEPS; ks++) {
-            i32x4 raw = {0, 0, 0, 0};
-            if (my_m < M) raw = gld16(qp + (int64_t)my_m * p.sq.s + (D <= 128 ? chunks.wrap(2 * ks + g) : 2 * ks + g) * 8);
-            qreg[ks] = as_vec<T8>(raw);
-        }
-    };
-    if (!STAGED || M <= 32) load_q();
+    for (int ks = 0; ks < C::KSTEPS; ks++) {
+        i32x4 raw = {0, 0, 0, 0};
+        if (my_m < M) raw = gld16(qp + (int64_t)my_m * p.sq.s + (D <= 128 ? chunks.wrap(2 * ks + g) : 2 * ks + g) * 8);
+        qreg[ks] = as_vec<T8>(raw);
+    }
     auto split_q = [&]() {
         if (D <= 128 && p.d_qk < D) {
 #pragma unroll
             for (int ks = 0; ks < C::KSTEPS; ks++) qreg[ks] = chunks.part(qreg[ks], 2 * ks + g, C::CPR);
         }
     };
-    if constexpr (!STAGED && TB != 0) split_q();  // (kernels of a bias tile have no registers for it later)
+    if constexpr (TB != 0) split_q();  // (kernels of a bias tile have no registers for it later)
 
     int n_steps = (N + BK - 1) / BK;
     if (CAUSAL) {
@@ -509,33 +506,16 @@ __global__ __launch_bounds__(256, (StreamCfg<D, fwd_stream_kind(BIAS, D), true>:
 
     auto run = [&](auto bv_tag) {
         constexpr int BV = decltype(bv_tag)::value;
-        if constexpr (STAGED) {
-            if (M > 32) {
-                const unsigned q_tile = ks_.stage_addr();
-                const unsigned saved_m0 = lds_copy_begin();
-                WR::issue(qp, p.sq.s, mw, M, q_tile, lane, [&](int c) { return D <= 128 ? chunks.wrap(c) : c; });
-                lds_copy_end(saved_m0);
-                ks_.template prologue<BV>();
-                WR::template arrived<KS::template prologue_copies<BV>()>();
-#pragma unroll
-                for (int ks = 0; ks < C::KSTEPS; ks++) qreg[ks] = SW::template row8_at<T8>(q_tile + rows_l, 0, ks);
-            } else {  // (a token or a few: 32 copies of the same rows cost a decode step at B=8 H=16 N=4097 1 %)
-                wait_vmcnt<0>();
-                ks_.template prologue<BV>();
-            }
-            split_q();
-        } else {
-            stage_row();
-            // The loads of this lane's rows issued above are the compiler's own.  Left in flight, they would
-            // make it wait for "all vector-memory operations" at their first use inside EVERY step of the
-            // loops (it cannot know that they land once), and that wait drains the queue of copies issued
-            // steps ahead.  Waiting for them here keeps the loops free of it.
-            wait_vmcnt<0>();
-            // (After the wait and not before the loads, where it would be one for the first copies too.  B=32 H=12 M=N=197 D=64, us
-            // per call, after / before: padding mask 13.45 / 13.96; no bias, B=8 H=16 S=512 15.4 / 15.9.)
-            ks_.template prologue<BV>();
-            if constexpr (TB == 0) split_q();  // (while the first copies are on their way)
-        }
+        stage_row();
+        // The loads of this lane's rows issued above are the compiler's own.  Left in flight, they would
+        // make it wait for "all vector-memory operations" at their first use inside EVERY step of the
+        // loops (it cannot know that they land once), and that wait drains the queue of copies issued
+        // steps ahead.  Waiting for them here keeps the loops free of it.
+        wait_vmcnt<0>();
+        // (After the wait and not before the loads, where it would be one for the first copies too.  B=32 H=12 M=N=197 D=64, us
+        // per call, after / before: padding mask 13.45 / 13.96; no bias, B=8 H=16 S=512 15.4 / 15.9.)
+        ks_.template prologue<BV>();
+        if constexpr (TB == 0) split_q();  // (while the first copies are on their way)
         // the leading fast steps whose copies stay inside the tensors issue them without clamps
         const int n_lean = (BV != kByElement || TB == 0) ? ks_.lean_steps(n_fast) : 0;
         int k = 0;
