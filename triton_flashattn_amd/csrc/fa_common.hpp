@@ -477,15 +477,17 @@ template <int D, int BIAS, bool WIDE = false> struct StreamCfg {
     // (half of one to a wave, or for waves 2 and 3 behind everything else), behind everything else, or in the wave's own ring
     // of bias slots, whose first copies then wait for them.  Head dim 256: nowhere, rows of dO would have to wait for those of Q to
     // be read (dQ, us, there / half slots: no bias B=32 H=12 S=192 causal 66.9 / 72.9, H=32 S=1001 60.6 / 64.2, B=2 H=4 S=64 12.0 /
-    // 13.8, row mask there 12.6 / 14.6, B=12 H=16 S=577 168 / 173, B=2 H=16 S=1024 90.8 / 92.0).  fp32 tiles up to 64, whose
-    // slices are the longest of those first copies: behind everything else at 64, where that is free, and nowhere below, where
-    // rows are so short that the lanes' own loads take less (dQ, us, own ring / here: D=64 B=8 H=12 S=256 12.9 / 12.6; D=32
-    // S=256 causal 11.8 / 11.2, S=128 7.6 / 7.2; D=16 32 x 12 pairs of 192 rows 16.8 / 16.4, B=8 H=12 S=256 10.3 / 9.5).
+    // 13.8, row mask there 12.6 / 14.6, B=12 H=16 S=577 168 / 173, B=2 H=16 S=1024 90.8 / 92.0).  Tiles up to 32:
+    // nowhere, rows are so short that the lanes' own loads take less than the first copies' wait (dQ, us, own ring / here: fp32,
+    // D=32 S=256 causal 11.8 / 11.2, S=128 7.6 / 7.2; D=16 32 x 12 pairs of 192 rows 16.8 / 16.4, B=8 H=12 S=256 10.3 / 9.5; byte
+    // mask, D=16 32 x 12 pairs of 192 rows 18.8 / 17.3, 16 x 12 of 197 13.4 / 12.0, D=32 13.4 / 13.1; bf16, D=16 19.3 / 18.4, 14.4 /
+    // 13.4, B=2 H=16 S=1024 causal 22.4 / 21.4, D=32 24.1 / 23.4).  fp32 tiles at 64, whose slices are the longest of those first
+    // copies: behind everything else, where that is free (B=8 H=12 S=256 12.9 / 12.6).
     enum Stage { kHalfSlots, kOwnRing, kBehind, kSlotsAndBehind, kNowhere };
     static constexpr Stage STAGE = D > 128                          ? kNowhere
                                    : NH == 2                        ? kHalfSlots
                                    : ES == 0                        ? kBehind
-                                   : ES == 4 && D <= 32             ? kNowhere
+                                   : ES != 0 && D <= 32             ? kNowhere
                                    : ES == 4 && D == 64             ? kBehind
                                    : NBS * BSLOT >= 64 * D          ? kOwnRing
                                                                     : kSlotsAndBehind;
