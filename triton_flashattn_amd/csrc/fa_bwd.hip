@@ -74,9 +74,11 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
     static_assert(!(FROM_DS && ROWB), "a row-broadcast bias has no dense dS");
 
     // Q and dO rows come through LDS (WaveRows) where StreamCfg has a place for them.  A place for dO beside that of Q where it
-    // costs no work-group on a CU; else one after the other.
+    // costs no work-group on a CU; else one after the other.  Not causal ALiBi at head dim 128 and a causal fp32 tile at 64 (us,
+    // the lanes' own loads / LDS: ALiBi H=16 S=2000 53.2 / 56.1, B=2 H=8 S=2048 55.5 / 57.6, H=32 S=1001 33.4 / 34.4, but B=16 H=12
+    // S=197 20.4 / 18.0; fp32 B=2 H=4 S=128 9.3 / 10.0, B=4 H=8 S=512 17.7 / 18.2, B=8 H=8 S=256 for all batches 13.0 / 13.9).
     typedef WaveRows<T, D> WR;
-    constexpr bool STAGED = C::STAGE != C::kNowhere && !FROM_DS;
+    constexpr bool STAGED = C::STAGE != C::kNowhere && !FROM_DS && !(CAUSAL && ((BIAS == 5 && D == 128) || (BIAS == 4 && D == 64)));
     constexpr bool BESIDE = STAGED && !ROWB && (C::LDS_BYTES + 4 * WR::BYTES) * C::ROOM <= 163840;
     constexpr int LDS_BYTES = STAGED ? C::LDS_BYTES : C::LOOP_BYTES;
     __shared__ __align__(1024) unsigned char smem[LDS_BYTES + (ROWB ? kRowBiasKeys * 4 : 0) + (BESIDE ? 4 * WR::BYTES : 0)];
