@@ -3,7 +3,7 @@ the fp32 oracle with the tolerances of the parity tests (out max-abs 2e-2, gradi
 import pytest
 import torch
 
-from oracle.attention_oracle import attention_backward, attention_forward
+from oracle.attention_oracle import attention_backward, attention_forward, reference_grads
 from triton_flashattn_amd import AlibiBias, flash_attention_fn
 
 pytestmark = pytest.mark.gpu
@@ -346,6 +346,27 @@ def test_host_path_with_hooks_views_and_transforms(gpu_device):
     # a transform is refused, also where it wraps none of the arguments
     with pytest.raises(RuntimeError):
         torch.func.vmap(lambda x: call(*one) * x)(rnd(3, 1))
+
+
+@pytest.mark.parametrize("D", [64, 72, 128])
+@pytest.mark.parametrize("causal", [False, True])
+def test_dq_of_few_rows(gpu_device, D, causal):
+    """Up to 64 query rows the dQ kernel takes rows of Q, dO and O by other loads than above: around that line, with every kind of
+    bias, by the kernel that forms delta itself and, with keys enough for several work-groups to share them, by shares."""
+    for M, N in ([(5, 5), (33, 33), (64, 64), (65, 65)] if causal else [(1, 70), (31, 2100), (63, 33), (64, 129), (65, 129), (97, 64)]):
+        g = torch.Generator().manual_seed(M + N)
+        q, k, v, do = (torch.randn(2, s, 3, D, generator=g).bfloat16().to(gpu_device) for s in (M, N, N, M))
+        ins = [t.requires_grad_(True) for t in (q, k, v)]
+        dense = torch.randn(2, 3, M, N, generator=g).to(gpu_device)
+        # (the first key is visible: scores of a row without a visible key are -1e6, rounded to 2^-4, and its weights off by 6 %)
+        mask = (dense > -1.5) | (torch.arange(N, device=gpu_device) == 0)
+        alibi = AlibiBias(torch.tensor([0.5, 0.25, 0.1], device=gpu_device))
+        for bias in (None, mask, dense.bfloat16(), dense, mask[:, :1, :1], dense[:1, :, :1].bfloat16(), alibi):
+            got = torch.autograd.grad(flash_attention_fn(*ins, bias, causal), ins, do)
+            full = alibi.materialize(M, N) if bias is alibi else bias
+            ref = reference_grads(*[t.detach() for t in ins], None if full is None else full.expand(2, 3, M, N), do, causal)
+            for name, a in zip(("dq", "dk", "dv"), got):
+                assert (a.float() - ref[name]).norm() <= 5e-2 * ref[name].norm(), (name, M, N, D, causal, type(bias))
 
 
 def test_ragged_fp32_bias_written_to_before_the_backward(gpu_device):

@@ -131,7 +131,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
     const T* dop = reinterpret_cast<const T*>(p.dout) + (int64_t)b * p.sdo.b + (int64_t)h * p.sdo.h;
     const T* outp = reinterpret_cast<const T*>(p.o) + (int64_t)b * p.so.b + (int64_t)h * p.so.h;
     T8 qreg[C::KSTEPS], doreg[C::KSTEPS];
-    if constexpr (!STAGED) {
+    auto load_rows = [&]() {
 #pragma unroll
         for (int ks = 0; ks < C::KSTEPS; ks++) {
             i32x4 rq = {0, 0, 0, 0}, rd = {0, 0, 0, 0};
@@ -141,7 +141,8 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
             qreg[ks] = as_vec<T8>(rq);
             doreg[ks] = as_vec<T8>(rd);
         }
-    }
+    };
+    if constexpr (!STAGED) load_rows();
     auto split_q = [&]() {
         if (D <= 128 && !FROM_DS && p.d_qk < D) {
 #pragma unroll
@@ -176,9 +177,9 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
             }
         }
     };
-    auto make_delta = [&](unsigned do_tile) {
+    auto make_delta = [&](unsigned do_tile, auto tile_tag) {  // tile_tag: dO stands in LDS
         if (!p.dq_makes_delta) return;
-        if constexpr (O_AS_TILE) {
+        if constexpr (O_AS_TILE && decltype(tile_tag)::value) {
             constexpr int RPI = 64 / CPR;  // rows of a copy
             float sum[WR::COPIES];
 #pragma unroll
@@ -225,7 +226,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
     };
     if constexpr (!STAGED && !FROM_DS) {
         if constexpr (TB != 0) split_q();  // (kernels of a bias tile have no registers for it later)
-        make_delta(0);
+        make_delta(0, std::false_type{});
     }
 
     int n_steps = (N + BK - 1) / BK;
@@ -489,6 +490,11 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
     // (query rows past M need no mask: a lane is one row, and such a row is not stored.  Run in masked steps, a
     // ragged last tile was the longest of a causal grid: B=1 H=16 M=N=6001 D=128 0.298 -> 0.218 ms)
     if (!(qk_scale > 0.f)) n_fast = 0;
+    // Up to 64 rows, half of a tile or less: the lanes' own loads.  Waves without rows of their own copy the last one over and
+    // over, and the longer way to the first step is all of such a call.  From head dim 64 on (us, LDS / own loads: D=128 B=2 H=4
+    // S=64 no bias 8.7 / 7.9, byte mask 9.4 / 8.7, row mask 9.4 / 8.3, causal fp32 10.1 / 9.1, H=8 M=32 N=1024 12.6 / 11.5; D=80 bf16
+    // B=2 H=4 S=64 10.0 / 9.2; D=64 no bias 6.2 / 5.6, fp32 for all batches 7.4 / 6.4; at 128 rows the two are even).
+    const bool few_rows = STAGED && D >= 64 && M <= 64;
     auto run = [&](auto bv_tag) {
         constexpr int BV = decltype(bv_tag)::value;
         auto stage_row = [&]() {
@@ -496,7 +502,14 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
                 stage_row_bias(reinterpret_cast<float*>(smem + LDS_BYTES), p.bias, p.row_bias_kind,
                                (int64_t)b * p.sbias.b + (int64_t)h * p.sbias.h + (int64_t)key0 * p.sbias.n, p.sbias.n, N, tid);
         };
-        if constexpr (STAGED) {
+        if (STAGED && few_rows) {
+            load_rows();
+            split_q();
+            make_delta(0, std::false_type{});
+            stage_row();
+            wait_vmcnt<0>();
+            ks_.template prologue<BV>();
+        } else if constexpr (STAGED) {
             constexpr bool FIRST_KV = C::STAGE != C::kOwnRing;  // the first copies of the stream need not wait for the rows
             constexpr int PRO = FIRST_KV ? KS::template prologue_copies<BV>() : 0;
             const unsigned q_tile = ks_.stage_addr(), do_tile = BESIDE ? ks_.lds_kv + LDS_BYTES + ks_.wave_s * WR::BYTES : q_tile;
@@ -526,7 +539,7 @@ __global__ __launch_bounds__(256, (StreamCfg<D, stream_kind(BIAS)>::MIN_BLOCKS))
                 doreg[ks] = as_vec<T8>(ks * 16 + 8 * g < p.d_v ? x : i32x4{0, 0, 0, 0});
             }
             split_q();
-            make_delta(do_tile);
+            make_delta(do_tile, std::true_type{});
             if constexpr (!FIRST_KV) {
                 WR::done();
                 ks_.template prologue<BV>();
