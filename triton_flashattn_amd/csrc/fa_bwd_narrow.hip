@@ -52,10 +52,12 @@ template <int D, int BIAS> struct NarrowCfg {
     static constexpr int LOOP_BYTES = OFF_DS + 4 * DS_BYTES;
     // Where the K and V rows of a wave stand before the first step (WaveRows): in the slots that the first copies leave free, of
     // Q and dO rows, half a slot to a wave, or in the wave's own bias slot; else behind everything else.  (V beside an fp32
-    // bias at D = 64: nowhere, there the lanes load it.)
+    // bias at D = 64: nowhere, there the lanes load it.  At D = 16, half a kilobyte to a wave, neither: us, LDS / own loads, fp32 for
+    // all batches 32 x 12 pairs of 192 rows 18.8 / 17.2, 16 x 12 of 197 14.3 / 13.3, fp32 H=8 M=32 N=1024 5.6 / 5.3, 192 rows 21.4 / 20.0,
+    // no bias B=12 H=16 S=577 causal 21.8 / 20.9.)
     enum Stage { kHalfSlots, kBiasSlot, kBehind, kNowhere };
-    static constexpr Stage K_STAGE = ES == 4 ? kBiasSlot : kHalfSlots;
-    static constexpr Stage V_STAGE = ES == 4 ? (128 * D <= BSLOT ? kBiasSlot : kNowhere) : 64 * D <= BSLOT ? kBiasSlot : kBehind;
+    static constexpr Stage K_STAGE = D == 16 ? kNowhere : ES == 4 ? kBiasSlot : kHalfSlots;
+    static constexpr Stage V_STAGE = D == 16 ? kNowhere : ES == 4 ? (128 * D <= BSLOT ? kBiasSlot : kNowhere) : 64 * D <= BSLOT ? kBiasSlot : kBehind;
     static constexpr int LDS_BYTES = LOOP_BYTES + (V_STAGE == kBehind ? 256 * D : 0);
     static constexpr int MIN_BLOCKS = D <= 32 && ES <= 1 ? 3 : 2;  // work-groups per CU
     static_assert(LDS_BYTES * MIN_BLOCKS <= 163840, "LDS of a CU");
@@ -195,13 +197,19 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
     // the way back at the end, us, before -> after: padding mask B=32 H=12 S=197 D=64 25.6 -> 21.9, with an fp32 table 31.1 ->
     // 27.6, B=8 H=16 S=257 D=80 22.1 -> 19.3, B=4 H=16 S=2048 D=64 causal 81.6 -> 78.2, B=4 H=32 M=N=4096 1105 -> 1078.
     typedef WaveRows<T, D> WR;
-    constexpr bool V_STAGED = C::V_STAGE != C::kNowhere;
+    constexpr bool K_STAGED = C::K_STAGE != C::kNowhere, V_STAGED = C::V_STAGE != C::kNowhere;
+    static_assert(K_STAGED || !V_STAGED, "V comes with K");
     T8 kreg[C::KSTEPS], vreg[C::KSTEPS];
     if constexpr (!V_STAGED) {
 #pragma unroll
         for (int ks = 0; ks < C::KSTEPS; ks++) {
             i32x4 rv = {0, 0, 0, 0};
             const int d = ks * 16 + 8 * g;
+            if constexpr (!K_STAGED) {
+                i32x4 rk = {0, 0, 0, 0};
+                if (my_n < N && d < p.d_qk) rk = gld16(kp + (int64_t)my_n * p.sk.s + d);
+                kreg[ks] = as_vec<T8>(rk);
+            }
             if (my_n < N && d < p.d_v) rv = gld16(vp + (int64_t)my_n * p.sv.s + d);
             vreg[ks] = as_vec<T8>(rv);
         }
@@ -403,7 +411,7 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
             const unsigned v_tile = C::V_STAGE == C::kBehind ? lds_base + C::LOOP_BYTES + (unsigned)wave * WR::BYTES
                                                              : bias_slot + (C::K_STAGE == C::kBiasSlot ? WR::BYTES : 0);
             const unsigned saved_m0 = lds_copy_begin();
-            WR::issue(kp, p.sk.s, nw, N, k_tile, lane, [&](int c) { return live_chunk(c, p.d_qk / 8); });
+            if constexpr (K_STAGED) WR::issue(kp, p.sk.s, nw, N, k_tile, lane, [&](int c) { return live_chunk(c, p.d_qk / 8); });
             if constexpr (V_STAGED) WR::issue(vp, p.sv.s, nw, N, v_tile, lane, [&](int c) { return live_chunk(c, p.d_v / 8); });
 #pragma unroll
             for (int i = 0; i < LA; i++) issue(t0 + i, bv_tag);
@@ -414,8 +422,10 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
 #pragma unroll
             for (int ks = 0; ks < C::KSTEPS; ks++) {
                 const int d = ks * 16 + 8 * g;
-                const i32x4 rk = as_raw(SW::template row8_at<T8>(k_tile + rows_l, 0, ks));
-                kreg[ks] = as_vec<T8>(d < p.d_qk ? rk : i32x4{0, 0, 0, 0});
+                if constexpr (K_STAGED) {
+                    const i32x4 rk = as_raw(SW::template row8_at<T8>(k_tile + rows_l, 0, ks));
+                    kreg[ks] = as_vec<T8>(d < p.d_qk ? rk : i32x4{0, 0, 0, 0});
+                }
                 if constexpr (V_STAGED) {
                     const i32x4 rv = as_raw(SW::template row8_at<T8>(v_tile + rows_l, 0, ks));
                     vreg[ks] = as_vec<T8>(d < p.d_v ? rv : i32x4{0, 0, 0, 0});
