@@ -646,11 +646,11 @@ __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) v
                 // used: operands of the first two products, then, under them, LSE, bias and the operands of the other two.  Left to
                 // the compiler, each read waited for the one before it in some of these kernels.  us, before -> after: D=32, fp32 and
                 // dBias B=2 H=12 M=N=1024 39.1 -> 36.2, B=8 154.8 -> 141.2; bf16 and dBias B=2 30.7 -> 29.5, causal H=8 28.0 -> 26.6;
-                // fp32 read B=16 H=8 M=N=256 10.6 -> 10.2; D=16, fp32 and dBias 38.0 -> 36.5.  (A 16-bit tile at D=16 that is only
-                // read has registers for three work-groups on a CU without them and for two with them.  Fetched ahead / not: B=8
-                // H=12 M=N=1024 50.5 / 46, 512 18.4 / 18.6, 16 x 12 pairs of 576 rows 36.8 / 33.7, but causal, where long tiles end
-                // alone, B=8 H=12 1024 37.0 / 37.6, 2048 117 / 121, and with dBias 28.0 / 29.4, 2048 355 / 374.)
-                constexpr bool AHEAD = D <= 32 && C::MIN_BLOCKS == 2 && !(D == 16 && C::ES == 2 && DBIAS != 1 && !CAUSAL);
+                // fp32 read B=16 H=8 M=N=256 10.6 -> 10.2; D=16, fp32 and dBias 38.0 -> 36.5.  (A 16-bit tile at D=16 has
+                // registers for three work-groups on a CU without them and for two with them.  Fetched ahead / not: read only, B=8 H=12
+                // M=N=1024 50.5 / 46, 16 x 12 pairs of 576 rows 36.8 / 33.7; dBias, 32 x 12 pairs of 192 rows 22.6 / 19.6, causal 23.6 /
+                // 19.7, but where few tiles end alone H=16 M=N=1024 29.1 / 29.4, B=12 H=16 S=577 77.9 / 77.3, B=8 H=12 2048 355 / 374.)
+                constexpr bool AHEAD = C::MIN_BLOCKS == 2 && (D == 32 || (D == 16 && C::ES == 4));
                 constexpr bool BIAS_AHEAD = AHEAD || (D == 64 && TB == 4 && DBIAS == 0);  // (16 registers)
                 constexpr int NP = 2 * C::DB;
                 auto fence = [&]() {
