@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from oracle.attention_oracle import attention_backward, attention_forward, reference_grads
-from triton_flashattn_amd import AlibiBias, flash_attention_fn
+from triton_flashattn_amd import AlibiBias, flash_attention_fn, flash_attention_qkvpacked_fn
 
 pytestmark = pytest.mark.gpu
 
@@ -366,6 +366,29 @@ def test_dq_of_few_rows(gpu_device, D, causal):
             full = alibi.materialize(M, N) if bias is alibi else bias
             ref = reference_grads(*[t.detach() for t in ins], None if full is None else full.expand(2, 3, M, N), do, causal)
             for name, a in zip(("dq", "dk", "dv"), got):
+                assert (a.float() - ref[name]).norm() <= 5e-2 * ref[name].norm(), (name, M, N, D, causal, type(bias))
+
+
+@pytest.mark.parametrize("D", [72, 80, 96])
+def test_dk_dv_of_few_keys_at_head_dim_96(gpu_device, D):
+    """Up to 64 keys the kernel of head dim 96 takes K and V in and gradients out by other ways than above: around that line,
+    waves without a key among them, and strided gradients (the packed function)."""
+    for M, N, causal in [(70, 5, False), (70, 31, False), (33, 33, True), (200, 64, False), (64, 64, True), (64, 65, False), (97, 97, True)]:
+        g = torch.Generator().manual_seed(M + N + D)
+        q, k, v, do = (torch.randn(2, s, 3, D, generator=g).bfloat16().to(gpu_device) for s in (M, N, N, M))
+        mask = torch.ones(2, 1, 1, N, dtype=torch.bool, device=gpu_device)
+        mask[1, ..., N // 2 + 1:] = False
+        for bias in (None, mask, AlibiBias(torch.tensor([0.5, 0.25, 0.1], device=gpu_device))):
+            ins = [t.detach().requires_grad_(True) for t in (q, k, v)]
+            got = torch.autograd.grad(flash_attention_fn(*ins, bias, causal), ins, do)
+            full = bias.materialize(M, N) if isinstance(bias, AlibiBias) else bias
+            ref = reference_grads(q, k, v, None if full is None else full.expand(2, 3, M, N), do, causal)
+            if M == N:
+                qkv = torch.stack((q, k, v), 2).requires_grad_(True)
+                packed, = torch.autograd.grad(flash_attention_qkvpacked_fn(qkv, bias, causal), qkv, do)
+                for i in range(3):
+                    assert torch.equal(packed[:, :, i], got[i]), (i, M, N, D, type(bias))
+            for name, a in zip(("dk", "dv"), got[1:]):
                 assert (a.float() - ref[name]).norm() <= 5e-2 * ref[name].norm(), (name, M, N, D, causal, type(bias))
 
 
