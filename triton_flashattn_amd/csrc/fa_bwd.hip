@@ -1626,9 +1626,13 @@ constexpr bool short_rows_built(int bias, int dbias) { return dbias == 0 || (dbi
 //   a byte mask, not causal, one tile to a CU of 1500 rows and more (N=512, H=16): M=1536 46.2 -> 44.5, M=4096 108 -> 101, 1088 rows
 //     35.0 -> 34.5; causal S=2000 57.6 -> 58.7.
 //   a dBias of the other 16-bit type: always one wave (M=N=1024 H=32 48 -> 37).
-// Rows of a dBias or its bias that allow no aligned 16-byte accesses: always a pair, whose stores go out of registers, 32 keys
-// of a row each, and which has 16 loads of a lane in flight, not 8 (fp32 dBias B=2 H=8 M=N=577 57 -> 38, bf16 q and fp16 dBias
-// B=2 H=16 M=N=1023 131 -> 59); an fp32 bias of such rows that is only read too (M=N=1023 68 -> 55).
+// A dBias whose rows allow no aligned 16-byte accesses, or a bias that is read element by element: always a pair, whose stores
+// go out of registers, 32 keys of a row each, and which has 16 loads of a lane in flight, not 8 (fp32 dBias B=2 H=8 M=N=577 57
+// -> 38, bf16 q and fp16 dBias B=2 H=16 M=N=1023 131 -> 59).
+// fp32 rows that are fetched 4 bytes to a lane (kByDword): by the lines above, though a block takes 16 copies there, not 4.  Of 144
+// cases (head dims 16 to 64, 8 to 960 tiles of 77 to 2049 rows, read only and dBias, causal and not) the other kernel is faster by
+// more than 3 % in 22, 10 % at most (one wave / pair: D=64 M=511 N=515 H=8 21.6 / 19.7, D=16 B=2 H=12 M=N=1001 dBias 45.5 / 41.4;
+// D=16 H=8 M=2049 N=2047 49.2 / 53.0, where the line takes the pair); with more tiles than CUs the pair loses up to half.
 // (measured at 256 CUs, B=1 where none is given)
 static bool pair_of_waves(const BwdParams& p, int D, int bias, int dbias, bool own_type, bool causal) {
     const int64_t tiles = (int64_t)p.n_ntiles * p.B * p.H;

@@ -136,8 +136,8 @@ __device__ __forceinline__ float row_bcast(float x, int i) {
     return row_bcast<15>(x);
 }
 
-// DBIAS as in fa_bwd_kernel: 0 = the bias is not trainable; 1 = dBias is written densely (rows of both that allow aligned
-// 16-byte accesses: fa_bwd_kernel takes the others); 2 = reduced: the sums of dS over the query rows, or (ALiBi) the slope's
+// DBIAS as in fa_bwd_kernel: 0 = the bias is not trainable; 1 = dBias is written densely (its rows allow aligned 16-byte
+// accesses, and those of the bias come by copies, of 16 bytes or of 4: fa_bwd_kernel takes the others); 2 = reduced: the sums of dS over the query rows, or (ALiBi) the slope's
 // gradient, one fp32 per (batch, head, key tile, wave).
 template <typename T, int D, int BIAS, bool CAUSAL, int DBIAS>
 __global__ __launch_bounds__(256, (NarrowCfg<D, tile_kind(BIAS)>::MIN_BLOCKS)) void fa_bwd_narrow_kernel(const BwdParams p) {

@@ -492,8 +492,7 @@ template <int D, int BIAS, bool WIDE = false> struct StreamCfg {
                                    : NBS * BSLOT >= 64 * D          ? kOwnRing
                                                                     : kSlotsAndBehind;
     // Work-groups on a CU that such a place must leave room for: three up to head dim 64 where the loops do, which the registers
-    // of most of those kernels allow (dQ, us, D=64 ALiBi, two / three: H=96 S=1024 54 / 51, causal 41 / 36; D=16 with an fp32 tile
-    // B=8 H=12 S=1024 108 / 95).
+    // of most of those kernels allow (dQ, us, D=64 ALiBi, two / three: H=96 S=1024 54 / 51, causal 41 / 36).
     static constexpr int ROOM = D <= 64 && 3 * LOOP_BYTES <= 163840 ? 3 : D <= 128 && LOOP_BYTES <= 81920 ? 2 : 1;
     static constexpr int LDS_BYTES = LOOP_BYTES + (STAGE == kBehind ? 256 * D : STAGE == kSlotsAndBehind ? 128 * D : 0);
     // 16-byte chunk c of bias row `row` is stored at chunk c ^ bswz(row): rows that share LDS banks

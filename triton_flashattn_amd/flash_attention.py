@@ -323,9 +323,13 @@ def _bias_rows_ok(b):
 def _empty_padded_rows(shape, dtype, device):
     """An uninitialised tensor of `shape` whose rows start at multiples of 16 bytes and own the rest
     of their last 16-byte chunk (a view of an allocation with a padded last dimension).  Padded rows of 512
-    bytes and more start at whole cache lines: the slices of 32 keys that the kernels read and write then touch no
-    line twice (us, 16 -> 128 bytes: fp32, B=2 H=12 M=N=1001 D=128, forward 41 -> 36; bf16, H=32 M=1001 N=8001
-    D=128, forward 228 -> 212, dQ 165 -> 145, dK/dV/dBias with the rest of its changes 427 -> 400)."""
+    bytes and more start at whole cache lines: no slice of 32 keys that the kernels read or write then straddles two
+    lines more than it must (us, 16 -> 128 bytes: fp32, B=2 H=12 M=N=1001 D=128, forward 41 -> 36; bf16, H=32 M=1001 N=8001
+    D=128, forward 228 -> 212, dQ 165 -> 145, dK/dV/dBias with the rest of its changes 427 -> 400).  The kernels of a training
+    step together, 16 and 96 (batch, head) pairs, 129 to 1001 keys, fp32 and bf16, head dims 64 and 128: rows below 1024 bytes
+    0.98 to 1.01 of the time, 0.993 in the mean, above 0.92 to 1.07, 0.992.  The padding costs memory, in copies and in
+    the gradients that are returned: at most 21 % more than with 16 bytes (129 fp32 keys: 528 -> 640 bytes a row), 12 %
+    from 1024 bytes on, 2 % at 1001 keys."""
     es = torch.empty((), dtype=dtype).element_size()
     row = shape[-1] * es
     lines = row % 16 != 0 and row >= 512 and shape[-2] * (row + 128) < 1 << 31  # (a (batch, head) slice stays below 2 GiB)
